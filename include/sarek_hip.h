@@ -626,7 +626,8 @@ int sarek_hip_gemm_f16(const uint16_t *a, const uint16_t *b, float *c, int m, in
                        sarek_hip_stream stream);
 
 /* Which kernel the three 16-bit GEMM entry points take for a shape under the
- * present tunables: 256 or 128 = the workgroup tile of the direct-to-LDS MFMA
+ * present tunables: 64 = the few-rows kernel (plain products, m <= 64 and k >= 32,
+ * where it is the faster one), 256 or 128 = the workgroup tile of the direct-to-LDS MFMA
  * kernels (the small tile where large ones would leave CUs idle; any n, any
  * k >= 64 and the multiples of 8 below, any alignment of a and b from k = 64
  * on), 0 = the one-thread-per-element kernel (k < 64 that is not a multiple
@@ -637,7 +638,7 @@ int sarek_hip_gemm16_tile(int m, int n, int k);
 /* Into how many pieces sarek_hip_gemm_bf16 / _f16 cut K for this shape now (1 =
  * none): products with few 128 x 128 tiles and a long K are spread over the
  * CUs that way, the partial tiles added up in a fixed order by a second
- * kernel.  Device memory for them: one 64 MiB block per stream, allocated at
+ * kernel (by the last workgroup of a tile in the few-rows kernel).  Device memory for them: one 64 MiB block per stream, allocated at
  * the first such call on the stream and kept until the process ends, for up
  * to 16 streams; calls on further streams, and calls under stream capture on
  * a stream that has no block yet, run unsplit (same result up to the order of

@@ -16,6 +16,7 @@
 //     column fragment is gathered by ds_read_b64_tr_b16.
 //   gemm16_m16_small_kernel: the same pipeline on a 128 x 128 tile (4 waves), two workgroups per CU, for products
 //     that do not fill the chip with large tiles; K split over several workgroups per tile where tiles are few.
+//   gemm16_rows_kernel (gemm16_rows.hip): plain products of at most 64 rows.
 //   gemm16_simple_kernel: any shape and alignment, one thread per C element (K below one LDS stage that is not a
 //     multiple of 8, or operands whose 256-row / 64-row panels span 2 GiB).
 //   gemm16_last_column_kernel: column N-1 of an odd N.
@@ -35,13 +36,8 @@
 namespace sarek_hip {
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 
 constexpr int BM = 256, BN = 256, BK = 64;
@@ -456,16 +452,6 @@ __global__ __launch_bounds__(64 * 2 * (8 / TJ)) void gemm16_dma_kernel(const uin
 //      the second group on the other 32-byte half of each 64-byte piece.
 // A slab is worked in two units of 16 MFMAs (rows 0-63 of the wave tile, then rows 64-127, same B fragments);
 // the barrier sits between them, and the second unit covers the fragment reads of the next slab.
-template <bool Bf16>
-__device__ __forceinline__ f32x4_t mfma16(u32x4 a, u32x4 b, f32x4_t c) {
-  if constexpr (Bf16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                   0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
-                                                  0, 0);
-}
-
 // Writes one wave's (16*TI) x 64 block held as TI x 4 tiles of 16 x 16 (register r of lane l: row 4*(l/16) + r, column
 // l%16 of its tile); TI = 8 in the 256 x 256 workgroup tile (2 x 4 waves), 4 in the 128 x 128 one (2 x 2 waves).
 // Fused form as in `epilogue`: per lane the sum over its four columns for each of its 4*TI rows, a halving butterfly
@@ -1292,13 +1278,7 @@ __global__ __launch_bounds__(64) void rowsum_fold_kernel(const float *__restrict
 // taken when that estimate is at least a tenth ahead (with every CU busy on a long K its extra operand traffic costs
 // clock under the power limit: 4096 x 2048 x 8192 gains 9 % where the estimate says 35 %).
 inline bool small_tile_wins(int m, int n) {
-  static const int cus = [] {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
-      v = 256;
-    return v;
-  }();
+  const int cus = compute_units();
   const int64_t large = static_cast<int64_t>((m + 255) / 256) * ((n + 255) / 256);
   const int64_t small = static_cast<int64_t>((m + 127) / 128) * ((n + 127) / 128);
   const double cost_large = static_cast<double>((large + cus - 1) / cus);
@@ -1350,13 +1330,7 @@ int splitk_for(int m, int n, int k) {
   const int64_t forced = tunable("gemm16.split_k", 0);
   // the planes are added 16 bytes at a time; a last piece below one stage needs K % 8 == 0
   if (forced == 1 || (static_cast<int64_t>(m) * n) % 4 != 0 || k % 8 != 0) return 1;
-  static const int cus = [] {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
-      v = 256;
-    return v;
-  }();
+  const int cus = compute_units();
   const double plane_mib = static_cast<double>(m) * n * 4 / (1 << 20);
   const int64_t fit = static_cast<int64_t>(static_cast<double>(kSplitWorkspaceBytes >> 20) / plane_mib);
   int64_t splits = 1;
@@ -1388,6 +1362,12 @@ inline bool gemm16_default_kernel() {
 #else
   return true;
 #endif
+}
+
+// Whether a plain product goes to the few-rows kernel: up to 64 rows, unless a knob asks for one of the tiled kernels.
+inline bool few_rows(int m, int n, int k) {
+  return gemm16_default_kernel() && tunable("gemm16.tile", 0) == 0 && tunable("gemm16.split_k", 0) == 0 &&
+         tunable("gemm16.force_simple", 0) == 0 && gemm16_rows_serves(m, n, k);
 }
 
 // The workgroup tile of the direct-to-LDS kernels for this shape under the present tunables (256 or 128), or 0 when
@@ -1492,6 +1472,9 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
 #endif
   // The kernels on v_mfma_f32_16x16x32 (256 x 256 or 128 x 128 tile) take any N, any K of at least one LDS stage and
   // any alignment of A and B in their Ragged form; below one stage K must be a multiple of 8 and A and B 16-byte aligned.
+  if constexpr (Epi == EPI_STORE) {
+    if (few_rows(m, n, k)) return launch_gemm16_rows(Bf16, a, b, c, m, n, k, st);
+  }
   const int tile_choice = gemm16_tile_for(m, n, k);
   const bool ab16 = reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
   const bool tiled = tile_choice != 0 && (k >= 64 || ab16);
@@ -1597,9 +1580,14 @@ using namespace sarek_hip;
 
 extern "C" {
 
-int sarek_hip_gemm16_tile(int m, int n, int k) { return gemm16_tile_for(m, n, k); }
+int sarek_hip_gemm16_tile(int m, int n, int k) {
+  return m >= 1 && n >= 1 && few_rows(m, n, k) ? 64 : gemm16_tile_for(m, n, k);
+}
 
-int sarek_hip_gemm16_k_splits(int m, int n, int k) { return gemm16_tile_for(m, n, k) == 128 ? splitk_for(m, n, k) : 1; }
+int sarek_hip_gemm16_k_splits(int m, int n, int k) {
+  if (m >= 1 && n >= 1 && few_rows(m, n, k)) return gemm16_rows_k_splits(m, n, k);
+  return gemm16_tile_for(m, n, k) == 128 ? splitk_for(m, n, k) : 1;
+}
 
 int sarek_hip_gemm_bf16(const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k,
                         sarek_hip_stream stream) {

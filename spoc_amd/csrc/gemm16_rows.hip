@@ -1,0 +1,315 @@
+// 16-bit-input (bf16 / fp16), f32-accumulate products of at most 64 rows:  C[M x N] = A[M x K] . B[K x N], row-major.
+//
+// What bounds it: B is read once and used M times, so the product is a read of B (16 x 8192 x 8192: 134 MB, 21 us at the
+// 6.3 TB/s large streams reach here) and a CU draws at most about 39 GB/s of L2 misses, so every CU has to take its
+// share.  The 128 x 128 tile of gemm16_m16_small_kernel fetches 128 rows of A whatever M is, adds its K pieces in a
+// second launch, and with an odd N runs the last column as a launch of its own.  Here:
+//   - No LDS on the way in.  A wave takes steps of 32 k x 128 columns of B, 8 KiB in eight 16-byte loads per lane: lane
+//     (l, g) = (lane % 16, lane / 16) gets rows 8g .. 8g+7 at columns 8l .. 8l+7.  v_perm_b32 turns that 8 x 8 block into
+//     eight operands of v_mfma_f32_16x16x32 (column 8l + c over k = 8g .. 8g+7, c = 0 .. 7), four instructions each; A's
+//     rows are the other operand, read as they lie.  The result puts 32 consecutive columns of one row of C in a lane.
+//   - The eight waves of a workgroup take the steps of its piece of K in turn, two in flight each, and add up through LDS.
+//   - K is cut over `splits` workgroups per column tile; each leaves its sums in a plane of the stream's workspace, past
+//     the L2s, and the one that takes a tile's last ticket adds the planes in order.  The order of all additions is fixed:
+//     the same bits on every run.
+//   - Workgroups start at different places of their piece: A's rows are a power of two apart in the usual case, and in
+//     step all workgroups would read them from the same L2 channels (64 x 8192 x 8192: 51 us in step, 38 rotated).
+// Measured, before (the 128 x 128 tile) and now, launches back to back on rotating operands:
+//   16 x 8192 x 8192 34.5 -> 25.7 us (5.2 TB/s), 16 x 2048 x 2048 10.4 -> 6.8, 16 x 40000 x 1024 21.1 -> 19.6,
+//   32 x 16384 x 4096 32.9 -> 27.4, 48 x 4096 x 4096 17.2 -> 13.8, 16 x 256 x 8192 12.8 -> 7.4; odd sizes:
+//   10 x 4161 x 4221 80 -> 12.6, 64 x 4097 x 4103 74 -> 20.5, 8 x 50257 x 1024 34.5 -> 28.0.
+// Tried: 4 waves with 2 to 4 steps in flight (5 to 10 % slower), tiles dealt so that neighbours share an XCD (no change),
+// 64-bit atomic stores and loads for the planes (4 planes of 64 x 8192: 3 us more than the 16-byte accesses).
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+#include <utility>
+
+#include "common.hpp"
+#include "gemm_common.hpp"
+#include "tunables.hpp"
+
+namespace sarek_hip {
+namespace {
+
+constexpr int kRowsMax = 64, kCols = 128, kStepK = 32, kWaves = 8;
+constexpr int kRedPitch = kCols + 4;   // floats per row of the waves' sums in LDS: 16 rows on different banks
+// Cache-policy bits of a buffer access: past the L2s, which the XCDs do not share; and non-temporal.
+constexpr int kDeviceScope = 16, kNonTemporal = 2;
+
+template <bool Bf16, int MT, int BPolicy>
+__global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t *__restrict__ A,
+                                                                  const uint16_t *__restrict__ B, float *__restrict__ C,
+                                                                  int M, int N, int K, int tiles, int splits,
+                                                                  int steps_per_split, float *__restrict__ partials,
+                                                                  unsigned *__restrict__ tickets) {
+  __shared__ __attribute__((aligned(16))) float red[kWaves][16 * kRedPitch];
+  __shared__ bool last;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int tile = blockIdx.x % tiles, split = blockIdx.x / tiles;
+  const int n0 = tile * kCols;
+  const int nsteps = (K + kStepK - 1) / kStepK;
+  const int s_begin = split * steps_per_split, s_end = min(nsteps, s_begin + steps_per_split);
+
+  const uint32_t row_bytes = static_cast<uint32_t>(N) * 2;
+  const int64_t b_bytes = static_cast<int64_t>(K) * row_bytes;
+  const uint32_t b_off = 8 * g * row_bytes + (n0 + 8 * l16) * 2u;
+  uint32_t a_off[MT];   // rows past M repeat the last one: what they produce is never stored
+#pragma unroll
+  for (int t = 0; t < MT; ++t) a_off[t] = (static_cast<uint32_t>(min(16 * t + l16, M - 1)) * K + 8 * g) * 2u;
+
+  // A step whose loads all lie inside A and B (columns past N bring the next rows' elements, and are never stored).
+  // !ok: the resources have no range, so every load returns zeros and fetches nothing; it keeps the count of loads in
+  // flight the same in every turn of the loop.
+  auto load = [&](int s, bool ok, u32x4 (&bf)[8], u32x4 (&af)[MT]) {
+    const uint32_t range = ok ? 0x80000000u : 0u;
+    const __amdgpu_buffer_rsrc_t b_rsrc =
+        make_rsrc(reinterpret_cast<const char *>(B) + static_cast<int64_t>(s) * kStepK * row_bytes, range);
+    const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(A + static_cast<int64_t>(s) * kStepK, range);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      bf[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, b_off, i * row_bytes, BPolicy));
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+      af[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off[t], 0, 0));
+  };
+  // A step at the end of B: B's range is exact, so what lies past it reads as zero; elements of A past K count as zero.
+  auto load_end = [&](int s, u32x4 (&bf)[8], u32x4 (&af)[MT]) {
+    const int64_t at = static_cast<int64_t>(s) * kStepK * row_bytes;
+    const __amdgpu_buffer_rsrc_t b_rsrc =
+        make_rsrc(reinterpret_cast<const char *>(B) + at,
+                  static_cast<uint32_t>(min(b_bytes - at, static_cast<int64_t>(0x7FFFFFFF))));
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      bf[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, b_off + i * row_bytes, 0, 0));
+    const int left = K - s * kStepK - 8 * g;   // elements of A this lane has before the end of K
+    const __amdgpu_buffer_rsrc_t a_rsrc =
+        make_rsrc(A + static_cast<int64_t>(s) * kStepK, static_cast<uint32_t>((static_cast<int64_t>(M) * K - s * kStepK) * 2));
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      af[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off[t], 0, 0));
+#pragma unroll
+      for (int d = 0; d < 4; ++d) af[t][d] &= left >= 2 * d + 2 ? 0xFFFFFFFFu : left == 2 * d + 1 ? 0xFFFFu : 0u;
+    }
+    // ranges are checked per dword: with an odd K the one that holds A[M-1][K-1] ends past A and read as zero ...
+    if ((K & 1) != 0 && s == nsteps - 1) {
+      const uint32_t v = A[static_cast<int64_t>(M) * K - 1];
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          if (16 * t + l16 >= M - 1 && left == 2 * d + 1) af[t][d] = v;
+    }
+    // ... and with an odd N the one that holds B[K-1][N-1]
+    if ((N & 1) != 0 && s == nsteps - 1) {
+      const int r = K - 1 - s * kStepK, c = N - 1 - n0;   // row in the step, column in the tile
+      if (g == r / 8 && c >= 0 && l16 == c / 8) {
+        const uint32_t v = B[static_cast<int64_t>(K - 1) * N + N - 1];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+            if (i == r % 8 && d == (c % 8) / 2) bf[i][d] = v;
+      }
+    }
+  };
+
+  f32x4_t acc[8][MT];
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[c][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](u32x4 (&bf)[8], u32x4 (&af)[MT]) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      u32x4 op;
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        op[d] = __builtin_amdgcn_perm(bf[2 * d + 1][c / 2], bf[2 * d][c / 2], c % 2 ? 0x07060302u : 0x05040100u);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) acc[c][t] = mfma16<Bf16>(op, af[t], acc[c][t]);
+    }
+  };
+
+  // The piece's plain steps: whole K, and at least one tile's width of B behind their last row's first element
+  const int64_t plain_rows = K - (kCols + N - 1) / N;
+  const int plain = max(min(s_end, plain_rows > 0 ? static_cast<int>(plain_rows / kStepK) : 0) - s_begin, 0);
+  const int first = plain > 0 ? (tile * kWaves) % plain : 0;
+  u32x4 bf[2][8], af[2][MT];
+  auto load_at = [&](int i, auto buffer) {
+    const int at = i + first;
+    load(s_begin + (at < plain ? at : at - plain), i < plain, bf[buffer], af[buffer]);
+  };
+  constexpr std::integral_constant<int, 0> b0{};
+  constexpr std::integral_constant<int, 1> b1{};
+  load_at(wave, b0);
+  for (int i = wave; i < plain; i += 2 * kWaves) {
+    load_at(i + kWaves, b1);
+    multiply(bf[0], af[0]);
+    load_at(i + 2 * kWaves, b0);
+    multiply(bf[1], af[1]);
+  }
+  for (int s = s_begin + plain + wave; s < s_end; s += kWaves) {
+    load_end(s, bf[0], af[0]);
+    multiply(bf[0], af[0]);
+  }
+
+  // Sums over the waves, 16 rows at a time: thread -> row `row`, columns col .. col + 3 of them
+  const int row = threadIdx.x >> 5, col = (threadIdx.x & 31) * 4;
+  auto put = [&](int t, f32x4_t v) {
+    const int m = 16 * t + row, n = n0 + col;
+    if (m >= M) return;
+    float *dst = C + static_cast<int64_t>(m) * N + n;
+    if (n + 4 <= N) {
+      *reinterpret_cast<f32x4_u *>(dst) = v;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (n + j < N) dst[j] = v[j];
+    }
+  };
+  // plane `split`: per tile 16 MT rows of kCols
+  const int plane_bytes = tiles * (MT * 16 * kCols * 4);
+  const __amdgpu_buffer_rsrc_t p_rsrc =
+      make_rsrc(partials + static_cast<int64_t>(tile) * (MT * 16 * kCols), 0x80000000u);
+  const int piece = (row * kCols + col) * 4;
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    if (t > 0) __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *reinterpret_cast<f32x4_t *>(&red[wave][l16 * kRedPitch + 32 * g + 8 * r + 4 * h]) =
+            f32x4_t{acc[4 * h][t][r], acc[4 * h + 1][t][r], acc[4 * h + 2][t][r], acc[4 * h + 3][t][r]};
+    __syncthreads();
+    f32x4_t v = *reinterpret_cast<const f32x4_t *>(&red[0][row * kRedPitch + col]);
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) v += *reinterpret_cast<const f32x4_t *>(&red[w][row * kRedPitch + col]);
+    if (splits == 1) put(t, v);
+    else
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), p_rsrc, piece + t * (16 * kCols * 4),
+                                             split * plane_bytes, kDeviceScope);
+  }
+  if (splits == 1) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's pieces are where the other XCDs read them
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(tickets + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+           static_cast<unsigned>(splits - 1);
+  __syncthreads();
+  if (!last) return;
+  f32x4_t sum[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) sum[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int q = 0; q < splits; q += 4) {   // four planes asked for before the first is added
+    f32x4_t v[4][MT];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        v[u][t] = __builtin_bit_cast(
+            f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(p_rsrc, piece + t * (16 * kCols * 4),
+                                                           min(q + u, splits - 1) * plane_bytes, kDeviceScope));
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (q + u < splits) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) sum[t] += v[u][t];
+      }
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) put(t, sum[t]);
+  if (threadIdx.x == 0) __hip_atomic_store(tickets + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Pieces of K per column tile, by an estimate in microseconds whose constants were fitted to sweeps of 1 to 31 pieces
+// over 12 shapes (within 1 us on those of 10 us and more): a CU's share of B and A at 39 GB/s in whole rounds of
+// workgroups, B from memory at 6.3 TB/s, the two merged smoothly; a split adds its planes, written and read at 2.7 TB/s,
+// a ticket, and a little per piece.  A wave keeps at least one step.  gemm16.rows_splits: 0 = this rule, n forces n.
+int rows_splits_for(int m, int n, int k) {
+  const int tiles = (n + kCols - 1) / kCols, steps = (k + kStepK - 1) / kStepK, mt = (m + 15) / 16;
+  const int64_t plane = static_cast<int64_t>(tiles) * mt * 16 * kCols * 4;
+  const int64_t fit = tiles > kSplitTickets ? 1 : static_cast<int64_t>(kSplitWorkspaceBytes) / plane;
+  const int64_t forced = tunable("gemm16.rows_splits", 0);
+  int64_t splits = 1;
+  if (forced > 0) {
+    splits = std::max<int64_t>(1, std::min<int64_t>({forced, steps, fit}));
+  } else {
+    const int cus = compute_units();
+    const double memory = static_cast<double>(k) * n * 2 / 6.3e6;
+    auto estimate = [&](int64_t s) {
+      const double cu = static_cast<double>((tiles * s + cus - 1) / cus) * steps / s * (8192 + 1024 * mt) / 39e3;
+      return std::cbrt(cu * cu * cu + memory * memory * memory) +
+             (s > 1 ? 1.0 + 0.15 * s + 2.0 * static_cast<double>(s * plane) / 2.7e6 : 0.0);
+    };
+    double best = estimate(1);
+    for (int64_t s = 2; s <= 64 && s <= fit && s * kWaves <= steps; ++s)
+      if (estimate(s) < best) best = estimate(s), splits = s;
+  }
+  const int64_t per = (steps + splits - 1) / splits;   // the count follows from the piece so that none is empty
+  return static_cast<int>((steps + per - 1) / per);
+}
+
+template <bool Bf16, int MT>
+int launch(const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k, hipStream_t st) {
+  const int tiles = (n + kCols - 1) / kCols, steps = (k + kStepK - 1) / kStepK;
+  int splits = rows_splits_for(m, n, k);
+  float *partials = nullptr;
+  if (splits > 1 && !(partials = splitk_workspace(st))) splits = 1;
+  const int per = (steps + splits - 1) / splits;
+  unsigned *tickets = partials ? splitk_tickets(partials) : nullptr;
+  // B past the caches from 64 MiB on where its rows are whole 16-byte pieces (100 MB: 20.2 us against 22.8, 134 MB: 26.4
+  // against 28.0, 34 MB: 15.8 against 13.2); rows at other offsets share lines between neighbouring loads, and lose
+  // (100 MB: 28.4 against 28.0)
+  const bool nt = n % 8 == 0 && static_cast<int64_t>(k) * n * 2 > (int64_t{64} << 20);
+  const dim3 grid(static_cast<unsigned>(tiles) * splits), block(64 * kWaves);
+  if (nt)
+    hipLaunchKernelGGL((gemm16_rows_kernel<Bf16, MT, kNonTemporal>), grid, block, 0, st, a, b, c, m, n, k, tiles, splits,
+                       per, partials, tickets);
+  else
+    hipLaunchKernelGGL((gemm16_rows_kernel<Bf16, MT, 0>), grid, block, 0, st, a, b, c, m, n, k, tiles, splits, per,
+                       partials, tickets);
+  return check_launch("gemm16 few-rows kernel launch");
+}
+
+template <bool Bf16>
+int launch_rows(const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k, hipStream_t st) {
+  switch ((m + 15) / 16) {
+    case 1: return launch<Bf16, 1>(a, b, c, m, n, k, st);
+    case 2: return launch<Bf16, 2>(a, b, c, m, n, k, st);
+    case 3: return launch<Bf16, 3>(a, b, c, m, n, k, st);
+    default: return launch<Bf16, 4>(a, b, c, m, n, k, st);
+  }
+}
+
+}  // namespace
+
+// Whether this kernel takes a product.  It can: up to 64 rows (four row tiles' sums fill the registers), K of at least one
+// step, 32 rows of B and all of A within the 32-bit load offsets.  Up to 16 rows it always should.  Beyond, a workgroup's
+// sums through LDS cost it 0.5 us per 16 rows and its registers leave room for one workgroup per CU, so short K and more
+// column tiles than CUs belong to the 128 x 128 tile unless that one would need its odd-N launch (us, 128 tile / here):
+//   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
+//   48 x 4096 x 256 6.2 / 6.1, 48 x 4096 x 1024 10.2 / 9.4, 48 x 40000 x 1024 23.0 / 26.4, 48 x 40001 x 1024 35.3 / 33.4
+//   64 x 4096 x 256 6.4 / 7.2, 64 x 4096 x 1024 10.5 / 10.5, 64 x 4096 x 4096 17.3 / 15.6, 64 x 40001 x 1024 36.3 / 37.0
+bool gemm16_rows_serves(int m, int n, int k) {
+  if (m > kRowsMax || k < kStepK || static_cast<int64_t>(n + kCols) * 2 * kStepK >= 0x7FFFFFFF ||
+      static_cast<int64_t>(m) * k * 2 >= 0x7FFFFFFF)
+    return false;
+  const bool odd = n % 2 != 0, one_round = (n + kCols - 1) / kCols <= compute_units();
+  switch ((m + 15) / 16) {
+    case 1: return true;
+    case 2: return odd || one_round;
+    case 3: return one_round ? odd || k >= 512 : odd && k >= 1024;
+    default: return one_round && (odd || k >= 1024);
+  }
+}
+
+int gemm16_rows_k_splits(int m, int n, int k) { return rows_splits_for(m, n, k); }
+
+int launch_gemm16_rows(bool bf16, const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k, hipStream_t st) {
+  return bf16 ? launch_rows<true>(a, b, c, m, n, k, st) : launch_rows<false>(a, b, c, m, n, k, st);
+}
+
+}  // namespace sarek_hip

@@ -10,8 +10,38 @@ namespace sarek_hip {
 constexpr size_t kSplitWorkspaceBytes = 64u << 20;
 float *splitk_workspace(hipStream_t st);
 int launch_splitk_reduce(const float *partials, float *c, int64_t mn, int splits, hipStream_t st);
+// Counters behind the planes of a block, zero between launches: one per tile for kernels whose last piece adds the planes.
+constexpr int kSplitTickets = 4096;
+inline unsigned *splitk_tickets(float *block) {
+  return reinterpret_cast<unsigned *>(reinterpret_cast<char *>(block) + kSplitWorkspaceBytes);
+}
+
+// Compute units of the current device (256 where it does not say).
+int compute_units();
+
+// 16-bit products of at most 64 rows (gemm16_rows.hip)
+bool gemm16_rows_serves(int m, int n, int k);
+int gemm16_rows_k_splits(int m, int n, int k);
+int launch_gemm16_rows(bool bf16, const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k, hipStream_t st);
 
 namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef f32x4_t f32x4_u __attribute__((aligned(4)));   // at any element's address
+typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+typedef __attribute__((ext_vector_type(2))) unsigned long long u64x2;
+
+template <bool Bf16>
+__device__ __forceinline__ f32x4_t mfma16(u32x4 a, u32x4 b, f32x4_t c) {
+  if constexpr (Bf16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                   0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
+                                                  0, 0);
+}
 
 #define LDS_PTR __attribute__((address_space(3)))
 

@@ -442,13 +442,7 @@ namespace {
 // fits one workgroup per CU.  `eff` is the MFMA issue efficiency measured for each shape.
 int gemm_f32_tile_for(int m, int n) {
   auto ntiles = [&](int t) { return static_cast<int64_t>((m + t - 1) / t) * ((n + t - 1) / t); };
-  static const int cus = [] {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
-      v = 256;
-    return v;
-  }();
+  const int cus = compute_units();
   auto cost = [&](int t, int occ, double eff) {
     const int64_t tiles = ntiles(t), slots = static_cast<int64_t>(cus) * occ;
     const int64_t full = tiles / slots, rest = tiles % slots;
@@ -466,13 +460,7 @@ int gemm_f32_tile_for(int m, int n) {
 int splitk_f32_for(int m, int n, int k) {
   const int64_t forced = tunable("gemm_f32.split_k", 0);
   if (forced == 1 || (static_cast<int64_t>(m) * n) % 4 != 0 || k % 32 != 0) return 1;
-  static const int cus = [] {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
-      v = 256;
-    return v;
-  }();
+  const int cus = compute_units();
   const int64_t tiles = static_cast<int64_t>((m + 63) / 64) * ((n + 63) / 64);
   const double plane_mib = static_cast<double>(m) * n * 4 / (1 << 20);
   const int64_t fit = static_cast<int64_t>(static_cast<double>(kSplitWorkspaceBytes >> 20) / plane_mib);

@@ -10,8 +10,6 @@
 namespace sarek_hip {
 namespace {
 
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-
 // Adds the `splits` partial planes into C, plane 0 first: a fixed order, so the result does not depend on which
 // workgroup finished when.  mn is a multiple of 4 and both pointers are 16-byte aligned (the callers' conditions).
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ partials, float *__restrict__ C,
@@ -23,9 +21,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
   *reinterpret_cast<f32x4_t *>(C + i) = acc;
 }
 
+__global__ __launch_bounds__(256) void zero_tickets_kernel(unsigned *tickets) {
+  tickets[blockIdx.x * 256 + threadIdx.x] = 0;
+}
+
 }  // namespace
 
-// One block of kSplitWorkspaceBytes per (device, stream), allocated at the first call that wants one on that stream and
+// One block of kSplitWorkspaceBytes and its tickets per (device, stream), allocated at the first call that wants one on that stream and
 // kept until the process ends (never grown or freed, so a pointer handed out stays good whatever other threads do):
 // calls on different streams never share one, calls on one stream are ordered by it.  nullptr (the caller then works
 // without one: no K split, row sums by atomicAdd) for a stream under capture -- a recorded graph would carry the
@@ -46,12 +48,24 @@ float *splitk_workspace(hipStream_t st) {
   if (it != blocks.end()) return static_cast<float *>(it->second);
   if (blocks.size() >= 16) return nullptr;
   void *p = nullptr;
-  if (hipMalloc(&p, kSplitWorkspaceBytes) != hipSuccess) {
+  if (hipMalloc(&p, kSplitWorkspaceBytes + kSplitTickets * sizeof(unsigned)) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
+  hipLaunchKernelGGL(zero_tickets_kernel, dim3(kSplitTickets / 256), dim3(256), 0, st, splitk_tickets(static_cast<float *>(p)));
   blocks[{dev, st}] = p;
   return static_cast<float *>(p);
+}
+
+int compute_units() {
+  static const int cus = [] {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0)
+      v = 256;
+    return v;
+  }();
+  return cus;
 }
 
 int launch_splitk_reduce(const float *partials, float *c, int64_t mn, int splits, hipStream_t st) {

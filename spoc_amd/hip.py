@@ -728,7 +728,7 @@ def gemm_bf16(a, b, out=None):
 
 
 def gemm16_tile(m, n, k):
-    """256 / 128: the workgroup tile the 16-bit GEMMs take for this shape now; 0: the staged or simple kernel."""
+    """256 / 128: the workgroup tile the 16-bit GEMMs take for this shape now; 64: the few-rows kernel; 0: the simple kernel."""
     return int(lib.sarek_hip_gemm16_tile(m, n, k))
 
 

@@ -715,3 +715,36 @@ def test_gemm_f32_split_k_rule(hip, torch_cuda):
                                   ((1024, 1024, 1024), False), ((2048, 2048, 2048), False), ((8192, 8192, 8192), False),
                                   ((1024, 1024, 8192), False), ((512, 512, 100), False)]:
         assert (hip.gemm_f32_k_splits(m, n, k) > 1) == want_split, (m, n, k)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 32), (16, 128, 256), (17, 129, 257), (15, 127, 33), (33, 3, 1000), (48, 264, 520),
+                                   (49, 255, 4129), (64, 1001, 1001), (64, 640, 2048), (65, 130, 96)])
+def test_gemm16_few_rows(hip, torch_cuda, kind, m, n, k):
+    """The few-rows kernel at the edges of its row tiles (16), columns (128) and steps of k (32), K whole and in pieces,
+    operands and result at odd offsets between NaNs and guard values, and 65 rows, which it leaves to the tiled kernels.
+    Against the float64 product: the sum of k products of exact factors, each addition rounded to half an ulp, is off by
+    at most k 2^-24 times the sum of their magnitudes."""
+    torch = torch_cuda
+    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    fn = hip.gemm_bf16 if kind == "bf16" else hip.gemm_f16
+    torch.manual_seed(m * n + k)
+    buf_a = torch.full((m * k + 64,), float("nan"), device="cuda").to(dt)
+    buf_b = torch.full((k * n + 64,), float("nan"), device="cuda").to(dt)
+    for off in (0, 3):
+        da, db = buf_a[off:off + m * k].view(m, k), buf_b[off:off + k * n].view(k, n)
+        da.copy_((torch.randn(m, k, device="cuda") * 0.02).to(dt))
+        db.copy_((torch.randn(k, n, device="cuda") * 0.02).to(dt))
+        ref, size = da.double() @ db.double(), da.double().abs() @ db.double().abs()
+        try:
+            for splits in (0, 1, 2, 5):
+                hip.set_tunable("gemm16.rows_splits", splits)
+                assert hip.gemm16_tile(m, n, k) == (64 if m <= 64 else 128)
+                guard = torch.full((m * n + 64,), 7.0, device="cuda")
+                c = guard[32 + off:32 + off + m * n].view(m, n)
+                fn(da, db, out=c)
+                assert bool((guard[:32 + off] == 7).all()) and bool((guard[32 + off + m * n:] == 7).all())
+                assert bool(((c.double() - ref).abs() <= k * 2.0 ** -24 * size).all()), (off, splits)
+                assert torch.equal(c, fn(da, db)), "the same bits on every run"
+        finally:
+            hip.set_tunable("gemm16.rows_splits", 0)
