@@ -16,10 +16,10 @@
 //     column fragment is gathered by ds_read_b64_tr_b16.
 //   gemm16_m16_small_kernel: the same pipeline on a 128 x 128 tile (4 waves), two workgroups per CU, for products
 //     that do not fill the chip with large tiles; K split over several workgroups per tile where tiles are few.
+//   gemm16_last_column_kernel: N = 1, and the column by which some N exceed whole tiles.
 //   gemm16_rows_kernel (gemm16_rows.hip): plain products of at most 64 rows.
 //   gemm16_simple_kernel: any shape and alignment, one thread per C element (K below one LDS stage that is not a
 //     multiple of 8, or operands whose 256-row / 64-row panels span 2 GiB).
-//   gemm16_last_column_kernel: column N-1 of an odd N.
 // A build with -DSAREK_HIP_MEASURE (libsarek_hip_measure.so, for bench.py --measure-build) also holds gemm16_dma_kernel,
 // the same pipeline on v_mfma_f32_32x32x16 in several ring and wave shapes, and variants of both MFMA kernels that leave
 // parts of the K loop out: what the power and ablation studies were measured with.  The product library has none of them.
@@ -452,17 +452,40 @@ __global__ __launch_bounds__(64 * 2 * (8 / TJ)) void gemm16_dma_kernel(const uin
 //      the second group on the other 32-byte half of each 64-byte piece.
 // A slab is worked in two units of 16 MFMAs (rows 0-63 of the wave tile, then rows 64-127, same B fragments);
 // the barrier sits between them, and the second unit covers the fragment reads of the next slab.
+template <bool Bf16>
+__device__ __forceinline__ float widen16(uint16_t bits) {
+  if constexpr (Bf16) return __uint_as_float(static_cast<uint32_t>(bits) << 16);
+  else return static_cast<float>(__builtin_bit_cast(_Float16, bits));
+}
+
+// The products A[row][K-1] B[K-1][N-1] of an odd N.  B is fetched in pairs of 16-bit elements from even columns on, and the
+// pair that holds B[K-1][N-1] ends two bytes past B: the buffer range ends right in front of it, its lanes bring zeros,
+// and in the workgroups of the last tile column (those that take the last k) epilogue16 adds what is missing: one product
+// per row of the tile, through LDS.  (A kernel of its own for the last column, a wave per row, took 9 us of
+// 2048 x 50257 x 1024's 282 and 20 of 64 x 4097 x 4096's 41.)
+template <bool Bf16, int TROWS>
+__device__ __forceinline__ void last_products(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, int M, int N,
+                                              int K, int m0, float *scratch) {
+  __syncthreads();   // every wave has left the K loop: the LDS ring is free
+  if (threadIdx.x < TROWS) {
+    const int row = min(m0 + static_cast<int>(threadIdx.x), M - 1);
+    scratch[threadIdx.x] = widen16<Bf16>(A[static_cast<int64_t>(row) * K + K - 1]) * widen16<Bf16>(B[static_cast<int64_t>(K) * N - 1]);
+  }
+  __syncthreads();
+}
+
 // Writes one wave's (16*TI) x 64 block held as TI x 4 tiles of 16 x 16 (register r of lane l: row 4*(l/16) + r, column
 // l%16 of its tile); TI = 8 in the 256 x 256 workgroup tile (2 x 4 waves), 4 in the 128 x 128 one (2 x 2 waves).
 // Fused form as in `epilogue`: per lane the sum over its four columns for each of its 4*TI rows, a halving butterfly
 // over the 16 lanes that share those rows (with TI = 8: 16+8+4+2 exchanges leave lane m with rows 2m, 2m+1 of the 32;
 // with TI = 4: 8+4+2+1 leave it with row m of the 16), the WNW waves along N through LDS.  The tile's sum of row r then
 // goes to rs_plane[r] when the launch has planes (one per tile column, added up in tile order by
-// rowsum_fold_kernel: the same bits on every run), else to rowsum[r] by atomicAdd.
-template <int Epi, int TI = 8, int WNW = 4>
+// rowsum_fold_kernel: the same bits on every run), else to rowsum[r] by atomicAdd.  add_last: the tile rows' last_products
+// lie in `scratch` and belong to column N - 1.
+template <int Epi, int TI, int WNW, bool Ragged>
 __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restrict__ C, const float *__restrict__ bias,
                                            float *__restrict__ rowsum, float *__restrict__ rs_plane, int M, int N, int ld,
-                                           int m0, int wm, int wn, int col0, int l16, int g, float *scratch) {
+                                           int m0, int wm, int wn, int col0, int l16, int g, float *scratch, bool add_last) {
   constexpr int WROWS = 16 * TI, TROWS = 2 * WROWS, NV = 4 * TI, E = NV / 16;
   static_assert(TI == 8 || TI == 4, "wave tiles of 128 or 64 rows");
   static_assert(WNW == 4 || WNW == 2, "four or two waves along N");
@@ -478,6 +501,8 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
   float rs[NV];
 #pragma unroll
   for (int i = 0; i < TI; ++i) {
+    f32x4_t last = {0.f, 0.f, 0.f, 0.f};
+    if (Ragged && add_last) last = *reinterpret_cast<const f32x4_t *>(scratch + wm * WROWS + i * 16 + 4 * g);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = row0 + i * 16 + 4 * g + r;
@@ -485,6 +510,7 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         float v = acc[i][j][r];
+        if (Ragged) v = add_last && col0 + j * 16 + l16 == N - 1 ? v + last[r] : v;
         if (Epi == EPI_BIAS_RELU_ROWSUM) {
           v += bj[j];
           v = v > 0.f ? v : 0.f;
@@ -611,7 +637,7 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
     b_in_last[i] = !Ragged || (move_last ? brow + BKB >= shared_k : brow < k_tail_b);
     b_in_prev[i] = !move_last || brow >= shared_k;
   }
-  const char *b_end = b_base + (static_cast<int64_t>(K - 1) * ld + N) * 2;   // the end of row K-1's N columns
+  const char *b_end = b_base + (static_cast<int64_t>(K - 1) * ld + N - (N & 1)) * 2;   // add_last_product brings an odd N's last element
   constexpr uint32_t kOutOfRange = 0x80000000u;
 
   f32x4_t acc[8][4];
@@ -774,8 +800,11 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
     ((full + Is < nslabs ? slab(std::integral_constant<int, Is>{}, full + Is) : (void)0), ...);
   }(std::make_integer_sequence<int, P - 1>{});
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // drain the (redundant) tail DMA before the LDS is released
-  epilogue16<Epi>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0, wm, wn,
-                  n0 + wn * 64, l16, g, reinterpret_cast<float *>(lds_ring<10, A_BYTES_S>));
+  float *scratch = reinterpret_cast<float *>(lds_ring<10, A_BYTES_S>);
+  const bool add_last = Ragged && (N & 1) != 0 && n0 + BN >= N;
+  if (add_last) last_products<Bf16, BM>(A, B, M, N, K, m0, scratch);
+  epilogue16<Epi, 8, 4, Ragged>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0, wm, wn,
+                  n0 + wn * 64, l16, g, scratch, add_last);
   if (kMeasureBuild && probe && tid == 0) {
     probe[2 * blockIdx.x] = static_cast<unsigned long long>(clock64() - probe_c0);
     probe[2 * blockIdx.x + 1] = static_cast<unsigned long long>(wall_clock64() - probe_t0);
@@ -805,7 +834,7 @@ __device__ __forceinline__ void mfma16_in_place(u32x4 a, u32x4 b, f32x4_t &c) {
 template <bool Bf16>
 __global__ __launch_bounds__(256) void gemm16_m16w4_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                            float *__restrict__ C, int M, int N, int K, int tiles_m,
-                                                           int tiles_n, int xcd_remap, int ld) {
+                                                           int tiles_n, int xcd_remap) {
   constexpr int BKA = 64, BKB = 32, NA = 2, NB = 4;
   constexpr int RA = BKA / BKB;
   constexpr int A_ROW = BKA * 2, A_CHUNKS = A_ROW / 16, A_ROWS_PER_DMA = 1024 / A_ROW;
@@ -839,10 +868,10 @@ __global__ __launch_bounds__(256) void gemm16_m16w4_kernel(const uint16_t *__res
     const int q = wave + NWAVES * i;
     const int brow = 2 * q + (lane >> 5);
     const int bchunk = (lane & 31) ^ b_swz(brow);
-    b_off[i] = (static_cast<uint32_t>(brow) * ld + min(n0 + bchunk * 8, N - 8)) * 2u;
+    b_off[i] = (static_cast<uint32_t>(brow) * N + min(n0 + bchunk * 8, N - 8)) * 2u;
   }
   const char *a_base = reinterpret_cast<const char *>(A + static_cast<int64_t>(m0) * K);
-  const int64_t b_slab_bytes = static_cast<int64_t>(BKB) * ld * 2;
+  const int64_t b_slab_bytes = static_cast<int64_t>(BKB) * N * 2;
   const int nstages = K / BKA, nslabs = K / BKB;
 
   f32x4_t acc[8][8];
@@ -962,7 +991,7 @@ __global__ __launch_bounds__(256) void gemm16_m16w4_kernel(const uint16_t *__res
     for (int r = 0; r < 4; ++r) {
       const int row = m0 + wm * 128 + i * 16 + 4 * g + r;
       if (row >= M) continue;
-      float *crow = C + static_cast<int64_t>(row) * ld + n0 + wn * 128 + l16;
+      float *crow = C + static_cast<int64_t>(row) * N + n0 + wn * 128 + l16;
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         if (n0 + wn * 128 + j * 16 + l16 < N) crow[j * 16] = acc[i][j][r];
@@ -1035,11 +1064,12 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     const int bcol = Ragged ? n0 + bchunk * 8 : min(n0 + bchunk * 8, N - 8);
     b_off[i] = (static_cast<uint32_t>(brow) * ld + bcol) * 2u;
   }
-  // K split over gridDim.y workgroups per tile (plain store only): this one takes k0 .. k0 + k_len - 1 and writes its
-  // partial tile to its own M x N plane of `partials`, which a second kernel adds up in a fixed order
+  // K split over gridDim.y workgroups per tile (plain store only): this one takes k0 .. k0 + k_len - 1, the last one what
+  // is left of K (at least a stage), and writes its partial tile to its own plane of `partials`, which a second kernel
+  // adds up in a fixed order
   const int k0 = blockIdx.y * k_chunk;
-  const int k_len = min(k_chunk, K - k0);
-  if (gridDim.y > 1) C = partials + static_cast<int64_t>(blockIdx.y) * M * ld;
+  const int k_len = blockIdx.y == gridDim.y - 1 ? K - k0 : k_chunk;
+  if (gridDim.y > 1) C = partials + blockIdx.y * splitk_plane_floats(M, ld);
   const char *a_base = reinterpret_cast<const char *>(A + static_cast<int64_t>(m0) * K + k0);
   const int64_t b_slab_bytes = static_cast<int64_t>(BKB) * ld * 2;
   // Ragged: K need not fill the last A stage.  A lane whose offset lies outside the buffer resource's range brings
@@ -1063,7 +1093,7 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     b_in_last[i] = !Ragged || (move_last ? brow + BKB >= shared_k : brow < k_tail_b);
     b_in_prev[i] = !move_last || brow >= shared_k;
   }
-  const char *b_end = reinterpret_cast<const char *>(B) + (static_cast<int64_t>(K - 1) * ld + N) * 2;
+  const char *b_end = reinterpret_cast<const char *>(B) + (static_cast<int64_t>(K - 1) * ld + N - (N & 1)) * 2;   // as above
   constexpr uint32_t kOutOfRange = 0x80000000u;
 
   f32x4_t acc[4][4];
@@ -1197,8 +1227,11 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     ((full + Is < nslabs ? slab(std::integral_constant<int, Is>{}, full + Is) : (void)0), ...);
   }(std::make_integer_sequence<int, P - 1>{});
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // drain the (redundant) tail DMA before the LDS is released
-  epilogue16<Epi, 4, WN>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0,
-                         wm, wn, n0 + wn * 64, l16, g, reinterpret_cast<float *>(lds_ring<30, A_BYTES_S>));
+  float *scratch = reinterpret_cast<float *>(lds_ring<30, A_BYTES_S>);
+  const bool add_last = Ragged && (N & 1) != 0 && n0 + SBN >= N && k0 + k_len == K;
+  if (add_last) last_products<Bf16, SBM>(A, B, M, N, K, m0, scratch);
+  epilogue16<Epi, 4, WN, Ragged>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0,
+                         wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
   if (kMeasureBuild && probe && tid == 0) {
     probe[2 * blockIdx.x] = static_cast<unsigned long long>(clock64() - probe_c0);
     probe[2 * blockIdx.x + 1] = static_cast<unsigned long long>(wall_clock64() - probe_t0);
@@ -1218,16 +1251,7 @@ __global__ __launch_bounds__(256) void gemm16_simple_kernel(const uint16_t *__re
   float acc = 0.f;
   if (row < M && col < N) {
     for (int k = 0; k < K; ++k) {
-      const uint16_t ab = A[static_cast<int64_t>(row) * K + k];
-      const uint16_t bb = B[static_cast<int64_t>(k) * N + col];
-      float af, bf;
-      if (Bf16) {
-        af = __builtin_bit_cast(float, static_cast<uint32_t>(ab) << 16);
-        bf = __builtin_bit_cast(float, static_cast<uint32_t>(bb) << 16);
-      } else {
-        af = static_cast<float>(__builtin_bit_cast(_Float16, ab));
-        bf = static_cast<float>(__builtin_bit_cast(_Float16, bb));
-      }
+      const float af = widen16<Bf16>(A[static_cast<int64_t>(row) * K + k]), bf = widen16<Bf16>(B[static_cast<int64_t>(k) * N + col]);
       acc = fmaf(af, bf, acc);
     }
     if (Epi == EPI_BIAS_RELU_ROWSUM) {
@@ -1286,10 +1310,9 @@ inline bool small_tile_wins(int m, int n) {
   return cost_small < 0.9 * cost_large;
 }
 
-// Column N-1 of C for an odd N, one wave per row: the direct-to-LDS kernels fetch B in pairs of 16-bit elements, and
-// with rows an odd number of elements apart the pair that holds B[K-1][N-1] ends two bytes past B, so they compute
-// the N-1 columns before it (their buffer range ends right in front of that pair) and this kernel the last one, with
-// the same epilogue.  Lane l takes k = l, l + 64, ...; the 64 partial sums are added in a fixed tree.
+// Column N-1 of C alone, one wave per row, with the same epilogue: N = 1, and an N of whole tiles and one column whose
+// extra tile column would cost a round of workgroups.  Lane l takes k = l, l + 64, ...; the 64 partial sums are added in
+// a fixed tree.
 template <bool Bf16, int Epi>
 __global__ __launch_bounds__(256) void gemm16_last_column_kernel(const uint16_t *__restrict__ A,
                                                                  const uint16_t *__restrict__ B, float *__restrict__ C,
@@ -1298,14 +1321,10 @@ __global__ __launch_bounds__(256) void gemm16_last_column_kernel(const uint16_t 
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= M) return;   // whole waves leave together
-  auto widen = [](uint16_t bits) {
-    if constexpr (Bf16) return __uint_as_float(static_cast<uint32_t>(bits) << 16);
-    else return static_cast<float>(__builtin_bit_cast(_Float16, bits));
-  };
   const uint16_t *a = A + static_cast<int64_t>(row) * K;
   const uint16_t *b = B + (N - 1);
   float sum = 0.f;
-  for (int k = lane; k < K; k += 64) sum += widen(a[k]) * widen(b[static_cast<int64_t>(k) * N]);
+  for (int k = lane; k < K; k += 64) sum += widen16<Bf16>(a[k]) * widen16<Bf16>(b[static_cast<int64_t>(k) * N]);
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
   if (lane == 0) {
@@ -1328,11 +1347,10 @@ __global__ __launch_bounds__(256) void gemm16_last_column_kernel(const uint16_t 
 int splitk_for(int m, int n, int k) {
   const int64_t tiles = static_cast<int64_t>((m + 127) / 128) * ((n + 127) / 128);
   const int64_t forced = tunable("gemm16.split_k", 0);
-  // the planes are added 16 bytes at a time; a last piece below one stage needs K % 8 == 0
-  if (forced == 1 || (static_cast<int64_t>(m) * n) % 4 != 0 || k % 8 != 0) return 1;
+  if (forced == 1) return 1;
   const int cus = compute_units();
   const double plane_mib = static_cast<double>(m) * n * 4 / (1 << 20);
-  const int64_t fit = static_cast<int64_t>(static_cast<double>(kSplitWorkspaceBytes >> 20) / plane_mib);
+  const int64_t fit = static_cast<int64_t>(kSplitWorkspaceBytes) / (splitk_plane_floats(m, n) * 4);
   int64_t splits = 1;
   if (forced >= 2) {
     splits = std::min<int64_t>({forced, static_cast<int64_t>(k / 64), fit});
@@ -1347,10 +1365,7 @@ int splitk_for(int m, int n, int k) {
       if (estimate(s) < best) best = estimate(s), splits = s;
     }
   }
-  if (splits < 2) return 1;
-  // whole K = 64 stages per piece; the count follows from the piece so that none is empty
-  const int chunk = static_cast<int>((((k + 63) / 64 + splits - 1) / splits) * 64);
-  return (k + chunk - 1) / chunk;
+  return splitk_pieces(k, 64, splits);
 }
 
 // The kernel on v_mfma_f32_16x16x32 with nothing switched off: what a call gets unless, in the measurement build, a sweep
@@ -1478,17 +1493,22 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   const int tile_choice = gemm16_tile_for(m, n, k);
   const bool ab16 = reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
   const bool tiled = tile_choice != 0 && (k >= 64 || ab16);
-  // an odd N: the tiled kernel takes the first N - 1 columns of the N-strided matrices, a matrix-vector kernel the last
-  const int nm = n - (n & 1);
+  // whole tile columns and one column more: that one goes to a kernel of its own where a tile column would add a round of
+  // workgroups (4096 x 4097 x 4096: 139 us against 184), and for N = 1
+  const int tile_slots = compute_units() * (tile_choice == 128 ? 2 : 1);
+  auto rounds = [&](int columns) {
+    return ((m + tile_choice - 1) / tile_choice * ceil_div(columns, tile_choice) + tile_slots - 1) / tile_slots;
+  };
+  const int nm = tiled && n % tile_choice == 1 && (n == 1 || rounds(n) > rounds(n - 1)) ? n - 1 : n;
 
-  // Row sums: every tile column (every 64 columns of the simple kernel, and the last column of an odd N) leaves its
-  // share of each row in a plane of its own, and rowsum_fold_kernel adds the planes in column order, in double, with one
-  // rounding: the same bits on every run.  The planes live in the stream's workspace block; a call that has none (under
+  // Row sums: every tile column (every 64 columns of the simple kernel; the last column on its own) leaves its share of
+  // each row in a plane of its own, and rowsum_fold_kernel adds the planes in column order, in double, with one rounding:
+  // the same bits on every run.  The planes live in the stream's workspace block; a call that has none (under
   // stream capture, past the sixteenth stream, planes beyond the block's size) adds with atomicAdd in arrival order.
   float *planes = nullptr;
   int n_planes = 0;
   if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
-    n_planes = !tiled ? (n + 63) / 64 : (nm > 0 ? (nm + tile_choice - 1) / tile_choice : 0) + (n & 1);
+    n_planes = tiled ? (nm + tile_choice - 1) / tile_choice + (n - nm) : (n + 63) / 64;
     if (static_cast<int64_t>(n_planes) * m * 4 <= static_cast<int64_t>(kSplitWorkspaceBytes)) planes = splitk_workspace(st);
     if (!planes) {
       hipLaunchKernelGGL(zero_f32_kernel, dim3((m + 255) / 256), dim3(256), 0, st, rowsum, m);
@@ -1510,10 +1530,8 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   const bool ragged = n % 8 != 0 || k % 64 != 0 || !ab16;   // the kernels' template flag
   const int remap = (int)tunable("gemm.xcd_remap", 1);
   int rc = SAREK_HIP_OK;
-  int tile_planes = 0;
   if (nm > 0 && tile_choice == 128) {
     const int sm = (m + 127) / 128, sn = (nm + 127) / 128;
-    tile_planes = sn;
     unsigned long long *sprobe = clock_probe(static_cast<int64_t>(sm) * sn);
     int splits = 1;
     float *partials = nullptr;
@@ -1523,8 +1541,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
       if (!partials) splits = 1;
     }
     if (splits > 1) {
-      const int64_t mn = static_cast<int64_t>(m) * n;
-      const int chunk = (((k + 63) / 64 + splits - 1) / splits) * 64;
+      const int chunk = splitk_chunk(k, 64, splits);
       if (ragged)
         hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, true>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
                            bias, rowsum, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, planes);
@@ -1533,7 +1550,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
                            bias, rowsum, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, planes);
       rc = check_launch("gemm16 kernel launch");
       if (rc != SAREK_HIP_OK) return rc;
-      rc = launch_splitk_reduce(partials, c, mn, splits, st);
+      rc = launch_splitk_reduce(partials, c, m, n, splits, st);
     } else {
       if (ragged)
         hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, true>), dim3(sm * sn), dim3(256), 0, st, a, b, c, bias,
@@ -1545,12 +1562,11 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
     }
   } else if (nm > 0) {
     const int tiles_m = (m + BM - 1) / BM, tiles_n = (nm + BN - 1) / BN;
-    tile_planes = tiles_n;
     unsigned long long *probe = clock_probe(static_cast<int64_t>(tiles_m) * tiles_n);
 #ifdef SAREK_HIP_MEASURE
     if (Epi == EPI_STORE && !ragged && tunable("gemm16.waves", 8) == 4) {
       hipLaunchKernelGGL((gemm16_m16w4_kernel<Bf16>), dim3(tiles_m * tiles_n), dim3(256), 0, st, a, b, c, m, nm, k, tiles_m,
-                         tiles_n, remap, n);
+                         tiles_n, remap);
     } else if (!ragged && tunable("gemm16.barriers", 2) == 1) {
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c,
                          bias, rowsum, m, nm, k, tiles_m, tiles_n, remap, probe, n, planes);
@@ -1567,7 +1583,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   if (rc != SAREK_HIP_OK) return rc;
   if (nm != n) {
     hipLaunchKernelGGL((gemm16_last_column_kernel<Bf16, Epi>), dim3((m + 3) / 4), dim3(256), 0, st, a, b, c, bias, rowsum,
-                       m, n, k, planes ? planes + static_cast<int64_t>(tile_planes) * m : nullptr);
+                       m, n, k, planes ? planes + static_cast<int64_t>(n_planes - 1) * m : nullptr);
     rc = check_launch("gemm16 last-column launch");
   }
   return finish(rc);

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
   const int s_begin = split * steps_per_split, s_end = min(nsteps, s_begin + steps_per_split);
 
   const uint32_t row_bytes = static_cast<uint32_t>(N) * 2;
-  const int64_t b_bytes = static_cast<int64_t>(K) * row_bytes;
+  const int64_t b_bytes = (static_cast<int64_t>(K) * N - (N & 1)) * 2;   // see load_end
   const uint32_t b_off = 8 * g * row_bytes + (n0 + 8 * l16) * 2u;
   uint32_t a_off[MT];   // rows past M repeat the last one: what they produce is never stored
 #pragma unroll
@@ -85,14 +85,14 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
       bf[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, b_off + i * row_bytes, 0, 0));
     const int left = K - s * kStepK - 8 * g;   // elements of A this lane has before the end of K
     const __amdgpu_buffer_rsrc_t a_rsrc =
-        make_rsrc(A + static_cast<int64_t>(s) * kStepK, static_cast<uint32_t>((static_cast<int64_t>(M) * K - s * kStepK) * 2));
+        make_rsrc(A + static_cast<int64_t>(s) * kStepK, static_cast<uint32_t>((static_cast<int64_t>(M) * K - (K & 1) - s * kStepK) * 2));
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       af[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off[t], 0, 0));
 #pragma unroll
       for (int d = 0; d < 4; ++d) af[t][d] &= left >= 2 * d + 2 ? 0xFFFFFFFFu : left == 2 * d + 1 ? 0xFFFFu : 0u;
     }
-    // ranges are checked per dword: with an odd K the one that holds A[M-1][K-1] ends past A and read as zero ...
+    // with an odd K the dword that holds A[M-1][K-1] ends past A: the range ends in front of it, it read as zero ...
     if ((K & 1) != 0 && s == nsteps - 1) {
       const uint32_t v = A[static_cast<int64_t>(M) * K - 1];
 #pragma unroll
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
         for (int d = 0; d < 4; ++d)
           if (16 * t + l16 >= M - 1 && left == 2 * d + 1) af[t][d] = v;
     }
-    // ... and with an odd N the one that holds B[K-1][N-1]
+    // ... and with an odd N the one that holds B[K-1][N-1] past B
     if ((N & 1) != 0 && s == nsteps - 1) {
       const int r = K - 1 - s * kStepK, c = N - 1 - n0;   // row in the step, column in the tile
       if (g == r / 8 && c >= 0 && l16 == c / 8) {
@@ -286,15 +286,15 @@ int launch_rows(const uint16_t *a, const uint16_t *b, float *c, int m, int n, in
 
 }  // namespace
 
-// Whether this kernel takes a product.  It can: up to 64 rows (four row tiles' sums fill the registers), K of at least one
-// step, 32 rows of B and all of A within the 32-bit load offsets.  Up to 16 rows it always should.  Beyond, a workgroup's
+// Whether this kernel takes a product.  It can: up to 64 rows (four row tiles' sums fill the registers), rows of B of at
+// least a pair of elements (load_end counts on it), K of at least one step, 32 rows of B and all of A within the 32-bit load offsets.  Up to 16 rows it always should.  Beyond, a workgroup's
 // sums through LDS cost it 0.5 us per 16 rows and its registers leave room for one workgroup per CU, so short K and more
 // column tiles than CUs belong to the 128 x 128 tile unless that one would need its odd-N launch (us, 128 tile / here):
 //   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
 //   48 x 4096 x 256 6.2 / 6.1, 48 x 4096 x 1024 10.2 / 9.4, 48 x 40000 x 1024 23.0 / 26.4, 48 x 40001 x 1024 35.3 / 33.4
 //   64 x 4096 x 256 6.4 / 7.2, 64 x 4096 x 1024 10.5 / 10.5, 64 x 4096 x 4096 17.3 / 15.6, 64 x 40001 x 1024 36.3 / 37.0
 bool gemm16_rows_serves(int m, int n, int k) {
-  if (m > kRowsMax || k < kStepK || static_cast<int64_t>(n + kCols) * 2 * kStepK >= 0x7FFFFFFF ||
+  if (m > kRowsMax || n < 2 || k < kStepK || static_cast<int64_t>(n + kCols) * 2 * kStepK >= 0x7FFFFFFF ||
       static_cast<int64_t>(m) * k * 2 >= 0x7FFFFFFF)
     return false;
   const bool odd = n % 2 != 0, one_round = (n + kCols - 1) / kCols <= compute_units();

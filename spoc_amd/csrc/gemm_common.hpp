@@ -9,7 +9,19 @@ namespace sarek_hip {
 // adds them into C in a fixed order.
 constexpr size_t kSplitWorkspaceBytes = 64u << 20;
 float *splitk_workspace(hipStream_t st);
-int launch_splitk_reduce(const float *partials, float *c, int64_t mn, int splits, hipStream_t st);
+int launch_splitk_reduce(const float *partials, float *c, int m, int n, int splits, hipStream_t st);
+// Floats from one partial plane to the next: planes start at 16 bytes.
+__host__ __device__ inline int64_t splitk_plane_floats(int m, int n) { return (static_cast<int64_t>(m) * n + 3) / 4 * 4; }
+// K in at most `splits` pieces of whole stages of `stage`: their length (the last one takes what is left, at least a
+// stage), and how many come out.
+inline int splitk_chunk(int k, int stage, int64_t splits) {
+  const int64_t stages = (k + stage - 1) / stage;
+  return static_cast<int>((stages + splits - 1) / splits) * stage;
+}
+inline int splitk_pieces(int k, int stage, int64_t splits) {
+  while (splits > 1 && k - splitk_chunk(k, stage, splits) * (splits - 1) < stage) --splits;
+  return static_cast<int>(splits);
+}
 // Counters behind the planes of a block, zero between launches: one per tile for kernels whose last piece adds the planes.
 constexpr int kSplitTickets = 4096;
 inline unsigned *splitk_tickets(float *block) {

@@ -225,11 +225,12 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
     const int col = Ragged ? n0 + chunk * 4 : min(n0 + chunk * 4, N - 4);
     b_off[i] = (static_cast<uint32_t>(brow) * N + col) * 4u;
   }
-  // K cut over gridDim.y workgroups per tile: this one takes k0 .. k0 + k_len - 1 and writes its partial tile to its
-  // own M x N plane of `partials`, which a second kernel adds up in a fixed order
+  // K cut over gridDim.y workgroups per tile: this one takes k0 .. k0 + k_len - 1, the last one what is left of K (at
+  // least a slab), and writes its partial tile to its own plane of `partials`, which a second kernel adds up in a fixed
+  // order
   const int k0 = blockIdx.y * k_chunk;
-  const int k_len = min(k_chunk, K - k0);
-  if (gridDim.y > 1) C = partials + static_cast<int64_t>(blockIdx.y) * M * N;
+  const int k_len = blockIdx.y == gridDim.y - 1 ? K - k0 : k_chunk;
+  if (gridDim.y > 1) C = partials + blockIdx.y * splitk_plane_floats(M, N);
   const char *a_base = reinterpret_cast<const char *>(A + static_cast<int64_t>(m0) * K + k0);
   const char *b_base = reinterpret_cast<const char *>(B + static_cast<int64_t>(k0) * N);
   const int64_t b_slab_bytes = static_cast<int64_t>(BKT) * N * 4;
@@ -459,11 +460,11 @@ int gemm_f32_tile_for(int m, int n) {
 // if it is a tenth below the whole product's.  gemm_f32.split_k: 0 = this rule, 1 = never, n >= 2 forces n.
 int splitk_f32_for(int m, int n, int k) {
   const int64_t forced = tunable("gemm_f32.split_k", 0);
-  if (forced == 1 || (static_cast<int64_t>(m) * n) % 4 != 0 || k % 32 != 0) return 1;
+  if (forced == 1) return 1;
   const int cus = compute_units();
   const int64_t tiles = static_cast<int64_t>((m + 63) / 64) * ((n + 63) / 64);
   const double plane_mib = static_cast<double>(m) * n * 4 / (1 << 20);
-  const int64_t fit = static_cast<int64_t>(static_cast<double>(kSplitWorkspaceBytes >> 20) / plane_mib);
+  const int64_t fit = static_cast<int64_t>(kSplitWorkspaceBytes) / (splitk_plane_floats(m, n) * 4);
   int64_t splits = 1;
   if (forced >= 2) {
     splits = std::min<int64_t>({forced, static_cast<int64_t>(k / 32), fit});
@@ -478,9 +479,7 @@ int splitk_f32_for(int m, int n, int k) {
       if (estimate(s) < best) best = estimate(s), splits = s;
     }
   }
-  if (splits < 2) return 1;
-  const int chunk = static_cast<int>(((k / 32 + splits - 1) / splits) * 32);
-  return (k + chunk - 1) / chunk;
+  return splitk_pieces(k, 32, splits);
 }
 }  // namespace
 
@@ -513,15 +512,15 @@ extern "C" int sarek_hip_gemm_f32(const float *a, const float *b, float *c, int 
     auto ntiles = [&](int t) { return static_cast<int64_t>((m + t - 1) / t) * ((n + t - 1) / t); };
     int tile = (int)tunable("gemm_f32.tile", 0);
     if (tile == 0) tile = gemm_f32_tile_for(m, n);
-    // K cut over idle CUs for the 64 x 64 tile (few tiles, long K): whole slabs per piece, planes added 16 bytes at a time
+    // K cut over idle CUs for the 64 x 64 tile (few tiles, long K): whole slabs per piece, the last one with the rest
     int splits = 1;
     float *partials = nullptr;
-    if (tile == 64 && k % 32 == 0 && reinterpret_cast<uintptr_t>(c) % 16 == 0) {
+    if (tile == 64 && reinterpret_cast<uintptr_t>(c) % 16 == 0) {
       splits = splitk_f32_for(m, n, k);
       if (splits > 1) partials = splitk_workspace(st);
       if (!partials) splits = 1;
     }
-    const int k_chunk = splits > 1 ? ((k / 32 + splits - 1) / splits) * 32 : k;
+    const int k_chunk = splits > 1 ? splitk_chunk(k, 32, splits) : k;
 #define SAREK_LAUNCH_F32(T, TI, TJ, WMW, WNW, BKT, RAGGED)                                         \
   hipLaunchKernelGGL((gemm_f32_dma_kernel<TI, TJ, WMW, WNW, BKT, 4, RAGGED>),                     \
                      dim3((unsigned)ntiles(T), splits), dim3(64 * WMW * WNW), 0, st, a, b, c, m, n, k, \
@@ -539,7 +538,7 @@ extern "C" int sarek_hip_gemm_f32(const float *a, const float *b, float *c, int 
 #undef SAREK_LAUNCH_F32
     const int rc = check_launch("gemm_f32 kernel launch");
     if (rc != SAREK_HIP_OK || splits == 1) return rc;
-    return launch_splitk_reduce(partials, c, static_cast<int64_t>(m) * n, splits, st);
+    return launch_splitk_reduce(partials, c, m, n, splits, st);
   }
   if (aligned && n % 4 == 0 && tunable("gemm_f32.force_simple", 0) == 0) {
     static bool attr_done = false;

@@ -11,14 +11,18 @@ namespace sarek_hip {
 namespace {
 
 // Adds the `splits` partial planes into C, plane 0 first: a fixed order, so the result does not depend on which
-// workgroup finished when.  mn is a multiple of 4 and both pointers are 16-byte aligned (the callers' conditions).
+// workgroup finished when.  C is 16-byte aligned (the callers' condition).
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ partials, float *__restrict__ C,
-                                                            int64_t mn, int splits) {
+                                                            int64_t mn, int64_t plane, int splits) {
   const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
   if (i >= mn) return;
   f32x4_t acc = *reinterpret_cast<const f32x4_t *>(partials + i);
-  for (int s = 1; s < splits; ++s) acc += *reinterpret_cast<const f32x4_t *>(partials + s * mn + i);
-  *reinterpret_cast<f32x4_t *>(C + i) = acc;
+  for (int s = 1; s < splits; ++s) acc += *reinterpret_cast<const f32x4_t *>(partials + s * plane + i);
+  if (i + 4 <= mn) {
+    *reinterpret_cast<f32x4_t *>(C + i) = acc;
+  } else {
+    for (int j = 0; i + j < mn; ++j) C[i + j] = acc[j];
+  }
 }
 
 __global__ __launch_bounds__(256) void zero_tickets_kernel(unsigned *tickets) {
@@ -68,9 +72,10 @@ int compute_units() {
   return cus;
 }
 
-int launch_splitk_reduce(const float *partials, float *c, int64_t mn, int splits, hipStream_t st) {
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>((mn / 4 + 255) / 256)), dim3(256), 0, st, partials,
-                     c, mn, splits);
+int launch_splitk_reduce(const float *partials, float *c, int m, int n, int splits, hipStream_t st) {
+  const int64_t mn = static_cast<int64_t>(m) * n;
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>((mn + 1023) / 1024)), dim3(256), 0, st, partials, c,
+                     mn, splitk_plane_floats(m, n), splits);
   return check_launch("split-K reduction launch");
 }
 

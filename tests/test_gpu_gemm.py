@@ -739,7 +739,7 @@ def test_gemm16_few_rows(hip, torch_cuda, kind, m, n, k):
         try:
             for splits in (0, 1, 2, 5):
                 hip.set_tunable("gemm16.rows_splits", splits)
-                assert hip.gemm16_tile(m, n, k) == (64 if m <= 64 else 128)
+                assert hip.gemm16_tile(m, n, k) == (64 if m <= 64 and n > 1 else 128)   # n = 1: a wave per row
                 guard = torch.full((m * n + 64,), 7.0, device="cuda")
                 c = guard[32 + off:32 + off + m * n].view(m, n)
                 fn(da, db, out=c)
@@ -748,3 +748,28 @@ def test_gemm16_few_rows(hip, torch_cuda, kind, m, n, k):
                 assert torch.equal(c, fn(da, db)), "the same bits on every run"
         finally:
             hip.set_tunable("gemm16.rows_splits", 0)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+@pytest.mark.parametrize("m,n,k", [(70, 1, 100), (300, 3, 65), (200, 129, 328), (513, 255, 4107), (4096, 4097, 72), (130, 4097, 2056)])
+def test_gemm16_odd_columns(hip, torch_cuda, kind, m, n, k):
+    """Odd N on the tiled kernels: the last element of B added in the epilogue of the last tile column (K whole and in
+    pieces whose last one is shorter or longer than the others), and the column that has a kernel of its own (n = 1; 4097
+    columns of 4096 rows, where a seventeenth tile column would be a second round).  Bound as for the few-rows kernel."""
+    torch = torch_cuda
+    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    torch.manual_seed(m + n * k)
+    da = (torch.randn(m, k, device="cuda") * 0.02).to(dt)
+    db = (torch.randn(k, n, device="cuda") * 0.02).to(dt)
+    ref, size = da.double() @ db.double(), da.double().abs() @ db.double().abs()
+    try:
+        for split in (0, 3) if m < 4096 else (0,):
+            hip.set_tunable("gemm16.split_k", split)
+            c = (hip.gemm_bf16 if kind == "bf16" else hip.gemm_f16)(da, db)
+            assert bool(((c.double() - ref).abs() <= k * 2.0 ** -24 * size).all()), split
+            if kind == "f16":
+                y, rs = hip.gemm_f16_bias_relu_rowsum(da, db, torch.zeros(n, device="cuda"))
+                assert bool(((y.double() - ref.relu()).abs() <= k * 2.0 ** -24 * size).all())
+                assert bool(((rs.double() - ref.relu().sum(1)).abs() <= (k + n) * 2.0 ** -24 * size.sum(1)).all())
+    finally:
+        hip.set_tunable("gemm16.split_k", 0)
