@@ -12,21 +12,18 @@
 #include "host/ir.hpp"
 #include "host/map_fuse.hpp"
 #include "plugin.hpp"
+#include "text_hash.hpp"
 
 namespace sarek_hip {
 namespace {
 // Every tagged text this process has handed out.  The recogniser matched the whole IR body before it wrote
 // the tag, so exactly these texts may be served by a hand-written kernel; any other text that starts with
 // the same line is somebody else's program.
-struct ViewHash {
-  using is_transparent = void;
-  size_t operator()(std::string_view v) const { return std::hash<std::string_view>{}(v); }
-};
 std::mutex g_tagged_mu;
-std::unordered_set<std::string, ViewHash, std::equal_to<>> g_tagged;
+std::unordered_set<std::string, TextHash, std::equal_to<>> g_tagged;
 constexpr size_t kTaggedMax = 4096;     // beyond this the set starts over: forgotten texts run as compiled
 // The element-wise kernels among them (tag map_f32), by their text: what run_source needs to rebuild them
-std::unordered_map<std::string, std::shared_ptr<MapEntry>, ViewHash, std::equal_to<>> g_maps;
+std::unordered_map<std::string, std::shared_ptr<MapEntry>, TextHash, std::equal_to<>> g_maps;
 }  // namespace
 
 std::shared_ptr<MapEntry> find_generated_map(const char *source) {

@@ -113,10 +113,9 @@ sarek_hip_kernel rebuilt_kernel(MapEntry &e, int reduce, bool nt, uint32_t pad_b
   return k;
 }
 
-int try_map(const char *source, const int block[3], const int grid[3], const sarek_hip_arg *a, int na,
+int try_map(const std::shared_ptr<MapEntry> &entry, const int block[3], const int grid[3], const sarek_hip_arg *a, int na,
             const sarek_hip_arg *red, int nred, const int rblock[3], const int rgrid[3], int *rc, bool red_is_max = false,
             uint32_t pad_bits = 0) {
-  const std::shared_ptr<MapEntry> entry = find_generated_map(source);
   if (!entry) return 0;
   const ir::MapKernel &m = entry->m;
   struct Slot {
@@ -185,8 +184,7 @@ int try_map(const char *source, const int block[3], const int grid[3], const sar
 
 // A block-256 tree sum or maximum with an element-wise expression in front (tags tree_sum_map_f32, tree_max_map_f32),
 // rebuilt in the hand block-256 kernel's shape.  Same conditions as for the plain tree: 256-thread blocks, exactly ceil(n / 256) of them.
-int try_tree_map(const char *source, const int block[3], const int grid[3], const sarek_hip_arg *a, int na, int *rc) {
-  const std::shared_ptr<MapEntry> entry = find_generated_map(source);
+int try_tree_map(const std::shared_ptr<MapEntry> &entry, const int block[3], const int grid[3], const sarek_hip_arg *a, int na, int *rc) {
   if (!entry) return 0;
   const ir::MapKernel &m = entry->m;
   struct Slot {
@@ -589,14 +587,14 @@ int try_specialised_pair(const std::string &tag0, const int block0[3], const int
 }
 
 // An element-wise kernel followed by the block-256 sum or maximum (fill value in the tag, as f32 bits) of its output
-int try_map_pair(const sarek_hip_launch &l0, const std::string &tag1, const sarek_hip_launch &l1, int *rc) {
+int try_map_pair(const std::shared_ptr<MapEntry> &entry, const sarek_hip_launch &l0, const std::string &tag1, const sarek_hip_launch &l1, int *rc) {
   if (tag1 == "reduce_sum_block256_f32")
-    return try_map(l0.source, l0.block, l0.grid, l0.args, l0.n_args, l1.args, l1.n_args, l1.block, l1.grid, rc);
+    return try_map(entry, l0.block, l0.grid, l0.args, l0.n_args, l1.args, l1.n_args, l1.block, l1.grid, rc);
   if (tag1.compare(0, 24, "reduce_max_block256_f32:") == 0 && tag1.size() == 32) {
     char *end = nullptr;
     const unsigned long bits = std::strtoul(tag1.c_str() + 24, &end, 16);
     if (*end != 0) return 0;
-    return try_map(l0.source, l0.block, l0.grid, l0.args, l0.n_args, l1.args, l1.n_args, l1.block, l1.grid, rc, true,
+    return try_map(entry, l0.block, l0.grid, l0.args, l0.n_args, l1.args, l1.n_args, l1.block, l1.grid, rc, true,
                    static_cast<uint32_t>(bits));
   }
   return 0;
@@ -606,64 +604,23 @@ int try_map_pair(const sarek_hip_launch &l0, const std::string &tag1, const sare
 
 }  // namespace sarek_hip
 
-using namespace sarek_hip;
+namespace sarek_hip {
 
-extern "C" {
-
-int sarek_hip_set_specialisation(int enabled) {
-  g_specialise = enabled ? 1 : 0;
-  return SAREK_HIP_OK;
+ResolvedText resolve_text(const char *source) {
+  ResolvedText r;
+  r.tag = read_tag(source);
+  if (!r.tag.empty() && !tag_is_ours(r.tag, source)) r.tag.clear();
+  if (!r.tag.empty()) r.map = find_generated_map(source);
+  return r;
 }
 
-const char *sarek_hip_last_run_path(void) { return t_last_path.c_str(); }
-
-int sarek_hip_run_sources(const sarek_hip_launch *launches, int n_launches, int *device_launches, int *completed) {
-  if (device_launches) *device_launches = 0;
-  if (completed) *completed = 0;
-  if (n_launches < 0 || (n_launches > 0 && !launches))
-    return fail(SAREK_HIP_E_INVALID_ARG, "run_sources: NULL or negative argument");
-  std::string path;
-  for (int i = 0; i < n_launches; ++i) {
-    const sarek_hip_launch &l0 = launches[i];
-    int served = 0;
-    if (i + 1 < n_launches && specialisation_enabled() && l0.source && launches[i + 1].source && l0.args &&
-        launches[i + 1].args) {
-      // two launches one hand-written kernel computes in a single pass over the data
-      const sarek_hip_launch &l1 = launches[i + 1];
-      const bool langs_ok = (l0.lang == SAREK_HIP_LANG_HIP_SOURCE || l0.lang == SAREK_HIP_LANG_CUDA_SOURCE) &&
-                            (l1.lang == SAREK_HIP_LANG_HIP_SOURCE || l1.lang == SAREK_HIP_LANG_CUDA_SOURCE);
-      const std::string tag0 = read_tag(l0.source), tag1 = read_tag(l1.source);
-      int rc = SAREK_HIP_OK;
-      if (langs_ok && !tag0.empty() && !tag1.empty() && tag_is_ours(tag0, l0.source) && tag_is_ours(tag1, l1.source) &&
-          (tag0 == "map_f32"
-               ? try_map_pair(l0, tag1, l1, &rc)
-               : try_specialised_pair(tag0, l0.block, l0.grid, l0.args, l0.n_args, tag1, l1.block, l1.grid, l1.args,
-                                      l1.n_args, &rc))) {
-        if (rc != SAREK_HIP_OK) return rc;
-        path += (path.empty() ? "" : ";") + tag0 + "+" + tag1;
-        served = 2;
-      }
-    }
-    if (!served) {
-      const int rc = sarek_hip_run_source(l0.source, l0.lang, l0.kernel_name, l0.block, l0.grid, l0.shared_mem_bytes,
-                                          l0.args, l0.n_args);
-      if (rc != SAREK_HIP_OK) return rc;
-      path += (path.empty() ? "" : ";") + t_last_path;
-      served = 1;
-    }
-    i += served - 1;
-    if (device_launches) ++*device_launches;
-    if (completed) *completed += served;
-  }
-  t_last_path = path.empty() ? "none" : path;
-  return SAREK_HIP_OK;
-}
-
-int sarek_hip_run_source(const char *source, int lang, const char *kernel_name, const int block[3],
-                         const int grid[3], int shared_mem_bytes, const sarek_hip_arg *args,
-                         int n_args) {
+int run_resolved(const sarek_hip_launch &l, const ResolvedText &text) {
+  const char *const source = l.source, *const kernel_name = l.kernel_name;
+  const int lang = l.lang, *const block = l.block, *const grid = l.grid, shared_mem_bytes = l.shared_mem_bytes,
+            n_args = l.n_args;
+  const sarek_hip_arg *const args = l.args;
   t_last_path = "none";
-  if (!source || !kernel_name || !block || !grid || n_args < 0 || (n_args > 0 && !args))
+  if (!source || !kernel_name || n_args < 0 || (n_args > 0 && !args))
     return fail(SAREK_HIP_E_INVALID_ARG, "run_source: NULL or negative argument");
   switch (lang) {
     case SAREK_HIP_LANG_HIP_SOURCE:
@@ -686,17 +643,14 @@ int sarek_hip_run_source(const char *source, int lang, const char *kernel_name, 
   if (shared_mem_bytes < 0)
     return fail(SAREK_HIP_E_INVALID_ARG, "run_source: negative shared memory size");
 
-  if (specialisation_enabled()) {
-    std::string tag = read_tag(source);
-    if (!tag.empty() && !tag_is_ours(tag, source)) tag.clear();
-    if (!tag.empty()) {
-      int rc = SAREK_HIP_OK;
-      if (tag == "map_f32"            ? try_map(source, block, grid, args, n_args, nullptr, 0, nullptr, nullptr, &rc)
-          : tag == "tree_sum_map_f32" || tag == "tree_max_map_f32" ? try_tree_map(source, block, grid, args, n_args, &rc)
-                                      : try_specialised(tag, block, grid, args, n_args, &rc)) {
-        t_last_path = tag;
-        return rc;
-      }
+  const std::string &tag = text.tag;
+  if (!tag.empty() && specialisation_enabled()) {
+    int rc = SAREK_HIP_OK;
+    if (tag == "map_f32"            ? try_map(text.map, block, grid, args, n_args, nullptr, 0, nullptr, nullptr, &rc)
+        : tag == "tree_sum_map_f32" || tag == "tree_max_map_f32" ? try_tree_map(text.map, block, grid, args, n_args, &rc)
+                                    : try_specialised(tag, block, grid, args, n_args, &rc)) {
+      t_last_path = tag;
+      return rc;
     }
   }
 
@@ -746,5 +700,83 @@ int sarek_hip_run_source(const char *source, int lang, const char *kernel_name, 
   rc = sarek_hip_kernel_launch(k, g, b, (unsigned)shared_mem_bytes, nullptr, params, n_args);
   if (rc == SAREK_HIP_OK) t_last_path = "jit";
   return rc;
+}
+
+int run_resolved_sequence(const sarek_hip_launch *launches, const ResolvedText *const *texts, int n_launches,
+                          int *device_launches, int *completed) {
+  if (device_launches) *device_launches = 0;
+  if (completed) *completed = 0;
+  std::string path;
+  for (int i = 0; i < n_launches; ++i) {
+    const sarek_hip_launch &l0 = launches[i];
+    int served = 0;
+    if (i + 1 < n_launches && specialisation_enabled() && l0.source && launches[i + 1].source && l0.args &&
+        launches[i + 1].args && !texts[i]->tag.empty() && !texts[i + 1]->tag.empty()) {
+      // two launches one hand-written kernel computes in a single pass over the data
+      const sarek_hip_launch &l1 = launches[i + 1];
+      const bool langs_ok = (l0.lang == SAREK_HIP_LANG_HIP_SOURCE || l0.lang == SAREK_HIP_LANG_CUDA_SOURCE) &&
+                            (l1.lang == SAREK_HIP_LANG_HIP_SOURCE || l1.lang == SAREK_HIP_LANG_CUDA_SOURCE);
+      const std::string &tag0 = texts[i]->tag, &tag1 = texts[i + 1]->tag;
+      int rc = SAREK_HIP_OK;
+      if (langs_ok &&
+          (tag0 == "map_f32"
+               ? try_map_pair(texts[i]->map, l0, tag1, l1, &rc)
+               : try_specialised_pair(tag0, l0.block, l0.grid, l0.args, l0.n_args, tag1, l1.block, l1.grid, l1.args,
+                                      l1.n_args, &rc))) {
+        if (rc != SAREK_HIP_OK) return rc;
+        path += (path.empty() ? "" : ";") + tag0 + "+" + tag1;
+        served = 2;
+      }
+    }
+    if (!served) {
+      const int rc = run_resolved(l0, *texts[i]);
+      if (rc != SAREK_HIP_OK) return rc;
+      path += (path.empty() ? "" : ";") + t_last_path;
+      served = 1;
+    }
+    i += served - 1;
+    if (device_launches) ++*device_launches;
+    if (completed) *completed += served;
+  }
+  t_last_path = path.empty() ? "none" : path;
+  return SAREK_HIP_OK;
+}
+
+}  // namespace sarek_hip
+
+using namespace sarek_hip;
+
+extern "C" {
+
+int sarek_hip_set_specialisation(int enabled) {
+  g_specialise = enabled ? 1 : 0;
+  return SAREK_HIP_OK;
+}
+
+const char *sarek_hip_last_run_path(void) { return t_last_path.c_str(); }
+
+int sarek_hip_run_sources(const sarek_hip_launch *launches, int n_launches, int *device_launches, int *completed) {
+  if (device_launches) *device_launches = 0;
+  if (completed) *completed = 0;
+  if (n_launches < 0 || (n_launches > 0 && !launches))
+    return fail(SAREK_HIP_E_INVALID_ARG, "run_sources: NULL or negative argument");
+  std::vector<ResolvedText> texts(n_launches);
+  std::vector<const ResolvedText *> pointers(n_launches);
+  for (int i = 0; i < n_launches; ++i) {
+    if (launches[i].source && specialisation_enabled()) texts[i] = resolve_text(launches[i].source);
+    pointers[i] = &texts[i];
+  }
+  return run_resolved_sequence(launches, pointers.data(), n_launches, device_launches, completed);
+}
+
+int sarek_hip_run_source(const char *source, int lang, const char *kernel_name, const int block[3],
+                         const int grid[3], int shared_mem_bytes, const sarek_hip_arg *args,
+                         int n_args) {
+  t_last_path = "none";
+  if (!source || !kernel_name || !block || !grid || n_args < 0 || (n_args > 0 && !args))
+    return fail(SAREK_HIP_E_INVALID_ARG, "run_source: NULL or negative argument");
+  const sarek_hip_launch l{source, lang, kernel_name, {block[0], block[1], block[2]}, {grid[0], grid[1], grid[2]},
+                           shared_mem_bytes, args, n_args};
+  return run_resolved(l, specialisation_enabled() ? resolve_text(source) : ResolvedText{});
 }
 }

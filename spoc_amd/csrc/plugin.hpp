@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "host/map_fuse.hpp"
+#include "sarek_hip.h"
 namespace sarek_hip {
 // First line of a generated source that a hand-written kernel can serve:
 // "// sarek-hip-specialise: <tag>".
@@ -30,6 +31,19 @@ struct MapEntry {
 // runtime.cpp: changes whenever sarek_hip_kernel_clear_cache has unloaded the cached kernels
 uint64_t kernel_cache_generation();
 std::shared_ptr<MapEntry> find_generated_map(const char *source);
+
+// plugin.cpp: what run_source finds out about a text before it looks at the arguments -- the specialise tag, if the text
+// carries one and is the library's own, and the rebuilt-class kernel behind it.  Both hold for a text as long as the
+// process lives, so whoever keeps a text (the dispatcher keeps one per distinct IR) keeps this with it.
+struct ResolvedText {
+  std::string tag;
+  std::shared_ptr<MapEntry> map;
+};
+ResolvedText resolve_text(const char *source);
+// sarek_hip_run_source / sarek_hip_run_sources for texts resolved before (`texts[i]` belongs to launches[i].source).
+int run_resolved(const sarek_hip_launch &l, const ResolvedText &text);
+int run_resolved_sequence(const sarek_hip_launch *launches, const ResolvedText *const *texts, int n_launches,
+                          int *device_launches, int *completed);
 
 // library_kernels.cpp: the texts sarek_hip_library_kernel_source hands out
 bool is_library_kernel_name(const std::string &name);

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "text_hash.hpp"
 
 struct sarek_hip_kernel_s {
   hipModule_t module = nullptr;
@@ -44,24 +45,6 @@ std::unordered_map<uint64_t, std::vector<CachedKernel>> g_kernel_cache;
 
 int rtc_fail(hiprtcResult r, const char *what) {
   return fail(1000 + static_cast<int>(r), "%s: %s", what, hiprtcGetErrorString(r));
-}
-
-// 64-bit hash of the source text, eight bytes a step, for the kernel cache (looked up at every
-// launch: a byte-at-a-time hash of a 2 KB source costs as much as the launch call itself).
-uint64_t hash_text(const char *p, size_t n) {
-  uint64_t h = 0x9E3779B97F4A7C15ull ^ n;
-  while (n >= 8) {
-    uint64_t w;
-    std::memcpy(&w, p, 8);
-    h = (h ^ w) * 0xFF51AFD7ED558CCDull;
-    h ^= h >> 32;
-    p += 8;
-    n -= 8;
-  }
-  uint64_t w = 0;
-  std::memcpy(&w, p, n);
-  h = (h ^ w) * 0xC4CEB9FE1A85EC53ull;
-  return h ^ (h >> 29);
 }
 
 void copy_log(const std::string &text, char *log, size_t log_len) {

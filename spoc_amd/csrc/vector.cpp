@@ -27,6 +27,7 @@
 #include "gpu_memory.hpp"
 #include "host/ir.hpp"
 #include "plugin.hpp"
+#include "text_hash.hpp"
 
 // The allocation behind a vector's host block; sub-vectors view their parent's, and it lives as
 // long as any of them (a Bigarray.Array1.sub keeps its parent's memory alive the same way).
@@ -215,6 +216,7 @@ int transfer_args(const sarek_hip_varg *args, int n, int dev) {
 
 // Execute.expand_to_run_source_args
 int expand_args(const sarek_hip_varg *args, int n, int dev, bool inject_lengths, std::vector<sarek_hip_arg> &out) {
+  out.reserve(2 * static_cast<size_t>(n));
   for (int i = 0; i < n; ++i) {
     sarek_hip_arg a;
     std::memset(&a, 0, sizeof(a));
@@ -265,7 +267,9 @@ void mark_stale(const sarek_hip_varg *args, int n, int dev) {
 // IR text -> (kernel name, source).  The reference regenerates and re-hashes the source at
 // every launch (Execute.ml:256); here one lowering per distinct IR text is kept.
 struct Lowered {
+  int block[3];                          // the text can depend on the block (sizes of shared arrays)
   std::string name, source;
+  ResolvedText text;                     // what run_source would find out about `source` at every launch
   // What each parameter takes: 'v' a vector (element size in bytes, 0 when the IR does not fix it: records), 'i' / 'l'
   // / 'f' / 'd' an int32 / int64 / float32 / float64 scalar, '?' anything (a record passed by value).
   struct Param {
@@ -318,24 +322,21 @@ int check_args(const Lowered &k, const sarek_hip_varg *args, int n, const char *
   return SAREK_HIP_OK;
 }
 std::mutex g_lowered_mu;
-std::unordered_map<std::string, std::shared_ptr<const Lowered>> g_lowered;
+std::unordered_map<std::string, std::vector<std::shared_ptr<const Lowered>>, TextHash, std::equal_to<>> g_lowered;
+size_t g_lowered_count = 0;
 
 // The lowering of (ir_text, block), made once: a launch loop calls this every time, so a hit
 // hands out the kept text without copying it.
 int lower(const char *ir_text, const int block[3], std::shared_ptr<const Lowered> &out) {
-  // the text can depend on the block (sizes of shared arrays): it is part of the key
-  thread_local std::string key;
-  char head[48];
-  const int head_len = std::snprintf(head, sizeof(head), "%d,%d,%d;", block[0], block[1], block[2]);
-  key.assign(head, static_cast<size_t>(head_len));
-  key.append(ir_text);
   {
     std::lock_guard<std::mutex> lock(g_lowered_mu);
-    auto it = g_lowered.find(key);
-    if (it != g_lowered.end()) {
-      out = it->second;
-      return SAREK_HIP_OK;
-    }
+    auto it = g_lowered.find(std::string_view(ir_text));
+    if (it != g_lowered.end())
+      for (const auto &k : it->second)
+        if (std::memcmp(k->block, block, sizeof(k->block)) == 0) {
+          out = k;
+          return SAREK_HIP_OK;
+        }
   }
   size_t needed = 0;
   int st = sarek_hip_generate_source(ir_text, block, nullptr, 0, &needed);
@@ -349,7 +350,9 @@ int lower(const char *ir_text, const int block[3], std::shared_ptr<const Lowered
   if (st != SAREK_HIP_OK) return st;
   src.resize(std::strlen(src.c_str()));
   auto made = std::make_shared<Lowered>();
-  made->source = src;
+  std::memcpy(made->block, block, sizeof(made->block));
+  made->text = resolve_text(src.c_str());
+  made->source = std::move(src);
   const ir::Kernel parsed = ir::parse_kernel(ir_text);
   made->name = parsed.name;
   for (const ir::Decl &d : parsed.params) {
@@ -372,8 +375,12 @@ int lower(const char *ir_text, const int block[3], std::shared_ptr<const Lowered
   }
   out = made;
   std::lock_guard<std::mutex> lock(g_lowered_mu);
-  if (g_lowered.size() > 256) g_lowered.clear();
-  g_lowered[key] = out;
+  if (g_lowered_count >= 256) {
+    g_lowered.clear();
+    g_lowered_count = 0;
+  }
+  g_lowered[ir_text].push_back(out);
+  ++g_lowered_count;
   return SAREK_HIP_OK;
 }
 
@@ -691,8 +698,9 @@ int sarek_hip_execute_run_vectors(const char *ir_text, const int block[3], const
   if ((st = check_args(*k, args, n_args, "run_vectors")) != SAREK_HIP_OK) return st;
   std::vector<sarek_hip_arg> rs;
   if ((st = expand_args(args, n_args, dev, true, rs)) != SAREK_HIP_OK) return st;
-  st = sarek_hip_run_source(k->source.c_str(), SAREK_HIP_LANG_HIP_SOURCE, k->name.c_str(), block, grid,
-                            shared_mem_bytes, rs.data(), static_cast<int>(rs.size()));
+  st = run_resolved({k->source.c_str(), SAREK_HIP_LANG_HIP_SOURCE, k->name.c_str(), {block[0], block[1], block[2]},
+                     {grid[0], grid[1], grid[2]}, shared_mem_bytes, rs.data(), static_cast<int>(rs.size())},
+                    k->text);
   if (st != SAREK_HIP_OK) return st;
   mark_stale(args, n_args, dev);
   return SAREK_HIP_OK;
@@ -714,6 +722,7 @@ int sarek_hip_execute_run_pipeline(const sarek_hip_pipeline_stage *stages, int n
   std::vector<std::shared_ptr<const Lowered>> lowered(n_stages);
   std::vector<std::vector<sarek_hip_arg>> expanded(n_stages);
   std::vector<sarek_hip_launch> seq(n_stages);
+  std::vector<const ResolvedText *> texts(n_stages);
   for (int i = 0; i < n_stages; ++i) {
     const sarek_hip_pipeline_stage &s = stages[i];
     if ((st = transfer_args(s.args, s.n_args, dev)) != SAREK_HIP_OK) return st;
@@ -726,6 +735,7 @@ int sarek_hip_execute_run_pipeline(const sarek_hip_pipeline_stage *stages, int n
     if ((st = expand_args(s.args, s.n_args, dev, true, expanded[i])) != SAREK_HIP_OK) return st;
     sarek_hip_launch &l = seq[i];
     l.source = lowered[i]->source.c_str();
+    texts[i] = &lowered[i]->text;
     l.lang = SAREK_HIP_LANG_HIP_SOURCE;
     l.kernel_name = lowered[i]->name.c_str();
     for (int d = 0; d < 3; ++d) {
@@ -737,7 +747,7 @@ int sarek_hip_execute_run_pipeline(const sarek_hip_pipeline_stage *stages, int n
     l.n_args = static_cast<int>(expanded[i].size());
   }
   int done = 0;
-  st = sarek_hip_run_sources(seq.data(), n_stages, launches, &done);
+  st = run_resolved_sequence(seq.data(), texts.data(), n_stages, launches, &done);
   for (int i = 0; i < done; ++i) mark_stale(stages[i].args, stages[i].n_args, dev);
   return st;
 }

@@ -597,6 +597,13 @@ class Transfer:
             hip.check(hip.lib.sarek_hip_stream_destroy(stream))
 
 
+def _served(result):
+    """What a launch call of hip._host returned: the code path, or the library's status."""
+    if type(result) is int:
+        hip.check(result)
+    return result
+
+
 class Execute:
     """sarek/sarek/Execute.ml: vector_arg constructors, run_vectors, run_source."""
 
@@ -676,29 +683,14 @@ class Execute:
     def run_vectors(ir, args, block, grid, shared_mem=0):
         """Execute.run_vectors ~ir ~args ~block ~grid ?shared_mem (); returns the code path that
         served the launch ("jit" or a hand kernel's tag)."""
-        a, n = Execute._args(args)
-        hip.check(hip.lib.sarek_hip_execute_run_vectors(ir.encode(), (C.c_int * 3)(*block), (C.c_int * 3)(*grid),
-                                                        shared_mem, a, n))
-        return hip.lib.sarek_hip_last_run_path().decode()
+        return _served(hip._host.run_vectors(ir, args, block, grid, shared_mem))
 
     @staticmethod
     def run_pipeline(stages):
         """A kernel list run in order: stages = [(ir, args, block, grid)] or [(ir, args, block, grid, shared_mem)],
         each what one run_vectors call takes.  Returns (code paths, device launches made); consecutive stages
         that one hand kernel serves count as one launch."""
-        arr = (hip.PipelineStage * max(len(stages), 1))()
-        keep = []
-        for st, stage in zip(arr, stages):
-            ir, args, block, grid = stage[:4]
-            a, n = Execute._args(args)
-            text = ir.encode()
-            keep.append((a, text))
-            st.ir_text, st.block, st.grid = text, (C.c_int * 3)(*block), (C.c_int * 3)(*grid)
-            st.shared_mem_bytes = stage[4] if len(stage) > 4 else 0
-            st.args, st.n_args = a, n
-        launches = C.c_int(0)
-        hip.check(hip.lib.sarek_hip_execute_run_pipeline(arr, len(stages), C.byref(launches)))
-        return hip.lib.sarek_hip_last_run_path().decode(), launches.value
+        return _served(hip._host.run_pipeline(stages))
 
     @staticmethod
     def library_kernel(name):
@@ -707,11 +699,7 @@ class Execute:
 
     @staticmethod
     def run_source(source, kernel_name, block, grid, args, lang=hip.LANG_HIP, shared_mem=0, inject_lengths=True):
-        a, n = Execute._args(args)
-        hip.check(hip.lib.sarek_hip_execute_run_source(source.encode(), lang, kernel_name.encode(),
-                                                       (C.c_int * 3)(*block), (C.c_int * 3)(*grid), shared_mem,
-                                                       int(inject_lengths), a, n))
-        return hip.lib.sarek_hip_last_run_path().decode()
+        return _served(hip._host.run_source(source, lang, kernel_name, block, grid, shared_mem, inject_lengths, args))
 
     @staticmethod
     def sync_vectors_to_cpu(args):
