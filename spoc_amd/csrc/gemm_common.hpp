@@ -31,6 +31,15 @@ inline unsigned *splitk_tickets(float *block) {
 // Compute units of the current device (256 where it does not say).
 int compute_units();
 
+// float32 products straight from memory to registers (gemm_f32_direct.hip): variants (row_blocks, waves) = (1, 8), (1, 4),
+// (2, 4)
+bool gemm_f32_direct_serves(int m, int n, int k);
+bool gemm_f32_direct_pays(int m, int n, int k);
+int gemm_f32_direct_pieces(int m, int n, int k, int row_blocks, int splits);
+double gemm_f32_direct_estimate(int m, int n, int k, int row_blocks, int waves, int splits);
+int launch_gemm_f32_direct(const float *a, const float *b, float *c, int m, int n, int k, int row_blocks, int waves,
+                           int splits, hipStream_t st);
+
 // 16-bit products of at most 64 rows (gemm16_rows.hip)
 bool gemm16_rows_serves(int m, int n, int k);
 int gemm16_rows_k_splits(int m, int n, int k);

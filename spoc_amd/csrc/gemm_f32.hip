@@ -19,6 +19,7 @@
 #include <utility>
 
 #include <algorithm>
+#include <cmath>
 
 #include "common.hpp"
 #include "gemm_common.hpp"
@@ -438,58 +439,75 @@ __global__ __launch_bounds__(256) void gemm_f32_simple_kernel(const float *__res
 using namespace sarek_hip;
 
 namespace {
-// Tile choice by a cost model of the launch: a CU holds `occ` workgroups of a tile shape at once (LDS ring), tiles run
-// in rounds of cus*occ, a workgroup that shares its CU takes occ times as long, and the tail round runs unshared when it
-// fits one workgroup per CU.  `eff` is the MFMA issue efficiency measured for each shape.
-int gemm_f32_tile_for(int m, int n) {
-  auto ntiles = [&](int t) { return static_cast<int64_t>((m + t - 1) / t) * ((n + t - 1) / t); };
-  const int cus = compute_units();
-  auto cost = [&](int t, int occ, double eff) {
-    const int64_t tiles = ntiles(t), slots = static_cast<int64_t>(cus) * occ;
-    const int64_t full = tiles / slots, rest = tiles % slots;
-    const double rounds = static_cast<double>(full) * occ + (rest == 0 ? 0 : rest <= cus ? 1 : occ);
-    return rounds * t * t / eff;
-  };
-  const double c256 = cost(256, 1, 1.0), c128 = cost(128, 2, 0.95), c64 = cost(64, 2, 0.80);
-  return (c256 <= c128 && c256 <= c64) ? 256 : (c128 <= c64 ? 128 : 64);
+// How a product is computed: straight from memory (row_blocks > 0; gemm_f32_direct.hip) or through the LDS ring in tiles
+// of `tile`, and into how many pieces K is cut (the 64 x 64 tile and the direct kernel).
+struct Plan {
+  int row_blocks, waves, tile, splits;
+};
+
+// K pieces for the 64 x 64 tile: whole slabs, planes within the workspace.
+int tile64_pieces(int m, int n, int k, int64_t splits) {
+  const int64_t fit = static_cast<int64_t>(kSplitWorkspaceBytes) / (splitk_plane_floats(m, n) * 4);
+  return splitk_pieces(k, 32, std::max<int64_t>(1, std::min<int64_t>({splits, static_cast<int64_t>(k / 32), fit})));
 }
 
-// K pieces for a product on the 64 x 64 tile; 1 = whole.  One such tile per CU runs at the rate of its MFMAs (0.45 us per
-// K = 32 slab, measured; two on a CU share the pipes), so pieces help while CUs are idle; against that stand the second
-// launch (5 us) and the partial planes (0.65 us per MiB).  The count in {2, 4, 8, 16} with the lowest estimate is taken
-// if it is a tenth below the whole product's.  gemm_f32.split_k: 0 = this rule, 1 = never, n >= 2 forces n.
-int splitk_f32_for(int m, int n, int k) {
-  const int64_t forced = tunable("gemm_f32.split_k", 0);
-  if (forced == 1) return 1;
-  const int cus = compute_units();
-  const int64_t tiles = static_cast<int64_t>((m + 63) / 64) * ((n + 63) / 64);
-  const double plane_mib = static_cast<double>(m) * n * 4 / (1 << 20);
-  const int64_t fit = static_cast<int64_t>(kSplitWorkspaceBytes) / (splitk_plane_floats(m, n) * 4);
-  int64_t splits = 1;
-  if (forced >= 2) {
-    splits = std::min<int64_t>({forced, static_cast<int64_t>(k / 32), fit});
-  } else {
-    auto estimate = [&](int64_t s) {
-      const double rounds = static_cast<double>((tiles * s + cus - 1) / cus);
-      return 8.0 + static_cast<double>(k) / 32 / s * 0.45 * rounds + (s > 1 ? 5.0 + s * plane_mib * 0.65 : 0.0);
-    };
-    double best = estimate(1) * 0.9;
-    for (int64_t s = 2; s <= 16; s *= 2) {
-      if (k / s < 256 || s > fit) break;
-      if (estimate(s) < best) best = estimate(s), splits = s;
+// Estimated time in us of the LDS kernels, fitted to the same drawn products as the direct kernel's estimate (3 % rms).
+// A 64 x 64 tile takes 0.49 us per K = 32 slab alone on its CU, and two on a CU share its matrix cores, so tiles count
+// in rounds of CUs; the larger ones take four and sixteen times as long less the operand traffic they save.  Pieces of
+// K cost the second launch and the planes.
+double ring_estimate(int m, int n, int k, int tile, int splits) {
+  const double tiles = static_cast<double>((m + tile - 1) / tile) * ((n + tile - 1) / tile);
+  const double rounds = std::ceil(tiles * splits / compute_units()), slabs = k / 32.0, c_mb = 4e-6 * m * n;
+  if (tile == 64)
+    return 3.16 + rounds * (slabs / splits * 0.487 + 0.915) + 0.208 * c_mb + (splits > 1 ? 3.41 + 0.127 * splits * c_mb : 0.0);
+  return 3.22 + rounds * (slabs * (tile == 128 ? 4 * 0.449 : 16 * 0.461) + 2.18) + 0.208 * c_mb;
+}
+
+// The variant and the pieces with the lowest estimate; the direct kernel, whose estimate is the less certain one, has to
+// be a twentieth ahead.  Against the best of all variants timed on the drawn products the choice loses 2.2 % on average.
+// Pieces are tried only while they leave every wave a step (direct) or four slabs (LDS), and while the workgroups they
+// make find CUs: more than four a CU never paid.
+// gemm_f32.direct: 1 = never, 18 / 14 / 24 = always, with (row_blocks, waves) these digits; gemm_f32.tile forces a tile,
+// gemm_f32.split_k the pieces (1 = whole) of the 64 x 64 tile or of a forced direct variant.  0 leaves the choice here.
+Plan plan_for(int m, int n, int k, bool ring_ok, bool c_aligned) {
+  constexpr int kPieces[] = {1, 2, 3, 4, 6, 8, 12, 16};
+  const int direct = static_cast<int>(tunable("gemm_f32.direct", 0)), forced = static_cast<int>(tunable("gemm_f32.tile", 0));
+  const int tile = forced == 0 || forced == 256 || forced == 128 ? forced : 64;
+  const int64_t split = tunable("gemm_f32.split_k", 0);
+  const bool direct_ok = gemm_f32_direct_serves(m, n, k);
+  if (direct > 1 && direct_ok)
+    return {direct / 10, direct % 10, 0, gemm_f32_direct_pieces(m, n, k, direct / 10, static_cast<int>(std::min<int64_t>(split, 64)))};
+  const int64_t most = 4ll * compute_units();
+  Plan best{0, 0, 0, 1};
+  double best_us = 1e300;
+  if (direct == 0 && direct_ok && (!ring_ok || (tile == 0 && split == 0 && gemm_f32_direct_pays(m, n, k))))
+    for (const auto [row_blocks, waves] : {std::pair{1, 8}, std::pair{1, 4}, std::pair{2, 4}}) {
+      const int64_t tiles = static_cast<int64_t>((m + 16 * row_blocks - 1) / (16 * row_blocks)) * ((n + 63) / 64);
+      for (const int pieces : kPieces) {
+        if (pieces > 1 && (k / 16 / pieces < waves || tiles * pieces > most)) break;
+        const int splits = gemm_f32_direct_pieces(m, n, k, row_blocks, pieces);
+        const double us = 1.05 * gemm_f32_direct_estimate(m, n, k, row_blocks, waves, splits);
+        if (us < best_us) best_us = us, best = {row_blocks, waves, 0, splits};
+      }
+    }
+  if (!ring_ok) return best;
+  for (const int t : {64, 128, 256}) {
+    if (tile != 0 && tile != t) continue;
+    const int64_t tiles = static_cast<int64_t>((m + t - 1) / t) * ((n + t - 1) / t);
+    for (const int pieces : kPieces) {
+      if (pieces > 1 && (t != 64 || split != 0 || !c_aligned || k / pieces < 128 || tiles * pieces > most)) break;
+      const int splits = t == 64 ? tile64_pieces(m, n, k, split >= 2 && c_aligned ? split : pieces) : 1;
+      const double us = ring_estimate(m, n, k, t, splits);
+      if (us < best_us) best_us = us, best = {0, 0, t, splits};
     }
   }
-  return splitk_pieces(k, 32, splits);
+  return best;
 }
 }  // namespace
 
 extern "C" int sarek_hip_gemm_f32_k_splits(int m, int n, int k) {
   if (m < 1 || n < 1 || k < 1) return 1;
-  // the split belongs to the 64 x 64 tile, which the launcher takes where its cost model says so
-  const int64_t forced_tile = tunable("gemm_f32.tile", 0);
-  if (forced_tile != 0 && forced_tile != 64) return 1;
-  if (forced_tile == 0 && gemm_f32_tile_for(m, n) != 64) return 1;
-  return splitk_f32_for(m, n, k);
+  return plan_for(m, n, k, k >= 32 || k % 4 == 0, true).splits;
 }
 
 extern "C" int sarek_hip_gemm_f32(const float *a, const float *b, float *c, int m, int n, int k,
@@ -507,19 +525,20 @@ extern "C" int sarek_hip_gemm_f32(const float *a, const float *b, float *c, int 
   // DMA offsets are 32-bit: 256 rows of A and 32 rows of B must span less than 2 GiB
   const bool offsets_ok = static_cast<int64_t>(k) * 256 * 4 < 0x7FFFFFFF &&
                           static_cast<int64_t>(n) * 32 * 4 < 0x7FFFFFFF;
-  if (ab_ok && offsets_ok && tunable("gemm_f32.force_simple", 0) == 0 && tunable("gemm_f32.force_staged", 0) == 0) {
-    const bool ragged = !aligned || n % 4 != 0 || k % 32 != 0 || reinterpret_cast<uintptr_t>(c) % 16 != 0;
+  const bool ring_ok = ab_ok && offsets_ok;
+  const bool c_aligned = reinterpret_cast<uintptr_t>(c) % 16 == 0;
+  const bool fallback = tunable("gemm_f32.force_simple", 0) != 0 || tunable("gemm_f32.force_staged", 0) != 0;
+  Plan plan{0, 0, 0, 1};
+  if (!fallback) plan = plan_for(m, n, k, ring_ok, c_aligned);
+  if (plan.row_blocks > 0) return launch_gemm_f32_direct(a, b, c, m, n, k, plan.row_blocks, plan.waves, plan.splits, st);
+  if (plan.tile > 0) {
+    const bool ragged = !aligned || n % 4 != 0 || k % 32 != 0 || !c_aligned;
     auto ntiles = [&](int t) { return static_cast<int64_t>((m + t - 1) / t) * ((n + t - 1) / t); };
-    int tile = (int)tunable("gemm_f32.tile", 0);
-    if (tile == 0) tile = gemm_f32_tile_for(m, n);
+    const int tile = plan.tile;
     // K cut over idle CUs for the 64 x 64 tile (few tiles, long K): whole slabs per piece, the last one with the rest
-    int splits = 1;
-    float *partials = nullptr;
-    if (tile == 64 && reinterpret_cast<uintptr_t>(c) % 16 == 0) {
-      splits = splitk_f32_for(m, n, k);
-      if (splits > 1) partials = splitk_workspace(st);
-      if (!partials) splits = 1;
-    }
+    int splits = plan.splits;
+    float *partials = splits > 1 ? splitk_workspace(st) : nullptr;
+    if (!partials) splits = 1;
     const int k_chunk = splits > 1 ? splitk_chunk(k, 32, splits) : k;
 #define SAREK_LAUNCH_F32(T, TI, TJ, WMW, WNW, BKT, RAGGED)                                         \
   hipLaunchKernelGGL((gemm_f32_dma_kernel<TI, TJ, WMW, WNW, BKT, 4, RAGGED>),                     \

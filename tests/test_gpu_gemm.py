@@ -773,3 +773,38 @@ def test_gemm16_odd_columns(hip, torch_cuda, kind, m, n, k):
                 assert bool(((rs.double() - ref.relu().sum(1)).abs() <= (k + n) * 2.0 ** -24 * size.sum(1)).all())
     finally:
         hip.set_tunable("gemm16.split_k", 0)
+
+
+@pytest.mark.parametrize("variant", [0, 18, 14, 24])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (16, 64, 16), (17, 65, 17), (15, 63, 31), (33, 3, 1001), (2, 1, 70), (32, 132, 256),
+                                   (70, 200, 4099), (129, 70, 530)])
+def test_gemm_f32_direct(hip, torch_cuda, variant, m, n, k):
+    """The f32 kernel without LDS staging at the edges of its rows (16, 32), columns (64) and steps of k (16): each variant
+    forced, K whole and in pieces, operands and result at odd offsets between NaNs and guard values, and the launcher's
+    own choice.  Against the float64 product: k products and at most 16 + 16 sums of waves and pieces, each addition
+    rounded to half an ulp, are off by at most (k + 32) 2^-24 times the sum of the products' magnitudes."""
+    torch = torch_cuda
+    torch.manual_seed(m * n + k)
+    buf_a = torch.full((m * k + 64,), float("nan"), device="cuda")
+    buf_b = torch.full((k * n + 64,), float("nan"), device="cuda")
+    try:
+        for off, splits in [(0, 0), (3, 1), (0, 2), (1, 5), (3, 16)]:
+            da, db = buf_a[off:off + m * k].view(m, k), buf_b[off:off + k * n].view(k, n)
+            da.copy_(torch.randn(m, k, device="cuda"))
+            db.copy_(torch.randn(k, n, device="cuda"))
+            ref, size = da.double() @ db.double(), da.double().abs() @ db.double().abs()
+            hip.set_tunable("gemm_f32.direct", variant)
+            hip.set_tunable("gemm_f32.split_k", splits if variant else 0)
+            if variant:
+                assert hip.gemm_f32_k_splits(m, n, k) <= max(splits, 1)
+            guard = torch.full((m * n + 64,), 7.0, device="cuda")
+            c = guard[32 + off:32 + off + m * n].view(m, n)
+            hip.gemm_f32(da, db, out=c)
+            assert bool((guard[:32 + off] == 7).all()) and bool((guard[32 + off + m * n:] == 7).all())
+            assert bool(((c.double() - ref).abs() <= (k + 32) * 2.0 ** -24 * size).all()), (off, splits)
+            assert torch.equal(c, hip.gemm_f32(da, db)), "the same bits on every run"
+            buf_a.fill_(float("nan"))
+            buf_b.fill_(float("nan"))
+    finally:
+        hip.set_tunable("gemm_f32.direct", 0)
+        hip.set_tunable("gemm_f32.split_k", 0)
