@@ -480,7 +480,9 @@ Plan plan_for(int m, int n, int k, bool ring_ok, bool c_aligned) {
   const int64_t most = 4ll * compute_units();
   Plan best{0, 0, 0, 1};
   double best_us = 1e300;
-  if (direct == 0 && direct_ok && (!ring_ok || (tile == 0 && split == 0 && gemm_f32_direct_pays(m, n, k))))
+  // (the clock probe of the measurement build is the ring kernels': a launch that it watches goes to them)
+  const bool probed = kMeasureBuild && clock_probe(1) != nullptr;
+  if (direct == 0 && direct_ok && !(probed && ring_ok) && (!ring_ok || (tile == 0 && split == 0 && gemm_f32_direct_pays(m, n, k))))
     for (const auto [row_blocks, waves] : {std::pair{1, 8}, std::pair{1, 4}, std::pair{2, 4}}) {
       const int64_t tiles = static_cast<int64_t>((m + 16 * row_blocks - 1) / (16 * row_blocks)) * ((n + 63) / 64);
       for (const int pieces : kPieces) {
