@@ -626,8 +626,8 @@ int sarek_hip_gemm_f16(const uint16_t *a, const uint16_t *b, float *c, int m, in
                        sarek_hip_stream stream);
 
 /* Which kernel the three 16-bit GEMM entry points take for a shape under the
- * present tunables: 64 = the few-rows kernel (plain products, m <= 64 and k >= 32,
- * where it is the faster one), 256 or 128 = the workgroup tile of the direct-to-LDS MFMA
+ * present tunables: 64 = the few-rows kernel (tiles of at most 64 rows, n >= 2 and
+ * k >= 32, for plain products where it is the faster one), 256 or 128 = the workgroup tile of the direct-to-LDS MFMA
  * kernels (the small tile where large ones would leave CUs idle; any n, any
  * k >= 64 and the multiples of 8 below, any alignment of a and b from k = 64
  * on), 0 = the one-thread-per-element kernel (k < 64 that is not a multiple
@@ -642,7 +642,8 @@ int sarek_hip_gemm16_tile(int m, int n, int k);
  * the first such call on the stream and kept until the process ends, for up
  * to 16 streams; calls on further streams, and calls under stream capture on
  * a stream that has no block yet, run unsplit (same result up to the order of
- * the f32 additions).  The fused-epilogue entry point never splits.         */
+ * the f32 additions).  The count is the plain products'; the fused entry point
+ * splits on the few-rows kernel only.                                       */
 int sarek_hip_gemm16_k_splits(int m, int n, int k);
 
 /* Fused epilogue chain: y = relu(A.B + bias[col]) (f32, [m x n]) and

@@ -1275,24 +1275,37 @@ __global__ void zero_f32_kernel(float *p, int n) {
   if (i < n) p[i] = 0.f;
 }
 
-// rowsum[r] = the per-tile-column sums planes[t * m + r], t = 0 .. count-1, added in that order in double and rounded
+// rowsum[r] = the per-tile-column sums planes[t * m + r], t = 0 .. count-1, added in double and rounded
 // once: the order is the tiles', not the order they finished in, so a product gives the same row sums on every run.
-__global__ __launch_bounds__(64) void rowsum_fold_kernel(const float *__restrict__ planes, int count, int m,
-                                                         float *__restrict__ rowsum) {
-  const int r = blockIdx.x * 64 + threadIdx.x;
-  if (r >= m) return;
+// A row is short and every load of it is a trip to another XCD's L2, so eight waves take the planes in turn with eight
+// loads in flight each (one thread per row: 6.3 us for 43 planes of 4095 rows).
+constexpr int kFoldParts = 8;
+__global__ __launch_bounds__(64 * kFoldParts) void rowsum_fold_kernel(const float *__restrict__ planes, int count, int m,
+                                                                      float *__restrict__ rowsum) {
+  __shared__ double part[kFoldParts][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = min(static_cast<int>(blockIdx.x) * 64 + lane, m - 1);
   double acc = 0.0;
-  // sixteen planes' values are asked for before the first is added (the loads are what takes the time: a row has one
-  // thread), the additions keep the planes' order
-  int t = 0;
-  for (; t + 16 <= count; t += 16) {
-    float v[16];
+  int t = wave;
+  for (; t + 7 * kFoldParts < count; t += 8 * kFoldParts) {
+    float v[8];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = planes[static_cast<int64_t>(t + u) * m + r];
+    for (int u = 0; u < 8; ++u) v[u] = planes[static_cast<int64_t>(t + u * kFoldParts) * m + r];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) acc += static_cast<double>(v[u]);
+    for (int u = 0; u < 8; ++u) acc += static_cast<double>(v[u]);
   }
-  for (; t < count; ++t) acc += static_cast<double>(planes[static_cast<int64_t>(t) * m + r]);
+  if (t < count) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = planes[static_cast<int64_t>(min(t + u * kFoldParts, count - 1)) * m + r];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc += t + u * kFoldParts < count ? static_cast<double>(v[u]) : 0.0;
+  }
+  part[wave][lane] = acc;
+  __syncthreads();
+  if (wave != 0 || static_cast<int>(blockIdx.x) * 64 + lane >= m) return;
+#pragma unroll
+  for (int w = 1; w < kFoldParts; ++w) acc += part[w][lane];
   rowsum[r] = static_cast<float>(acc);
 }
 
@@ -1379,10 +1392,24 @@ inline bool gemm16_default_kernel() {
 #endif
 }
 
-// Whether a plain product goes to the few-rows kernel: up to 64 rows, unless a knob asks for one of the tiled kernels.
-inline bool few_rows(int m, int n, int k) {
-  return gemm16_default_kernel() && tunable("gemm16.tile", 0) == 0 && tunable("gemm16.split_k", 0) == 0 &&
-         tunable("gemm16.force_simple", 0) == 0 && gemm16_rows_serves(m, n, k);
+// Microseconds of a product on the 128 x 128 tile with at most a workgroup per CU, by an estimate: its slabs by how A's and
+// B's rows lie (on 16 bytes, on 4, on 2), the K pieces it would take.
+double small_tile_time(int m, int n, int k, bool fused) {
+  const double slab = k % 8 == 0 && n % 8 == 0 ? 0.19 : k % 2 == 0 && n % 2 == 0 ? 0.24 : 0.33;
+  const int splits = fused ? 1 : splitk_for(m, n, k);
+  return 5.5 + static_cast<double>(k) / 32 / splits * slab +
+         (splits > 1 ? 3.0 + splits * (static_cast<double>(m) * n * 4 / (1 << 20)) * 0.65 : 0.0);
+}
+
+// Whether a product goes to the few-rows kernel, unless a knob asks for one of the tiled kernels.  gemm16.rows: 0 = by
+// size, 1 = never, 2 = wherever it can.
+inline bool few_rows(int m, int n, int k, bool fused) {
+  const int64_t asked = tunable("gemm16.rows", 0);
+  return asked != 1 && gemm16_default_kernel() && tunable("gemm16.tile", 0) == 0 && tunable("gemm16.split_k", 0) == 0 &&
+         tunable("gemm16.force_simple", 0) == 0 && gemm16_rows_serves(m, n, k) &&
+         !(kMeasureBuild && m > 64 && clock_probe(1)) &&   // the probe is the tiled kernels'
+        
+         (asked == 2 || gemm16_rows_pays(m, n, k, fused, small_tile_time(m, n, k, fused)));
 }
 
 // The workgroup tile of the direct-to-LDS kernels for this shape under the present tunables (256 or 128), or 0 when
@@ -1488,7 +1515,9 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   // The kernels on v_mfma_f32_16x16x32 (256 x 256 or 128 x 128 tile) take any N, any K of at least one LDS stage and
   // any alignment of A and B in their Ragged form; below one stage K must be a multiple of 8 and A and B 16-byte aligned.
   if constexpr (Epi == EPI_STORE) {
-    if (few_rows(m, n, k)) return launch_gemm16_rows(Bf16, a, b, c, m, n, k, st);
+    if (few_rows(m, n, k, false)) return launch_gemm16_rows(Bf16, a, b, c, m, n, k, st);
+  } else if constexpr (!Bf16) {
+    if (few_rows(m, n, k, true)) return launch_gemm16_rows_fused(a, b, bias, c, rowsum, m, n, k, st);
   }
   const int tile_choice = gemm16_tile_for(m, n, k);
   const bool ab16 = reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
@@ -1511,15 +1540,13 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
     n_planes = tiled ? (nm + tile_choice - 1) / tile_choice + (n - nm) : (n + 63) / 64;
     if (static_cast<int64_t>(n_planes) * m * 4 <= static_cast<int64_t>(kSplitWorkspaceBytes)) planes = splitk_workspace(st);
     if (!planes) {
-      hipLaunchKernelGGL(zero_f32_kernel, dim3((m + 255) / 256), dim3(256), 0, st, rowsum, m);
-      const int rc = check_launch("rowsum clear launch");
+      const int rc = launch_zero_f32(rowsum, m, st);
       if (rc != SAREK_HIP_OK) return rc;
     }
   }
   auto finish = [&](int rc) {
     if (rc != SAREK_HIP_OK || !planes) return rc;
-    hipLaunchKernelGGL(rowsum_fold_kernel, dim3((m + 63) / 64), dim3(64), 0, st, planes, n_planes, m, rowsum);
-    return check_launch("rowsum fold launch");
+    return launch_rowsum_fold(planes, n_planes, m, rowsum, st);
   };
 
   if (!tiled) {
@@ -1590,6 +1617,17 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
 }
 
 }  // namespace
+
+int launch_zero_f32(float *p, int n, hipStream_t st) {
+  hipLaunchKernelGGL(zero_f32_kernel, dim3((n + 255) / 256), dim3(256), 0, st, p, n);
+  return check_launch("rowsum clear launch");
+}
+
+int launch_rowsum_fold(const float *planes, int count, int m, float *rowsum, hipStream_t st) {
+  hipLaunchKernelGGL(rowsum_fold_kernel, dim3((m + 63) / 64), dim3(64 * kFoldParts), 0, st, planes, count, m, rowsum);
+  return check_launch("rowsum fold launch");
+}
+
 }  // namespace sarek_hip
 
 using namespace sarek_hip;
@@ -1597,11 +1635,11 @@ using namespace sarek_hip;
 extern "C" {
 
 int sarek_hip_gemm16_tile(int m, int n, int k) {
-  return m >= 1 && n >= 1 && few_rows(m, n, k) ? 64 : gemm16_tile_for(m, n, k);
+  return m >= 1 && n >= 1 && few_rows(m, n, k, false) ? 64 : gemm16_tile_for(m, n, k);
 }
 
 int sarek_hip_gemm16_k_splits(int m, int n, int k) {
-  if (m >= 1 && n >= 1 && few_rows(m, n, k)) return gemm16_rows_k_splits(m, n, k);
+  if (m >= 1 && n >= 1 && few_rows(m, n, k, false)) return gemm16_rows_k_splits(m, n, k);
   return gemm16_tile_for(m, n, k) == 128 ? splitk_for(m, n, k) : 1;
 }
 

@@ -1,4 +1,5 @@
-// 16-bit-input (bf16 / fp16), f32-accumulate products of at most 64 rows:  C[M x N] = A[M x K] . B[K x N], row-major.
+// 16-bit-input (bf16 / fp16), f32-accumulate products in tiles of at most 64 rows:  C[M x N] = A[M x K] . B[K x N],
+// row-major; for the fp16 product with bias, ReLU and row sums as well.
 //
 // What bounds it: B is read once and used M times, so the product is a read of B (16 x 8192 x 8192: 134 MB, 21 us at the
 // 6.3 TB/s large streams reach here) and a CU draws at most about 39 GB/s of L2 misses, so every CU has to take its
@@ -18,6 +19,10 @@
 //   16 x 8192 x 8192 34.5 -> 25.7 us (5.2 TB/s), 16 x 2048 x 2048 10.4 -> 6.8, 16 x 40000 x 1024 21.1 -> 19.6,
 //   32 x 16384 x 4096 32.9 -> 27.4, 48 x 4096 x 4096 17.2 -> 13.8, 16 x 256 x 8192 12.8 -> 7.4; odd sizes:
 //   10 x 4161 x 4221 80 -> 12.6, 64 x 4097 x 4103 74 -> 20.5, 8 x 50257 x 1024 34.5 -> 28.0.
+// More rows are more row tiles.  Where all tiles find a CU of their own the product is bound by the latency of its steps,
+// not by what is read, and the 128 x 128 tile has one wave per SIMD to hide it and, with the fused epilogue, no K pieces:
+//   77 x 2332 x 1920 22.7 -> 10.0, 97 x 1633 x 1090 16.1 -> 11.0; fused 220 x 256 x 4444 47.8 -> 16.0,
+//   537 x 259 x 3648 40.7 -> 18.0, 214 x 1088 x 3264 25.3 -> 17.1, 224 x 256 x 2368 18.9 -> 14.4.
 // Tried: 4 waves with 2 to 4 steps in flight (5 to 10 % slower), tiles dealt so that neighbours share an XCD (no change),
 // 64-bit atomic stores and loads for the planes (4 planes of 64 x 8192: 3 us more than the 16-byte accesses).
 #include <algorithm>
@@ -32,23 +37,38 @@
 namespace sarek_hip {
 namespace {
 
-constexpr int kRowsMax = 64, kCols = 128, kStepK = 32, kWaves = 8;
+constexpr int kTileRows = 64, kCols = 128, kStepK = 32, kWaves = 8;
 constexpr int kRedPitch = kCols + 4;   // floats per row of the waves' sums in LDS: 16 rows on different banks
 // Cache-policy bits of a buffer access: past the L2s, which the XCDs do not share; and non-temporal.
 constexpr int kDeviceScope = 16, kNonTemporal = 2;
 
-template <bool Bf16, int MT, int BPolicy>
+template <bool Bf16, int MT, int BPolicy, bool Fused>
 __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t *__restrict__ A,
                                                                   const uint16_t *__restrict__ B, float *__restrict__ C,
-                                                                  int M, int N, int K, int tiles, int splits,
-                                                                  int steps_per_split, float *__restrict__ partials,
+                                                                  const float *__restrict__ bias,
+                                                                  float *__restrict__ rowsum, int M, int N, int K,
+                                                                  int row_tiles, int col_tiles, int splits,
+                                                                  int steps_per_split, float *__restrict__ rs_planes,
+                                                                  float *__restrict__ partials,
                                                                   unsigned *__restrict__ tickets) {
   __shared__ __attribute__((aligned(16))) float red[kWaves][16 * kRedPitch];
   __shared__ bool last;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, g = lane >> 4;
-  const int tile = blockIdx.x % tiles, split = blockIdx.x / tiles;
-  const int n0 = tile * kCols;
+  // The row tiles of a column tile read the same piece of B: they are neighbours in an XCD's run of workgroups.
+  int index = blockIdx.x;
+  if (row_tiles > 1) {
+    const int xcd = index % NUM_XCD, nb = gridDim.x;
+    index = xcd * (nb / NUM_XCD) + min(xcd, nb % NUM_XCD) + index / NUM_XCD;
+  }
+  const int row_tile = index % row_tiles, col_tile = index / row_tiles % col_tiles;
+  const int split = index / (row_tiles * col_tiles);
+  const int tile = col_tile * row_tiles + row_tile, tiles = row_tiles * col_tiles;
+  const int n0 = col_tile * kCols, m0 = row_tile * (16 * MT);
+  A += static_cast<int64_t>(m0) * K;
+  M -= m0;   // from here on rows count from the tile's first
+  C += static_cast<int64_t>(m0) * N;
+
   const int nsteps = (K + kStepK - 1) / kStepK;
   const int s_begin = split * steps_per_split, s_end = min(nsteps, s_begin + steps_per_split);
 
@@ -85,7 +105,9 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
       bf[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, b_off + i * row_bytes, 0, 0));
     const int left = K - s * kStepK - 8 * g;   // elements of A this lane has before the end of K
     const __amdgpu_buffer_rsrc_t a_rsrc =
-        make_rsrc(A + static_cast<int64_t>(s) * kStepK, static_cast<uint32_t>((static_cast<int64_t>(M) * K - (K & 1) - s * kStepK) * 2));
+        make_rsrc(A + static_cast<int64_t>(s) * kStepK,
+                  static_cast<uint32_t>(min((static_cast<int64_t>(M) * K - (K & 1) - s * kStepK) * 2,
+                                            static_cast<int64_t>(0x7FFFFFFF))));
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
       af[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off[t], 0, 0));
@@ -135,7 +157,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
   // The piece's plain steps: whole K, and at least one tile's width of B behind their last row's first element
   const int64_t plain_rows = K - (kCols + N - 1) / N;
   const int plain = max(min(s_end, plain_rows > 0 ? static_cast<int>(plain_rows / kStepK) : 0) - s_begin, 0);
-  const int first = plain > 0 ? (tile * kWaves) % plain : 0;
+  const int first = plain > 0 ? (col_tile * kWaves) % plain : 0;
   u32x4 bf[2][8], af[2][MT];
   auto load_at = [&](int i, auto buffer) {
     const int at = i + first;
@@ -157,8 +179,30 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
 
   // Sums over the waves, 16 rows at a time: thread -> row `row`, columns col .. col + 3 of them
   const int row = threadIdx.x >> 5, col = (threadIdx.x & 31) * 4;
+  // (Fused: bias, ReLU, and the row's sum over the tile's columns, added by the 32 lanes that hold it, to its plane)
+  f32x4_t bias4 = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (Fused) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (n0 + col + j < N) bias4[j] = bias[n0 + col + j];
+  }
   auto put = [&](int t, f32x4_t v) {
     const int m = 16 * t + row, n = n0 + col;
+    if constexpr (Fused) {
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[j] += bias4[j];
+        v[j] = v[j] > 0.f ? v[j] : 0.f;
+        sum += n + j < N ? v[j] : 0.f;
+      }
+#pragma unroll
+      for (int o = 16; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
+      if (m < M && (lane & 31) == 0) {
+        if (rs_planes) rs_planes[static_cast<int64_t>(col_tile) * (M + m0) + m0 + m] = sum;
+        else atomicAdd(rowsum + m0 + m, sum);
+      }
+    }
     if (m >= M) return;
     float *dst = C + static_cast<int64_t>(m) * N + n;
     if (n + 4 <= N) {
@@ -224,92 +268,161 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
   if (threadIdx.x == 0) __hip_atomic_store(tickets + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Pieces of K per column tile, by an estimate in microseconds whose constants were fitted to sweeps of 1 to 31 pieces
+// Rows per tile: as few tiles of at most 64 as there can be, of equal height, in blocks of 16.
+inline int row_blocks_for(int m) {
+  const int tiles = (m + kTileRows - 1) / kTileRows;
+  return ((m + tiles - 1) / tiles + 15) / 16;
+}
+
+struct Shape {
+  int mt, row_tiles, col_tiles, steps;
+  int64_t tiles, plane, rs_floats;   // bytes of a partial plane; floats of the row sums' planes, whole 256-byte pieces
+};
+inline Shape shape_of(int m, int n, int k, bool fused) {
+  Shape s;
+  s.mt = row_blocks_for(m);
+  s.row_tiles = (m + 16 * s.mt - 1) / (16 * s.mt);
+  s.col_tiles = (n + kCols - 1) / kCols;
+  s.steps = (k + kStepK - 1) / kStepK;
+  s.tiles = static_cast<int64_t>(s.row_tiles) * s.col_tiles;
+  s.plane = s.tiles * s.mt * 16 * kCols * 4;
+  s.rs_floats = fused ? (static_cast<int64_t>(s.col_tiles) * m + 63) / 64 * 64 : 0;
+  return s;
+}
+
+double rows_time(const Shape &s, int n, int k, int64_t splits) {
+  const int cus = compute_units();
+  const double memory = static_cast<double>(k) * n * 2 / 6.3e6;
+  const double cu = static_cast<double>((s.tiles * splits + cus - 1) / cus) * s.steps / splits * (8192 + 1024 * s.mt) / 39e3;
+  return std::cbrt(cu * cu * cu + memory * memory * memory) +
+         (splits > 1 ? 1.0 + 0.15 * splits + 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0);
+}
+
+// Pieces of K per tile, by an estimate in microseconds whose constants were fitted to sweeps of 1 to 31 pieces
 // over 12 shapes (within 1 us on those of 10 us and more): a CU's share of B and A at 39 GB/s in whole rounds of
 // workgroups, B from memory at 6.3 TB/s, the two merged smoothly; a split adds its planes, written and read at 2.7 TB/s,
 // a ticket, and a little per piece.  A wave keeps at least one step.  gemm16.rows_splits: 0 = this rule, n forces n.
-int rows_splits_for(int m, int n, int k) {
-  const int tiles = (n + kCols - 1) / kCols, steps = (k + kStepK - 1) / kStepK, mt = (m + 15) / 16;
-  const int64_t plane = static_cast<int64_t>(tiles) * mt * 16 * kCols * 4;
-  const int64_t fit = tiles > kSplitTickets ? 1 : static_cast<int64_t>(kSplitWorkspaceBytes) / plane;
+int rows_splits_for(const Shape &s, int n, int k) {
+  const int64_t fit = s.tiles > kSplitTickets
+                          ? 1
+                          : (static_cast<int64_t>(kSplitWorkspaceBytes) - s.rs_floats * 4) / s.plane;
   const int64_t forced = tunable("gemm16.rows_splits", 0);
   int64_t splits = 1;
   if (forced > 0) {
-    splits = std::max<int64_t>(1, std::min<int64_t>({forced, steps, fit}));
+    splits = std::max<int64_t>(1, std::min<int64_t>({forced, s.steps, fit}));
   } else {
-    const int cus = compute_units();
-    const double memory = static_cast<double>(k) * n * 2 / 6.3e6;
-    auto estimate = [&](int64_t s) {
-      const double cu = static_cast<double>((tiles * s + cus - 1) / cus) * steps / s * (8192 + 1024 * mt) / 39e3;
-      return std::cbrt(cu * cu * cu + memory * memory * memory) +
-             (s > 1 ? 1.0 + 0.15 * s + 2.0 * static_cast<double>(s * plane) / 2.7e6 : 0.0);
-    };
-    double best = estimate(1);
-    for (int64_t s = 2; s <= 64 && s <= fit && s * kWaves <= steps; ++s)
-      if (estimate(s) < best) best = estimate(s), splits = s;
+    double best = rows_time(s, n, k, 1);
+    for (int64_t t = 2; t <= 64 && t <= fit && t * kWaves <= s.steps; ++t)
+      if (rows_time(s, n, k, t) < best) best = rows_time(s, n, k, t), splits = t;
   }
-  const int64_t per = (steps + splits - 1) / splits;   // the count follows from the piece so that none is empty
-  return static_cast<int>((steps + per - 1) / per);
+  const int64_t per = (s.steps + splits - 1) / splits;   // the count follows from the piece so that none is empty
+  return static_cast<int>((s.steps + per - 1) / per);
 }
 
-template <bool Bf16, int MT>
-int launch(const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k, hipStream_t st) {
-  const int tiles = (n + kCols - 1) / kCols, steps = (k + kStepK - 1) / kStepK;
-  int splits = rows_splits_for(m, n, k);
-  float *partials = nullptr;
-  if (splits > 1 && !(partials = splitk_workspace(st))) splits = 1;
-  const int per = (steps + splits - 1) / splits;
-  unsigned *tickets = partials ? splitk_tickets(partials) : nullptr;
+struct Call {
+  const uint16_t *a, *b;
+  float *c;
+  const float *bias;
+  float *rowsum;
+  int m, n, k;
+  hipStream_t st;
+};
+
+template <bool Bf16, bool Fused, int MT>
+int launch(const Call &q, const Shape &s) {
+  int splits = rows_splits_for(s, q.n, q.k);
+  float *block = nullptr;
+  if (Fused || splits > 1) block = splitk_workspace(q.st);
+  if (!block) splits = 1;
+  const int per = (s.steps + splits - 1) / splits;
+  float *rs_planes = nullptr;
+  if constexpr (Fused) {
+    if (s.rs_floats * 4 <= static_cast<int64_t>(kSplitWorkspaceBytes)) rs_planes = block;
+    if (!rs_planes) {
+      const int rc = launch_zero_f32(q.rowsum, q.m, q.st);
+      if (rc != SAREK_HIP_OK) return rc;
+    }
+  }
+  float *partials = splits > 1 ? block + s.rs_floats : nullptr;
+  unsigned *tickets = splits > 1 ? splitk_tickets(block) : nullptr;
   // B past the caches from 64 MiB on where its rows are whole 16-byte pieces (100 MB: 20.2 us against 22.8, 134 MB: 26.4
   // against 28.0, 34 MB: 15.8 against 13.2); rows at other offsets share lines between neighbouring loads, and lose
-  // (100 MB: 28.4 against 28.0)
-  const bool nt = n % 8 == 0 && static_cast<int64_t>(k) * n * 2 > (int64_t{64} << 20);
-  const dim3 grid(static_cast<unsigned>(tiles) * splits), block(64 * kWaves);
+  // (100 MB: 28.4 against 28.0), and so does what several row tiles read
+  const bool nt = s.row_tiles == 1 && q.n % 8 == 0 && static_cast<int64_t>(q.k) * q.n * 2 > (int64_t{64} << 20);
+  const dim3 grid(static_cast<unsigned>(s.tiles * splits)), block_dim(64 * kWaves);
   if (nt)
-    hipLaunchKernelGGL((gemm16_rows_kernel<Bf16, MT, kNonTemporal>), grid, block, 0, st, a, b, c, m, n, k, tiles, splits,
-                       per, partials, tickets);
+    hipLaunchKernelGGL((gemm16_rows_kernel<Bf16, MT, kNonTemporal, Fused>), grid, block_dim, 0, q.st, q.a, q.b, q.c, q.bias,
+                       q.rowsum, q.m, q.n, q.k, s.row_tiles, s.col_tiles, splits, per, rs_planes, partials, tickets);
   else
-    hipLaunchKernelGGL((gemm16_rows_kernel<Bf16, MT, 0>), grid, block, 0, st, a, b, c, m, n, k, tiles, splits, per,
-                       partials, tickets);
-  return check_launch("gemm16 few-rows kernel launch");
+    hipLaunchKernelGGL((gemm16_rows_kernel<Bf16, MT, 0, Fused>), grid, block_dim, 0, q.st, q.a, q.b, q.c, q.bias,
+                       q.rowsum, q.m, q.n, q.k, s.row_tiles, s.col_tiles, splits, per, rs_planes, partials, tickets);
+  const int rc = check_launch("gemm16 few-rows kernel launch");
+  if (!rs_planes || rc != SAREK_HIP_OK) return rc;
+  return launch_rowsum_fold(rs_planes, s.col_tiles, q.m, q.rowsum, q.st);
 }
 
-template <bool Bf16>
-int launch_rows(const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k, hipStream_t st) {
-  switch ((m + 15) / 16) {
-    case 1: return launch<Bf16, 1>(a, b, c, m, n, k, st);
-    case 2: return launch<Bf16, 2>(a, b, c, m, n, k, st);
-    case 3: return launch<Bf16, 3>(a, b, c, m, n, k, st);
-    default: return launch<Bf16, 4>(a, b, c, m, n, k, st);
+template <bool Bf16, bool Fused>
+int launch_rows(const Call &q) {
+  const Shape s = shape_of(q.m, q.n, q.k, Fused);
+  switch (s.mt) {
+    case 1: return launch<Bf16, Fused, 1>(q, s);
+    case 2: return launch<Bf16, Fused, 2>(q, s);
+    case 3: return launch<Bf16, Fused, 3>(q, s);
+    default: return launch<Bf16, Fused, 4>(q, s);
   }
 }
 
 }  // namespace
 
-// Whether this kernel takes a product.  It can: up to 64 rows (four row tiles' sums fill the registers), rows of B of at
-// least a pair of elements (load_end counts on it), K of at least one step, 32 rows of B and all of A within the 32-bit load offsets.  Up to 16 rows it always should.  Beyond, a workgroup's
+// Whether this kernel can take a product: rows of B of at least a pair of elements (load_end counts on it), K of at least
+// one step, 32 rows of B and 64 of A within the 32-bit load offsets.
+bool gemm16_rows_serves(int m, int n, int k) {
+  return m >= 1 && n >= 2 && k >= kStepK && static_cast<int64_t>(n + kCols) * 2 * kStepK < 0x7FFFFFFF &&
+         static_cast<int64_t>(kTileRows) * k * 2 < 0x7FFFFFFF && shape_of(m, n, k, false).tiles * 64 < 0x7FFFFFFF;
+}
+
+// Whether it should.  Up to 16 rows always.  To 64 a workgroup's
 // sums through LDS cost it 0.5 us per 16 rows and its registers leave room for one workgroup per CU, so short K and more
-// column tiles than CUs belong to the 128 x 128 tile unless that one would need its odd-N launch (us, 128 tile / here):
+// column tiles than CUs belong to the 128 x 128 tile unless N is odd (us, 128 tile / here):
 //   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
 //   48 x 4096 x 256 6.2 / 6.1, 48 x 4096 x 1024 10.2 / 9.4, 48 x 40000 x 1024 23.0 / 26.4, 48 x 40001 x 1024 35.3 / 33.4
 //   64 x 4096 x 256 6.4 / 7.2, 64 x 4096 x 1024 10.5 / 10.5, 64 x 4096 x 4096 17.3 / 15.6, 64 x 40001 x 1024 36.3 / 37.0
-bool gemm16_rows_serves(int m, int n, int k) {
-  if (m > kRowsMax || n < 2 || k < kStepK || static_cast<int64_t>(n + kCols) * 2 * kStepK >= 0x7FFFFFFF ||
-      static_cast<int64_t>(m) * k * 2 >= 0x7FFFFFFF)
-    return false;
-  const bool odd = n % 2 != 0, one_round = (n + kCols - 1) / kCols <= compute_units();
-  switch ((m + 15) / 16) {
-    case 1: return true;
-    case 2: return odd || one_round;
-    case 3: return one_round ? odd || k >= 512 : odd && k >= 1024;
-    default: return one_round && (odd || k >= 1024);
+// Beyond 64 rows, and with the fused epilogue at any number, where its tiles fit the CUs in one round (882 x 2401 x 4259,
+// 266 tiles: 50 us on the other tile, 108 here), at least half of the waves have a step, and its time is below the 128 x 128
+// tile's by both estimates.  They were read off 50 drawn products (up to 20 % and a microsecond apart from them, the
+// better kernel taken on 45, at most 8 % lost on the others): a step costs by how A's and B's rows lie, on 16 bytes, on 4, on 2.
+// `other`: what the tiled kernel is estimated at.
+bool gemm16_rows_pays(int m, int n, int k, bool fused, double other) {
+  if (m <= kTileRows && !fused) {
+    const bool odd = n % 2 != 0, one_round = (n + kCols - 1) / kCols <= compute_units();
+    switch ((m + 15) / 16) {
+      case 1: return true;
+      case 2: return odd || one_round;
+      case 3: return one_round ? odd || k >= 512 : odd && k >= 1024;
+      default: return one_round && (odd || k >= 1024);
+    }
   }
+  const Shape s = shape_of(m, n, k, fused);
+  if (s.tiles > compute_units() || 2 * s.steps < kWaves) return false;
+  const int splits = rows_splits_for(s, n, k);
+  const bool on16 = k % 8 == 0 && n % 8 == 0;
+  const double step = (on16 ? 0.055 : k % 2 == 0 && n % 2 == 0 ? 0.07 : 0.12) * s.mt;
+  const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
+  const double here = (on16 ? 6.0 : 4.5) + rounds * s.steps / splits * step +
+                      (splits > 1 ? 2.5 + 0.15 * splits + 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0);
+  return here < other;
 }
 
-int gemm16_rows_k_splits(int m, int n, int k) { return rows_splits_for(m, n, k); }
+int gemm16_rows_k_splits(int m, int n, int k) { return rows_splits_for(shape_of(m, n, k, false), n, k); }
 
 int launch_gemm16_rows(bool bf16, const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k, hipStream_t st) {
-  return bf16 ? launch_rows<true>(a, b, c, m, n, k, st) : launch_rows<false>(a, b, c, m, n, k, st);
+  const Call q{a, b, c, nullptr, nullptr, m, n, k, st};
+  return bf16 ? launch_rows<true, false>(q) : launch_rows<false, false>(q);
+}
+
+int launch_gemm16_rows_fused(const uint16_t *a, const uint16_t *b, const float *bias, float *c, float *rowsum, int m, int n,
+                             int k, hipStream_t st) {
+  return launch_rows<false, true>({a, b, c, bias, rowsum, m, n, k, st});
 }
 
 }  // namespace sarek_hip

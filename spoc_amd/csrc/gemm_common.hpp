@@ -40,10 +40,16 @@ double gemm_f32_direct_estimate(int m, int n, int k, int row_blocks, int waves, 
 int launch_gemm_f32_direct(const float *a, const float *b, float *c, int m, int n, int k, int row_blocks, int waves,
                            int splits, hipStream_t st);
 
-// 16-bit products of at most 64 rows (gemm16_rows.hip)
+// 16-bit products in tiles of at most 64 rows, straight from memory to registers (gemm16_rows.hip)
 bool gemm16_rows_serves(int m, int n, int k);
+bool gemm16_rows_pays(int m, int n, int k, bool fused, double other);
 int gemm16_rows_k_splits(int m, int n, int k);
 int launch_gemm16_rows(bool bf16, const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k, hipStream_t st);
+int launch_gemm16_rows_fused(const uint16_t *a, const uint16_t *b, const float *bias, float *c, float *rowsum, int m, int n,
+                             int k, hipStream_t st);
+// Row sums of the fused products (gemm16.hip): zeroes, and rowsum[r] = planes[r] + planes[m + r] + ... in plane order
+int launch_zero_f32(float *p, int n, hipStream_t st);
+int launch_rowsum_fold(const float *planes, int count, int m, float *rowsum, hipStream_t st);
 
 namespace {
 

@@ -750,6 +750,46 @@ def test_gemm16_few_rows(hip, torch_cuda, kind, m, n, k):
             hip.set_tunable("gemm16.rows_splits", 0)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 2, 32), (16, 128, 257), (33, 130, 65), (64, 255, 520), (65, 2, 33), (81, 257, 1001),
+                                   (128, 384, 256), (129, 129, 700), (300, 131, 4099)])
+def test_gemm16_few_rows_tiles_and_epilogue(hip, torch_cuda, m, n, k):
+    """Several row tiles of the few-rows kernel, whole and ragged, with K whole and in pieces, and its fused form: operands,
+    bias and results at odd offsets between NaNs and guard values.  Bounds as above; a row sum adds n terms more."""
+    torch = torch_cuda
+    torch.manual_seed(m * n + k)
+    nan = lambda count, dt: torch.full((count + 64,), float("nan"), device="cuda").to(dt)  # noqa: E731
+    buf_a, buf_b, buf_bias = nan(m * k, torch.float16), nan(k * n, torch.float16), nan(n, torch.float32)
+    for off in (0, 3):
+        da, db, bias = buf_a[off:off + m * k].view(m, k), buf_b[off:off + k * n].view(k, n), buf_bias[off:off + n]
+        da.copy_((torch.randn(m, k, device="cuda") * 0.02).half())
+        db.copy_((torch.randn(k, n, device="cuda") * 0.02).half())
+        bias.copy_(torch.randn(n, device="cuda") * 0.01)
+        ref, size = da.double() @ db.double(), da.double().abs() @ db.double().abs()
+        fused, fused_size = (ref + bias.double()).relu(), size + bias.double().abs()
+        try:
+            hip.set_tunable("gemm16.rows", 2)
+            assert hip.gemm16_tile(m, n, k) == 64
+            for splits in (0, 1, 3):
+                hip.set_tunable("gemm16.rows_splits", splits)
+                guards = [torch.full((count + 64,), 7.0, device="cuda") for count in (m * n, m * n, m)]
+                c, y, rs = (g[32 + off:32 + off + g.numel() - 64] for g in guards)
+                c, y = c.view(m, n), y.view(m, n)
+                hip.gemm_f16(da, db, out=c)
+                hip.check(hip.lib.sarek_hip_gemm_f16_bias_relu_rowsum(
+                    da.data_ptr(), db.data_ptr(), bias.data_ptr(), y.data_ptr(), rs.data_ptr(), m, n, k,
+                    torch.cuda.current_stream().cuda_stream))
+                for g in guards:
+                    assert bool((g[:32 + off] == 7).all()) and bool((g[g.numel() - 32 + off:] == 7).all())
+                assert bool(((c.double() - ref).abs() <= k * 2.0 ** -24 * size).all()), (off, splits)
+                assert bool(((y.double() - fused).abs() <= (k + 1) * 2.0 ** -24 * fused_size).all()), (off, splits)
+                assert bool(((rs.double() - fused.sum(1)).abs() <= (k + n) * 2.0 ** -24 * fused_size.sum(1)).all())
+                y2, rs2 = hip.gemm_f16_bias_relu_rowsum(da, db, bias)
+                assert torch.equal(y, y2) and torch.equal(rs, rs2), "the same bits on every run"
+        finally:
+            hip.set_tunable("gemm16.rows", 0)
+            hip.set_tunable("gemm16.rows_splits", 0)
+
+
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(70, 1, 100), (300, 3, 65), (200, 129, 328), (513, 255, 4107), (4096, 4097, 72), (130, 4097, 2056)])
 def test_gemm16_odd_columns(hip, torch_cuda, kind, m, n, k):
