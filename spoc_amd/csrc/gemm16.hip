@@ -465,11 +465,12 @@ __device__ __forceinline__ float widen16(uint16_t bits) {
 // 2048 x 50257 x 1024's 282 and 20 of 64 x 4097 x 4096's 41.)
 template <bool Bf16, int TROWS>
 __device__ __forceinline__ void last_products(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, int M, int N,
-                                              int K, int m0, float *scratch) {
+                                              int K, int ld, int m0, float *scratch) {
   __syncthreads();   // every wave has left the K loop: the LDS ring is free
   if (threadIdx.x < TROWS) {
     const int row = min(m0 + static_cast<int>(threadIdx.x), M - 1);
-    scratch[threadIdx.x] = widen16<Bf16>(A[static_cast<int64_t>(row) * K + K - 1]) * widen16<Bf16>(B[static_cast<int64_t>(K) * N - 1]);
+    scratch[threadIdx.x] = widen16<Bf16>(A[static_cast<int64_t>(row) * K + K - 1]) *
+                           widen16<Bf16>(B[static_cast<int64_t>(K - 1) * ld + N - 1]);
   }
   __syncthreads();
 }
@@ -802,7 +803,7 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // drain the (redundant) tail DMA before the LDS is released
   float *scratch = reinterpret_cast<float *>(lds_ring<10, A_BYTES_S>);
   const bool add_last = Ragged && (N & 1) != 0 && n0 + BN >= N;
-  if (add_last) last_products<Bf16, BM>(A, B, M, N, K, m0, scratch);
+  if (add_last) last_products<Bf16, BM>(A, B, M, N, K, ld, m0, scratch);
   epilogue16<Epi, 8, 4, Ragged>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0, wm, wn,
                   n0 + wn * 64, l16, g, scratch, add_last);
   if (kMeasureBuild && probe && tid == 0) {
@@ -1229,7 +1230,7 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // drain the (redundant) tail DMA before the LDS is released
   float *scratch = reinterpret_cast<float *>(lds_ring<30, A_BYTES_S>);
   const bool add_last = Ragged && (N & 1) != 0 && n0 + SBN >= N && k0 + k_len == K;
-  if (add_last) last_products<Bf16, SBM>(A, B, M, N, K, m0, scratch);
+  if (add_last) last_products<Bf16, SBM>(A, B, M, N, K, ld, m0, scratch);
   epilogue16<Epi, 4, WN, Ragged>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0,
                          wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
   if (kMeasureBuild && probe && tid == 0) {
@@ -1321,6 +1322,27 @@ inline bool small_tile_wins(int m, int n) {
   const double cost_large = static_cast<double>((large + cus - 1) / cus);
   const double cost_small = 0.65 * static_cast<double>((small + 2 * cus - 1) / (2 * cus));
   return cost_small < 0.9 * cost_large;
+}
+
+// How many of n columns the 256 x 256 tiles take when the last round of workgroups would hold few of them: the tile columns
+// of whole rounds; the rest goes to the 128 x 128 tile in a second launch.  n where that does not pay.  The results are the
+// same bits: both kernels add an element's products in the same order.
+// A round of a few large tiles takes nearly as long as a full one (a CU works its tile alone); as small tiles, one to a CU,
+// the same columns take half of that.  Measured, us, without and with the cut: 2048 rows, 8448 / 9216 / 10240 columns
+// (32 / 128 / 256 small tiles) K = 512 35.5 -> 32.1 / 35.8 -> 33.4 / 38.5 -> 35.2, K = 1024 53.3 -> 45.6 / 53.9 -> 46.9 /
+// 56.7 -> 48.7, K = 4096 157 -> 134 / 169 -> 141 / 172 -> 146; 4096 x 4100 x 4096 187 -> 155; fused 4096 x 4352 x 4096
+// 169 -> 140; 2048 x 50257 x 1024 274 -> 264.  From there on two small tiles share a CU and nothing is left to gain: 11264
+// columns 39.7 -> 39.6, 56.8 -> 55.2, 174 -> 175; 12288 40.0 -> 40.1, 59.5 -> 58.4, 177 -> 181.
+// gemm16.cut: 0 = this rule, 1 = never, s >= 2: a rest of up to s small tiles.
+inline int whole_round_columns(int m, int n) {
+  const int64_t asked = tunable("gemm16.cut", 0);
+  if (asked == 1 || tunable("gemm16.tile", 0) != 0) return n;
+  const int cus = compute_units();
+  const int64_t tiles_m = ceil_div(m, 256), tiles_n = ceil_div(n, 256), over = tiles_m * tiles_n % cus;
+  const int64_t columns = tiles_n - ceil_div(over, tiles_m);
+  if (over == 0 || columns < 1) return n;
+  const int64_t rest = ceil_div(m, 128) * ceil_div(n - columns * 256, 128);
+  return rest <= (asked >= 2 ? asked : cus) ? static_cast<int>(columns * 256) : n;
 }
 
 // Column N-1 of C alone, one wave per row, with the same epilogue: N = 1, and an N of whole tiles and one column whose
@@ -1536,8 +1558,9 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   // stream capture, past the sixteenth stream, planes beyond the block's size) adds with atomicAdd in arrival order.
   float *planes = nullptr;
   int n_planes = 0;
+  const int cut = tiled && tile_choice == 256 && nm > 0 && !(kMeasureBuild && clock_probe(1)) ? whole_round_columns(m, nm) : nm;
   if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
-    n_planes = tiled ? (nm + tile_choice - 1) / tile_choice + (n - nm) : (n + 63) / 64;
+    n_planes = tiled ? (cut + tile_choice - 1) / tile_choice + (nm - cut + 127) / 128 + (n - nm) : (n + 63) / 64;
     if (static_cast<int64_t>(n_planes) * m * 4 <= static_cast<int64_t>(kSplitWorkspaceBytes)) planes = splitk_workspace(st);
     if (!planes) {
       const int rc = launch_zero_f32(rowsum, m, st);
@@ -1588,24 +1611,36 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
       rc = check_launch("gemm16 kernel launch");
     }
   } else if (nm > 0) {
-    const int tiles_m = (m + BM - 1) / BM, tiles_n = (nm + BN - 1) / BN;
+    const int tiles_m = (m + BM - 1) / BM, tiles_n = (cut + BN - 1) / BN;
     unsigned long long *probe = clock_probe(static_cast<int64_t>(tiles_m) * tiles_n);
 #ifdef SAREK_HIP_MEASURE
     if (Epi == EPI_STORE && !ragged && tunable("gemm16.waves", 8) == 4) {
-      hipLaunchKernelGGL((gemm16_m16w4_kernel<Bf16>), dim3(tiles_m * tiles_n), dim3(256), 0, st, a, b, c, m, nm, k, tiles_m,
+      hipLaunchKernelGGL((gemm16_m16w4_kernel<Bf16>), dim3(tiles_m * tiles_n), dim3(256), 0, st, a, b, c, m, cut, k, tiles_m,
                          tiles_n, remap);
     } else if (!ragged && tunable("gemm16.barriers", 2) == 1) {
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c,
-                         bias, rowsum, m, nm, k, tiles_m, tiles_n, remap, probe, n, planes);
+                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
     } else
 #endif
     if (ragged)
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c, bias,
-                         rowsum, m, nm, k, tiles_m, tiles_n, remap, probe, n, planes);
+                         rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
     else
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c, bias,
-                         rowsum, m, nm, k, tiles_m, tiles_n, remap, probe, n, planes);
+                         rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
     rc = check_launch("gemm16 kernel launch");
+    if (rc == SAREK_HIP_OK && cut < nm) {
+      const int rest = nm - cut, sm = (m + 127) / 128, sn = (rest + 127) / 128;
+      float *const rest_planes = planes ? planes + static_cast<int64_t>(tiles_n) * m : nullptr;
+      const float *const rest_bias = Epi == EPI_BIAS_RELU_ROWSUM ? bias + cut : nullptr;
+      if (ragged)
+        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, true>), dim3(sm * sn), dim3(256), 0, st, a, b + cut, c + cut,
+                           rest_bias, rowsum, m, rest, k, sm, sn, remap, nullptr, k, nullptr, n, rest_planes);
+      else
+        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, false>), dim3(sm * sn), dim3(256), 0, st, a, b + cut, c + cut,
+                           rest_bias, rowsum, m, rest, k, sm, sn, remap, nullptr, k, nullptr, n, rest_planes);
+      rc = check_launch("gemm16 kernel launch");
+    }
   }
   if (rc != SAREK_HIP_OK) return rc;
   if (nm != n) {
