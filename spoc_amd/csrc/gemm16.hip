@@ -499,11 +499,20 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
     cok[j] = col < N;
     bj[j] = (Epi == EPI_BIAS_RELU_ROWSUM && cok[j]) ? bias[col] : 0.f;
   }
+  // a branch of its own: selects in the loop below cost every ragged product 3 % at 2880 x 42688 x 431
+  if (Ragged && add_last) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      const f32x4_t last = *reinterpret_cast<const f32x4_t *>(scratch + wm * WROWS + i * 16 + 4 * g);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] = col0 + j * 16 + l16 == N - 1 ? acc[i][j][r] + last[r] : acc[i][j][r];
+    }
+  }
   float rs[NV];
 #pragma unroll
   for (int i = 0; i < TI; ++i) {
-    f32x4_t last = {0.f, 0.f, 0.f, 0.f};
-    if (Ragged && add_last) last = *reinterpret_cast<const f32x4_t *>(scratch + wm * WROWS + i * 16 + 4 * g);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = row0 + i * 16 + 4 * g + r;
@@ -511,7 +520,6 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         float v = acc[i][j][r];
-        if (Ragged) v = add_last && col0 + j * 16 + l16 == N - 1 ? v + last[r] : v;
         if (Epi == EPI_BIAS_RELU_ROWSUM) {
           v += bj[j];
           v = v > 0.f ? v : 0.f;
