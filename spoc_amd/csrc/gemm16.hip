@@ -463,14 +463,23 @@ __device__ __forceinline__ float widen16(uint16_t bits) {
 // and in the workgroups of the last tile column (those that take the last k) epilogue16 adds what is missing: one product
 // per row of the tile, through LDS.  (A kernel of its own for the last column, a wave per row, took 9 us of
 // 2048 x 50257 x 1024's 282 and 20 of 64 x 4097 x 4096's 41.)
+// An infinite A[row][K-1] has met the zero: its accumulator is NaN whatever the row holds, so the sum from k0 on is formed
+// here, serially, and takes the accumulator's place.  scratch: TROWS addends, then per row whether it replaces the
+// accumulator (1) or is added to it (0).
 template <bool Bf16, int TROWS>
 __device__ __forceinline__ void last_products(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B, int M, int N,
-                                              int K, int ld, int m0, float *scratch) {
+                                              int K, int ld, int m0, int k0, float *scratch) {
   __syncthreads();   // every wave has left the K loop: the LDS ring is free
   if (threadIdx.x < TROWS) {
-    const int row = min(m0 + static_cast<int>(threadIdx.x), M - 1);
-    scratch[threadIdx.x] = widen16<Bf16>(A[static_cast<int64_t>(row) * K + K - 1]) *
-                           widen16<Bf16>(B[static_cast<int64_t>(K - 1) * ld + N - 1]);
+    const uint16_t *a = A + static_cast<int64_t>(min(m0 + static_cast<int>(threadIdx.x), M - 1)) * K;
+    const uint16_t *b = B + N - 1;
+    const float last = widen16<Bf16>(a[K - 1]);
+    float sum = last * widen16<Bf16>(b[static_cast<int64_t>(K - 1) * ld]);
+    const bool replace = __builtin_isinf(last);
+    if (replace)
+      for (int k = k0; k < K - 1; ++k) sum += widen16<Bf16>(a[k]) * widen16<Bf16>(b[static_cast<int64_t>(k) * ld]);
+    scratch[threadIdx.x] = sum;
+    scratch[TROWS + threadIdx.x] = replace ? 1.f : 0.f;
   }
   __syncthreads();
 }
@@ -504,10 +513,12 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
 #pragma unroll
     for (int i = 0; i < TI; ++i) {
       const f32x4_t last = *reinterpret_cast<const f32x4_t *>(scratch + wm * WROWS + i * 16 + 4 * g);
+      const f32x4_t only = *reinterpret_cast<const f32x4_t *>(scratch + TROWS + wm * WROWS + i * 16 + 4 * g);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i][j][r] = col0 + j * 16 + l16 == N - 1 ? acc[i][j][r] + last[r] : acc[i][j][r];
+        for (int r = 0; r < 4; ++r)
+          if (col0 + j * 16 + l16 == N - 1) acc[i][j][r] = (only[r] != 0.f ? 0.f : acc[i][j][r]) + last[r];
     }
   }
   float rs[NV];
@@ -811,7 +822,7 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // drain the (redundant) tail DMA before the LDS is released
   float *scratch = reinterpret_cast<float *>(lds_ring<10, A_BYTES_S>);
   const bool add_last = Ragged && (N & 1) != 0 && n0 + BN >= N;
-  if (add_last) last_products<Bf16, BM>(A, B, M, N, K, ld, m0, scratch);
+  if (add_last) last_products<Bf16, BM>(A, B, M, N, K, ld, m0, 0, scratch);
   epilogue16<Epi, 8, 4, Ragged>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0, wm, wn,
                   n0 + wn * 64, l16, g, scratch, add_last);
   if (kMeasureBuild && probe && tid == 0) {
@@ -1238,7 +1249,7 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // drain the (redundant) tail DMA before the LDS is released
   float *scratch = reinterpret_cast<float *>(lds_ring<30, A_BYTES_S>);
   const bool add_last = Ragged && (N & 1) != 0 && n0 + SBN >= N && k0 + k_len == K;
-  if (add_last) last_products<Bf16, SBM>(A, B, M, N, K, ld, m0, scratch);
+  if (add_last) last_products<Bf16, SBM>(A, B, M, N, K, ld, m0, k0, scratch);
   epilogue16<Epi, 4, WN, Ragged>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0,
                          wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
   if (kMeasureBuild && probe && tid == 0) {

@@ -844,6 +844,36 @@ def test_gemm16_odd_columns(hip, torch_cuda, kind, m, n, k):
         hip.set_tunable("gemm16.split_k", 0)
 
 
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+@pytest.mark.parametrize("m,n,k,split", [(300, 129, 200, 0), (300, 129, 333, 3), (16, 129, 200, 0), (1024, 16379, 136, 0)])
+def test_gemm16_odd_columns_infinities(hip, torch_cuda, kind, m, n, k, split):
+    """Infinities and NaN in the last k, whose products with the last element of B the tiled kernels add after the loop:
+    the same infinities and NaN as the float64 product of the same values."""
+    torch = torch_cuda
+    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    torch.manual_seed(m + n * k)
+    inf, nan = float("inf"), float("nan")
+    da, db = torch.randn(m, k, device="cuda"), torch.randn(k, n, device="cuda")
+    da[:5, k - 1] = torch.tensor([inf, -inf, inf, nan, 0.0], device="cuda")
+    da[2, k - 2] = nan
+    for last in (1.5, -2.0, 0.0, inf):
+        db[k - 1, n - 1] = last
+        a, b = da.to(dt), db.to(dt)
+        ref = a.double() @ b.double()
+        hip.set_tunable("gemm16.split_k", split)
+        try:
+            c = (hip.gemm_bf16 if kind == "bf16" else hip.gemm_f16)(a, b).double()
+            y = hip.gemm_f16_bias_relu_rowsum(a, b, torch.zeros(n, device="cuda"))[0].double() if kind == "f16" else None
+        finally:
+            hip.set_tunable("gemm16.split_k", 0)
+        odd = ~ref.isfinite()
+        assert torch.equal(c.isnan(), ref.isnan()) and torch.equal(c.isinf(), ref.isinf()), last
+        assert torch.equal(c[ref.isinf()], ref[ref.isinf()])
+        assert bool((c - ref)[~odd].abs().max() <= k * 2.0 ** -24 * (a[5:].double().abs() @ b[:, :-1].double().abs()).max())
+        if y is not None:
+            assert torch.equal(y.isinf(), ref == inf) and bool((y[ref.isnan()] == 0).all())   # ReLU of NaN is 0
+
+
 @pytest.mark.parametrize("variant", [0, 18, 14, 24])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (16, 64, 16), (17, 65, 17), (15, 63, 31), (33, 3, 1001), (2, 1, 70), (32, 132, 256),
                                    (70, 200, 4099), (129, 70, 530)])
