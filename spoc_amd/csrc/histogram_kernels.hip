@@ -264,6 +264,25 @@ int compute_units() {
   return cus;
 }
 
+// Tile of the scatter by key count (the numbers of radix_scatter.tile).  A tile costs its latency, and what its global
+// atomics wait for those of the others, whether it is the only one of its CU or not; so up to two rounds of the chip the
+// tile is the smallest (12 to 32 keys a thread, fewer gain nothing) that leaves no tile for another round.  Beyond, 16 keys:
+// two workgroups per CU cover each other's latency; from 2^27 keys on 32 keys, where the atomics are most of it
+// (2^28 keys 648 us with 16, 573 with 32).  Measured, before (512 x 16 below 2^22 keys, 1024 x 16 from there) and now, us a
+// launch and a 1 KiB copy of 3.6 us: 10007 keys 10.2 / 9.3, 1000003 10.3 / 9.6, 2560000 15.7 / 13.1, 3200001 17.2 / 14.5,
+// 4300003 18.5 / 16.9, 6000000 20.7 / 19.3, 8000000 25.1 / 23.1, 10000019 30.9 / 28.6, 13000000 39.3 / 34.2,
+// 16000000 43.5 / 39.0; 22 10^6 keys 54.2 with 16, 53.5 with 32, 50 10^6 94.2 and 109.  Keys of one value (10^7) 56.9 / 54.3,
+// of 16 values 25.1 / 26.7.
+int scatter_shape(int64_t n) {
+  constexpr int kShapes[] = {5, 2, 6, 7, 8, 4};   // 12, 16, 20, 24, 28, 32 keys a thread
+  const int64_t round = static_cast<int64_t>(compute_units()) * 1024;
+  if (n <= 2 * 32 * round) {
+    const int64_t keys = ceil_div(n, n <= 32 * round ? round : 2 * round);
+    return kShapes[keys <= 12 ? 0 : (keys - 9) / 4];
+  }
+  return n >= (int64_t{1} << 27) ? 4 : 2;
+}
+
 template <class Bin>
 int launch(int *histogram, const int *keys, int64_t n, int bins, Bin bin, hipStream_t st) {
   // one workgroup per 64 KiB of keys until every CU has `per_cu` of them
@@ -323,16 +342,17 @@ int sarek_hip_radix_scatter_i32(int32_t *out, int64_t out_len, int32_t *counters
     return fail(SAREK_HIP_E_INVALID_ARG, "radix scatter: mask %d outside 0..%d", mask, kBins - 1);
   if (n == 0) return SAREK_HIP_OK;
   hipStream_t st = as_stream(stream);
-  // Measured on MI355X: 16384-key tiles from about 4M keys on (half the global atomics of 8192-key tiles:
-  // 95 against 142 us at 50M keys), 8192-key tiles below (more workgroups than CUs sooner), 32768-key tiles
-  // from 2^27 keys on (573 against 648 us at 2^28 keys; 111 against 100 us at 50M).
   int64_t shape = tunable("radix_scatter.tile", 0);
-  if (shape == 0) shape = n >= (int64_t{1} << 27) ? 4 : n >= (int64_t{1} << 22) ? 2 : 1;
+  if (shape == 0) shape = scatter_shape(n);
   switch (shape) {
     case 1: return launch_scatter<512, 16>(out, out_len, counters, keys, n, shift, mask, st);
     case 2: return launch_scatter<1024, 16>(out, out_len, counters, keys, n, shift, mask, st);
     case 3: return launch_scatter<512, 32>(out, out_len, counters, keys, n, shift, mask, st);
     case 4: return launch_scatter<1024, 32>(out, out_len, counters, keys, n, shift, mask, st);
+    case 5: return launch_scatter<1024, 12>(out, out_len, counters, keys, n, shift, mask, st);
+    case 6: return launch_scatter<1024, 20>(out, out_len, counters, keys, n, shift, mask, st);
+    case 7: return launch_scatter<1024, 24>(out, out_len, counters, keys, n, shift, mask, st);
+    case 8: return launch_scatter<1024, 28>(out, out_len, counters, keys, n, shift, mask, st);
     default: return launch_scatter<512, 16>(out, out_len, counters, keys, n, shift, mask, st);
   }
 }

@@ -172,6 +172,25 @@ def test_radix_scatter_tile_shapes(hip, torch_cuda, oracle, n, shape):
     assert check_scatter(out.cpu().numpy(), counters.cpu().numpy(), keys, n, starts, shift, mask, oracle) == 0
 
 
+@pytest.mark.parametrize("n,shape", [(12288, 5), (12289, 5), (20479, 6), (40961, 6), (24577, 7), (57343, 8), (1, 0), (3, 0),
+                                     (256 * 12288 + 1, 0), (256 * 32768, 0), (256 * 32768 + 1, 0), (512 * 32768 + 1, 0)])
+def test_radix_scatter_tiles_that_fit_the_rounds(hip, torch_cuda, n, shape):
+    """Tiles of 12, 20, 24 and 28 keys a thread at whole tiles and one key more or less, and key counts at the edges of the
+    rule that chooses: the keys of an 8-bit digit sorted, the counters at their ends, nothing past the output."""
+    torch = torch_cuda
+    torch.manual_seed(n)
+    keys = torch.randint(0, 256, (n,), device="cuda", dtype=torch.int32)
+    counts = torch.bincount(keys, minlength=256)
+    ends = counts.cumsum(0).int()
+    counters, out = ends - counts.int(), torch.full((n + 64,), -1, dtype=torch.int32, device="cuda")
+    hip.set_tunable("radix_scatter.tile", shape)
+    try:
+        hip.radix_scatter(keys, out, counters, 0, 255)
+    finally:
+        hip.set_tunable("radix_scatter.tile", 0)
+    assert torch.equal(out[:n], keys.sort().values) and torch.equal(counters, ends) and bool((out[n:] == -1).all())
+
+
 def test_radix_scatter_skips_positions_outside_the_output(hip, torch_cuda, oracle):
     """Counters that start 40 too high push the last keys of the last digit past the output: those
     stores are dropped (the slots behind the output keep their contents), the counters still advance."""
