@@ -154,8 +154,8 @@ def test_radix_scatter_sizes(hip, torch_cuda, oracle, n, shift, mask):
 
 @pytest.mark.parametrize("n,shape", [(100_003, 2), (100_003, 3), (100_003, 4), (40_000, 4), ((1 << 22) + 4099, 0)])
 def test_radix_scatter_tile_shapes(hip, torch_cuda, oracle, n, shape):
-    """Every tile shape of the kernel (8192 to 32768 keys; 0 = the library's choice, which from 2^22 keys on
-    is the 16384-key tile), ragged last tiles included."""
+    """Every tile shape of the kernel (8192 to 32768 keys; 0 = the library's choice, just past 2^22 keys
+    the 20480-key tile), ragged last tiles included."""
     torch = torch_cuda
     shift, mask = 8, 255
     keys = keys_of(n, shape, 1, 2**31 - 1)
