@@ -458,6 +458,24 @@ __device__ __forceinline__ float widen16(uint16_t bits) {
   else return static_cast<float>(__builtin_bit_cast(_Float16, bits));
 }
 
+// Zeroes the first `count` (1 .. 7) of the eight elements this lane brought to each of its places of an A stage, if `mine`.
+// The caller has waited for the transfers and passes a barrier afterwards: no other wave reads the stage in between.  Once
+// a tile; a mask on the fragments instead would be in every turn of the K loop.
+template <int DA, int NWAVES>
+__device__ __forceinline__ void clear_piece_heads(char *sa, int wave, int lane, bool mine, int count) {
+  if (mine) {
+    u32x4 keep;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) keep[d] = count <= 2 * d ? 0xFFFFFFFFu : count == 2 * d + 1 ? 0xFFFF0000u : 0u;
+#pragma unroll
+    for (int i = 0; i < DA; ++i) {
+      u32x4 *piece = reinterpret_cast<u32x4 *>(sa + (wave + NWAVES * i) * 1024 + lane * 16);
+      *piece = *piece & keep;
+    }
+  }
+  wait_lds();
+}
+
 // The products A[row][K-1] B[K-1][N-1] of an odd N.  B is fetched in pairs of 16-bit elements from even columns on, and the
 // pair that holds B[K-1][N-1] ends two bytes past B: the buffer range ends right in front of it, its lanes bring zeros,
 // and in the workgroups of the last tile column (those that take the last k) epilogue16 adds what is missing: one product
@@ -639,17 +657,19 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   // Ragged: K need not fill the last A stage.  A lane whose offset lies outside the buffer resource's range brings
   // zeros into LDS, so k that must not count are a per-lane choice between the usual offset and one past the range.
   // From one whole stage on (K >= 64) the last stage is moved back to end at K: its A pieces then hold nothing but
-  // elements of their own rows, at whatever alignment, and the B rows it shares with the stage before it are the
-  // lanes sent out of range, in the first of its two slabs and, past 32 shared rows, in the second.  Below one stage
-  // (K % 8 == 0) the A pieces and B rows past K are.  A lane's k piece is the same for all its transfers of a stage
-  // (rows 16 apart share the swizzle).
+  // elements of their own rows, at whatever alignment, and the k it shares with the stage before it are sent out of
+  // range, in A as in B: an infinity times the other's zero would be NaN.  Of B they are rows of the first of the
+  // stage's two slabs and, past 32, of the second; of A whole pieces of 8, and the rest of a piece that holds shared k
+  // and others (shared_k % 8 != 0) is zeroed in LDS by the lane that brought it (clear_shared).  Below one stage
+  // (K % 8 == 0) the A pieces and B rows past K are out of range.  A lane's k piece is the same for all its transfers of
+  // a stage (rows 16 apart share the swizzle).
   const int nstages = (K + BKA - 1) / BKA;
   const bool move_last = Ragged && K >= BKA && K % BKA != 0;
   const int nslabs = move_last ? RA * nstages : (K + BKB - 1) / BKB;
   const int k_tail_a = K - (nstages - 1) * BKA, k_tail_b = K - (nslabs - 1) * BKB;   // single stage
   const int shared_k = nstages * BKA - K;                                               // moved stage
-  const bool a_lane_in_k = !Ragged || move_last ||
-                           (((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3) < k_tail_a;
+  const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3;
+  const bool a_lane_in_k = !Ragged || (move_last ? a_lane_k + 8 > shared_k : a_lane_k < k_tail_a);
   bool b_in_last[DB], b_in_prev[DB];   // the lanes that count in the last slab and in the one before it
 #pragma unroll
   for (int i = 0; i < DB; ++i) {
@@ -684,6 +704,10 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
 #pragma unroll
     for (int i = 0; i < DA; ++i)
       dma16(a_rsrc, (!Ragged || whole || a_lane_in_k) ? a_off[i] : kOutOfRange, a_so, sa + (wave + NWAVES * i) * 1024);
+  };
+  const int clear_stage = move_last && shared_k % 8 != 0 ? nstages - 1 : -1;
+  auto clear_shared = [&](char *sa) {
+    clear_piece_heads<DA, NWAVES>(sa, wave, lane, a_lane_k < shared_k && shared_k < a_lane_k + 8, shared_k % 8);
   };
   // B slabs are issued in order 0, 1, 2, ...: the source of the next one is a running pointer (two scalar adds per
   // slab instead of a 64-bit multiply) that stops at the last slab, which the tail of the K loop re-issues into
@@ -777,6 +801,8 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
     if constexpr (!HalfBarriers || I % RA == RA - 1) {
       __builtin_amdgcn_s_waitcnt(
           waitcnt_vm_lgkm0(dma_allowed_in_flight(I, RA, NA, NB, DA, DB, HalfBarriers ? 2 : 1)));
+      if constexpr (Ragged && I % RA == RA - 1)
+        if (s / RA + 1 == clear_stage) clear_shared(lds_ring<10 + ian, A_BYTES_S>);
       barrier_no_fence();
     }
     if constexpr (I % RA == RA - 1) issue_a(lds_ring<10 + ia, A_BYTES_S>, s / RA + NA);
@@ -1095,17 +1121,19 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   // Ragged: K need not fill the last A stage.  A lane whose offset lies outside the buffer resource's range brings
   // zeros into LDS, so k that must not count are a per-lane choice between the usual offset and one past the range.
   // From one whole stage on (K >= 64) the last stage is moved back to end at K: its A pieces then hold nothing but
-  // elements of their own rows, at whatever alignment, and the B rows it shares with the stage before it are the
-  // lanes sent out of range, in the first of its two slabs and, past 32 shared rows, in the second.  Below one stage
-  // (K % 8 == 0) the A pieces and B rows past K are.  A lane's k piece is the same for all its transfers of a stage
-  // (rows 16 apart share the swizzle).
+  // elements of their own rows, at whatever alignment, and the k it shares with the stage before it are sent out of
+  // range, in A as in B: an infinity times the other's zero would be NaN.  Of B they are rows of the first of the
+  // stage's two slabs and, past 32, of the second; of A whole pieces of 8, and the rest of a piece that holds shared k
+  // and others (shared_k % 8 != 0) is zeroed in LDS by the lane that brought it (clear_shared).  Below one stage
+  // (K % 8 == 0) the A pieces and B rows past K are out of range.  A lane's k piece is the same for all its transfers of
+  // a stage (rows 16 apart share the swizzle).
   const int nstages = (k_len + BKA - 1) / BKA;
   const bool move_last = Ragged && k_len >= BKA && k_len % BKA != 0;
   const int nslabs = move_last ? RA * nstages : (k_len + BKB - 1) / BKB;
   const int k_tail_a = k_len - (nstages - 1) * BKA, k_tail_b = k_len - (nslabs - 1) * BKB;   // single stage
   const int shared_k = nstages * BKA - k_len;                                               // moved stage
-  const bool a_lane_in_k = !Ragged || move_last ||
-                           (((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3) < k_tail_a;
+  const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3;
+  const bool a_lane_in_k = !Ragged || (move_last ? a_lane_k + 8 > shared_k : a_lane_k < k_tail_a);
   bool b_in_last[DB], b_in_prev[DB];   // the lanes that count in the last slab and in the one before it
 #pragma unroll
   for (int i = 0; i < DB; ++i) {
@@ -1136,6 +1164,10 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
 #pragma unroll
     for (int i = 0; i < DA; ++i)
       dma16(a_rsrc, (!Ragged || whole || a_lane_in_k) ? a_off[i] : kOutOfRange, a_so, sa + (wave + NWAVES * i) * 1024);
+  };
+  const int clear_stage = move_last && shared_k % 8 != 0 ? nstages - 1 : -1;
+  auto clear_shared = [&](char *sa) {
+    clear_piece_heads<DA, NWAVES>(sa, wave, lane, a_lane_k < shared_k && shared_k < a_lane_k + 8, shared_k % 8);
   };
   // B slabs go out in order; the source is a running pointer that stops at the last slab (the tail of the K loop
   // re-issues it into stages nobody reads any more, so the count of transfers in flight keeps its pattern)
@@ -1210,6 +1242,8 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     mfma_range(std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{}, af[I & 1], bf[I & 1]);
     spread(std::integral_constant<int, DB>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{});
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(dma_allowed_in_flight(I, RA, NA, NB, DA, DB)));
+    if constexpr (Ragged && I % RA == RA - 1)
+      if (s / RA + 1 == clear_stage) clear_shared(lds_ring<30 + ian, A_BYTES_S>);
     barrier_no_fence();
     if constexpr (I % RA == RA - 1) issue_a(lds_ring<30 + ia, A_BYTES_S>, s / RA + NA);
     // the next slab's fragments in the order its first MFMAs need them

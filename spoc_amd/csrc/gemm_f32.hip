@@ -237,19 +237,23 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
   const int64_t b_slab_bytes = static_cast<int64_t>(BKT) * N * 4;
   const int nslabs = (k_len + BKT - 1) / BKT;
   // The end of K inside the last slab.  With K >= BKT the last slab is moved back to end at K (its A pieces then hold
-  // nothing but elements of their own row, at whatever alignment) and the B rows it shares with the slab before it
-  // are the ones left out; with a single slab (K < BKT, K % 4 == 0) the A pieces and B rows past K are.  A lane's k
-  // piece is the same for all its A transfers: rows NWAVES * A_ROWS_PER_DMA apart share the swizzle.
+  // nothing but elements of their own row, at whatever alignment) and the k it shares with the slab before it are left
+  // out, in A as in B (an infinity times the other's zero would be NaN): rows of B, whole pieces of A, and the rest of a
+  // piece that holds shared k and others is zeroed in LDS by the lane that brought it, once a tile, before the barrier
+  // behind which the slab is read.  With a single slab (K < BKT, K % 4 == 0) the A pieces and B rows past K are left out.
+  // A lane's k piece is the same for all its A transfers: rows NWAVES * A_ROWS_PER_DMA apart share the swizzle.
   const int k_tail = k_len - (nslabs - 1) * BKT;
   const bool move_last = Ragged && k_len >= BKT && k_tail != BKT;
   const int k_last = move_last ? k_len - BKT : (nslabs - 1) * BKT;   // first k of the last slab, from k0
-  const bool a_lane_in_k =
-      !Ragged || move_last || (((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 2) < k_tail;
+  const int shared_k = BKT - k_tail;   // moved slab
+  const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 2;
+  const bool a_lane_in_k = !Ragged || (move_last ? a_lane_k + 4 > shared_k : a_lane_k < k_tail);
+  const int clear_slab = move_last && shared_k % 4 != 0 ? nslabs - 1 : -1;
   bool b_lane_in_k[B_DMA];
 #pragma unroll
   for (int i = 0; i < B_DMA; ++i) {
     const int brow = (wave + NWAVES * i) * B_ROWS_PER_DMA + lane / B_CHUNKS;
-    b_lane_in_k[i] = !Ragged || (move_last ? brow >= BKT - k_tail : brow < k_tail);
+    b_lane_in_k[i] = !Ragged || (move_last ? brow >= shared_k : brow < k_tail);
   }
   const char *b_end = reinterpret_cast<const char *>(B) + static_cast<int64_t>(K) * N * 4;
   constexpr uint32_t kOutOfRange = 0x80000000u;
@@ -337,7 +341,19 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
   f32x4 af[2][TI];
   bvec_t bf[2][4];
 
-  auto slab = [&](char *ca, char *cb, const char *na, const char *nb, int s) {
+  auto clear_shared = [&](char *sa) {
+    if (a_lane_k < shared_k && shared_k < a_lane_k + 4) {
+#pragma unroll
+      for (int i = 0; i < A_DMA; ++i) {
+        float *piece = reinterpret_cast<float *>(sa + (wave + NWAVES * i) * 1024 + lane * 16);
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+          if (a_lane_k + d < shared_k) piece[d] = 0.f;
+      }
+    }
+    wait_lds();
+  };
+  auto slab = [&](char *ca, char *cb, char *na, const char *nb, int s) {
     asm volatile("" : "+v"(a_addr0), "+v"(b_addr0));   // keep per-stage addresses out of registers
 #pragma unroll
     for (int kk = 0; kk + 1 < KK; ++kk) {
@@ -346,6 +362,8 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
       interleave(std::integral_constant<int, 0>{});
     }
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NS - 2) * (A_DMA + B_DMA)));
+    if constexpr (Ragged)
+      if (s + 1 == clear_slab) clear_shared(na);
     barrier_no_fence();
     issue(ca, cb, s + NS);
     load_frags(na, nb, 0, af[0], bf[0]);

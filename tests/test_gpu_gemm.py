@@ -907,3 +907,47 @@ def test_gemm_f32_direct(hip, torch_cuda, variant, m, n, k):
     finally:
         hip.set_tunable("gemm_f32.direct", 0)
         hip.set_tunable("gemm_f32.split_k", 0)
+
+
+@pytest.mark.parametrize("kind,tunables", [("bf16", {"gemm16.tile": 256}), ("f16", {"gemm16.tile": 256}),
+                                           ("bf16", {"gemm16.tile": 128}), ("f16", {"gemm16.tile": 128}),
+                                           ("f16", {"gemm16.tile": 128, "gemm16.split_k": 2}),
+                                           ("f16", {"gemm16.rows": 2}),
+                                           ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 64}),
+                                           ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 64, "gemm_f32.split_k": 2}),
+                                           ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 128}),
+                                           ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 256}),
+                                           ("f32", {"gemm_f32.direct": 18})])
+@pytest.mark.parametrize("m,n,k", [(70, 131, 200), (140, 264, 200), (129, 129, 77), (300, 257, 333), (66, 136, 131),
+                                   (65, 260, 190)])
+def test_gemm_infinity_at_every_k(hip, torch_cuda, kind, tunables, m, n, k):
+    """An infinity in A at one k per row, every k of the last stages among them (the stage at the end of K is moved back
+    over the one before it: what the two share must count once and no product of it be formed twice), and rows of NaN-free
+    finite values beside them: the infinities, NaN and zeros of the float64 product, and its finite values within k 2^-24 of
+    the products' magnitudes.  B holds no zeros, so that an infinity is an infinity in every column."""
+    torch = torch_cuda
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[kind]
+    torch.manual_seed(m + n * k)
+    da = (torch.randn(m, k, device="cuda") * 0.1).to(dt)
+    db = (torch.rand(k, n, device="cuda") + 0.5).to(dt)
+    db[:, 1::3] *= -1
+    ks = torch.arange(k - 1, k - 1 - (m - 1), -1, device="cuda") % k   # row i + 1: k - 1 - i; row 0 stays finite
+    da[torch.arange(1, m, device="cuda"), ks] = float("inf")
+    da[1::2] *= -1
+    ref, size = da.double() @ db.double(), da.double().abs() @ db.double().abs()
+    bias = torch.zeros(n, device="cuda")
+    y = None
+    try:
+        for name, value in tunables.items():
+            hip.set_tunable(name, value)
+        c = {"bf16": hip.gemm_bf16, "f16": hip.gemm_f16, "f32": hip.gemm_f32}[kind](da, db)
+        if kind == "f16":
+            y, rs = hip.gemm_f16_bias_relu_rowsum(da, db, bias)
+    finally:
+        for name in tunables:
+            hip.set_tunable(name, 0)
+    assert bool(ref[1:].isinf().all()) and bool(ref[0].isfinite().all())
+    assert torch.equal(c[1:].double(), ref[1:])
+    assert bool(((c[0].double() - ref[0]).abs() <= (k + 32) * 2.0 ** -24 * size[0]).all())
+    if y is not None:
+        assert torch.equal(y[1:].double(), ref[1:].relu()) and bool(rs[1:].isinf().all())
