@@ -458,12 +458,12 @@ __device__ __forceinline__ float widen16(uint16_t bits) {
   else return static_cast<float>(__builtin_bit_cast(_Float16, bits));
 }
 
-// Zeroes the first `count` (1 .. 7) of the eight elements this lane brought to each of its places of an A stage, if `mine`.
+// Zeroes the first `count` (0 .. 7, the lane's own) of the eight elements this lane brought to each of its places of an A stage.
 // The caller has waited for the transfers and passes a barrier afterwards: no other wave reads the stage in between.  Once
 // a tile; a mask on the fragments instead would be in every turn of the K loop.
 template <int DA, int NWAVES>
-__device__ __forceinline__ void clear_piece_heads(char *sa, int wave, int lane, bool mine, int count) {
-  if (mine) {
+__device__ __forceinline__ void clear_piece_heads(char *sa, int wave, int lane, int count) {
+  if (count > 0) {
     u32x4 keep;
 #pragma unroll
     for (int d = 0; d < 4; ++d) keep[d] = count <= 2 * d ? 0xFFFFFFFFu : count == 2 * d + 1 ? 0xFFFF0000u : 0u;
@@ -660,7 +660,7 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   // elements of their own rows, at whatever alignment, and the k it shares with the stage before it are sent out of
   // range, in A as in B: an infinity times the other's zero would be NaN.  Of B they are rows of the first of the
   // stage's two slabs and, past 32, of the second; of A whole pieces of 8, and the rest of a piece that holds shared k
-  // and others (shared_k % 8 != 0) is zeroed in LDS by the lane that brought it (clear_shared).  Below one stage
+  // and others (shared_k % 8 != 0) is zeroed in LDS by the lane that brought it (clear).  Below one stage
   // (K % 8 == 0) the A pieces and B rows past K are out of range.  A lane's k piece is the same for all its transfers of
   // a stage (rows 16 apart share the swizzle).
   const int nstages = (K + BKA - 1) / BKA;
@@ -669,16 +669,19 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   const int k_tail_a = K - (nstages - 1) * BKA, k_tail_b = K - (nslabs - 1) * BKB;   // single stage
   const int shared_k = nstages * BKA - K;                                               // moved stage
   const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3;
-  const bool a_lane_in_k = !Ragged || (move_last ? a_lane_k + 8 > shared_k : a_lane_k < k_tail_a);
-  bool b_in_last[DB], b_in_prev[DB];   // the lanes that count in the last slab and in the one before it
+  const uint32_t a_out = (move_last ? a_lane_k + 8 <= shared_k : a_lane_k >= k_tail_a) ? 0x80000000u : 0u;
+  constexpr uint32_t kOutOfRange = 0x80000000u;
+  // A lane whose row does not count has bit 31 set for the last slab and bit 30 for the one before it, and its offset
+  // gets bit 31 from there.  (As lane masks they took what scalar registers the loop has left.  Offsets of their own to
+  // select from became branches in the loop: four times the time.)
+  uint32_t b_out[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i) {
     const int brow = 2 * (wave + NWAVES * i) + (lane >> 5);
-    b_in_last[i] = !Ragged || (move_last ? brow + BKB >= shared_k : brow < k_tail_b);
-    b_in_prev[i] = !move_last || brow >= shared_k;
+    b_out[i] = (move_last ? brow + BKB < shared_k : brow >= k_tail_b) ? kOutOfRange : 0u;
+    if (move_last && brow < shared_k) b_out[i] |= kOutOfRange >> 1;
   }
-  const char *b_end = b_base + (static_cast<int64_t>(K - 1) * ld + N - (N & 1)) * 2;   // add_last_product brings an odd N's last element
-  constexpr uint32_t kOutOfRange = 0x80000000u;
+  const char *b_end = b_base + (static_cast<int64_t>(K - 1) * ld + N - (N & 1)) * 2;   // last_products bring an odd N's last element
 
   f32x4_t acc[8][4];
 #pragma unroll
@@ -703,12 +706,9 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
     const uint32_t a_so = static_cast<uint32_t>(!whole && move_last ? K - BKA : min(stage, nstages - 1) * BKA) * 2u;
 #pragma unroll
     for (int i = 0; i < DA; ++i)
-      dma16(a_rsrc, (!Ragged || whole || a_lane_in_k) ? a_off[i] : kOutOfRange, a_so, sa + (wave + NWAVES * i) * 1024);
+      dma16(a_rsrc, Ragged ? a_off[i] | (whole ? 0u : a_out) : a_off[i], a_so, sa + (wave + NWAVES * i) * 1024);
   };
-  const int clear_stage = move_last && shared_k % 8 != 0 ? nstages - 1 : -1;
-  auto clear_shared = [&](char *sa) {
-    clear_piece_heads<DA, NWAVES>(sa, wave, lane, a_lane_k < shared_k && shared_k < a_lane_k + 8, shared_k % 8);
-  };
+  const int clear = move_last && a_lane_k < shared_k && shared_k < a_lane_k + 8 ? shared_k - a_lane_k : 0;
   // B slabs are issued in order 0, 1, 2, ...: the source of the next one is a running pointer (two scalar adds per
   // slab instead of a 64-bit multiply) that stops at the last slab, which the tail of the K loop re-issues into
   // stages nobody reads any more so that the count of outstanding transfers follows the same pattern throughout
@@ -719,13 +719,13 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
     (void)slab;   // == b_next
     const bool last = b_next >= nslabs - 1, prev = b_next == nslabs - 2;
     if (move_last && prev) b_src = b_base + static_cast<int64_t>(K - BKA) * ld * 2;
+    const int place = last ? 0 : prev ? 1 : 2;
     const int64_t b_left = b_end - b_src;
     const __amdgpu_buffer_rsrc_t b_rsrc =
         make_rsrc(b_src, Ragged && b_left < 0x80000000ll ? static_cast<uint32_t>(b_left) : kOutOfRange);
 #pragma unroll
     for (int i = 0; i < DB; ++i)
-      dma16(b_rsrc, (!Ragged || (last ? b_in_last[i] : prev ? b_in_prev[i] : true)) ? b_off[i] : kOutOfRange, 0u,
-            sb + (wave + NWAVES * i) * 1024);
+      dma16(b_rsrc, Ragged ? b_off[i] | ((b_out[i] << place) & kOutOfRange) : b_off[i], 0u, sb + (wave + NWAVES * i) * 1024);
     ++b_next;
     if (b_next < nslabs) b_src += b_slab_bytes;
   };
@@ -802,7 +802,7 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
       __builtin_amdgcn_s_waitcnt(
           waitcnt_vm_lgkm0(dma_allowed_in_flight(I, RA, NA, NB, DA, DB, HalfBarriers ? 2 : 1)));
       if constexpr (Ragged && I % RA == RA - 1)
-        if (s / RA + 1 == clear_stage) clear_shared(lds_ring<10 + ian, A_BYTES_S>);
+        if (s / RA + 1 == nstages - 1) clear_piece_heads<DA, NWAVES>(lds_ring<10 + ian, A_BYTES_S>, wave, lane, clear);
       barrier_no_fence();
     }
     if constexpr (I % RA == RA - 1) issue_a(lds_ring<10 + ia, A_BYTES_S>, s / RA + NA);
@@ -1124,7 +1124,7 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   // elements of their own rows, at whatever alignment, and the k it shares with the stage before it are sent out of
   // range, in A as in B: an infinity times the other's zero would be NaN.  Of B they are rows of the first of the
   // stage's two slabs and, past 32, of the second; of A whole pieces of 8, and the rest of a piece that holds shared k
-  // and others (shared_k % 8 != 0) is zeroed in LDS by the lane that brought it (clear_shared).  Below one stage
+  // and others (shared_k % 8 != 0) is zeroed in LDS by the lane that brought it (clear).  Below one stage
   // (K % 8 == 0) the A pieces and B rows past K are out of range.  A lane's k piece is the same for all its transfers of
   // a stage (rows 16 apart share the swizzle).
   const int nstages = (k_len + BKA - 1) / BKA;
@@ -1133,16 +1133,16 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   const int k_tail_a = k_len - (nstages - 1) * BKA, k_tail_b = k_len - (nslabs - 1) * BKB;   // single stage
   const int shared_k = nstages * BKA - k_len;                                               // moved stage
   const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3;
-  const bool a_lane_in_k = !Ragged || (move_last ? a_lane_k + 8 > shared_k : a_lane_k < k_tail_a);
-  bool b_in_last[DB], b_in_prev[DB];   // the lanes that count in the last slab and in the one before it
+  const uint32_t a_out = (move_last ? a_lane_k + 8 <= shared_k : a_lane_k >= k_tail_a) ? 0x80000000u : 0u;
+  constexpr uint32_t kOutOfRange = 0x80000000u;
+  uint32_t b_out[DB];   // as in the large tile
 #pragma unroll
   for (int i = 0; i < DB; ++i) {
     const int brow = (wave + NWAVES * i) * B_ROWS_PER_DMA + lane / B_CHUNKS;
-    b_in_last[i] = !Ragged || (move_last ? brow + BKB >= shared_k : brow < k_tail_b);
-    b_in_prev[i] = !move_last || brow >= shared_k;
+    b_out[i] = (move_last ? brow + BKB < shared_k : brow >= k_tail_b) ? kOutOfRange : 0u;
+    if (move_last && brow < shared_k) b_out[i] |= kOutOfRange >> 1;
   }
   const char *b_end = reinterpret_cast<const char *>(B) + (static_cast<int64_t>(K - 1) * ld + N - (N & 1)) * 2;   // as above
-  constexpr uint32_t kOutOfRange = 0x80000000u;
 
   f32x4_t acc[4][4];
 #pragma unroll
@@ -1163,12 +1163,9 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     const uint32_t a_so = static_cast<uint32_t>(!whole && move_last ? k_len - BKA : min(stage, nstages - 1) * BKA) * 2u;
 #pragma unroll
     for (int i = 0; i < DA; ++i)
-      dma16(a_rsrc, (!Ragged || whole || a_lane_in_k) ? a_off[i] : kOutOfRange, a_so, sa + (wave + NWAVES * i) * 1024);
+      dma16(a_rsrc, Ragged ? a_off[i] | (whole ? 0u : a_out) : a_off[i], a_so, sa + (wave + NWAVES * i) * 1024);
   };
-  const int clear_stage = move_last && shared_k % 8 != 0 ? nstages - 1 : -1;
-  auto clear_shared = [&](char *sa) {
-    clear_piece_heads<DA, NWAVES>(sa, wave, lane, a_lane_k < shared_k && shared_k < a_lane_k + 8, shared_k % 8);
-  };
+  const int clear = move_last && a_lane_k < shared_k && shared_k < a_lane_k + 8 ? shared_k - a_lane_k : 0;
   // B slabs go out in order; the source is a running pointer that stops at the last slab (the tail of the K loop
   // re-issues it into stages nobody reads any more, so the count of transfers in flight keeps its pattern)
   const char *b_src = reinterpret_cast<const char *>(B + static_cast<int64_t>(k0) * ld);
@@ -1176,13 +1173,13 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   auto issue_b = [&](char *sb) {
     const bool last = b_next >= nslabs - 1, prev = b_next == nslabs - 2;
     if (move_last && prev) b_src = reinterpret_cast<const char *>(B + static_cast<int64_t>(k0 + k_len - BKA) * ld);
+    const int place = last ? 0 : prev ? 1 : 2;
     const int64_t b_left = b_end - b_src;
     const __amdgpu_buffer_rsrc_t b_rsrc =
         make_rsrc(b_src, Ragged && b_left < 0x80000000ll ? static_cast<uint32_t>(b_left) : kOutOfRange);
 #pragma unroll
     for (int i = 0; i < DB; ++i)
-      dma16(b_rsrc, (!Ragged || (last ? b_in_last[i] : prev ? b_in_prev[i] : true)) ? b_off[i] : kOutOfRange, 0u,
-            sb + (wave + NWAVES * i) * 1024);
+      dma16(b_rsrc, Ragged ? b_off[i] | ((b_out[i] << place) & kOutOfRange) : b_off[i], 0u, sb + (wave + NWAVES * i) * 1024);
     ++b_next;
     if (b_next < nslabs) b_src += b_slab_bytes;
   };
@@ -1243,7 +1240,7 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     spread(std::integral_constant<int, DB>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{});
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(dma_allowed_in_flight(I, RA, NA, NB, DA, DB)));
     if constexpr (Ragged && I % RA == RA - 1)
-      if (s / RA + 1 == clear_stage) clear_shared(lds_ring<30 + ian, A_BYTES_S>);
+      if (s / RA + 1 == nstages - 1) clear_piece_heads<DA, NWAVES>(lds_ring<30 + ian, A_BYTES_S>, wave, lane, clear);
     barrier_no_fence();
     if constexpr (I % RA == RA - 1) issue_a(lds_ring<30 + ia, A_BYTES_S>, s / RA + NA);
     // the next slab's fragments in the order its first MFMAs need them

@@ -248,7 +248,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
   const int shared_k = BKT - k_tail;   // moved slab
   const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 2;
   const bool a_lane_in_k = !Ragged || (move_last ? a_lane_k + 4 > shared_k : a_lane_k < k_tail);
-  const int clear_slab = move_last && shared_k % 4 != 0 ? nslabs - 1 : -1;
+  const int clear = move_last && a_lane_k < shared_k && shared_k < a_lane_k + 4 ? shared_k - a_lane_k : 0;
   bool b_lane_in_k[B_DMA];
 #pragma unroll
   for (int i = 0; i < B_DMA; ++i) {
@@ -342,13 +342,13 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
   bvec_t bf[2][4];
 
   auto clear_shared = [&](char *sa) {
-    if (a_lane_k < shared_k && shared_k < a_lane_k + 4) {
+    if (clear > 0) {
 #pragma unroll
       for (int i = 0; i < A_DMA; ++i) {
         float *piece = reinterpret_cast<float *>(sa + (wave + NWAVES * i) * 1024 + lane * 16);
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-          if (a_lane_k + d < shared_k) piece[d] = 0.f;
+          if (d < clear) piece[d] = 0.f;
       }
     }
     wait_lds();
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
     }
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NS - 2) * (A_DMA + B_DMA)));
     if constexpr (Ragged)
-      if (s + 1 == clear_slab) clear_shared(na);
+      if (s + 1 == nslabs - 1) clear_shared(na);
     barrier_no_fence();
     issue(ca, cb, s + NS);
     load_frags(na, nb, 0, af[0], bf[0]);
