@@ -485,11 +485,14 @@ double ring_estimate(int m, int n, int k, int tile, int splits) {
 // be a twentieth ahead.  Against the best of all variants timed on the drawn products the choice loses 2.2 % on average.
 // Pieces are tried only while they leave every wave a step (direct) or four slabs (LDS), and while the workgroups they
 // make find CUs: more than four a CU never paid.
-// gemm_f32.direct: 1 = never, 18 / 14 / 24 = always, with (row_blocks, waves) these digits; gemm_f32.tile forces a tile,
-// gemm_f32.split_k the pieces (1 = whole) of the 64 x 64 tile or of a forced direct variant.  0 leaves the choice here.
+// gemm_f32.direct: 1 = never, 18 / 14 / 24 = always, with (row_blocks, waves) these digits, any other value as 0;
+// gemm_f32.tile forces a tile, gemm_f32.split_k the pieces (1 = whole) of the 64 x 64 tile or of a forced direct variant.
+// 0 leaves the choice here.
 Plan plan_for(int m, int n, int k, bool ring_ok, bool c_aligned) {
   constexpr int kPieces[] = {1, 2, 3, 4, 6, 8, 12, 16};
-  const int direct = static_cast<int>(tunable("gemm_f32.direct", 0)), forced = static_cast<int>(tunable("gemm_f32.tile", 0));
+  const int64_t asked = tunable("gemm_f32.direct", 0);
+  const int direct = asked == 1 || asked == 18 || asked == 14 || asked == 24 ? static_cast<int>(asked) : 0;
+  const int forced = static_cast<int>(tunable("gemm_f32.tile", 0));
   const int tile = forced == 0 || forced == 256 || forced == 128 ? forced : 64;
   const int64_t split = tunable("gemm_f32.split_k", 0);
   const bool direct_ok = gemm_f32_direct_serves(m, n, k);

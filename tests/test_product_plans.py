@@ -1,0 +1,43 @@
+"""How the products say they will be computed, for knobs of any value: whole-number answers, no device needed."""
+import pytest
+
+
+@pytest.fixture
+def knobs(hip):
+    """set(name, value), undone afterwards."""
+    seen = set()
+
+    def put(name, value):
+        seen.add(name)
+        hip.set_tunable(name, value)
+    yield put
+    for name in seen:
+        hip.set_tunable(name, 0)
+
+
+@pytest.mark.parametrize("value", [-1, 2, 3, 9, 10, 12, 16, 20, 28, 34, 48, 64, 99, 18 + 2 ** 32])
+def test_f32_direct_knob_of_no_variant_counts_as_zero(hip, knobs, value):
+    """gemm_f32.direct names a variant by its digits; a number that names none (2: no rows at all; 34, 64: rows the kernel
+    has no form for, and fewer tickets than its tiles draw) leaves the choice to the library."""
+    shapes = [(1, 1, 1), (128, 128, 128), (68, 119, 3328), (153, 1216, 1920), (4096, 2048, 512), (2049, 4097, 3000)]
+    for split_k in (0, 2, 16):
+        knobs("gemm_f32.split_k", split_k)
+        knobs("gemm_f32.direct", 0)
+        own = [hip.gemm_f32_k_splits(*s) for s in shapes]
+        knobs("gemm_f32.direct", value)
+        assert [hip.gemm_f32_k_splits(*s) for s in shapes] == own
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [2, 34])
+def test_f32_direct_knob_of_no_variant_computes_the_same_product(hip, torch_cuda, knobs, value):
+    """The same bits as with the knob at 0, K left whole and cut, where the direct kernel is the library's choice."""
+    torch = torch_cuda
+    torch.manual_seed(value)
+    a, b = torch.randn(153, 1921, device="cuda"), torch.randn(1921, 1217, device="cuda")
+    for split_k in (0, 3):
+        knobs("gemm_f32.split_k", split_k)
+        knobs("gemm_f32.direct", 0)
+        c = hip.gemm_f32(a, b)
+        knobs("gemm_f32.direct", value)
+        assert torch.equal(hip.gemm_f32(a, b), c)
