@@ -1438,7 +1438,7 @@ int splitk_for(int m, int n, int k) {
   const int64_t fit = static_cast<int64_t>(kSplitWorkspaceBytes) / (splitk_plane_floats(m, n) * 4);
   int64_t splits = 1;
   if (forced >= 2) {
-    splits = std::min<int64_t>({forced, static_cast<int64_t>(k / 64), fit});
+    splits = std::max<int64_t>(1, std::min<int64_t>({forced, static_cast<int64_t>(k / 64), fit}));
   } else {
     auto estimate = [&](int64_t s) {
       const double slabs = static_cast<double>(k) / 32 / s;

@@ -28,6 +28,17 @@ def test_f32_direct_knob_of_no_variant_counts_as_zero(hip, knobs, value):
         assert [hip.gemm_f32_k_splits(*s) for s in shapes] == own
 
 
+@pytest.mark.parametrize("m,n,k,room", [(200, 200, 40, False), (100, 64, 32, False), (200, 200, 63, False), (8192, 4096, 4096, False),
+                                         (300, 520, 448, True), (200, 200, 64, False), (200, 200, 127, False)])
+@pytest.mark.parametrize("forced", [2, 7])
+def test_16_bit_pieces_forced_where_there_is_no_room(hip, knobs, m, n, k, room, forced):
+    """A forced count of K pieces is cut to whole stages of 64 and to planes that fit the workspace, and to no less than the
+    one piece that says K stays whole."""
+    knobs("gemm16.tile", 128)
+    knobs("gemm16.split_k", forced)
+    assert hip.gemm16_k_splits(m, n, k) == (forced if room else 1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("value", [2, 34])
 def test_f32_direct_knob_of_no_variant_computes_the_same_product(hip, torch_cuda, knobs, value):
