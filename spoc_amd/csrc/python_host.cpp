@@ -179,32 +179,33 @@ PyObject *run_source(PyObject *, PyObject *const *a, Py_ssize_t n) {
 // run_pipeline([(ir, args, block, grid[, shared_mem]), ...]) -> (path, launches) | status
 PyObject *run_pipeline(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!bound() || !arity(n, 1, "run_pipeline")) return nullptr;
-  PyObject *seq = PySequence_Fast(a[0], "stages is a sequence of (ir, args, block, grid[, shared_mem])");
+  PyObject *seq = PySequence_Tuple(a[0]);
   if (!seq) return nullptr;
-  const size_t count = static_cast<size_t>(PySequence_Fast_GET_SIZE(seq));
+  const size_t count = static_cast<size_t>(PyTuple_GET_SIZE(seq));
   std::vector<sarek_hip_pipeline_stage> stages(count);
   std::vector<std::vector<sarek_hip_varg>> args(count);
-  std::vector<PyObject *> held;   // the stages' own sequences: they keep the IR texts
+  // The stages as tuples of their own: they keep the IR texts, which the library reads while other threads run and may
+  // change a stage that is a list.
+  std::vector<PyObject *> held;
   bool ok = true;
   for (size_t i = 0; i < count && ok; ++i) {
-    PyObject *stage = PySequence_Fast(PySequence_Fast_GET_ITEM(seq, static_cast<Py_ssize_t>(i)), "a stage is a sequence");
+    PyObject *stage = PySequence_Tuple(PyTuple_GET_ITEM(seq, static_cast<Py_ssize_t>(i)));
     if (!stage) {
       ok = false;
       break;
     }
     held.push_back(stage);
-    const Py_ssize_t parts = PySequence_Fast_GET_SIZE(stage);
+    const Py_ssize_t parts = PyTuple_GET_SIZE(stage);
     if (parts < 4) {
       PyErr_Format(PyExc_ValueError, "not enough values to unpack (expected 4, got %zd)", parts);
       ok = false;
       break;
     }
-    PyObject **p = PySequence_Fast_ITEMS(stage);
     sarek_hip_pipeline_stage &s = stages[i];
-    s.ir_text = PyUnicode_AsUTF8(p[0]);
+    s.ir_text = PyUnicode_AsUTF8(PyTuple_GET_ITEM(stage, 0));
     s.shared_mem_bytes = 0;
-    ok = s.ir_text && as_args(p[1], args[i]) && as_dims(p[2], s.block) && as_dims(p[3], s.grid) &&
-         (parts == 4 || as_int(p[4], &s.shared_mem_bytes));
+    ok = s.ir_text && as_args(PyTuple_GET_ITEM(stage, 1), args[i]) && as_dims(PyTuple_GET_ITEM(stage, 2), s.block) &&
+         as_dims(PyTuple_GET_ITEM(stage, 3), s.grid) && (parts == 4 || as_int(PyTuple_GET_ITEM(stage, 4), &s.shared_mem_bytes));
     s.args = args[i].data();
     s.n_args = static_cast<int>(args[i].size());
   }

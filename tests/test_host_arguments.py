@@ -1,0 +1,44 @@
+"""The launch calls' argument lists (spoc_amd._host) against what the caller's objects do meanwhile: the entry points are
+replaced by functions of the test that look at what arrives, so no device is needed."""
+import ctypes as C
+
+import pytest
+
+NAMES = ("sarek_hip_execute_run_vectors", "sarek_hip_execute_run_source", "sarek_hip_execute_run_pipeline",
+         "sarek_hip_last_run_path", "sarek_hip_fold_partials_f64")
+
+
+@pytest.fixture
+def entries(hip):
+    """entries(name=function): those entry points call the function until the test ends."""
+    def addresses(**replaced):
+        return [C.cast(replaced.get(n, getattr(hip.lib, n)), C.c_void_p).value for n in NAMES]
+    yield lambda **replaced: hip._host.bind(*addresses(**replaced))
+    hip._host.bind(*addresses())
+
+
+def stage_text(word, length=4000):
+    """A text of its own (not interned, not shared)."""
+    return "".join([word] * (length // len(word)))
+
+
+def test_pipeline_keeps_the_stages_texts(hip, entries):
+    """A stage given as a list may be changed by another thread while the library works on it: the text it was given is
+    the one it reads."""
+    from spoc_amd.sarek import Execute
+    stage = [stage_text("first"), [Execute.Int(7)], (1, 1, 1), (1, 1, 1)]
+    stages = [stage]
+    want = stage[0].encode()
+    seen, other = [], []
+
+    @C.CFUNCTYPE(C.c_int, C.POINTER(hip.PipelineStage), C.c_int, C.POINTER(C.c_int))
+    def run(given, n, launches):
+        stage[0] = "gone"
+        stages[0] = None
+        other.extend(stage_text("other") for _ in range(64))     # takes the place of a text that was given back
+        address = C.c_void_p.from_buffer(given.contents, hip.PipelineStage.ir_text.offset).value
+        seen.append((C.string_at(address, len(want)), given.contents.n_args, given.contents.args[0].i32))
+        return hip.OK
+    entries(sarek_hip_execute_run_pipeline=run)
+    Execute.run_pipeline(stages)
+    assert seen == [(want, 1, 7)]
