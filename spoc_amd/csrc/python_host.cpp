@@ -43,16 +43,18 @@ bool as_int(PyObject *o, int *out) {
   return true;
 }
 
+// Sequences are read as tuples: a conversion below may run the caller's code (__index__), which may change a list.
+
 // block or grid: up to three integers, missing ones zero
 bool as_dims(PyObject *o, int out[3]) {
-  PyObject *seq = PySequence_Fast(o, "block and grid are sequences of three integers");
+  PyObject *seq = PySequence_Tuple(o);
   if (!seq) return false;
-  const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+  const Py_ssize_t n = PyTuple_GET_SIZE(seq);
   bool ok = n <= 3;
   if (!ok) PyErr_SetString(PyExc_IndexError, "invalid index");
   for (Py_ssize_t i = 0; i < 3 && ok; ++i) {
     out[i] = 0;
-    if (i < n) ok = as_int(PySequence_Fast_GET_ITEM(seq, i), out + i);
+    if (i < n) ok = as_int(PyTuple_GET_ITEM(seq, i), out + i);
   }
   Py_DECREF(seq);
   return ok;
@@ -79,24 +81,24 @@ bool as_handle(PyObject *vector, sarek_hip_vector *out) {
 
 // [(kind, value), ...] as Execute.Vec, .Int, ... make them
 bool as_args(PyObject *o, std::vector<sarek_hip_varg> &out) {
-  PyObject *seq = PySequence_Fast(o, "args is a sequence of Execute.Vec, Execute.Int, ...");
+  PyObject *seq = PySequence_Tuple(o);
   if (!seq) return false;
-  const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+  const Py_ssize_t n = PyTuple_GET_SIZE(seq);
   out.resize(static_cast<size_t>(n));
   bool ok = true;
   for (Py_ssize_t i = 0; i < n && ok; ++i) {
-    PyObject *item = PySequence_Fast(PySequence_Fast_GET_ITEM(seq, i), "an argument is a pair of kind and value");
+    PyObject *item = PySequence_Tuple(PyTuple_GET_ITEM(seq, i));
     if (!item) {
       ok = false;
       break;
     }
-    if (PySequence_Fast_GET_SIZE(item) != 2) {
+    if (PyTuple_GET_SIZE(item) != 2) {
       PyErr_SetString(PyExc_ValueError, "an argument is a pair of kind and value");
       Py_DECREF(item);
       ok = false;
       break;
     }
-    PyObject *kind = PySequence_Fast_GET_ITEM(item, 0), *value = PySequence_Fast_GET_ITEM(item, 1);
+    PyObject *kind = PyTuple_GET_ITEM(item, 0), *value = PyTuple_GET_ITEM(item, 1);
     sarek_hip_varg &a = out[static_cast<size_t>(i)];
     std::memset(&a, 0, sizeof(a));
     const char *k = PyUnicode_Check(kind) ? PyUnicode_AsUTF8(kind) : "";

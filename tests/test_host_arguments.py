@@ -42,3 +42,31 @@ def test_pipeline_keeps_the_stages_texts(hip, entries):
     entries(sarek_hip_execute_run_pipeline=run)
     Execute.run_pipeline(stages)
     assert seen == [(want, 1, 7)]
+
+
+class Changes:
+    """An integer that changes a list when it is asked for its value."""
+
+    def __init__(self, value, change):
+        self.value, self.change = value, change
+
+    def __index__(self):
+        self.change()
+        return self.value
+
+
+def test_arguments_are_those_the_list_held(hip, entries):
+    """Whatever __index__ of an argument, or of a block's size, does to the list that is being read."""
+    from spoc_amd.sarek import Execute
+    args, block = [], []
+    args += [("i32", Changes(1, args.clear)), ("i32", 2), ("i64", 3)]
+    block += [Changes(8, block.clear), 4, 2]
+    seen = []
+
+    @C.CFUNCTYPE(C.c_int, C.c_char_p, C.POINTER(C.c_int), C.POINTER(C.c_int), C.c_int, C.POINTER(hip.VArg), C.c_int)
+    def run(ir, block, grid, shared, given, n):
+        seen.append((list(block[:3]), [given[0].i32, given[1].i32, given[2].i64], n))
+        return hip.OK
+    entries(sarek_hip_execute_run_vectors=run)
+    Execute.run_vectors("(kernel)", args, block, (1, 1, 1))
+    assert seen == [([8, 4, 2], [1, 2, 3], 3)]
