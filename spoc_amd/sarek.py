@@ -699,7 +699,7 @@ class Execute:
 
     @staticmethod
     def run_source(source, kernel_name, block, grid, args, lang=hip.LANG_HIP, shared_mem=0, inject_lengths=True):
-        return _served(hip._host.run_source(source, lang, kernel_name, block, grid, shared_mem, inject_lengths, args))
+        return _served(hip._host.run_source(source, lang, kernel_name, block, grid, shared_mem, int(inject_lengths), args))
 
     @staticmethod
     def sync_vectors_to_cpu(args):

@@ -2,6 +2,7 @@
 replaced by functions of the test that look at what arrives, so no device is needed."""
 import ctypes as C
 
+import numpy as np
 import pytest
 
 NAMES = ("sarek_hip_execute_run_vectors", "sarek_hip_execute_run_source", "sarek_hip_execute_run_pipeline",
@@ -70,3 +71,18 @@ def test_arguments_are_those_the_list_held(hip, entries):
     entries(sarek_hip_execute_run_vectors=run)
     Execute.run_vectors("(kernel)", args, block, (1, 1, 1))
     assert seen == [([8, 4, 2], [1, 2, 3], 3)]
+
+
+@pytest.mark.parametrize("given,want", [(True, 1), (False, 0), (np.True_, 1), (np.False_, 0), (1.0, 1)])
+def test_inject_lengths_is_any_truth_value_that_is_a_number(hip, entries, given, want):
+    """numpy's booleans have no __index__, and what int() takes was always taken."""
+    from spoc_amd.sarek import Execute
+    seen = []
+
+    @C.CFUNCTYPE(C.c_int, C.c_char_p, C.c_int, C.c_char_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_int)
+    def run(source, lang, name, block, grid, shared, inject, args, n):
+        seen.append(inject)
+        return hip.OK
+    entries(sarek_hip_execute_run_source=run)
+    Execute.run_source("text", "name", (1, 1, 1), (1, 1, 1), [], inject_lengths=given)
+    assert seen == [want]
