@@ -75,7 +75,7 @@ def test_arguments_are_those_the_list_held(hip, entries):
 
 @pytest.mark.parametrize("given,want", [(True, 1), (False, 0), (np.True_, 1), (np.False_, 0), (1.0, 1)])
 def test_inject_lengths_is_any_truth_value_that_is_a_number(hip, entries, given, want):
-    """numpy's booleans have no __index__, and what int() takes was always taken."""
+    """What int() takes: a float too, and numpy's booleans without the warning that their __index__ gives."""
     from spoc_amd.sarek import Execute
     seen = []
 
