@@ -3,6 +3,8 @@ No compute call is made here (this file runs without a GPU)."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -228,3 +230,19 @@ def test_bench_refuses_more_than_one_gpu_without_touching_one():
     import sys
     run = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert run.returncode == 2 and "one GPU" in run.stderr and run.stdout == ""
+
+
+def test_library_builds_without_python_headers(tmp_path):
+    """`make` plans libsarek_hip.so alone, and says so, where the Python it is given is missing or has no headers: C and
+    OCaml programs need nothing of _host.so."""
+    csrc = os.path.join(ROOT, "spoc_amd", "csrc")
+    bare = tmp_path / "python"
+    bare.write_text(f"#!/bin/sh\necho {tmp_path}\n")
+    bare.chmod(0o755)
+
+    def plan(python):
+        return subprocess.run(["make", "-C", csrc, "-n", "-B", f"PYTHON={python}"], capture_output=True, text=True, check=True).stdout
+    assert "-o ../_host.so" in plan(sys.executable)
+    for python in (bare, "/nonexistent/python"):
+        out = plan(python)
+        assert "-o ../libsarek_hip.so" in out and "-o ../_host.so" not in out and "_host.so is not built" in out
