@@ -640,8 +640,8 @@ int sarek_hip_gemm16_tile(int m, int n, int k);
  * CUs that way, the partial tiles added up in a fixed order by a second
  * kernel (by the last workgroup of a tile in the few-rows kernel).  Device memory for them: one 64 MiB block per stream, allocated at
  * the first such call on the stream and kept until the process ends, for up
- * to 16 streams; calls on further streams, and calls under stream capture on
- * a stream that has no block yet, run unsplit (same result up to the order of
+ * to 16 streams; calls on further streams or on hipStreamPerThread, and calls
+ * under stream capture, run unsplit (same result up to the order of
  * the f32 additions).  The count is the plain products'; the fused entry point
  * splits on the few-rows kernel only.                                       */
 int sarek_hip_gemm16_k_splits(int m, int n, int k);

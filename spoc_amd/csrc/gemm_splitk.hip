@@ -31,13 +31,15 @@ __global__ __launch_bounds__(256) void zero_tickets_kernel(unsigned *tickets) {
 
 }  // namespace
 
-// One block of kSplitWorkspaceBytes and its tickets per (device, stream), allocated at the first call that wants one on that stream and
-// kept until the process ends (never grown or freed, so a pointer handed out stays good whatever other threads do):
+// One block of kSplitWorkspaceBytes and its tickets per (device, stream), allocated at the first call that wants one on
+// that stream and kept until the process ends (never grown or freed, so a pointer handed out stays good whatever other threads do):
 // calls on different streams never share one, calls on one stream are ordered by it.  nullptr (the caller then works
 // without one: no K split, row sums by atomicAdd) for a stream under capture -- a recorded graph would carry the
-// block's address to wherever it is replayed, next to eager calls or other replays that use the same block --, past 16
-// streams, or when the allocation fails.
+// block's address to wherever it is replayed, next to eager calls or other replays that use the same block --, for
+// hipStreamPerThread (one handle, a stream to each thread: their launches are not ordered by it), past 16 streams, or when
+// the allocation fails.
 float *splitk_workspace(hipStream_t st) {
+  if (st == hipStreamPerThread) return nullptr;
   static std::mutex mu;
   static std::map<std::pair<int, hipStream_t>, void *> blocks;
   int dev = 0;

@@ -951,3 +951,39 @@ def test_gemm_infinity_at_every_k(hip, torch_cuda, kind, tunables, m, n, k):
     assert bool(((c[0].double() - ref[0]).abs() <= (k + 32) * 2.0 ** -24 * size[0]).all())
     if y is not None:
         assert torch.equal(y[1:].double(), ref[1:].relu()) and bool(rs[1:].isinf().all())
+
+
+@pytest.mark.parametrize("kind,m,n,k", [("bf16", 16, 512, 8192), ("f32", 16, 64, 4096), ("f16", 128, 128, 8192)])
+def test_products_on_the_stream_per_thread(hip, torch_cuda, kind, m, n, k):
+    """hipStreamPerThread is one handle for as many streams as there are threads: a block of device memory kept by the handle
+    would be written by all of them at once.  Products that are cut along K elsewhere are left whole there: threads at work
+    together get the bits of the whole product."""
+    import ctypes
+    import threading
+    torch = torch_cuda
+    torch.manual_seed(m + n + k)
+    dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[kind]
+    count = {"f32": hip.gemm_f32_k_splits}.get(kind, hip.gemm16_k_splits)
+    entry = {"bf16": hip.lib.sarek_hip_gemm_bf16, "f16": hip.lib.sarek_hip_gemm_f16, "f32": hip.lib.sarek_hip_gemm_f32}[kind]
+    per_thread = ctypes.c_void_p(2)
+    assert count(m, n, k) > 1
+
+    def product(a, b, c):
+        hip.check(entry(*(ctypes.c_void_p(t.data_ptr()) for t in (a, b, c)), m, n, k, per_thread))
+    work = [(torch.randn(m, k, device="cuda").to(dt), torch.randn(k, n, device="cuda").to(dt),
+             [torch.full((m, n), float("nan"), device="cuda") for _ in range(20)]) for _ in range(4)]
+    whole = [torch.empty(m, n, device="cuda") for _ in work]
+    torch.cuda.synchronize()
+    for (a, b, _), c in zip(work, whole):
+        product(a, b, c)
+        torch.cuda.synchronize()
+    threads = [threading.Thread(target=lambda w=w: [product(w[0], w[1], c) for c in w[2]]) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for (a, b, outs), c in zip(work, whole):
+        ref, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+        assert bool(((c.double() - ref).abs() <= (k + 32) * 2.0 ** -24 * size).all())
+        assert all(torch.equal(o, c) for o in outs)
