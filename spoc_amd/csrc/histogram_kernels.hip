@@ -152,6 +152,12 @@ __global__ __launch_bounds__(kThreads) void histogram_kernel(int *__restrict__ h
 // exactly as it leaves them.  8 bytes per key.  What is left of the atomics still sets the pace below
 // HBM speed: the 256 counters share eight cache lines, and the L2 retires about one 4-byte atomic per
 // clock and line (15 ns per tile, whatever the tile size; 64-bit atomics on counter pairs cost the same).
+// The lanes of an LDS atomic that meet on one address are served one after the other, so keys of few values (sorted keys,
+// a later digit) cost a CU by the keys it holds, and larger tiles made them slower; so a digit has Threads / 256 counters,
+// and neighbouring threads count on different ones.  Measured, one counter a digit and now, us a launch and a 1 KiB copy of
+// 3.6 us: 10^5 keys of one value 16.7 / 9.0, of 16 values 11.1 / 9.1, of 256 9.3 / 8.8; 8 10^6 keys 43.2 / 22.7, 30.3 /
+// 24.9, 22.9 / 22.7, sorted 42.0 / 21.4; 10^7 keys 54.4 / 29.2, 37.5 / 31.4, 28.5 / 28.3, sorted 53.5 / 28.2; 2^28 keys
+// 1186 / 551, 714 / 559, 584 / 576.
 // out_len guards the stores: a position outside [0, out_len) (counters that do not leave room for the
 // keys) is skipped, where the reference's kernel would write out of bounds.  The tile (Threads * Keys
 // keys) is staged in dynamic LDS.
@@ -161,15 +167,16 @@ __global__ __launch_bounds__(Threads) void radix_scatter_kernel(int *__restrict_
                                                                 const int *__restrict__ keys, int64_t n, int shift,
                                                                 int mask) {
   constexpr int kTile = Threads * Keys;
+  constexpr int kCopies = Threads / kBins;   // counters per digit: a thread has one of them to scan
   extern __shared__ int stage[];    // kTile keys, ordered by digit
-  __shared__ int count[kBins];      // keys of the tile per digit
-  __shared__ int start[kBins];      // first slot of the digit in `stage` (exclusive scan of count)
+  __shared__ int count[Threads];    // keys of the tile per digit and copy
+  __shared__ int start[Threads];    // first slot of the digit's copy in `stage` (exclusive scan of count)
   __shared__ int base[kBins];       // position in `out` of the digit's first key of this tile, less its slot
-  __shared__ int wave_total[kBins / 64];
+  __shared__ int wave_total[Threads / 64];
   const int t = threadIdx.x, lane = t & 63;
   const int64_t tile = static_cast<int64_t>(blockIdx.x) * kTile;
   const int valid = n - tile < kTile ? static_cast<int>(n - tile) : kTile;
-  if (t < kBins) count[t] = 0;
+  count[t] = 0;
   __syncthreads();
 
   // slot j of thread t is key tile + (j / 4 * Threads + t) * 4 + j % 4: 16-byte loads
@@ -192,35 +199,35 @@ __global__ __launch_bounds__(Threads) void radix_scatter_kernel(int *__restrict_
     }
   }
   auto in_tile = [&](int j) { return ((j >> 2) * Threads + t) * 4 + (j & 3) < valid; };
+  auto counter = [&](int j) { return ((key[j] >> shift) & mask) * kCopies + t % kCopies; };
 #pragma unroll
-  for (int j = 0; j < Keys; ++j)
-    rank[j] = in_tile(j) ? atomicAdd(&count[(key[j] >> shift) & mask], 1) : 0;
+  for (int j = 0; j < Keys; ++j) rank[j] = in_tile(j) ? atomicAdd(&count[counter(j)], 1) : 0;
   __syncthreads();
 
-  if (t < kBins) {
-    const int c = count[t];
-    int incl = c;
+  const int c = count[t];
+  int incl = c;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int up = __shfl_up(incl, o);
-      if (lane >= o) incl += up;
-    }
-    if (lane == 63) wave_total[t >> 6] = incl;
-    start[t] = incl - c;                       // within the wave; the waves before are added below
-    base[t] = c != 0 ? atomicAdd(&counters[t], c) : 0;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int up = __shfl_up(incl, o);
+    if (lane >= o) incl += up;
   }
+  const int of_digit = __shfl(incl, lane | (kCopies - 1)) - (incl - c);   // in the lane of the digit's first copy
+  if (lane == 63) wave_total[t >> 6] = incl;
+  int first = 0;
+  if (t % kCopies == 0 && of_digit != 0) first = atomicAdd(&counters[t / kCopies], of_digit);
   __syncthreads();
-  if (t < kBins) {
-    int before = 0;
-    for (int w = 0; w < (t >> 6); ++w) before += wave_total[w];
-    start[t] += before;
-    base[t] -= start[t];                       // slot s of digit t goes to out[base[t] + s]
-  }
+  // the waves before this one, one to a lane (all in each lane's registers took the occupancy of the 16-key tile)
+  int before = lane < (t >> 6) ? wave_total[lane] : 0;
+#pragma unroll
+  for (int o = Threads / 128; o >= 1; o >>= 1) before += __shfl_xor(before, o);
+  const int slot = incl - c + __builtin_amdgcn_readfirstlane(before);
+  start[t] = slot;
+  if (t % kCopies == 0) base[t / kCopies] = first - slot;   // slot s of the digit goes to out[base + s]
   __syncthreads();
 
 #pragma unroll
   for (int j = 0; j < Keys; ++j)
-    if (in_tile(j)) stage[start[(key[j] >> shift) & mask] + rank[j]] = key[j];
+    if (in_tile(j)) stage[start[counter(j)] + rank[j]] = key[j];
   __syncthreads();
 
   for (int s = t; s < valid; s += Threads) {
@@ -236,7 +243,7 @@ int launch_scatter(int *out, int64_t out_len, int *counters, const int *keys, in
                    hipStream_t st) {
   constexpr int kTile = Threads * Keys;
   constexpr int kLds = kTile * 4;
-  static_assert(Threads >= kBins && Threads % 64 == 0 && Keys % 4 == 0, "tile shape");
+  static_assert(Threads % kBins == 0 && 64 % (Threads / kBins) == 0 && Keys % 4 == 0, "tile shape");
   const int64_t tiles = ceil_div(n, static_cast<int64_t>(kTile));
   if (tiles > 0x7FFFFFFF) return fail(SAREK_HIP_E_INVALID_ARG, "radix scatter: vector too long for one launch");
   auto kern = radix_scatter_kernel<Threads, Keys>;
@@ -271,8 +278,8 @@ int compute_units() {
 // (2^28 keys 648 us with 16, 573 with 32).  Measured, before (512 x 16 below 2^22 keys, 1024 x 16 from there) and now, us a
 // launch and a 1 KiB copy of 3.6 us: 10007 keys 10.2 / 9.3, 1000003 10.3 / 9.6, 2560000 15.7 / 13.1, 3200001 17.2 / 14.5,
 // 4300003 18.5 / 16.9, 6000000 20.7 / 19.3, 8000000 25.1 / 23.1, 10000019 30.9 / 28.6, 13000000 39.3 / 34.2,
-// 16000000 43.5 / 39.0; 22 10^6 keys 54.2 with 16, 53.5 with 32, 50 10^6 94.2 and 109.  Keys of one value (10^7) 56.9 / 54.3,
-// of 16 values 25.1 / 26.7.
+// 16000000 43.5 / 39.0; 22 10^6 keys 54.2 with 16, 53.5 with 32, 50 10^6 94.2 and 109 (random bytes; with keys of few values
+// 16 keys are up to a sixth ahead at 8 and 16 10^6, both well ahead of what either was with one counter a digit).
 int scatter_shape(int64_t n) {
   constexpr int kShapes[] = {5, 2, 6, 7, 8, 4};   // 12, 16, 20, 24, 28, 32 keys a thread
   const int64_t round = static_cast<int64_t>(compute_units()) * 1024;

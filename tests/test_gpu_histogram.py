@@ -191,6 +191,28 @@ def test_radix_scatter_tiles_that_fit_the_rounds(hip, torch_cuda, n, shape):
     assert torch.equal(out[:n], keys.sort().values) and torch.equal(counters, ends) and bool((out[n:] == -1).all())
 
 
+@pytest.mark.parametrize("shape", [1, 2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("values,shift,mask", [(1, 0, 255), (2, 0, 255), (3, 8, 15), (256, 0, 255)])
+def test_radix_scatter_keys_of_few_values(hip, torch_cuda, oracle, shape, values, shift, mask):
+    """A digit's keys are counted in several places of a tile: one value for all keys, few, digits at both ends of the mask,
+    sorted keys, over a whole tile and a ragged one."""
+    torch = torch_cuda
+    n = 33_333
+    digits = np.linspace(mask, 0, values).astype(np.int64)[np.arange(n) * 7919 % values]
+    for keys in (digits << shift, np.sort(digits << shift)):
+        keys = (keys | (np.arange(n) << (shift + 12) & 0x7F000000)).astype(np.int32)
+        counts = np.bincount((keys >> shift) & mask, minlength=256)
+        starts = np.concatenate(([0], np.cumsum(counts)[:-1])).astype(np.int32)
+        out = torch.full((n + 64,), -1, dtype=torch.int32, device="cuda")
+        counters = torch.from_numpy(starts.copy()).cuda()
+        hip.set_tunable("radix_scatter.tile", shape)
+        try:
+            hip.radix_scatter(torch.from_numpy(keys).cuda(), out, counters, shift, mask)
+        finally:
+            hip.set_tunable("radix_scatter.tile", 0)
+        assert check_scatter(out.cpu().numpy(), counters.cpu().numpy(), keys, n, starts, shift, mask, oracle) == 0
+
+
 def test_radix_scatter_skips_positions_outside_the_output(hip, torch_cuda, oracle):
     """Counters that start 40 too high push the last keys of the last digit past the output: those
     stores are dropped (the slots behind the output keep their contents), the counters still advance."""
