@@ -24,6 +24,7 @@
 // the same pipeline on v_mfma_f32_32x32x16 in several ring and wave shapes, and variants of both MFMA kernels that leave
 // parts of the K loop out: what the power and ablation studies were measured with.  The product library has none of them.
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -1473,6 +1474,18 @@ double small_tile_time(int m, int n, int k, bool fused) {
          (splits > 1 ? 3.0 + splits * (static_cast<double>(m) * n * 4 / (1 << 20)) * 0.65 : 0.0);
 }
 
+// The same for 17 to 64 rows, from 1046 drawn products of that many (8 % rms): the slabs of a CU's workgroups, against B from
+// memory.  K that is no whole number of stages goes to the tile's ragged form.
+double narrow_tile_time(int m, int n, int k, bool fused) {
+  const double slab = k % 64 == 0 && n % 8 == 0 ? 0.128 : k % 8 == 0 && n % 8 == 0 ? 0.216 : k % 2 == 0 && n % 2 == 0 ? 0.228 : 0.276;
+  const int splits = fused ? 1 : splitk_for(m, n, k);
+  const int64_t per_cu = ceil_div(ceil_div(n, 128) * splits, compute_units());
+  const double slabs = static_cast<double>(k) / 32 / splits * slab * static_cast<double>(per_cu);
+  const double memory = static_cast<double>(k) * n * 2e-6 * 0.115, c_mb = static_cast<double>(m) * n * 4e-6;
+  return 5.06 + std::cbrt(slabs * slabs * slabs + memory * memory * memory) + 0.14 * c_mb +
+         (splits > 1 ? 3.85 + 0.22 * splits * c_mb : 0.0);
+}
+
 // Whether a product goes to the few-rows kernel, unless a knob asks for one of the tiled kernels.  gemm16.rows: 0 = by
 // size, 1 = never, 2 = wherever it can.
 inline bool few_rows(int m, int n, int k, bool fused) {
@@ -1480,8 +1493,7 @@ inline bool few_rows(int m, int n, int k, bool fused) {
   return asked != 1 && gemm16_default_kernel() && tunable("gemm16.tile", 0) == 0 && tunable("gemm16.split_k", 0) == 0 &&
          tunable("gemm16.force_simple", 0) == 0 && gemm16_rows_serves(m, n, k) &&
          !(kMeasureBuild && m > 64 && clock_probe(1)) &&   // the probe is the tiled kernels'
-        
-         (asked == 2 || gemm16_rows_pays(m, n, k, fused, small_tile_time(m, n, k, fused)));
+         (asked == 2 || gemm16_rows_pays(m, n, k, fused, small_tile_time, narrow_tile_time));
 }
 
 // The workgroup tile of the direct-to-LDS kernels for this shape under the present tunables (256 or 128), or 0 when

@@ -381,36 +381,62 @@ bool gemm16_rows_serves(int m, int n, int k) {
          static_cast<int64_t>(kTileRows) * k * 2 < 0x7FFFFFFF && shape_of(m, n, k, false).tiles * 64 < 0x7FFFFFFF;
 }
 
+// Microseconds of a product of 17 to 64 rows, by an estimate read off 1046 drawn ones (9 % rms): the steps of the CU with the
+// most workgroups by how A's and B's rows lie, against B from memory (whose stream the registers of more row blocks leave
+// fewer loads in flight), and the sums.
+double narrow_time(const Shape &s, int n, int k, int splits) {
+  const int align = k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2;
+  constexpr double kStep[] = {0.0174, 0.0146, 0.0316}, kMegabyte[] = {0.114, 0.131, 0.140};
+  const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
+  const double steps = rounds * s.steps / splits * kStep[align] * (3.9 + s.mt);
+  const double memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[align] * (1 + 0.168 * s.mt);
+  return 2.6 + 0.88 * s.mt * rounds + std::cbrt(steps * steps * steps + memory * memory * memory) +
+         (splits > 1 ? 1.3 + 0.24 * splits : 0.0);
+}
+
 // Whether it should.  Up to 16 rows always.  To 64 a workgroup's
 // sums through LDS cost it 0.5 us per 16 rows and its registers leave room for one workgroup per CU, so short K and more
 // column tiles than CUs belong to the 128 x 128 tile unless N is odd (us, 128 tile / here):
 //   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
 //   48 x 4096 x 256 6.2 / 6.1, 48 x 4096 x 1024 10.2 / 9.4, 48 x 40000 x 1024 23.0 / 26.4, 48 x 40001 x 1024 35.3 / 33.4
 //   64 x 4096 x 256 6.4 / 7.2, 64 x 4096 x 1024 10.5 / 10.5, 64 x 4096 x 4096 17.3 / 15.6, 64 x 40001 x 1024 36.3 / 37.0
+// and so does what the estimates of both kernels (narrow_other: the tile's) put 5 % apart the other way, products of one to
+// two hundred column tiles and 33 to 64 rows most of all: 64 x 20992 x 4160 31.3 / 49.4, 64 x 27136 x 2432 23.5 / 32.3,
+// 48 x 11840 x 5568 28.5 / 33.5.  Of 900 products drawn afresh 97 were more than 5 % slower here than there without the
+// estimates and 29 are with them; 11 are that much slower than they were (profiles/gemm16_rows_vs_tile.txt).  An odd N of
+// few column tiles stays here whatever they say (49 x 255 x 4129 13.5 / 15.1, 64 x 1001 x 1001 15.7 / 11.4), 17 to 32 rows
+// against up to 96 column tiles do (one of 576 more than 10 % slower), and so does a product whose pieces gemm16.rows_splits sets.
 // Beyond 64 rows, and with the fused epilogue at any number, where its tiles fit the CUs in one round (882 x 2401 x 4259,
-// 266 tiles: 50 us on the other tile, 108 here), at least half of the waves have a step, and its time is below the 128 x 128
-// tile's by both estimates.  They were read off 50 drawn products (up to 20 % and a microsecond apart from them, the
-// better kernel taken on 45, at most 8 % lost on the others): a step costs by how A's and B's rows lie, on 16 bytes, on 4, on 2.
-// `other`: what the tiled kernel is estimated at.
-bool gemm16_rows_pays(int m, int n, int k, bool fused, double other) {
-  if (m <= kTileRows && !fused) {
-    const bool odd = n % 2 != 0, one_round = (n + kCols - 1) / kCols <= compute_units();
-    switch ((m + 15) / 16) {
-      case 1: return true;
-      case 2: return odd || one_round;
-      case 3: return one_round ? odd || k >= 512 : odd && k >= 1024;
-      default: return one_round && (odd || k >= 1024);
-    }
-  }
+// 266 tiles: 50 us on the other tile, 108 here), at least half of the waves have a step (in tiles of 64 rows some wave has
+// two: 256 x 1280 x 191 6.8 / 8.4, 723 x 1702 x 256 7.2 / 7.9, as 21 of 118 drawn products, all but 3 of them so short), and its
+// time is below the 128 x 128 tile's by both estimates.  They were read off 50 drawn products (up to 20 % and a microsecond
+// apart from them, the better kernel taken on 45, at most 8 % lost on the others): a step costs by how A's and B's rows lie, on
+// 16 bytes, on 4, on 2.  `other`: what the tiled kernel is estimated at.
+bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other, Gemm16Estimate narrow_other) {
   const Shape s = shape_of(m, n, k, fused);
-  if (s.tiles > compute_units() || 2 * s.steps < kWaves) return false;
+  if (m <= kTileRows && !fused) {
+    const bool odd = n % 2 != 0, one_round = s.col_tiles <= compute_units();
+    bool here = true;
+    switch (s.mt) {
+      case 1: return true;
+      case 2: here = odd || one_round; break;
+      case 3: here = one_round ? odd || k >= 512 : odd && k >= 1024; break;
+      default: here = one_round && (odd || k >= 1024);
+    }
+    if (!here) return false;
+  }
+  if (m > 16 && m <= kTileRows && s.col_tiles > (s.mt == 2 ? 96 : n % 2 != 0 ? 8 : 0) && tunable("gemm16.rows_splits", 0) == 0 &&
+      narrow_time(s, n, k, rows_splits_for(s, n, k)) >= 1.05 * narrow_other(m, n, k, fused))
+    return false;
+  if (m <= kTileRows && !fused) return true;
+  if (s.tiles > compute_units() || 2 * s.steps < kWaves || (s.mt == 4 && s.steps <= kWaves)) return false;
   const int splits = rows_splits_for(s, n, k);
   const bool on16 = k % 8 == 0 && n % 8 == 0;
   const double step = (on16 ? 0.055 : k % 2 == 0 && n % 2 == 0 ? 0.07 : 0.12) * s.mt;
   const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
   const double here = (on16 ? 6.0 : 4.5) + rounds * s.steps / splits * step +
                       (splits > 1 ? 2.5 + 0.15 * splits + 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0);
-  return here < other;
+  return here < other(m, n, k, fused);
 }
 
 int gemm16_rows_k_splits(int m, int n, int k) { return rows_splits_for(shape_of(m, n, k, false), n, k); }
