@@ -1384,8 +1384,13 @@ inline bool small_tile_wins(int m, int n) {
 // 56.7 -> 48.7, K = 4096 157 -> 134 / 169 -> 141 / 172 -> 146; 4096 x 4100 x 4096 187 -> 155; fused 4096 x 4352 x 4096
 // 169 -> 140; 2048 x 50257 x 1024 274 -> 264.  From there on two small tiles share a CU and nothing is left to gain: 11264
 // columns 39.7 -> 39.6, 56.8 -> 55.2, 174 -> 175; 12288 40.0 -> 40.1, 59.5 -> 58.4, 177 -> 181.
-// gemm16.cut: 0 = this rule, 1 = never, s >= 2: a rest of up to s small tiles.
-inline int whole_round_columns(int m, int n) {
+// A short K, and the more so the more rounds there are (their tiles no longer end together, and some CUs take the few that are
+// over while others finish), gives the second launch nothing to win: 7232 x 13568 (6 rounds) K = 82 85.0 -> 91.2, 512 128 ->
+// 132; 3712 x 39176 (9 rounds) 82 149 -> 155, 768 302 -> 313; 4160 x 8000 (2 rounds) 126 39.2 -> 42.2, 768 66.8 -> 64.7;
+// 2048 x 8448 (1 round) 82 22.6 -> 22.2, 256 24.9 -> 23.9.  So K has to be 128 times the whole rounds: of 417 drawn products
+// of up to 8192 rows the cut cost 48 more than 2 % without that and costs 6 with it.
+// gemm16.cut: 0 = this rule, 1 = never, s >= 2: a rest of up to s small tiles, whatever K.
+inline int whole_round_columns(int m, int n, int k) {
   const int64_t asked = tunable("gemm16.cut", 0);
   if (asked == 1 || tunable("gemm16.tile", 0) != 0) return n;
   const int cus = compute_units();
@@ -1393,7 +1398,16 @@ inline int whole_round_columns(int m, int n) {
   const int64_t columns = tiles_n - ceil_div(over, tiles_m);
   if (over == 0 || columns < 1) return n;
   const int64_t rest = ceil_div(m, 128) * ceil_div(n - columns * 256, 128);
+  if (asked < 2 && k < tiles_m * tiles_n / cus * 128) return n;
   return rest <= (asked >= 2 ? asked : cus) ? static_cast<int>(columns * 256) : n;
+}
+
+// The columns that are left to the tiles when gemm16_last_column_kernel takes the last one: n - 1 for N = 1 and for whole
+// tile columns and one column more that would add a round of workgroups (4096 x 4097 x 4096: 139 us against 184).
+inline int tiled_columns(int m, int n, int tile) {
+  const int64_t slots = compute_units() * (tile == 128 ? 2 : 1);
+  auto rounds = [&](int columns) { return ceil_div(ceil_div(m, tile) * ceil_div(columns, tile), slots); };
+  return n % tile == 1 && (n == 1 || rounds(n) > rounds(n - 1)) ? n - 1 : n;
 }
 
 // Column N-1 of C alone, one wave per row, with the same epilogue: N = 1, and an N of whole tiles and one column whose
@@ -1606,13 +1620,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   const int tile_choice = gemm16_tile_for(m, n, k);
   const bool ab16 = reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
   const bool tiled = tile_choice != 0 && (k >= 64 || ab16);
-  // whole tile columns and one column more: that one goes to a kernel of its own where a tile column would add a round of
-  // workgroups (4096 x 4097 x 4096: 139 us against 184), and for N = 1
-  const int tile_slots = compute_units() * (tile_choice == 128 ? 2 : 1);
-  auto rounds = [&](int columns) {
-    return ((m + tile_choice - 1) / tile_choice * ceil_div(columns, tile_choice) + tile_slots - 1) / tile_slots;
-  };
-  const int nm = tiled && n % tile_choice == 1 && (n == 1 || rounds(n) > rounds(n - 1)) ? n - 1 : n;
+  const int nm = tiled ? tiled_columns(m, n, tile_choice) : n;
 
   // Row sums: every tile column (every 64 columns of the simple kernel; the last column on its own) leaves its share of
   // each row in a plane of its own, and rowsum_fold_kernel adds the planes in column order, in double, with one rounding:
@@ -1620,7 +1628,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   // stream capture, past the sixteenth stream, planes beyond the block's size) adds with atomicAdd in arrival order.
   float *planes = nullptr;
   int n_planes = 0;
-  const int cut = tiled && tile_choice == 256 && nm > 0 && !(kMeasureBuild && clock_probe(1)) ? whole_round_columns(m, nm) : nm;
+  const int cut = tiled && tile_choice == 256 && nm > 0 && !(kMeasureBuild && clock_probe(1)) ? whole_round_columns(m, nm, k) : nm;
   if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
     n_planes = tiled ? (cut + tile_choice - 1) / tile_choice + (nm - cut + 127) / 128 + (n - nm) : (n + 63) / 64;
     if (static_cast<int64_t>(n_planes) * m * 4 <= static_cast<int64_t>(kSplitWorkspaceBytes)) planes = splitk_workspace(st);
@@ -1733,6 +1741,13 @@ extern "C" {
 
 int sarek_hip_gemm16_tile(int m, int n, int k) {
   return m >= 1 && n >= 1 && few_rows(m, n, k, false) ? 64 : gemm16_tile_for(m, n, k);
+}
+
+int sarek_hip_gemm16_tile_columns(int m, int n, int k) {
+  const int tile = sarek_hip_gemm16_tile(m, n, k);
+  if (tile != 256 && tile != 128) return n;
+  const int columns = tiled_columns(m, n, tile);
+  return tile == 256 && columns > 0 ? whole_round_columns(m, columns, k) : columns;
 }
 
 int sarek_hip_gemm16_k_splits(int m, int n, int k) {

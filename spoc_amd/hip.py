@@ -147,6 +147,7 @@ SYMBOLS = {
     "sarek_hip_gemm_f32_k_splits": (_i, [_i, _i, _i]),
     "sarek_hip_gemm16_tile": (_i, [_i, _i, _i]),
     "sarek_hip_gemm16_k_splits": (_i, [_i, _i, _i]),
+    "sarek_hip_gemm16_tile_columns": (_i, [_i, _i, _i]),
     "sarek_hip_gemm_f16_bias_relu_rowsum": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "sarek_hip_cast_f32_to_bf16": (_i, [_vp, _vp, _i64, _vp]),
     "sarek_hip_cast_f32_to_f16": (_i, [_vp, _vp, _i64, _vp]),
@@ -748,6 +749,11 @@ def gemm_bf16(a, b, out=None):
 def gemm16_tile(m, n, k):
     """256 / 128: the workgroup tile the 16-bit GEMMs take for this shape now; 64: the few-rows kernel; 0: the simple kernel."""
     return int(lib.sarek_hip_gemm16_tile(m, n, k))
+
+
+def gemm16_tile_columns(m, n, k):
+    """How many of the n columns that tile takes; the rest goes to the 128 x 128 tile or, one column, to a kernel of its own."""
+    return int(lib.sarek_hip_gemm16_tile_columns(m, n, k))
 
 
 def gemm16_k_splits(m, n, k):

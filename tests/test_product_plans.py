@@ -48,6 +48,21 @@ def test_16_bit_products_of_few_rows_go_where_they_are_faster(hip, m, n, k, kern
     assert hip.gemm16_tile(m, n, k) == kernel
 
 
+@pytest.mark.parametrize("m,n,k,columns", [
+    (2048, 8448, 4096, 8192), (2048, 8448, 128, 8192), (2048, 8448, 127, 8448), (2048, 50257, 1024, 49152), (2048, 12288, 4096, 12288),
+    (7232, 13568, 82, 13568), (7232, 13568, 767, 13568), (7232, 13568, 768, 52 * 256), (3712, 39176, 768, 39176),
+    (4160, 8000, 126, 8000), (4160, 8000, 256, 30 * 256), (4096, 4097, 4096, 4096), (8192, 8192, 8192, 8192), (100, 1, 64, 0),
+    (16, 8192, 8192, 8192)])
+def test_columns_past_whole_rounds_of_large_tiles(hip, knobs, m, n, k, columns):
+    """The cut wants K to be 128 times the whole rounds of workgroups; gemm16.cut = 1 never cuts, a count cuts whatever K."""
+    assert hip.gemm16_tile_columns(m, n, k) == columns
+    knobs("gemm16.cut", 1)
+    assert hip.gemm16_tile_columns(m, n, k) == (n if n not in (1, 4097) else n - 1)
+    if (m, n) in ((2048, 8448), (4160, 8000), (7232, 13568)):
+        knobs("gemm16.cut", 256)
+        assert hip.gemm16_tile_columns(m, n, k) < n
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("value", [2, 34])
 def test_f32_direct_knob_of_no_variant_computes_the_same_product(hip, torch_cuda, knobs, value):
