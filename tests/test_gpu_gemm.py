@@ -385,33 +385,41 @@ def test_gemm16_both_tile_sizes(hip, oracle, torch_cuda, kind, m, n, k):
     assert np.array_equal(got[128], got[256])
 
 
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(2048, 8448, 64), (2047, 8195, 72), (1921, 8703, 131), (2048, 10240, 65),
                                    (8192, 2050, 70), (2300, 7425, 200)])
-def test_gemm16_columns_past_whole_rounds_of_large_tiles(hip, oracle, torch_cuda, m, n, k):
-    """Products whose last round of 256 x 256 tiles would hold few: its columns go to the 128 x 128 tile.  The same bits as
-    without the cut, rows of the result against the oracle, the row sums against those of y, nothing stored outside."""
+def test_gemm16_columns_past_whole_rounds_of_large_tiles(hip, oracle, torch_cuda, kind, m, n, k):
+    """Products whose last round of 256 x 256 tiles would hold few: its columns go to the 128 x 128 tile (reported as columns
+    that the large tile does not keep).  The same bits as without the cut, rows of the result against the oracle, the row
+    sums of both against those of y, nothing stored outside."""
     torch = torch_cuda
-    a, b = normal16(oracle, (m, k), m + 3, "f16"), normal16(oracle, (k, n), n + 4, "f16")
+    a, b = normal16(oracle, (m, k), m + 3, kind), normal16(oracle, (k, n), n + 4, kind)
     bias = oracle.fill_uniform(n, seed=n + 2, lo=-0.1, hi=0.1)
-    da, db, dbias = dev(torch, a).half(), dev(torch, b).half(), dev(torch, bias)
+    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    da, db, dbias = dev(torch, a).to(dt), dev(torch, b).to(dt), dev(torch, bias)
     assert hip.gemm16_tile(m, n, k) == 256
     got = []
     try:
-        for cut in (0, 1):
+        for cut in (256, 1):
             hip.set_tunable("gemm16.cut", cut)
+            columns = hip.gemm16_tile_columns(m, n, k)
+            assert columns % 256 == 0 and 0 < columns < n if cut == 256 else columns == n
             guard = torch.full((m * n + 64,), 7.0, device="cuda")
             c = guard[32:32 + m * n].view(m, n)
-            hip.gemm_f16(da, db, out=c)
+            (hip.gemm_bf16 if kind == "bf16" else hip.gemm_f16)(da, db, out=c)
             assert bool((guard[:32] == 7).all()) and bool((guard[32 + m * n:] == 7).all())
-            got.append((c,) + hip.gemm_f16_bias_relu_rowsum(da, db, dbias))
+            got.append((c,) + (hip.gemm_f16_bias_relu_rowsum(da, db, dbias) if kind == "f16" else ()))
     finally:
         hip.set_tunable("gemm16.cut", 0)
-    (c, y, rs), (c1, y1, _) = got
-    assert torch.equal(c, c1) and torch.equal(y, y1)
+    assert torch.equal(got[0][0], got[1][0])
     rows = np.r_[0:3, m // 2, m - 3:m]
     ref = oracle.gemm(np.ascontiguousarray(a[rows]), b)
-    assert np.abs(c[dev(torch, rows)].cpu().numpy() - ref).max() / np.abs(ref).max() < 1e-4
-    assert rowsums_ok(rs.cpu().numpy(), y.double().sum(1).cpu().numpy())
+    assert np.abs(got[0][0][dev(torch, rows)].cpu().numpy() - ref).max() / np.abs(ref).max() < 1e-4
+    if kind == "f16":
+        (_, y, rs), (_, y1, rs1) = got
+        assert torch.equal(y, y1)
+        for sums in (rs, rs1):
+            assert rowsums_ok(sums.cpu().numpy(), y.double().sum(1).cpu().numpy())
 
 
 def test_gemm16_tile_choice_by_shape(hip, torch_cuda):
