@@ -17,7 +17,7 @@
 //   gemm16_m16_small_kernel: the same pipeline on a 128 x 128 tile (4 waves), two workgroups per CU, for products
 //     that do not fill the chip with large tiles; K split over several workgroups per tile where tiles are few.
 //   gemm16_last_column_kernel: N = 1, and the column by which some N exceed whole tiles.
-//   gemm16_rows_kernel (gemm16_rows.hip): plain products of at most 64 rows.
+//   gemm16_rows_kernel (gemm16_rows.hip): products of few tiles, plain or fused, in tiles of at most 64 rows.
 //   gemm16_simple_kernel: any shape and alignment, one thread per C element (K below one LDS stage that is not a
 //     multiple of 8, or operands whose 256-row / 64-row panels span 2 GiB).
 // A build with -DSAREK_HIP_MEASURE (libsarek_hip_measure.so, for bench.py --measure-build) also holds gemm16_dma_kernel,
@@ -436,23 +436,6 @@ __global__ __launch_bounds__(64 * 2 * (8 / TJ)) void gemm16_dma_kernel(const uin
 
 #endif  // SAREK_HIP_MEASURE
 
-// ---- direct-to-LDS kernel on v_mfma_f32_16x16x32 ---------------------------------------
-// The same tile, rings and transfers as gemm16_dma_kernel<.., 64, 32, 2, 4, 2> (256 x 256 per workgroup, 8 waves
-// of 128 x 64, A in 2 stages of K = 64, B in 4 slabs of K = 32, one barrier per B slab), but the products go
-// through the 16 x 16 x 32 instruction: 8 x 4 accumulator tiles of 16 x 16 per wave instead of 4 x 2 of 32 x 32.
-// On N(0, 0.02) data under the package power limit a bare stream of the 16 x 16 x 32 instruction runs 17 % faster
-// than one of the 32 x 32 x 16 instruction (2.09 against 1.79 PFLOP/s; on zeros both reach 2.45): it writes half as
-// many accumulator values per flop.  The LDS bytes read per flop are the same (the wave tile is).
-//
-// Operands: lane (m = lane%16, g = lane/16) supplies k = 8g..8g+7 of row m (A) / column m (B) and receives
-// rows 4g..4g+3 of column m of the 16 x 16 result.
-//   A: one ds_read_b128 per 16-row tile: chunk 4*ks + g of the row (ks = the B slab's place in the A stage).
-//   B: two ds_read_b64_tr_b16 per 16-column tile: rows 8g + {0..3} and 8g + {4..7} of the slab, 16 columns.
-//      A 32-lane phase of that read holds two k groups (rows r and r + 8): the B swizzle of the 32 x 32 kernel
-//      (slot ^= (row & 3) << 2, rows 64 bytes apart) is extended by slot ^= ((row >> 3) & 1) << 1, which puts
-//      the second group on the other 32-byte half of each 64-byte piece.
-// A slab is worked in two units of 16 MFMAs (rows 0-63 of the wave tile, then rows 64-127, same B fragments);
-// the barrier sits between them, and the second unit covers the fragment reads of the next slab.
 template <bool Bf16>
 __device__ __forceinline__ float widen16(uint16_t bits) {
   if constexpr (Bf16) return __uint_as_float(static_cast<uint32_t>(bits) << 16);
@@ -595,6 +578,23 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
   }
 }
 
+// ---- direct-to-LDS kernel on v_mfma_f32_16x16x32 ---------------------------------------
+// The same tile, rings and transfers as gemm16_dma_kernel<.., 64, 32, 2, 4, 2> (256 x 256 per workgroup, 8 waves
+// of 128 x 64, A in 2 stages of K = 64, B in 4 slabs of K = 32, one barrier per B slab), but the products go
+// through the 16 x 16 x 32 instruction: 8 x 4 accumulator tiles of 16 x 16 per wave instead of 4 x 2 of 32 x 32.
+// On N(0, 0.02) data under the package power limit a bare stream of the 16 x 16 x 32 instruction runs 17 % faster
+// than one of the 32 x 32 x 16 instruction (2.09 against 1.79 PFLOP/s; on zeros both reach 2.45): it writes half as
+// many accumulator values per flop.  The LDS bytes read per flop are the same (the wave tile is).
+//
+// Operands: lane (m = lane%16, g = lane/16) supplies k = 8g..8g+7 of row m (A) / column m (B) and receives
+// rows 4g..4g+3 of column m of the 16 x 16 result.
+//   A: one ds_read_b128 per 16-row tile: chunk 4*ks + g of the row (ks = the B slab's place in the A stage).
+//   B: two ds_read_b64_tr_b16 per 16-column tile: rows 8g + {0..3} and 8g + {4..7} of the slab, 16 columns.
+//      A 32-lane phase of that read holds two k groups (rows r and r + 8): the B swizzle of the 32 x 32 kernel
+//      (slot ^= (row & 3) << 2, rows 64 bytes apart) is extended by slot ^= ((row >> 3) & 1) << 1, which puts
+//      the second group on the other 32-byte half of each 64-byte piece.
+// A slab is worked in two units of 16 MFMAs (rows 0-63 of the wave tile, then rows 64-127, same B fragments);
+// the barrier sits between them, and the second unit covers the fragment reads of the next slab.
 template <bool Bf16, int Epi, int Ablate = 0, bool Ragged = false, bool HalfBarriers = false>
 __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                          float *__restrict__ C, const float *__restrict__ bias,

@@ -236,7 +236,8 @@ bool gemm_f32_direct_serves(int m, int n, int k) {
 }
 
 // Up to 10 GFLOP: above, the LDS kernel is level at best (1280 x 2712 x 1792, 12 GFLOP: 134 us here, 104 there;
-// 2049 x 4097 x 3000, 50: 437 and 430).
+// 2049 x 4097 x 3000, 50: 437 and 430), but for products that leave its tiles a round nearly empty (578 x 3308 x 5773, 22 GFLOP,
+// 520 tiles of 64 x 64: 183 us here, 305 there; profiles/gemm_f32_plans.txt has more).
 bool gemm_f32_direct_pays(int m, int n, int k) { return static_cast<double>(m) * n * k <= 5e9; }
 
 // At most `splits` pieces of K: of whole steps, none empty, their planes within the workspace and a ticket per tile.

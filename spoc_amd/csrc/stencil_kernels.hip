@@ -126,10 +126,10 @@ __device__ __forceinline__ void zero_row(float *__restrict__ out, int w, int y, 
 // untouched.  Box = true: the mean of the 3 x 3 cells round (x, y) there, 0 on the border.  4 * blockIdx.x + wave is
 // the strip, blockIdx.y the band of `rows` output rows.  Every lane of a wave stays in the loop (the shuffles need
 // them all); lanes past the last column neither load nor store.  Four rows are asked for before any is used: a band of
-// four (the usual one) brings all its six input rows in one trip to memory, where two at a time take two more.  With
-// the divide of the sums by `over`, start of the change / two rows / four, us a call: box filter 2048 x 2048 9.5 / 8.4 /
-// 8.1, 8192 x 8192 104 / 97 / 97, 1001 x 3001 8.6 / 7.8 / 7.3, 4096 x 2048 (bands of 8) 16.7 / 13.8 / 13.5; mean of five
-// 2048 x 2048 8.9 / 8.3 / 7.7.
+// four (the usual one) brings all its six input rows in one trip to memory, where two at a time take two more.  Two rows
+// and a full divide / four and `over`, us a launch back to back over one pair of grids: box filter 2048 x 2048 7.4 / 6.2, 8192 x
+// 8192 86 / 83, 1001 x 3001 7.3 / 6.1, 4096 x 2048 (bands of 8) 14.3 / 12.6; mean of five 2048 x 2048 6.5 / 5.6, 8192 x 8192
+// 92 / 83.  Over inputs that change from launch to launch the box filter of 2048 x 2048 takes 8.8 / 7.7.
 template <bool Box>
 __global__ __launch_bounds__(kBlock) void neighbourhood_kernel(const float *__restrict__ in, float *__restrict__ out,
                                                                int w, int h, int rows) {
