@@ -345,10 +345,11 @@ int launch(const Call &q, const Shape &s) {
   }
   float *partials = splits > 1 ? block + s.rs_floats : nullptr;
   unsigned *tickets = splits > 1 ? splitk_tickets(block) : nullptr;
-  // B past the caches from 64 MiB on where its rows are whole 16-byte pieces (100 MB: 20.2 us against 22.8, 134 MB: 26.4
+  // B past the caches from 64 MiB on where its rows are whole 128-byte lines (100 MB: 20.2 us against 22.8, 134 MB: 26.4
   // against 28.0, 34 MB: 15.8 against 13.2); rows at other offsets share lines between neighbouring loads, and lose
-  // (100 MB: 28.4 against 28.0), and so does what several row tiles read
-  const bool nt = s.row_tiles == 1 && q.n % 8 == 0 && static_cast<int64_t>(q.k) * q.n * 2 > (int64_t{64} << 20);
+  // (16 x 30000 x 4096 53.1 against 49.9, 8 x 24632 x 3072 35.2 and 33.4, 16 x 22000 x 1536 18.2 and 17.5, operands new to the
+  // caches), and so does what several row tiles read
+  const bool nt = s.row_tiles == 1 && q.n % 64 == 0 && static_cast<int64_t>(q.k) * q.n * 2 > (int64_t{64} << 20);
   const dim3 grid(static_cast<unsigned>(s.tiles * splits)), block_dim(64 * kWaves);
   if (nt)
     hipLaunchKernelGGL((gemm16_rows_kernel<Bf16, MT, kNonTemporal, Fused>), grid, block_dim, 0, q.st, q.a, q.b, q.c, q.bias,
@@ -394,7 +395,9 @@ double narrow_time(const Shape &s, int n, int k, int splits) {
          (splits > 1 ? 1.3 + 0.24 * splits : 0.0);
 }
 
-// Whether it should.  Up to 16 rows always.  To 64 a workgroup's
+// Whether it should.  Up to 16 rows always, but for more than 128 MiB of B in one piece of K whose rows, of an even N, share
+// lines: there the tile's transfers into LDS come in better (16 x 30000 x 4096 43.2 on the tile, 49.9 here; elsewhere the tile was
+// the faster by 4 % on 4 of 400 drawn products, operands new to the caches, this kernel by a quarter on average).  To 64 a workgroup's
 // sums through LDS cost it 0.5 us per 16 rows and its registers leave room for one workgroup per CU, so short K and more
 // column tiles than CUs belong to the 128 x 128 tile unless N is odd (us, 128 tile / here):
 //   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
@@ -418,7 +421,9 @@ bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other, Gem
     const bool odd = n % 2 != 0, one_round = s.col_tiles <= compute_units();
     bool here = true;
     switch (s.mt) {
-      case 1: return true;
+      case 1:
+        return n % 64 == 0 || odd || static_cast<int64_t>(k) * n * 2 <= (int64_t{128} << 20) || rows_splits_for(s, n, k) > 1 ||
+               tunable("gemm16.rows_splits", 0) != 0;
       case 2: here = odd || one_round; break;
       case 3: here = one_round ? odd || k >= 512 : odd && k >= 1024; break;
       default: here = one_round && (odd || k >= 1024);
