@@ -1488,16 +1488,17 @@ double small_tile_time(int m, int n, int k, bool fused) {
          (splits > 1 ? 3.0 + splits * (static_cast<double>(m) * n * 4 / (1 << 20)) * 0.65 : 0.0);
 }
 
-// The same for 17 to 64 rows, from 1046 drawn products of that many (8 % rms): the slabs of a CU's workgroups, against B from
-// memory.  K that is no whole number of stages goes to the tile's ragged form.
+// The same for 17 to 64 rows and a B that is new to the caches, from 800 drawn products of that many (8 % rms): the slabs of a
+// CU's workgroups, against B from memory.  K that is no whole number of stages goes to the tile's ragged form.
 double narrow_tile_time(int m, int n, int k, bool fused) {
-  const double slab = k % 64 == 0 && n % 8 == 0 ? 0.128 : k % 8 == 0 && n % 8 == 0 ? 0.216 : k % 2 == 0 && n % 2 == 0 ? 0.228 : 0.276;
+  const int align = k % 64 == 0 && n % 8 == 0 ? 0 : k % 8 == 0 && n % 8 == 0 ? 1 : k % 2 == 0 && n % 2 == 0 ? 2 : 3;
+  constexpr double kSlab[] = {0.172, 0.257, 0.272, 0.334}, kMegabyte[] = {0.156, 0.125, 0.134, 0.155};
   const int splits = fused ? 1 : splitk_for(m, n, k);
   const int64_t per_cu = ceil_div(ceil_div(n, 128) * splits, compute_units());
-  const double slabs = static_cast<double>(k) / 32 / splits * slab * static_cast<double>(per_cu);
-  const double memory = static_cast<double>(k) * n * 2e-6 * 0.115, c_mb = static_cast<double>(m) * n * 4e-6;
-  return 5.06 + std::cbrt(slabs * slabs * slabs + memory * memory * memory) + 0.14 * c_mb +
-         (splits > 1 ? 3.85 + 0.22 * splits * c_mb : 0.0);
+  const double slabs = static_cast<double>(k) / 32 / splits * kSlab[align] * static_cast<double>(per_cu);
+  const double memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[align], c_mb = static_cast<double>(m) * n * 4e-6;
+  return 5.17 + std::cbrt(slabs * slabs * slabs + memory * memory * memory) + 0.28 * c_mb +
+         (splits > 1 ? 4.0 + 0.38 * splits * c_mb : 0.0);
 }
 
 // Whether a product goes to the few-rows kernel, unless a knob asks for one of the tiled kernels.  gemm16.rows: 0 = by

@@ -382,17 +382,17 @@ bool gemm16_rows_serves(int m, int n, int k) {
          static_cast<int64_t>(kTileRows) * k * 2 < 0x7FFFFFFF && shape_of(m, n, k, false).tiles * 64 < 0x7FFFFFFF;
 }
 
-// Microseconds of a product of 17 to 64 rows, by an estimate read off 1046 drawn ones (9 % rms): the steps of the CU with the
+// Microseconds of a product of 17 to 64 rows whose B is new to the caches, by an estimate read off 800 drawn ones (9 % rms): the steps of the CU with the
 // most workgroups by how A's and B's rows lie, against B from memory (whose stream the registers of more row blocks leave
 // fewer loads in flight), and the sums.
 double narrow_time(const Shape &s, int n, int k, int splits) {
   const int align = k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2;
-  constexpr double kStep[] = {0.0174, 0.0146, 0.0316}, kMegabyte[] = {0.114, 0.131, 0.140};
+  constexpr double kStep[] = {0.0125, 0.0147, 0.0288}, kMegabyte[] = {0.124, 0.147, 0.164};
   const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
-  const double steps = rounds * s.steps / splits * kStep[align] * (3.9 + s.mt);
-  const double memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[align] * (1 + 0.168 * s.mt);
-  return 2.6 + 0.88 * s.mt * rounds + std::cbrt(steps * steps * steps + memory * memory * memory) +
-         (splits > 1 ? 1.3 + 0.24 * splits : 0.0);
+  const double steps = rounds * s.steps / splits * kStep[align] * (4.0 + s.mt);
+  const double memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[align] * (1 + 0.182 * s.mt);
+  return 2.94 + 0.97 * s.mt * rounds + std::cbrt(steps * steps * steps + memory * memory * memory) +
+         (splits > 1 ? 1.17 + 0.31 * splits : 0.0);
 }
 
 // Whether it should.  Up to 16 rows always, but for more than 128 MiB of B in one piece of K whose rows, of an even N, share
@@ -403,10 +403,11 @@ double narrow_time(const Shape &s, int n, int k, int splits) {
 //   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
 //   48 x 4096 x 256 6.2 / 6.1, 48 x 4096 x 1024 10.2 / 9.4, 48 x 40000 x 1024 23.0 / 26.4, 48 x 40001 x 1024 35.3 / 33.4
 //   64 x 4096 x 256 6.4 / 7.2, 64 x 4096 x 1024 10.5 / 10.5, 64 x 4096 x 4096 17.3 / 15.6, 64 x 40001 x 1024 36.3 / 37.0
-// and so does what the estimates of both kernels (narrow_other: the tile's) put 5 % apart the other way, products of one to
-// two hundred column tiles and 33 to 64 rows most of all: 64 x 20992 x 4160 31.3 / 49.4, 64 x 27136 x 2432 23.5 / 32.3,
-// 48 x 11840 x 5568 28.5 / 33.5.  Of 900 products drawn afresh 97 were more than 5 % slower here than there without the
-// estimates and 29 are with them; 11 are that much slower than they were (profiles/gemm16_rows_vs_tile.txt).  An odd N of
+// and so does what the estimates of both kernels (narrow_other: the tile's) put 5 % apart the other way, B being new to the
+// caches as in a program's loop over its weights (again and again the same B favours the tile more): 33 to 64 rows against one
+// to two hundred column tiles most of all (us, tile / here): 64 x 29028 x 2725 45.2 / 51.8, 51 x 7969 x 5857 29.5 / 34.4.  Of
+// 900 products drawn afresh 85 were more than 5 % slower here than there without the estimates and 43 are with them; nine are
+// that much slower than they were, by at most 15 % (profiles/gemm16_rows_vs_tile.txt).  An odd N of
 // few column tiles stays here whatever they say (49 x 255 x 4129 13.5 / 15.1, 64 x 1001 x 1001 15.7 / 11.4), 17 to 32 rows
 // against up to 96 column tiles do (one of 576 more than 10 % slower), and so does a product whose pieces gemm16.rows_splits sets.
 // Beyond 64 rows, and with the fused epilogue at any number, where its tiles fit the CUs in one round (882 x 2401 x 4259,
