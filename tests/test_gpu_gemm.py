@@ -534,6 +534,53 @@ def test_gemm16_split_k_under_graph_capture(hip, torch_cuda):
         assert torch.equal(got, want), seed
 
 
+@pytest.mark.parametrize("kind,m,n,k", [("bf16", 16, 512, 8192), ("f32", 68, 119, 3328), ("fused", 128, 1024, 4246)])
+def test_products_cut_along_k_without_lds_under_graph_capture(hip, torch_cuda, kind, m, n, k):
+    """The kernels that add their own K pieces by tickets, captured after they have run on the stream: a graph holds no
+    address of that stream's block, so K is whole there; replays beside eager calls on the same stream give the product of
+    the inputs of that moment.  Bound as for the kernels: an addition is off by half an ulp."""
+    torch = torch_cuda
+    torch.manual_seed(m + n + k)
+    dt = {"bf16": torch.bfloat16, "f32": torch.float32, "fused": torch.float16}[kind]
+    assert (hip.gemm_f32_k_splits if kind == "f32" else hip.gemm16_k_splits)(m, n, k) > 1
+    a, b, bias = torch.empty(m, k, device="cuda", dtype=dt), torch.empty(k, n, device="cuda", dtype=dt), torch.rand(n, device="cuda")
+    c, rs = torch.empty(m, n, device="cuda"), torch.empty(m, device="cuda")
+
+    def product(out, sums):
+        if kind == "fused":
+            hip.gemm_f16_bias_relu_rowsum(a, b, bias, out=out, rowsum=sums)
+        else:
+            {"bf16": hip.gemm_bf16, "f32": hip.gemm_f32}[kind](a, b, out=out)
+
+    def fill():
+        a.copy_(torch.randn(m, k, device="cuda") * 0.02)
+        b.copy_(torch.randn(k, n, device="cuda") * 0.02)
+    fill()
+    stream = side_stream(torch)
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        product(c, rs)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            product(c, rs)
+        for _ in range(3):
+            fill()
+            eager, eager_rs = torch.empty_like(c), torch.empty_like(rs)
+            c.fill_(float("nan"))
+            graph.replay()
+            product(eager, eager_rs)
+            graph.replay()
+            torch.cuda.synchronize()
+            ref, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+            if kind == "fused":
+                ref, size = (ref + bias.double()).relu(), size + bias.double().abs()
+            for got, sums in ((c, rs), (eager, eager_rs)):
+                assert bool(((got.double() - ref).abs() <= (k + 33) * 2.0 ** -24 * size).all())
+                if kind == "fused":
+                    assert bool(((sums.double() - ref.sum(1)).abs() <= (k + n) * 2.0 ** -24 * size.sum(1)).all())
+
+
 RAGGED_SHAPES = [(1, 1, 8), (3, 5, 8), (37, 51, 24), (130, 137, 40), (256, 255, 64), (257, 1001, 1000),
                  (300, 262, 136), (512, 514, 4104), (777, 1003, 328), (64, 4100, 96), (1000, 3, 2056),
                  (130, 137, 65), (257, 1001, 1001), (300, 263, 75), (64, 65, 67), (512, 514, 4107), (33, 40, 127),
