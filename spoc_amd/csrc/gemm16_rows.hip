@@ -3,8 +3,8 @@
 //
 // What bounds it: B is read once and used M times, so the product is a read of B (16 x 8192 x 8192: 134 MB, 21 us at the
 // 6.3 TB/s large streams reach here) and a CU draws at most about 39 GB/s of L2 misses, so every CU has to take its
-// share.  The 128 x 128 tile of gemm16_m16_small_kernel fetches 128 rows of A whatever M is, adds its K pieces in a
-// second launch, and with an odd N runs the last column as a launch of its own.  Here:
+// share.  The 128 x 128 tile of gemm16_m16_small_kernel fetches 128 rows of A whatever M is and adds its K pieces in a
+// second launch.  Here:
 //   - No LDS on the way in.  A wave takes steps of 32 k x 128 columns of B, 8 KiB in eight 16-byte loads per lane: lane
 //     (l, g) = (lane % 16, lane / 16) gets rows 8g .. 8g+7 at columns 8l .. 8l+7.  v_perm_b32 turns that 8 x 8 block into
 //     eight operands of v_mfma_f32_16x16x32 (column 8l + c over k = 8g .. 8g+7, c = 0 .. 7), four instructions each; A's
@@ -15,7 +15,7 @@
 //     the same bits on every run.
 //   - Workgroups start at different places of their piece: A's rows are a power of two apart in the usual case, and in
 //     step all workgroups would read them from the same L2 channels (64 x 8192 x 8192: 51 us in step, 38 rotated).
-// Measured, before (the 128 x 128 tile) and now, launches back to back on rotating operands:
+// Measured, before (the 128 x 128 tile, which then took the last column of an odd N in a launch of its own) and now, launches back to back on rotating operands:
 //   16 x 8192 x 8192 34.5 -> 25.7 us (5.2 TB/s), 16 x 2048 x 2048 10.4 -> 6.8, 16 x 40000 x 1024 21.1 -> 19.6,
 //   32 x 16384 x 4096 32.9 -> 27.4, 48 x 4096 x 4096 17.2 -> 13.8, 16 x 256 x 8192 12.8 -> 7.4; odd sizes:
 //   10 x 4161 x 4221 80 -> 12.6, 64 x 4097 x 4103 74 -> 20.5, 8 x 50257 x 1024 34.5 -> 28.0.
