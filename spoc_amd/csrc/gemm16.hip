@@ -442,19 +442,19 @@ __device__ __forceinline__ float widen16(uint16_t bits) {
   else return static_cast<float>(__builtin_bit_cast(_Float16, bits));
 }
 
-// Zeroes the first `count` (0 .. 7, the lane's own) of the eight elements this lane brought to each of its places of an A stage.
-// The caller has waited for the transfers and passes a barrier afterwards: no other wave reads the stage in between.  Once
-// a tile; a mask on the fragments instead would be in every turn of the K loop.
+// Zeroes all but the first `keep` (1 .. 7; 0: nothing to do) of the eight elements this lane brought to each of its places
+// of an A stage.  The caller has waited for the transfers and passes a barrier afterwards: no other wave reads the stage in
+// between.
 template <int DA, int NWAVES>
-__device__ __forceinline__ void clear_piece_heads(char *sa, int wave, int lane, int count) {
-  if (count > 0) {
-    u32x4 keep;
+__device__ __forceinline__ void clear_piece_tails(char *sa, int wave, int lane, int keep) {
+  if (keep > 0) {
+    u32x4 mask;
 #pragma unroll
-    for (int d = 0; d < 4; ++d) keep[d] = count <= 2 * d ? 0xFFFFFFFFu : count == 2 * d + 1 ? 0xFFFF0000u : 0u;
+    for (int d = 0; d < 4; ++d) mask[d] = keep >= 2 * d + 2 ? 0xFFFFFFFFu : keep == 2 * d + 1 ? 0x0000FFFFu : 0u;
 #pragma unroll
     for (int i = 0; i < DA; ++i) {
       u32x4 *piece = reinterpret_cast<u32x4 *>(sa + (wave + NWAVES * i) * 1024 + lane * 16);
-      *piece = *piece & keep;
+      *piece = *piece & mask;
     }
   }
   wait_lds();
@@ -655,34 +655,22 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   const char *a_base = reinterpret_cast<const char *>(A + static_cast<int64_t>(m0) * K);
   const char *b_base = reinterpret_cast<const char *>(B);
   const int64_t b_slab_bytes = static_cast<int64_t>(BKB) * ld * 2;
-  // Ragged: K need not fill the last A stage.  A lane whose offset lies outside the buffer resource's range brings
-  // zeros into LDS, so k that must not count are a per-lane choice between the usual offset and one past the range.
-  // From one whole stage on (K >= 64) the last stage is moved back to end at K: its A pieces then hold nothing but
-  // elements of their own rows, at whatever alignment, and the k it shares with the stage before it are sent out of
-  // range, in A as in B: an infinity times the other's zero would be NaN.  Of B they are rows of the first of the
-  // stage's two slabs and, past 32, of the second; of A whole pieces of 8, and the rest of a piece that holds shared k
-  // and others (shared_k % 8 != 0) is zeroed in LDS by the lane that brought it (clear).  Below one stage
-  // (K % 8 == 0) the A pieces and B rows past K are out of range.  A lane's k piece is the same for all its transfers of
-  // a stage (rows 16 apart share the swizzle).
+  // Ragged: K need not be whole A stages.  What is over them, K's first `head` elements, is a stage of its own in front of
+  // the others, which then end at K: their pieces of A hold nothing but elements of their own rows, at whatever alignment,
+  // and the K loop is the aligned form's.  A lane whose offset lies outside the buffer resource's range brings zeros into
+  // LDS, so pieces of A and rows of B past `head` are sent out of range, in A as in B (they belong to the next stage, and
+  // an infinity times the other's zero would be NaN); the rest of a piece of A that holds k on both sides of `head` is
+  // zeroed in LDS by the lane that brought it (keep).  A lane's k piece is the same for all its transfers of a stage (rows
+  // 16 apart share the swizzle).  With the odd stage at the end, moved back over the one before it, the loop had masks to
+  // apply and a branch: 2048 x 2048 x 2040 26.6 us, now 24.5; 1024 x 1024 x 1000 12.9, 11.0; 120 x 9000 x 520 9.7, 8.7;
+  // 4096 x 4095 x 4093 123, 119.
   const int nstages = (K + BKA - 1) / BKA;
-  const bool move_last = Ragged && K >= BKA && K % BKA != 0;
-  const int nslabs = move_last ? RA * nstages : (K + BKB - 1) / BKB;
-  const int k_tail_a = K - (nstages - 1) * BKA, k_tail_b = K - (nslabs - 1) * BKB;   // single stage
-  const int shared_k = nstages * BKA - K;                                               // moved stage
-  const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3;
-  const uint32_t a_out = (move_last ? a_lane_k + 8 <= shared_k : a_lane_k >= k_tail_a) ? 0x80000000u : 0u;
+  const int head = Ragged ? K - (nstages - 1) * BKA : BKA;
+  const int nslabs = Ragged && nstages > 1 ? RA * nstages : (K + BKB - 1) / BKB;
   constexpr uint32_t kOutOfRange = 0x80000000u;
-  // A lane whose row does not count has bit 31 set for the last slab and bit 30 for the one before it, and its offset
-  // gets bit 31 from there.  (As lane masks they took what scalar registers the loop has left.  Offsets of their own to
-  // select from became branches in the loop: four times the time.)
-  uint32_t b_out[DB];
-#pragma unroll
-  for (int i = 0; i < DB; ++i) {
-    const int brow = 2 * (wave + NWAVES * i) + (lane >> 5);
-    b_out[i] = (move_last ? brow + BKB < shared_k : brow >= k_tail_b) ? kOutOfRange : 0u;
-    if (move_last && brow < shared_k) b_out[i] |= kOutOfRange >> 1;
-  }
-  const char *b_end = b_base + (static_cast<int64_t>(K - 1) * ld + N - (N & 1)) * 2;   // last_products bring an odd N's last element
+  const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3;
+  const int keep = Ragged && a_lane_k < head && head < a_lane_k + 8 ? head - a_lane_k : 0;
+  int64_t b_left = (static_cast<int64_t>(K - 1) * ld + N - (N & 1)) * 2;   // last_products bring an odd N's last element
 
   f32x4_t acc[8][4];
 #pragma unroll
@@ -700,35 +688,35 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   const int b_r = l16 >> 2;
   int b_addr0 = (g * 8 + b_r) * 512 + ((wn * 128 + (l16 & 3) * 8) ^ ((b_r << 6) | ((g & 1) << 5)));
 
-  const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(a_base, 0x80000000u);
-  auto issue_a = [&](char *sa, int stage) {
+  // Past the last stage or slab a transfer has an empty range: it fetches nothing, and the count of transfers in flight
+  // keeps its pattern.  `at`: the stage or slab where it is known at compile time (the prologue's), -1 in the K loop.
+  auto issue_a = [&](auto at, char *sa, int stage) {
+    constexpr bool first = Ragged && decltype(at)::value == 0;
     if (stage >= NA && (Ablate & 1)) return;
-    const bool whole = stage < nstages - 1;
-    const uint32_t a_so = static_cast<uint32_t>(!whole && move_last ? K - BKA : min(stage, nstages - 1) * BKA) * 2u;
+    const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(a_base, stage < nstages ? kOutOfRange : 0u);
+    const uint32_t a_so = first ? 0u : static_cast<uint32_t>((stage - 1) * BKA + head) * 2u;
 #pragma unroll
     for (int i = 0; i < DA; ++i)
-      dma16(a_rsrc, Ragged ? a_off[i] | (whole ? 0u : a_out) : a_off[i], a_so, sa + (wave + NWAVES * i) * 1024);
+      dma16(a_rsrc, first && a_lane_k >= head ? kOutOfRange : a_off[i], a_so, sa + (wave + NWAVES * i) * 1024);
   };
-  const int clear = move_last && a_lane_k < shared_k && shared_k < a_lane_k + 8 ? shared_k - a_lane_k : 0;
-  // B slabs are issued in order 0, 1, 2, ...: the source of the next one is a running pointer (two scalar adds per
-  // slab instead of a 64-bit multiply) that stops at the last slab, which the tail of the K loop re-issues into
-  // stages nobody reads any more so that the count of outstanding transfers follows the same pattern throughout
+  // B slabs are issued in order 0, 1, 2, ...: the source of the next one is a running pointer
   const char *b_src = b_base;
   int b_next = 0;
-  auto issue_b = [&](char *sb, int slab) {
-    if (slab >= NB && (Ablate & 1)) return;
-    (void)slab;   // == b_next
-    const bool last = b_next >= nslabs - 1, prev = b_next == nslabs - 2;
-    if (move_last && prev) b_src = b_base + static_cast<int64_t>(K - BKA) * ld * 2;
-    const int place = last ? 0 : prev ? 1 : 2;
-    const int64_t b_left = b_end - b_src;
-    const __amdgpu_buffer_rsrc_t b_rsrc =
-        make_rsrc(b_src, Ragged && b_left < 0x80000000ll ? static_cast<uint32_t>(b_left) : kOutOfRange);
+  auto issue_b = [&](auto at, char *sb) {
+    constexpr int At = decltype(at)::value;
+    constexpr bool first = Ragged && At >= 0 && At < RA;   // a slab of the first stage
+    if (At < 0 && (Ablate & 1)) return;
+    const int32_t left_hi = static_cast<int32_t>(b_left >> 32);
+    const uint32_t left = left_hi > 0 ? kOutOfRange : left_hi < 0 ? 0u : min(static_cast<uint32_t>(b_left), kOutOfRange);
+    const __amdgpu_buffer_rsrc_t b_rsrc = make_rsrc(b_src, Ragged ? left : b_next < nslabs ? kOutOfRange : 0u);
 #pragma unroll
     for (int i = 0; i < DB; ++i)
-      dma16(b_rsrc, Ragged ? b_off[i] | ((b_out[i] << place) & kOutOfRange) : b_off[i], 0u, sb + (wave + NWAVES * i) * 1024);
+      dma16(b_rsrc, first && 2 * (wave + NWAVES * i) + (lane >> 5) >= head - At * BKB ? kOutOfRange : b_off[i], 0u,
+            sb + (wave + NWAVES * i) * 1024);
     ++b_next;
-    if (b_next < nslabs) b_src += b_slab_bytes;
+    const int64_t step = first && At == RA - 1 ? static_cast<int64_t>(head - At * BKB) * ld * 2 : b_slab_bytes;
+    b_src += step;
+    b_left -= step;
   };
   // half: rows 0-63 (0) or 64-127 (1) of the wave tile
   bool frags_loaded = false;
@@ -795,18 +783,17 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
     constexpr int ks = I % RA, ksn = In % RA;
     (void)ib;
     asm volatile("" : "+v"(a_addr0), "+v"(b_addr0));
-    issue_b(lds_ring<20 + ibp, B_BYTES_S>, s - BEHIND + NB);
+    issue_b(std::integral_constant<int, -1>{}, lds_ring<20 + ibp, B_BYTES_S>);
     load_a(lds_ring<10 + ia, A_BYTES_S>, ks, 1, af[1]);
     mfma_range(std::integral_constant<int, 0>{}, std::integral_constant<int, 16>{}, af, bf[I & 1]);
     spread(std::integral_constant<int, DB>{}, std::integral_constant<int, 4>{}, std::integral_constant<int, 16>{});
     if constexpr (!HalfBarriers || I % RA == RA - 1) {
       __builtin_amdgcn_s_waitcnt(
           waitcnt_vm_lgkm0(dma_allowed_in_flight(I, RA, NA, NB, DA, DB, HalfBarriers ? 2 : 1)));
-      if constexpr (Ragged && I % RA == RA - 1)
-        if (s / RA + 1 == nstages - 1) clear_piece_heads<DA, NWAVES>(lds_ring<10 + ian, A_BYTES_S>, wave, lane, clear);
       barrier_no_fence();
     }
-    if constexpr (I % RA == RA - 1) issue_a(lds_ring<10 + ia, A_BYTES_S>, s / RA + NA);
+    if constexpr (I % RA == RA - 1)
+      issue_a(std::integral_constant<int, -1>{}, lds_ring<10 + ia, A_BYTES_S>, s / RA + NA);
     // the next slab's fragments in the order its first MFMAs need them: A tile 0, the four B tiles, A tiles 1-3.
     // (The barrier was also tried after 8 and after 12 MFMAs, with the low-half A registers reloaded behind their
     // last readers: 1 % slower.)
@@ -821,12 +808,13 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   };
 
   [&]<int... Is>(std::integer_sequence<int, Is...>) {
-    (issue_a(lds_ring<10 + Is, A_BYTES_S>, Is), ...);
+    (issue_a(std::integral_constant<int, Is>{}, lds_ring<10 + Is, A_BYTES_S>, Is), ...);
   }(std::make_integer_sequence<int, NA>{});
   [&]<int... Is>(std::integer_sequence<int, Is...>) {
-    (issue_b(lds_ring<20 + Is, B_BYTES_S>, Is), ...);
+    (issue_b(std::integral_constant<int, Is>{}, lds_ring<20 + Is, B_BYTES_S>), ...);
   }(std::make_integer_sequence<int, NB - BEHIND>{});
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
+  if constexpr (Ragged) clear_piece_tails<DA, NWAVES>(lds_ring<10, A_BYTES_S>, wave, lane, keep);
   barrier_no_fence();
   load_a(lds_ring<10, A_BYTES_S>, 0, 0, af[0]);
   load_b(lds_ring<20, B_BYTES_S>, bf[0]);
@@ -1119,31 +1107,14 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   if (gridDim.y > 1) C = partials + blockIdx.y * splitk_plane_floats(M, ld);
   const char *a_base = reinterpret_cast<const char *>(A + static_cast<int64_t>(m0) * K + k0);
   const int64_t b_slab_bytes = static_cast<int64_t>(BKB) * ld * 2;
-  // Ragged: K need not fill the last A stage.  A lane whose offset lies outside the buffer resource's range brings
-  // zeros into LDS, so k that must not count are a per-lane choice between the usual offset and one past the range.
-  // From one whole stage on (K >= 64) the last stage is moved back to end at K: its A pieces then hold nothing but
-  // elements of their own rows, at whatever alignment, and the k it shares with the stage before it are sent out of
-  // range, in A as in B: an infinity times the other's zero would be NaN.  Of B they are rows of the first of the
-  // stage's two slabs and, past 32, of the second; of A whole pieces of 8, and the rest of a piece that holds shared k
-  // and others (shared_k % 8 != 0) is zeroed in LDS by the lane that brought it (clear).  Below one stage
-  // (K % 8 == 0) the A pieces and B rows past K are out of range.  A lane's k piece is the same for all its transfers of
-  // a stage (rows 16 apart share the swizzle).
+  // Ragged: K's first `head` elements as a stage of their own, as in the large tile
   const int nstages = (k_len + BKA - 1) / BKA;
-  const bool move_last = Ragged && k_len >= BKA && k_len % BKA != 0;
-  const int nslabs = move_last ? RA * nstages : (k_len + BKB - 1) / BKB;
-  const int k_tail_a = k_len - (nstages - 1) * BKA, k_tail_b = k_len - (nslabs - 1) * BKB;   // single stage
-  const int shared_k = nstages * BKA - k_len;                                               // moved stage
-  const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3;
-  const uint32_t a_out = (move_last ? a_lane_k + 8 <= shared_k : a_lane_k >= k_tail_a) ? 0x80000000u : 0u;
+  const int head = Ragged ? k_len - (nstages - 1) * BKA : BKA;
+  const int nslabs = Ragged && nstages > 1 ? RA * nstages : (k_len + BKB - 1) / BKB;
   constexpr uint32_t kOutOfRange = 0x80000000u;
-  uint32_t b_out[DB];   // as in the large tile
-#pragma unroll
-  for (int i = 0; i < DB; ++i) {
-    const int brow = (wave + NWAVES * i) * B_ROWS_PER_DMA + lane / B_CHUNKS;
-    b_out[i] = (move_last ? brow + BKB < shared_k : brow >= k_tail_b) ? kOutOfRange : 0u;
-    if (move_last && brow < shared_k) b_out[i] |= kOutOfRange >> 1;
-  }
-  const char *b_end = reinterpret_cast<const char *>(B) + (static_cast<int64_t>(K - 1) * ld + N - (N & 1)) * 2;   // as above
+  const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 3;
+  const int keep = Ragged && a_lane_k < head && head < a_lane_k + 8 ? head - a_lane_k : 0;
+  int64_t b_left = (static_cast<int64_t>(K - k0 - 1) * ld + N - (N & 1)) * 2;   // as above
 
   f32x4_t acc[4][4];
 #pragma unroll
@@ -1158,31 +1129,33 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   const int b_r = l16 >> 2;
   int b_addr0 = (g * 8 + b_r) * B_ROW + ((wn * 128 + (l16 & 3) * 8) ^ ((b_r << 6) | ((g & 1) << 5)));
 
-  const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(a_base, 0x80000000u);
-  auto issue_a = [&](char *sa, int stage) {
-    const bool whole = stage < nstages - 1;
-    const uint32_t a_so = static_cast<uint32_t>(!whole && move_last ? k_len - BKA : min(stage, nstages - 1) * BKA) * 2u;
+  // Past the last stage or slab a transfer has an empty range: it fetches nothing, and the count of transfers in flight
+  // keeps its pattern.  `at`: the stage or slab where it is known at compile time (the prologue's), -1 in the K loop.
+  auto issue_a = [&](auto at, char *sa, int stage) {
+    constexpr bool first = Ragged && decltype(at)::value == 0;
+    const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(a_base, stage < nstages ? kOutOfRange : 0u);
+    const uint32_t a_so = first ? 0u : static_cast<uint32_t>((stage - 1) * BKA + head) * 2u;
 #pragma unroll
     for (int i = 0; i < DA; ++i)
-      dma16(a_rsrc, Ragged ? a_off[i] | (whole ? 0u : a_out) : a_off[i], a_so, sa + (wave + NWAVES * i) * 1024);
+      dma16(a_rsrc, first && a_lane_k >= head ? kOutOfRange : a_off[i], a_so, sa + (wave + NWAVES * i) * 1024);
   };
-  const int clear = move_last && a_lane_k < shared_k && shared_k < a_lane_k + 8 ? shared_k - a_lane_k : 0;
-  // B slabs go out in order; the source is a running pointer that stops at the last slab (the tail of the K loop
-  // re-issues it into stages nobody reads any more, so the count of transfers in flight keeps its pattern)
+  // B slabs are issued in order 0, 1, 2, ...: the source of the next one is a running pointer
   const char *b_src = reinterpret_cast<const char *>(B + static_cast<int64_t>(k0) * ld);
   int b_next = 0;
-  auto issue_b = [&](char *sb) {
-    const bool last = b_next >= nslabs - 1, prev = b_next == nslabs - 2;
-    if (move_last && prev) b_src = reinterpret_cast<const char *>(B + static_cast<int64_t>(k0 + k_len - BKA) * ld);
-    const int place = last ? 0 : prev ? 1 : 2;
-    const int64_t b_left = b_end - b_src;
-    const __amdgpu_buffer_rsrc_t b_rsrc =
-        make_rsrc(b_src, Ragged && b_left < 0x80000000ll ? static_cast<uint32_t>(b_left) : kOutOfRange);
+  auto issue_b = [&](auto at, char *sb) {
+    constexpr int At = decltype(at)::value;
+    constexpr bool first = Ragged && At >= 0 && At < RA;   // a slab of the first stage
+    const int32_t left_hi = static_cast<int32_t>(b_left >> 32);
+    const uint32_t left = left_hi > 0 ? kOutOfRange : left_hi < 0 ? 0u : min(static_cast<uint32_t>(b_left), kOutOfRange);
+    const __amdgpu_buffer_rsrc_t b_rsrc = make_rsrc(b_src, Ragged ? left : b_next < nslabs ? kOutOfRange : 0u);
 #pragma unroll
     for (int i = 0; i < DB; ++i)
-      dma16(b_rsrc, Ragged ? b_off[i] | ((b_out[i] << place) & kOutOfRange) : b_off[i], 0u, sb + (wave + NWAVES * i) * 1024);
+      dma16(b_rsrc, first && (wave + NWAVES * i) * B_ROWS_PER_DMA + lane / B_CHUNKS >= head - At * BKB ? kOutOfRange : b_off[i],
+            0u, sb + (wave + NWAVES * i) * 1024);
     ++b_next;
-    if (b_next < nslabs) b_src += b_slab_bytes;
+    const int64_t step = first && At == RA - 1 ? static_cast<int64_t>(head - At * BKB) * ld * 2 : b_slab_bytes;
+    b_src += step;
+    b_left -= step;
   };
   auto load_a1 = [&](const char *sa, int ks, int i, u32x4 &af) {
     af = *reinterpret_cast<const u32x4 *>(sa + (a_addr0 ^ (ks << 6)) + i * 16 * A_ROW);
@@ -1236,14 +1209,13 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     constexpr int ian = (In / RA) % NA, ibn = In % NB;
     constexpr int ksn = In % RA;
     asm volatile("" : "+v"(a_addr0), "+v"(b_addr0));
-    issue_b(lds_ring<40 + ibp, B_BYTES_S>);
+    issue_b(std::integral_constant<int, -1>{}, lds_ring<40 + ibp, B_BYTES_S>);
     mfma_range(std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{}, af[I & 1], bf[I & 1]);
     spread(std::integral_constant<int, DB>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{});
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(dma_allowed_in_flight(I, RA, NA, NB, DA, DB)));
-    if constexpr (Ragged && I % RA == RA - 1)
-      if (s / RA + 1 == nstages - 1) clear_piece_heads<DA, NWAVES>(lds_ring<30 + ian, A_BYTES_S>, wave, lane, clear);
     barrier_no_fence();
-    if constexpr (I % RA == RA - 1) issue_a(lds_ring<30 + ia, A_BYTES_S>, s / RA + NA);
+    if constexpr (I % RA == RA - 1)
+      issue_a(std::integral_constant<int, -1>{}, lds_ring<30 + ia, A_BYTES_S>, s / RA + NA);
     // the next slab's fragments in the order its first MFMAs need them
     load_a1(lds_ring<30 + ian, A_BYTES_S>, ksn, 0, af[In & 1][0]);
     load_b(lds_ring<40 + ibn, B_BYTES_S>, bf[In & 1]);
@@ -1257,12 +1229,13 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
 
   // prologue: fill both rings except the last B stage (the top of slab 0 issues it) and wait for all of it
   [&]<int... Is>(std::integer_sequence<int, Is...>) {
-    (issue_a(lds_ring<30 + Is, A_BYTES_S>, Is), ...);
+    (issue_a(std::integral_constant<int, Is>{}, lds_ring<30 + Is, A_BYTES_S>, Is), ...);
   }(std::make_integer_sequence<int, NA>{});
   [&]<int... Is>(std::integer_sequence<int, Is...>) {
-    (issue_b(lds_ring<40 + Is, B_BYTES_S>), ...);
+    (issue_b(std::integral_constant<int, Is>{}, lds_ring<40 + Is, B_BYTES_S>), ...);
   }(std::make_integer_sequence<int, NB - 1>{});
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));
+  if constexpr (Ragged) clear_piece_tails<DA, NWAVES>(lds_ring<30, A_BYTES_S>, wave, lane, keep);
   barrier_no_fence();
 #pragma unroll
   for (int i = 0; i < 4; ++i) load_a1(lds_ring<30, A_BYTES_S>, 0, i, af[0][i]);

@@ -1008,6 +1008,16 @@ def test_gemm_infinity_at_every_k(hip, torch_cuda, kind, tunables, m, n, k):
         assert torch.equal(y[1:].double(), ref[1:].relu()) and bool(rs[1:].isinf().all())
 
 
+@pytest.mark.parametrize("kind,tunables", [("bf16", {"gemm16.tile": 256}), ("f16", {"gemm16.tile": 128}),
+                                           ("f16", {"gemm16.tile": 128, "gemm16.split_k": 2})])
+@pytest.mark.parametrize("n,k", [(256, 65), (131, 71), (200, 72), (77, 95), (264, 96), (130, 97), (128, 127), (300, 129),
+                                 (257, 193), (96, 40), (96, 8)])
+def test_gemm_infinity_where_the_first_stage_ends(hip, torch_cuda, kind, tunables, n, k):
+    """K over whole stages is a stage of its own at the start of K: an infinity at every k, one to a row, over first stages of
+    1 to 63, whole and part pieces of eight among them."""
+    test_gemm_infinity_at_every_k(hip, torch_cuda, kind, tunables, k + 2, n, k)
+
+
 @pytest.mark.parametrize("kind,m,n,k", [("bf16", 16, 512, 8192), ("f32", 16, 64, 4096), ("f16", 128, 128, 8192)])
 def test_products_on_the_stream_per_thread(hip, torch_cuda, kind, m, n, k):
     """hipStreamPerThread is one handle for as many streams as there are threads: a block of device memory kept by the handle
