@@ -12,7 +12,13 @@
 //
 // Blocks the caller allocated with sarek_hip_host_alloc are pinned already and go to the
 // DMA engines directly.
+//
+// A vector of a few hundred elements (a histogram, a table of offsets) is bound by none of that but by what the driver
+// takes for a copy of any size: 11 us, and as much again for the launch that waits behind an upload.  put_small sends such
+// a vector in a kernel's argument block, in the order of the default stream and without a wait; get_small has a kernel
+// write it to pinned memory, with a mark that the host looks for.
 #include <algorithm>
+#include <chrono>
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
@@ -21,6 +27,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "transfer.hpp"
 #include "tunables.hpp"
 
 namespace sarek_hip {
@@ -236,7 +243,97 @@ int staged_copy(bool upload, void *dst, const void *src, size_t bytes, const cha
   return check_hip(crew().run(job), what);
 }
 
+// ---- vectors of at most kSmallBytes ------------------------------------------------------------------------------
+
+template <int Words>
+struct Payload {
+  uint32_t words[Words];
+};
+
+__device__ __forceinline__ void copy_words(uint32_t *dst, const uint32_t *src, int bytes) {
+  const int words = bytes >> 2;
+  for (int i = threadIdx.x; i < words; i += blockDim.x) dst[i] = src[i];
+  if (static_cast<int>(threadIdx.x) < (bytes & 3))
+    reinterpret_cast<uint8_t *>(dst + words)[threadIdx.x] = static_cast<uint8_t>(src[words] >> (8 * threadIdx.x));
+}
+
+template <int Words>
+__global__ __launch_bounds__(256) void put_kernel(uint32_t *dst, Payload<Words> data, int bytes) {
+  copy_words(dst, data.words, bytes);
+}
+
+// `src` is a vector's device block: whole words may be read past an end inside one (device allocations are multiples of 256
+// bytes).  The mark follows the data, for whoever reads host memory.
+__global__ __launch_bounds__(256) void get_kernel(uint32_t *host, const uint32_t *src, int bytes, uint32_t *mark, uint32_t value) {
+  copy_words(host, src, bytes);
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(mark, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+struct Window {               // per device; lives until the process ends
+  std::mutex mu;
+  uint32_t *host = nullptr;   // pinned: kSmallBytes of data, then the mark
+  uint32_t count = 0;
+  bool failed = false;
+};
+Window g_windows[kMaxDevices];
+constexpr auto kLook = std::chrono::milliseconds(2);   // how long the host looks for a mark before it waits for the stream
+
+template <int Words>
+int put(void *dst, const void *src, size_t bytes) {
+  Payload<Words> data;
+  std::memcpy(data.words, src, bytes);
+  hipLaunchKernelGGL(put_kernel<Words>, dim3(1), dim3(256), 0, nullptr, static_cast<uint32_t *>(dst), data,
+                     static_cast<int>(bytes));
+  return hipGetLastError() == hipSuccess ? SAREK_HIP_OK : SAREK_HIP_E_UNSUPPORTED;
+}
+
 }  // namespace
+
+// One launch of 2.2 us against 11 for the driver's copy (1 KiB); the next kernel on the stream starts 2 us later for it.
+int put_small(void *dst, const void *src, size_t bytes) {
+  if (bytes == 0 || bytes > kSmallBytes || tunable("transfer.small", 1) == 0) return SAREK_HIP_E_UNSUPPORTED;
+  return bytes <= 1024 ? put<256>(dst, src, bytes) : put<kSmallBytes / 4>(dst, src, bytes);
+}
+
+// A launch and its 1 KiB back in host memory in 10.4 us against 14.3 with the driver's copy, which is a wait for the stream.
+int get_small(void *dst, const void *src, size_t bytes, int dev) {
+  if (bytes == 0 || bytes > kSmallBytes || dev < 0 || dev >= kMaxDevices || tunable("transfer.small", 1) == 0)
+    return SAREK_HIP_E_UNSUPPORTED;
+  Window &w = g_windows[dev];
+  std::unique_lock<std::mutex> lock(w.mu, std::try_to_lock);
+  if (!lock.owns_lock() || w.failed) return SAREK_HIP_E_UNSUPPORTED;
+  if (!w.host) {
+    void *p = nullptr;
+    if (hipHostMalloc(&p, kSmallBytes + 64, hipHostMallocCoherent) != hipSuccess) {
+      (void)hipGetLastError();
+      w.failed = true;
+      return SAREK_HIP_E_UNSUPPORTED;
+    }
+    w.host = static_cast<uint32_t *>(p);
+    w.host[kSmallBytes / 4] = 0;
+  }
+  uint32_t *mark = w.host + kSmallBytes / 4;
+  const uint32_t value = ++w.count;
+  hipLaunchKernelGGL(get_kernel, dim3(1), dim3(256), 0, nullptr, w.host, static_cast<const uint32_t *>(src),
+                     static_cast<int>(bytes), mark, value);
+  if (hipGetLastError() != hipSuccess) return SAREK_HIP_E_UNSUPPORTED;
+  const auto until = std::chrono::steady_clock::now() + kLook;
+  while (__atomic_load_n(mark, __ATOMIC_ACQUIRE) != value) {
+    for (int i = 0; i < 64 && __atomic_load_n(mark, __ATOMIC_RELAXED) != value; ++i) __builtin_ia32_pause();
+    if (std::chrono::steady_clock::now() > until) {
+      // a long kernel in front of it, or one that failed
+      const hipError_t e = hipStreamSynchronize(nullptr);
+      if (e != hipSuccess) w.failed = true;   // the kernel may still write: the window is not used again
+      if (e != hipSuccess) return check_hip(e, "download of a small vector");
+      break;
+    }
+  }
+  std::memcpy(dst, w.host, bytes);
+  return SAREK_HIP_OK;
+}
+
 }  // namespace sarek_hip
 
 using namespace sarek_hip;

@@ -28,6 +28,7 @@
 #include "host/ir.hpp"
 #include "plugin.hpp"
 #include "text_hash.hpp"
+#include "transfer.hpp"
 
 // The allocation behind a vector's host block; sub-vectors view their parent's, and it lives as
 // long as any of them (a Bigarray.Array1.sub keeps its parent's memory alive the same way).
@@ -57,6 +58,8 @@ struct sarek_hip_vector_s {
   int location = SAREK_HIP_LOC_CPU;
   int device = -1;                       // the device of a non-CPU location
   std::map<int, void *> buffers;         // device id -> device block (vec.device_buffers)
+  bool shown = false;                    // a caller knows a device block's address (vector_device_ptr)
+  bool in_order = false;                 // an upload was left to the order of the default stream (put_small)
 };
 
 namespace sarek_hip {
@@ -128,7 +131,14 @@ int to_device(sarek_hip_vector_s *v, int dev) {
   int st = ensure_buffer(v, dev, &buf);
   if (st != SAREK_HIP_OK) return st;
   if (!v->zero_copy) {
-    st = sarek_hip_memcpy_htod(buf, v->host, bytes_of(v));
+    // A block whose address nobody was given is used by the default stream alone, so a small upload need only be in its
+    // order; any other copy is complete on return.
+    int current = -1;
+    st = SAREK_HIP_E_UNSUPPORTED;
+    if (!v->shown && bytes_of(v) <= kSmallBytes && hipGetDevice(&current) == hipSuccess && current == dev)
+      st = put_small(buf, v->host, bytes_of(v));
+    v->in_order |= st == SAREK_HIP_OK;
+    if (st == SAREK_HIP_E_UNSUPPORTED) st = sarek_hip_memcpy_htod(buf, v->host, bytes_of(v));
     if (st != SAREK_HIP_OK) return st;
   }
   v->location = SAREK_HIP_LOC_BOTH;
@@ -149,7 +159,12 @@ int to_cpu(sarek_hip_vector_s *v, bool force) {
   if (it == v->buffers.end()) return fail(SAREK_HIP_E_INVALID_ARG, "to_cpu: no device buffer to transfer from");
   // A copy waits for the launches before it; a zero-copy vector has nothing to copy, but the
   // kernel that wrote the host block must have finished before the host reads it.
-  int st = v->zero_copy ? sarek_hip_device_synchronize() : sarek_hip_memcpy_dtoh(v->host, it->second, bytes_of(v));
+  int st = SAREK_HIP_E_UNSUPPORTED, current = -1;
+  if (v->zero_copy)
+    st = sarek_hip_device_synchronize();
+  else if (bytes_of(v) <= kSmallBytes && hipGetDevice(&current) == hipSuccess && current == v->device)
+    st = get_small(v->host, it->second, bytes_of(v), current);
+  if (st == SAREK_HIP_E_UNSUPPORTED) st = sarek_hip_memcpy_dtoh(v->host, it->second, bytes_of(v));
   if (st != SAREK_HIP_OK) return st;
   v->location = SAREK_HIP_LOC_BOTH;
   return SAREK_HIP_OK;
@@ -586,6 +601,17 @@ int sarek_hip_vector_device_ptr(sarek_hip_vector v, void **dptr) {
   if (st != SAREK_HIP_OK) return st;
   auto it = v->buffers.find(dev);
   *dptr = it == v->buffers.end() ? nullptr : it->second;
+  if (*dptr) v->shown = true;
+  if (*dptr && v->in_order) {
+    // From here on other streams may read the block: what the default stream was given is waited for, a caller's stream
+    // capture left alone.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    SAREK_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    const hipError_t e = hipStreamSynchronize(nullptr);
+    SAREK_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    SAREK_HIP_TRY(e);
+    v->in_order = false;
+  }
   return SAREK_HIP_OK;
 }
 
