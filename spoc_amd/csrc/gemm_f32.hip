@@ -170,12 +170,12 @@ __global__ __launch_bounds__(THREADS) void gemm_f32_staged_kernel(const float *_
 //
 // Ragged = false: N % 4 == 0, K % BKT == 0, A, B and C 16-byte aligned.  Ragged = true: any N, any K >= BKT (or a multiple of
 // 4 below it), any alignment.  A lane whose offset lies outside the buffer resource's range brings zeros into LDS, the range
-// is checked per dword and the address needs no alignment beyond the element's, so B rows that must not count are a per-lane
-// choice between the usual offset and one past the range, B's range ends with its last element, pieces past column N bring
-// the next row's elements into columns that are never stored, and C is stored element by element.
-// PieceHeads: K % 4 != 0, so a 16-byte piece of A can hold k that the last two slabs share and others (a form of its own: the
-// test for that slab in every turn of the loop took 0.6 % of 2049 x 4097 x 3000).
-template <int TI, int TJ, int WMW, int WNW, int BKT, int NS, bool Ragged, bool PieceHeads>
+// is checked per dword and the address needs no alignment beyond the element's, so B's range ends with its last element,
+// pieces past column N bring the next row's elements into columns that are never stored, and C is stored element by element.
+// What K is over whole slabs is at its start, outside the K loop: with it in a slab at the end, moved back over the one
+// before, every turn of the loop chose its offsets by masks (64 x 64 tile: 2049 x 4097 x 3000 428 us, now 404; 2031 x 1792 x
+// 2211 143, 135; 1500^3 77, 72).
+template <int TI, int TJ, int WMW, int WNW, int BKT, int NS, bool Ragged>
 __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
     const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int M, int N,
     int K, int tiles_m, int tiles_n, int xcd_remap, unsigned long long *probe, int k_chunk,
@@ -235,29 +235,17 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
   const int k_len = blockIdx.y == gridDim.y - 1 ? K - k0 : k_chunk;
   if (gridDim.y > 1) C = partials + blockIdx.y * splitk_plane_floats(M, N);
   const char *a_base = reinterpret_cast<const char *>(A + static_cast<int64_t>(m0) * K + k0);
-  const char *b_base = reinterpret_cast<const char *>(B + static_cast<int64_t>(k0) * N);
   const int64_t b_slab_bytes = static_cast<int64_t>(BKT) * N * 4;
   const int nslabs = (k_len + BKT - 1) / BKT;
-  // The end of K inside the last slab.  With K >= BKT the last slab is moved back to end at K (its A pieces then hold
-  // nothing but elements of their own row, at whatever alignment) and the k it shares with the slab before it are left
-  // out, in A as in B (an infinity times the other's zero would be NaN): rows of B, whole pieces of A, and the rest of a
-  // piece that holds shared k and others is zeroed in LDS by the lane that brought it, once a tile, before the barrier
-  // behind which the slab is read.  With a single slab (K < BKT, K % 4 == 0) the A pieces and B rows past K are left out.
-  // A lane's k piece is the same for all its A transfers: rows NWAVES * A_ROWS_PER_DMA apart share the swizzle.
-  const int k_tail = k_len - (nslabs - 1) * BKT;
-  const bool move_last = Ragged && k_len >= BKT && k_tail != BKT;
-  const int k_last = move_last ? k_len - BKT : (nslabs - 1) * BKT;   // first k of the last slab, from k0
-  const int shared_k = BKT - k_tail;   // moved slab
+  // Ragged: K need not be whole slabs.  What is over them, the first `head` elements, is a slab of its own in front of the
+  // others, which then end at K (their A pieces hold nothing but elements of their own rows, at whatever alignment), and
+  // the K loop is the aligned form's.  Pieces of A and rows of B past `head` are sent out of range, in A as in B (they belong
+  // to the next slab, and an infinity times the other's zero would be NaN); the rest of a piece of A that holds k on both
+  // sides of `head` is zeroed in LDS by the lane that brought it (keep).  A lane's k piece is the same for all its A
+  // transfers: rows NWAVES * A_ROWS_PER_DMA apart share the swizzle.
+  const int head = Ragged ? k_len - (nslabs - 1) * BKT : BKT;
   const int a_lane_k = ((lane % A_CHUNKS) ^ a_swz(wave * A_ROWS_PER_DMA + lane / A_CHUNKS)) << 2;
-  const bool a_lane_in_k = !Ragged || (move_last ? a_lane_k + 4 > shared_k : a_lane_k < k_tail);
-  const int clear = move_last && a_lane_k < shared_k && shared_k < a_lane_k + 4 ? shared_k - a_lane_k : 0;
-  bool b_lane_in_k[B_DMA];
-#pragma unroll
-  for (int i = 0; i < B_DMA; ++i) {
-    const int brow = (wave + NWAVES * i) * B_ROWS_PER_DMA + lane / B_CHUNKS;
-    b_lane_in_k[i] = !Ragged || (move_last ? brow >= shared_k : brow < k_tail);
-  }
-  const char *b_end = reinterpret_cast<const char *>(B) + static_cast<int64_t>(K) * N * 4;
+  const int keep = Ragged && a_lane_k < head && head < a_lane_k + 4 ? head - a_lane_k : 0;
   constexpr uint32_t kOutOfRange = 0x80000000u;
 
   f32x16 acc[TI][TJ];
@@ -281,21 +269,30 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
 
   // A: one resource for the tile's row panel, the slab selects a scalar byte offset.
   // B: the resource is rebased to the slab's first row (keeps every offset below 2^31).
-  const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(a_base, 0x80000000u);
-  auto issue = [&](char *sa, char *sb, int slab) {
-    const int sl = min(slab, nslabs - 1);   // the tail re-issues the last slab: constant vmcnt
-    const bool whole = !Ragged || slab < nslabs - 1;
-    const char *b_src = whole ? b_base + sl * b_slab_bytes : b_base + static_cast<int64_t>(k_last) * N * 4;
-    const int64_t b_left = b_end - b_src;
-    const __amdgpu_buffer_rsrc_t b_rsrc =
-        make_rsrc(b_src, Ragged && b_left < 0x80000000ll ? static_cast<uint32_t>(b_left) : kOutOfRange);
-    const uint32_t a_so = static_cast<uint32_t>(whole ? sl * BKT : k_last) * 4u;
+  // Past the last slab a transfer has an empty range: it fetches nothing, and the count of transfers in flight keeps its
+  // pattern.  Slabs are issued in order; `at` is 0 for the first.
+  const char *b_src = reinterpret_cast<const char *>(B + static_cast<int64_t>(k0) * N);
+  int64_t b_left = static_cast<int64_t>(K - k0) * N * 4;
+  uint32_t a_so = 0;
+  int to_issue = nslabs;
+  auto issue = [&](auto at, char *sa, char *sb) {
+    constexpr bool first = Ragged && decltype(at)::value == 0;
+    const int32_t left_hi = static_cast<int32_t>(b_left >> 32);
+    const uint32_t left = left_hi > 0 ? kOutOfRange : left_hi < 0 ? 0u : min(static_cast<uint32_t>(b_left), kOutOfRange);
+    const __amdgpu_buffer_rsrc_t a_rsrc = make_rsrc(a_base, to_issue > 0 ? kOutOfRange : 0u);
+    const __amdgpu_buffer_rsrc_t b_rsrc = make_rsrc(b_src, Ragged ? left : to_issue > 0 ? kOutOfRange : 0u);
 #pragma unroll
     for (int i = 0; i < A_DMA; ++i)
-      dma16(a_rsrc, (whole || a_lane_in_k) ? a_off[i] : kOutOfRange, a_so, sa + (wave + NWAVES * i) * 1024);
+      dma16(a_rsrc, first && a_lane_k >= head ? kOutOfRange : a_off[i], a_so, sa + (wave + NWAVES * i) * 1024);
 #pragma unroll
     for (int i = 0; i < B_DMA; ++i)
-      dma16(b_rsrc, (whole || b_lane_in_k[i]) ? b_off[i] : kOutOfRange, 0u, sb + (wave + NWAVES * i) * 1024);
+      dma16(b_rsrc, first && (wave + NWAVES * i) * B_ROWS_PER_DMA + lane / B_CHUNKS >= head ? kOutOfRange : b_off[i], 0u,
+            sb + (wave + NWAVES * i) * 1024);
+    --to_issue;
+    const int64_t step = first ? static_cast<int64_t>(head) * N * 4 : b_slab_bytes;
+    b_src += step;
+    b_left -= step;
+    a_so += first ? head * 4u : BKT * 4u;
   };
   auto load_frags = [&](const char *sa, const char *sb, int kk, f32x4 (&af)[TI], bvec_t (&bf)[4]) {
     const char *pa = sa + (a_addr0 ^ (kk << 5));
@@ -343,19 +340,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
   f32x4 af[2][TI];
   bvec_t bf[2][4];
 
-  auto clear_shared = [&](char *sa) {
-    if (clear > 0) {
-#pragma unroll
-      for (int i = 0; i < A_DMA; ++i) {
-        float *piece = reinterpret_cast<float *>(sa + (wave + NWAVES * i) * 1024 + lane * 16);
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-          if (d < clear) piece[d] = 0.f;
-      }
-    }
-    wait_lds();
-  };
-  auto slab = [&](char *ca, char *cb, char *na, const char *nb, int s) {
+  auto slab = [&](char *ca, char *cb, char *na, const char *nb) {
     asm volatile("" : "+v"(a_addr0), "+v"(b_addr0));   // keep per-stage addresses out of registers
 #pragma unroll
     for (int kk = 0; kk + 1 < KK; ++kk) {
@@ -364,31 +349,36 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
       interleave(std::integral_constant<int, 0>{});
     }
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NS - 2) * (A_DMA + B_DMA)));
-    if constexpr (PieceHeads)
-      if (s + 1 == nslabs - 1) clear_shared(na);
     barrier_no_fence();
-    issue(ca, cb, s + NS);
+    issue(std::integral_constant<int, -1>{}, ca, cb);
     load_frags(na, nb, 0, af[0], bf[0]);
     mfma_step(af[(KK - 1) & 1], bf[(KK - 1) & 1]);
     interleave(std::integral_constant<int, A_DMA + B_DMA>{});
   };
 
-  issue(lds_ring<0, A_BYTES_S>, lds_ring<1, B_BYTES_S>, 0);
-  issue(lds_ring<2, A_BYTES_S>, lds_ring<3, B_BYTES_S>, 1);
-  if constexpr (NS == 4) {
-    issue(lds_ring<4, A_BYTES_S>, lds_ring<5, B_BYTES_S>, 2);
-    issue(lds_ring<6, A_BYTES_S>, lds_ring<7, B_BYTES_S>, 3);
-  }
+  [&]<int... Is>(std::integer_sequence<int, Is...>) {
+    (issue(std::integral_constant<int, Is>{}, lds_ring<2 * Is, A_BYTES_S>, lds_ring<2 * Is + 1, B_BYTES_S>), ...);
+  }(std::make_integer_sequence<int, NS>{});
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NS - 1) * (A_DMA + B_DMA)));
+  if (keep > 0) {
+#pragma unroll
+    for (int i = 0; i < A_DMA; ++i) {
+      float *piece = reinterpret_cast<float *>(lds_ring<0, A_BYTES_S> + (wave + NWAVES * i) * 1024 + lane * 16);
+#pragma unroll
+      for (int d = 1; d < 4; ++d)
+        if (d >= keep) piece[d] = 0.f;
+    }
+    wait_lds();
+  }
   barrier_no_fence();
   load_frags(lds_ring<0, A_BYTES_S>, lds_ring<1, B_BYTES_S>, 0, af[0], bf[0]);
   __builtin_amdgcn_sched_barrier(0);
 
-  auto ring_slab = [&](auto st_c, int s) {
+  auto ring_slab = [&](auto st_c) {
     constexpr int st = decltype(st_c)::value;
     constexpr int nx = (st + 1) % NS;
     slab(lds_ring<2 * st, A_BYTES_S>, lds_ring<2 * st + 1, B_BYTES_S>, lds_ring<2 * nx, A_BYTES_S>,
-         lds_ring<2 * nx + 1, B_BYTES_S>, s);
+         lds_ring<2 * nx + 1, B_BYTES_S>);
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
@@ -396,19 +386,19 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_f32_dma_kernel(
   using I3 = std::integral_constant<int, 3>;
   const int full = nslabs - nslabs % NS;
   for (int s = 0; s < full; s += NS) {
-    ring_slab(I0{}, s);
-    ring_slab(I1{}, s + 1);
+    ring_slab(I0{});
+    ring_slab(I1{});
     if constexpr (NS == 4) {
-      ring_slab(I2{}, s + 2);
-      ring_slab(I3{}, s + 3);
+      ring_slab(I2{});
+      ring_slab(I3{});
     }
   }
-  if (full < nslabs) ring_slab(I0{}, full);
+  if (full < nslabs) ring_slab(I0{});
   if constexpr (NS == 4) {
-    if (full + 1 < nslabs) ring_slab(I1{}, full + 1);
-    if (full + 2 < nslabs) ring_slab(I2{}, full + 2);
+    if (full + 1 < nslabs) ring_slab(I1{});
+    if (full + 2 < nslabs) ring_slab(I2{});
   }
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // drain the redundant tail DMA
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // drain the tail's (empty) transfers
   if constexpr (kTwoChains) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[0][0][r] += acc_odd[r];
@@ -566,23 +556,19 @@ extern "C" int sarek_hip_gemm_f32(const float *a, const float *b, float *c, int 
     float *partials = splits > 1 ? splitk_workspace(st) : nullptr;
     if (!partials) splits = 1;
     const int k_chunk = splits > 1 ? splitk_chunk(k, 32, splits) : k;
-#define SAREK_LAUNCH_F32(T, TI, TJ, WMW, WNW, BKT, RAGGED, HEADS)                                  \
-  hipLaunchKernelGGL((gemm_f32_dma_kernel<TI, TJ, WMW, WNW, BKT, 4, RAGGED, HEADS>),              \
+#define SAREK_LAUNCH_F32(T, TI, TJ, WMW, WNW, BKT, RAGGED)                                  \
+  hipLaunchKernelGGL((gemm_f32_dma_kernel<TI, TJ, WMW, WNW, BKT, 4, RAGGED>),              \
                      dim3((unsigned)ntiles(T), splits), dim3(64 * WMW * WNW), 0, st, a, b, c, m, n, k, \
                      (m + T - 1) / T, (n + T - 1) / T, remap, splits > 1 ? nullptr : clock_probe(ntiles(T)), k_chunk, \
                      partials)
-    if (ragged && k % 4 != 0) {
-      if (tile == 256) SAREK_LAUNCH_F32(256, 4, 2, 2, 4, 16, true, true);
-      else if (tile == 128) SAREK_LAUNCH_F32(128, 2, 2, 2, 2, 16, true, true);
-      else SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, true, true);
-    } else if (ragged) {
-      if (tile == 256) SAREK_LAUNCH_F32(256, 4, 2, 2, 4, 16, true, false);
-      else if (tile == 128) SAREK_LAUNCH_F32(128, 2, 2, 2, 2, 16, true, false);
-      else SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, true, false);
+    if (ragged) {
+      if (tile == 256) SAREK_LAUNCH_F32(256, 4, 2, 2, 4, 16, true);
+      else if (tile == 128) SAREK_LAUNCH_F32(128, 2, 2, 2, 2, 16, true);
+      else SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, true);
     } else {
-      if (tile == 256) SAREK_LAUNCH_F32(256, 4, 2, 2, 4, 16, false, false);
-      else if (tile == 128) SAREK_LAUNCH_F32(128, 2, 2, 2, 2, 16, false, false);
-      else SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, false, false);
+      if (tile == 256) SAREK_LAUNCH_F32(256, 4, 2, 2, 4, 16, false);
+      else if (tile == 128) SAREK_LAUNCH_F32(128, 2, 2, 2, 2, 16, false);
+      else SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, false);
     }
 #undef SAREK_LAUNCH_F32
     const int rc = check_launch("gemm_f32 kernel launch");

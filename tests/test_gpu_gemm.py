@@ -1009,7 +1009,10 @@ def test_gemm_infinity_at_every_k(hip, torch_cuda, kind, tunables, m, n, k):
 
 
 @pytest.mark.parametrize("kind,tunables", [("bf16", {"gemm16.tile": 256}), ("f16", {"gemm16.tile": 128}),
-                                           ("f16", {"gemm16.tile": 128, "gemm16.split_k": 2})])
+                                           ("f16", {"gemm16.tile": 128, "gemm16.split_k": 2}),
+                                           ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 64}),
+                                           ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 128}),
+                                           ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 256})])
 @pytest.mark.parametrize("n,k", [(256, 65), (131, 71), (200, 72), (77, 95), (264, 96), (130, 97), (128, 127), (300, 129),
                                  (257, 193), (96, 40), (96, 8)])
 def test_gemm_infinity_where_the_first_stage_ends(hip, torch_cuda, kind, tunables, n, k):
