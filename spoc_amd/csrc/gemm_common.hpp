@@ -85,19 +85,24 @@ constexpr int NUM_XCD = 8;   // XCDs of an MI355X; workgroup ids are dealt to th
 // brings past its L2 the others find in the memory-side cache.  Measured on bf16 products against bands of 8:
 // 8192^3 0.729 against 0.740 ms, 8192 x 4096 x 8192 0.365 against 0.374, 16384 x 8192 x 2048 0.442 against 0.474,
 // nothing lost on 3072^3, 4096^3, the fp16 epilogue shape and the f32 8192^3 product; bands of 2, 16 or 32 are slower.
+// block: the workgroup's id, or what stands for it where not every tile has a workgroup of its own.
 __device__ __forceinline__ void tile_of_block(int tiles_m, int tiles_n, int xcd_remap, int &tm,
-                                              int &tn) {
+                                              int &tn, int block) {
   const int GROUP = xcd_remap > 1 ? xcd_remap : 4;   // tile-rows per raster band
   const int nblocks = tiles_m * tiles_n;
-  const int xcd = blockIdx.x % NUM_XCD, slot = blockIdx.x / NUM_XCD;
+  const int xcd = block % NUM_XCD, slot = block / NUM_XCD;
   int tile = xcd * (nblocks / NUM_XCD) + min(xcd, nblocks % NUM_XCD) + slot;
-  if (xcd_remap == 0) tile = blockIdx.x;
+  if (xcd_remap == 0) tile = block;
   const int per_group = GROUP * tiles_n;
   const int g = tile / per_group;
   const int rows_in_group = min(GROUP, tiles_m - g * GROUP);
   const int in_g = tile - g * per_group;
   tm = g * GROUP + in_g % rows_in_group;
   tn = in_g / rows_in_group;
+}
+
+__device__ __forceinline__ void tile_of_block(int tiles_m, int tiles_n, int xcd_remap, int &tm, int &tn) {
+  tile_of_block(tiles_m, tiles_n, xcd_remap, tm, tn, static_cast<int>(blockIdx.x));
 }
 
 // One static LDS array per ring stage and operand: distinct objects, so the compiler can

@@ -235,10 +235,9 @@ bool gemm_f32_direct_serves(int m, int n, int k) {
   return tiles <= kMaxBlocks && static_cast<int64_t>(m) * k * 4 < 0x7FFFFFFF && static_cast<int64_t>(n) * 2 * kStepK * 4 < 0x7FFFFFFF;
 }
 
-// Up to 10 GFLOP: above, the LDS kernel is level at best (1280 x 2712 x 1792, 12 GFLOP: 134 us here, 104 there;
-// 2049 x 4097 x 3000, 50: 437 and 430), but for products that leave its tiles a round nearly empty (578 x 3308 x 5773, 22 GFLOP,
-// 520 tiles of 64 x 64: 183 us here, 305 there; profiles/gemm_f32_plans.txt has more).
-bool gemm_f32_direct_pays(int m, int n, int k) { return static_cast<double>(m) * n * k <= 5e9; }
+// Up to 6 GFLOP: above, the LDS kernel with its last tiles cut is level or ahead (1280 x 1644 x 960, 4 GFLOP: 41 us here, 36
+// there; 1500^3, 7: 62 and 57; 2049 x 4097 x 3000, 50: 408 and 388).
+bool gemm_f32_direct_pays(int m, int n, int k) { return static_cast<double>(m) * n * k <= 3e9; }
 
 // At most `splits` pieces of K: of whole steps, none empty, their planes within the workspace and a ticket per tile.
 int gemm_f32_direct_pieces(int m, int n, int k, int row_blocks, int splits) {

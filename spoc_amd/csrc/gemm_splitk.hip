@@ -1,5 +1,6 @@
-// What the GEMMs share when a product with few tiles and a long K is cut along K over several workgroups per tile:
-// device memory for the partial M x N planes, and the kernel that adds them up.
+// What the GEMMs share when tiles are cut along K over several workgroups each: device memory for the partial tiles and
+// tickets for the kernels whose last workgroup of a tile adds them, and, for the 16-bit tiles, the kernel that adds partial
+// M x N planes up.
 #include <map>
 #include <mutex>
 #include <utility>

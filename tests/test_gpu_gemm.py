@@ -801,6 +801,47 @@ def test_gemm_f32_split_k_rule(hip, torch_cuda):
         assert (hip.gemm_f32_k_splits(m, n, k) > 1) == want_split, (m, n, k)
 
 
+@pytest.mark.parametrize("tile,cut", [(64, 2), (64, 3), (64, 5), (128, 2), (128, 4)])
+@pytest.mark.parametrize("m,n,k", [(1088, 1024, 256), (1030, 1051, 333), (2100, 2113, 130), (300, 130, 200), (4100, 130, 97),
+                                   (1, 17000, 128), (2049, 2300, 517)])
+def test_gemm_f32_tiles_past_whole_turns(hip, torch_cuda, tile, cut, m, n, k):
+    """The tiles past whole turns of the CUs in pieces of K (all of them where there is no whole turn; fewer pieces where K
+    has no more), whole and ragged, C at an odd offset between guard values: the float64 product within k 2^-24 of the
+    products' magnitudes, the same bits on every run, on another stream and replayed beside eager calls; under capture no
+    tile is cut."""
+    torch = torch_cuda
+    torch.manual_seed(m + n * k + cut)
+    da, db = torch.rand(m, k, device="cuda") * 2 - 1, torch.rand(k, n, device="cuda") * 2 - 1
+    ref, size = da.double() @ db.double(), da.double().abs() @ db.double().abs()
+    good = lambda c: bool(((c.double() - ref).abs() <= (k + 32) * 2.0 ** -24 * size).all())  # noqa: E731
+    try:
+        for name, value in (("gemm_f32.direct", 1), ("gemm_f32.tile", tile), ("gemm_f32.cut", cut)):
+            hip.set_tunable(name, value)
+        guard = torch.full((m * n + 64,), 7.0, device="cuda")
+        c = guard[33:33 + m * n].view(m, n)
+        hip.gemm_f32(da, db, out=c)
+        assert bool((guard[:33] == 7).all()) and bool((guard[33 + m * n:] == 7).all()) and good(c)
+        for _ in range(3):
+            assert torch.equal(hip.gemm_f32(da, db), c)
+        side = side_stream(torch)
+        side.wait_stream(torch.cuda.current_stream())
+        captured, graph = torch.empty(m, n, device="cuda"), torch.cuda.CUDAGraph()
+        with torch.cuda.stream(side):
+            assert torch.equal(hip.gemm_f32(da, db), c)
+            with torch.cuda.graph(graph, stream=side):
+                hip.gemm_f32(da, db, out=captured)
+        side.synchronize()
+        for _ in range(3):
+            captured.fill_(float("nan"))
+            graph.replay()
+            again = hip.gemm_f32(da, db)
+            torch.cuda.synchronize()
+            assert good(captured) and torch.equal(again, c)
+    finally:
+        for name in ("gemm_f32.direct", "gemm_f32.tile", "gemm_f32.cut"):
+            hip.set_tunable(name, 0)
+
+
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 32), (16, 128, 256), (17, 129, 257), (15, 127, 33), (33, 3, 1000), (48, 264, 520),
                                    (49, 255, 4129), (64, 1001, 1001), (64, 640, 2048), (65, 130, 96)])
