@@ -741,9 +741,10 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   auto mfma_range = [&](auto first_c, auto count_c, u32x4 (&af)[2][4], u32x4 (&bf)[4]) {
     constexpr int First = decltype(first_c)::value, Count = decltype(count_c)::value;
     [&]<int... Ts>(std::integer_sequence<int, Ts...>) {
-      ((acc[(First + Ts) / 4][(First + Ts) % 4] = mfma16<Bf16>(af[(First + Ts) / 16][((First + Ts) / 4) % 4],
-                                                              bf[(First + Ts) % 4],
-                                                              acc[(First + Ts) / 4][(First + Ts) % 4])),
+      (([&] {
+         constexpr int i = (First + Ts) / 4, j = i % 2 ? 3 - (First + Ts) % 4 : (First + Ts) % 4;
+         acc[i][j] = mfma16<Bf16>(af[i / 4][i % 4], bf[j], acc[i][j]);
+       }()),
        ...);
     }(std::make_integer_sequence<int, Count>{});
   };
@@ -1180,8 +1181,10 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   auto mfma_range = [&](auto first_c, auto count_c, u32x4 (&af)[4], u32x4 (&bf)[4]) {
     constexpr int First = decltype(first_c)::value, Count = decltype(count_c)::value;
     [&]<int... Ts>(std::integer_sequence<int, Ts...>) {
-      ((acc[(First + Ts) / 4][(First + Ts) % 4] =
-            mfma16<Bf16>(af[(First + Ts) / 4], bf[(First + Ts) % 4], acc[(First + Ts) / 4][(First + Ts) % 4])),
+      (([&] {
+         constexpr int i = (First + Ts) / 4, j = i % 2 ? 3 - (First + Ts) % 4 : (First + Ts) % 4;
+         acc[i][j] = mfma16<Bf16>(af[i], bf[j], acc[i][j]);
+       }()),
        ...);
     }(std::make_integer_sequence<int, Count>{});
   };
