@@ -222,12 +222,14 @@ __global__ __launch_bounds__(Threads) void radix_scatter_kernel(int *__restrict_
   for (int o = Threads / 128; o >= 1; o >>= 1) before += __shfl_xor(before, o);
   const int slot = incl - c + __builtin_amdgcn_readfirstlane(before);
   start[t] = slot;
-  if (t % kCopies == 0) base[t / kCopies] = first - slot;   // slot s of the digit goes to out[base + s]
   __syncthreads();
 
 #pragma unroll
   for (int j = 0; j < Keys; ++j)
     if (in_tile(j)) stage[start[counter(j)] + rank[j]] = key[j];
+  // What the global atomics answer is waited for only here: in front of the staging (us, with a 1 KiB copy) 3000001 keys 13.7,
+  // here 12.6, 5000000 17.2 / 15.1, 10000019 28.2 / 26.7, 16000000 38.5 / 35.5, 50000000 as before.
+  if (t % kCopies == 0) base[t / kCopies] = first - slot;   // slot s of the digit goes to out[base + s]
   __syncthreads();
 
   for (int s = t; s < valid; s += Threads) {
