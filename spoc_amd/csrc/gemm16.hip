@@ -487,18 +487,18 @@ __device__ __forceinline__ void last_products(const uint16_t *__restrict__ A, co
 }
 
 // Writes one wave's (16*TI) x 64 block held as TI x 4 tiles of 16 x 16 (register r of lane l: row 4*(l/16) + r, column
-// l%16 of its tile); TI = 8 in the 256 x 256 workgroup tile (2 x 4 waves), 4 in the 128 x 128 one (2 x 2 waves).
+// l%16 of its tile); TI = 8 in the 256 x 256 workgroup tile (2 x 4 waves) and the 128 x 256 one (1 x 4), 4 in the 128 x 128 one (2 x 2).
 // Fused form as in `epilogue`: per lane the sum over its four columns for each of its 4*TI rows, a halving butterfly
 // over the 16 lanes that share those rows (with TI = 8: 16+8+4+2 exchanges leave lane m with rows 2m, 2m+1 of the 32;
 // with TI = 4: 8+4+2+1 leave it with row m of the 16), the WNW waves along N through LDS.  The tile's sum of row r then
 // goes to rs_plane[r] when the launch has planes (one per tile column, added up in tile order by
 // rowsum_fold_kernel: the same bits on every run), else to rowsum[r] by atomicAdd.  add_last: the tile rows' last_products
 // lie in `scratch` and belong to column N - 1.
-template <int Epi, int TI, int WNW, bool Ragged>
+template <int Epi, int TI, int WNW, bool Ragged, int WMW = 2>   // WMW, WNW: waves along M, N
 __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restrict__ C, const float *__restrict__ bias,
                                            float *__restrict__ rowsum, float *__restrict__ rs_plane, int M, int N, int ld,
                                            int m0, int wm, int wn, int col0, int l16, int g, float *scratch, bool add_last) {
-  constexpr int WROWS = 16 * TI, TROWS = 2 * WROWS, NV = 4 * TI, E = NV / 16;
+  constexpr int WROWS = 16 * TI, TROWS = WMW * WROWS, NV = 4 * TI, E = NV / 16;
   static_assert(TI == 8 || TI == 4, "wave tiles of 128 or 64 rows");
   static_assert(WNW == 4 || WNW == 2, "four or two waves along N");
   const int row0 = m0 + wm * WROWS;
@@ -595,22 +595,28 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
 //      the second group on the other 32-byte half of each 64-byte piece.
 // A slab is worked in two units of 16 MFMAs (rows 0-63 of the wave tile, then rows 64-127, same B fragments);
 // the barrier sits between them, and the second unit covers the fragment reads of the next slab.
-template <bool Bf16, int Epi, int Ablate = 0, bool Ragged = false, bool HalfBarriers = false>
-__global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
+//
+// WM = 1: the upper half of the tile alone, 128 x 256 on 4 waves, with the LDS that the other half would take in deeper rings
+// (three stages of A and six slabs of B, 144 KiB): a wave has its SIMD to itself and nobody to cover a late transfer for it.
+// With two stages and four slabs, two such workgroups to a CU, it was slower than the small tile everywhere.
+template <bool Bf16, int Epi, int Ablate = 0, bool Ragged = false, bool HalfBarriers = false, int WM = 2>
+__global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                          float *__restrict__ C, const float *__restrict__ bias,
                                                          float *__restrict__ rowsum, int M, int N, int K, int tiles_m,
                                                          int tiles_n, int xcd_remap, unsigned long long *probe, int ld,
                                                          float *__restrict__ rs_planes) {
+  static_assert(WM == 2 || (WM == 1 && !HalfBarriers), "the whole tile or its upper half");
   // HalfBarriers: one barrier per A stage (K = 64) instead of one per B slab (K = 32).  A transfer may then only
   // overwrite the slab before the previous one (the waves are a whole stage apart at most), so the top of slab j
   // issues B(j - 2 + NB) and the ring is two slabs deeper, 160 KiB of LDS in all.
-  constexpr int BKA = 64, BKB = 32, NA = 2, NB = HalfBarriers ? 6 : 4;
+  constexpr int BKA = 64, BKB = 32, NA = WM == 1 ? 3 : 2, NB = HalfBarriers || WM == 1 ? 6 : 4;
   constexpr int BEHIND = HalfBarriers ? 2 : 1;   // the slab whose stage the top of a slab refills lies this far back
   constexpr int RA = BKA / BKB;                  // B slabs per A stage
   static_assert(!HalfBarriers || RA == 2, "the barrier sits in the second slab of an A stage");
   constexpr int A_ROW = BKA * 2, A_CHUNKS = A_ROW / 16, A_ROWS_PER_DMA = 1024 / A_ROW;
-  constexpr int A_BYTES_S = BM * A_ROW, B_BYTES_S = BKB * BN * 2;
-  constexpr int NWAVES = 8, WN = 4;
+  constexpr int TBM = 128 * WM;
+  constexpr int A_BYTES_S = TBM * A_ROW, B_BYTES_S = BKB * BN * 2;
+  constexpr int NWAVES = 4 * WM, WN = 4;
   constexpr int DA = A_BYTES_S / 1024 / NWAVES, DB = B_BYTES_S / 1024 / NWAVES;
   constexpr int P = lcm_int(NB, RA * NA);
   static_assert(P % 2 == 0, "the B fragment buffers alternate by slab parity");
@@ -623,7 +629,7 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   const int l16 = lane & 15, g = lane >> 4;
   int tm, tn;
   tile_of_block(tiles_m, tiles_n, xcd_remap, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * TBM, n0 = tn * BN;
   long long probe_c0 = 0, probe_t0 = 0;
   if (kMeasureBuild && probe) {
     probe_c0 = clock64();
@@ -845,9 +851,9 @@ __global__ __launch_bounds__(512) void gemm16_m16_kernel(const uint16_t *__restr
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // drain the (redundant) tail DMA before the LDS is released
   float *scratch = reinterpret_cast<float *>(lds_ring<10, A_BYTES_S>);
   const bool add_last = Ragged && (N & 1) != 0 && n0 + BN >= N;
-  if (add_last) last_products<Bf16, BM>(A, B, M, N, K, ld, m0, 0, scratch);
-  epilogue16<Epi, 8, 4, Ragged>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0, wm, wn,
-                  n0 + wn * 64, l16, g, scratch, add_last);
+  if (add_last) last_products<Bf16, TBM>(A, B, M, N, K, ld, m0, 0, scratch);
+  epilogue16<Epi, 8, 4, Ragged, WM>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N,
+                                    ld, m0, wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
   if (kMeasureBuild && probe && tid == 0) {
     probe[2 * blockIdx.x] = static_cast<unsigned long long>(clock64() - probe_c0);
     probe[2 * blockIdx.x + 1] = static_cast<unsigned long long>(wall_clock64() - probe_t0);
@@ -1362,22 +1368,45 @@ inline bool small_tile_wins(int m, int n) {
   return cost_small < 0.9 * cost_large;
 }
 
+// Whether n columns go to the 128 x 256 tile: where a workgroup of it per CU takes them all and 128 x 128 tiles would share
+// CUs.  Two small tiles on a CU move 64 KiB per K = 64 between them, one of these 48 (some 60 bytes a nanosecond reach a CU's
+// LDS, whichever the tile), and the 256 x 256 tile leaves CUs idle.  Measured, us, on the better of those two and on this:
+// 4096 x 2048 x 8192 118 -> 108, 2048 x 4096 x 4096 60.0 -> 57.3, 4096 x 1935 x 5504 96 -> 86, 1673 x 3642 x 7005 129 -> 101,
+// 392 x 12497 x 4079 82 -> 66, 3130 x 1656 x 2304 33.9 -> 30.1, 128 x 35072 x 7296 157 -> 122.  More such tiles than CUs run in
+// two rounds and lose to the large tile (3072^3 76 us against 55), fewer than half of them leave the CUs to the small one
+// (2048^3 27 against 21).  Its prologue and its epilogue, with one wave per SIMD, take 2 us more: K = 640 15.1 -> 15.5, 1024
+// 15.2 -> 16.6 and 19.0 -> 18.2, 1274 27.2 -> 23.9, 1600 24.7 -> 24.0.  The same after whole rounds of large tiles, in the
+// second launch: one round, 2048 x 12288 x 4096 159 -> 154, x 1024 51.8 -> 51.9, x 256 25.1 -> 27.7, 2880 x 6912 x 7168 262 ->
+// 236, 6361 x 3264 x 1425 74.7 -> 70.0; two, 2880 x 13120 x 1755 137 -> 132, 5888 x 6400 x 640 60.2 -> 62.0; four, 2880 x
+// 23971 x 1579 234 -> 237; six, 5248 x 20113 x 2313 500 -> 495.  So K has to be 600 for each round and for one more; a
+// product of no whole round counts as of one.
+// gemm16.half: 0 = this rule, 1 = never, 2 = wherever a workgroup per CU takes the columns, whatever K.
+inline bool half_tile_pays(int m, int n, int k, int64_t rounds) {
+  const int64_t asked = tunable("gemm16.half", 0);
+  if (asked == 1 || tunable("gemm16.split_k", 0) != 0 || (kMeasureBuild && clock_probe(1))) return false;
+  const int cus = compute_units();
+  const int64_t rows = ceil_div(m, 128);
+  if (rows * ceil_div(n, 256) > cus) return false;
+  return asked == 2 || (tunable("gemm16.tile", 0) == 0 && rows * ceil_div(n, 128) > cus && k >= 600 * (rounds + 1));
+}
+
 // How many of n columns the 256 x 256 tiles take when the last round of workgroups would hold few of them: the tile columns
-// of whole rounds; the rest goes to the 128 x 128 tile in a second launch.  n where that does not pay.  The results are the
-// same bits: both kernels add an element's products in the same order.
+// of whole rounds; the rest goes to a smaller tile in a second launch.  n where that does not pay.  The results are the
+// same bits: all tiles add an element's products in the same order.
 // A round of a few large tiles takes nearly as long as a full one (a CU works its tile alone); as small tiles, one to a CU,
 // the same columns take half of that.  Measured, us, without and with the cut: 2048 rows, 8448 / 9216 / 10240 columns
 // (32 / 128 / 256 small tiles) K = 512 35.5 -> 32.1 / 35.8 -> 33.4 / 38.5 -> 35.2, K = 1024 53.3 -> 45.6 / 53.9 -> 46.9 /
 // 56.7 -> 48.7, K = 4096 157 -> 134 / 169 -> 141 / 172 -> 146; 4096 x 4100 x 4096 187 -> 155; fused 4096 x 4352 x 4096
-// 169 -> 140; 2048 x 50257 x 1024 274 -> 264.  From there on two small tiles share a CU and nothing is left to gain: 11264
-// columns 39.7 -> 39.6, 56.8 -> 55.2, 174 -> 175; 12288 40.0 -> 40.1, 59.5 -> 58.4, 177 -> 181.
+// 169 -> 140; 2048 x 50257 x 1024 274 -> 264.  From there on two small tiles would share a CU, with nothing left to gain (11264
+// columns 39.7 -> 39.6, 56.8 -> 55.2, 174 -> 175; 12288 40.0 -> 40.1, 59.5 -> 58.4, 177 -> 181): the 128 x 256 tile, where that
+// pays (half).
 // A short K, and the more so the more rounds there are (their tiles no longer end together, and some CUs take the few that are
 // over while others finish), gives the second launch nothing to win: 7232 x 13568 (6 rounds) K = 82 85.0 -> 91.2, 512 128 ->
 // 132; 3712 x 39176 (9 rounds) 82 149 -> 155, 768 302 -> 313; 4160 x 8000 (2 rounds) 126 39.2 -> 42.2, 768 66.8 -> 64.7;
 // 2048 x 8448 (1 round) 82 22.6 -> 22.2, 256 24.9 -> 23.9.  So K has to be 128 times the whole rounds: of 417 drawn products
 // of up to 8192 rows the cut cost 48 more than 2 % without that and costs 6 with it.
 // gemm16.cut: 0 = this rule, 1 = never, s >= 2: a rest of up to s small tiles, whatever K.
-inline int whole_round_columns(int m, int n, int k) {
+inline int whole_round_columns(int m, int n, int k, bool &half) {
   const int64_t asked = tunable("gemm16.cut", 0);
   if (asked == 1 || tunable("gemm16.tile", 0) != 0) return n;
   const int cus = compute_units();
@@ -1386,7 +1415,9 @@ inline int whole_round_columns(int m, int n, int k) {
   if (over == 0 || columns < 1) return n;
   const int64_t rest = ceil_div(m, 128) * ceil_div(n - columns * 256, 128);
   if (asked < 2 && k < tiles_m * tiles_n / cus * 128) return n;
-  return rest <= (asked >= 2 ? asked : cus) ? static_cast<int>(columns * 256) : n;
+  if (rest <= (asked >= 2 ? asked : cus)) return static_cast<int>(columns * 256);
+  half = asked < 2 && half_tile_pays(m, n - static_cast<int>(columns * 256), k, tiles_m * tiles_n / cus);
+  return half ? static_cast<int>(columns * 256) : n;
 }
 
 // The columns that are left to the tiles when gemm16_last_column_kernel takes the last one: n - 1 for N = 1 and for whole
@@ -1616,9 +1647,13 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   // stream capture, past the sixteenth stream, planes beyond the block's size) adds with atomicAdd in arrival order.
   float *planes = nullptr;
   int n_planes = 0;
-  const int cut = tiled && tile_choice == 256 && nm > 0 && !(kMeasureBuild && clock_probe(1)) ? whole_round_columns(m, nm, k) : nm;
+  bool half = tiled && tile_choice == 128 && half_tile_pays(m, nm, k, 1);
+  const int cut = tiled && tile_choice == 256 && nm > 0 && !(kMeasureBuild && clock_probe(1))
+                      ? whole_round_columns(m, nm, k, half) : nm;
   if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
-    n_planes = tiled ? (cut + tile_choice - 1) / tile_choice + (nm - cut + 127) / 128 + (n - nm) : (n + 63) / 64;
+    const int rest_tile = half ? 256 : 128;   // the columns of the tiles that take [cut, nm), or all where tile_choice is 128
+    const int first = tiled && tile_choice == 128 ? 0 : cut;
+    n_planes = tiled ? (first + 255) / 256 + (nm - first + rest_tile - 1) / rest_tile + (n - nm) : (n + 63) / 64;
     if (static_cast<int64_t>(n_planes) * m * 4 <= static_cast<int64_t>(kSplitWorkspaceBytes)) planes = splitk_workspace(st);
     if (!planes) {
       const int rc = launch_zero_f32(rowsum, m, st);
@@ -1638,7 +1673,21 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   const bool ragged = n % 8 != 0 || k % 64 != 0 || !ab16;   // the kernels' template flag
   const int remap = (int)tunable("gemm.xcd_remap", 1);
   int rc = SAREK_HIP_OK;
-  if (nm > 0 && tile_choice == 128) {
+  // columns [first, first + count) on the 128 x 256 tile
+  auto launch_half = [&](int first, int count, float *count_planes) {
+    const int sm = (m + 127) / 128, sn = (count + 255) / 256;
+    const float *const part_bias = Epi == EPI_BIAS_RELU_ROWSUM ? bias + first : nullptr;
+    if (ragged)
+      hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, true, false, 1>), dim3(sm * sn), dim3(256), 0, st, a, b + first,
+                         c + first, part_bias, rowsum, m, count, k, sm, sn, remap, nullptr, n, count_planes);
+    else
+      hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false, false, 1>), dim3(sm * sn), dim3(256), 0, st, a, b + first,
+                         c + first, part_bias, rowsum, m, count, k, sm, sn, remap, nullptr, n, count_planes);
+    return check_launch("gemm16 kernel launch");
+  };
+  if (nm > 0 && half && tile_choice == 128) {
+    rc = launch_half(0, nm, planes);
+  } else if (nm > 0 && tile_choice == 128) {
     const int sm = (m + 127) / 128, sn = (nm + 127) / 128;
     unsigned long long *sprobe = clock_probe(static_cast<int64_t>(sm) * sn);
     int splits = 1;
@@ -1691,13 +1740,15 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
       const int rest = nm - cut, sm = (m + 127) / 128, sn = (rest + 127) / 128;
       float *const rest_planes = planes ? planes + static_cast<int64_t>(tiles_n) * m : nullptr;
       const float *const rest_bias = Epi == EPI_BIAS_RELU_ROWSUM ? bias + cut : nullptr;
-      if (ragged)
+      if (half)
+        rc = launch_half(cut, rest, rest_planes);
+      else if (ragged)
         hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, true>), dim3(sm * sn), dim3(256), 0, st, a, b + cut, c + cut,
                            rest_bias, rowsum, m, rest, k, sm, sn, remap, nullptr, k, nullptr, n, rest_planes);
       else
         hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, false>), dim3(sm * sn), dim3(256), 0, st, a, b + cut, c + cut,
                            rest_bias, rowsum, m, rest, k, sm, sn, remap, nullptr, k, nullptr, n, rest_planes);
-      rc = check_launch("gemm16 kernel launch");
+      if (!half) rc = check_launch("gemm16 kernel launch");
     }
   }
   if (rc != SAREK_HIP_OK) return rc;
@@ -1735,7 +1786,9 @@ int sarek_hip_gemm16_tile_columns(int m, int n, int k) {
   const int tile = sarek_hip_gemm16_tile(m, n, k);
   if (tile != 256 && tile != 128) return n;
   const int columns = tiled_columns(m, n, tile);
-  return tile == 256 && columns > 0 ? whole_round_columns(m, columns, k) : columns;
+  bool half = false;
+  const int cut = tile == 256 && columns > 0 ? whole_round_columns(m, columns, k, half) : columns;
+  return half ? columns : cut;
 }
 
 int sarek_hip_gemm16_k_splits(int m, int n, int k) {

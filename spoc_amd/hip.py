@@ -747,12 +747,14 @@ def gemm_bf16(a, b, out=None):
 
 
 def gemm16_tile(m, n, k):
-    """256 / 128: the workgroup tile the 16-bit GEMMs take for this shape now; 64: the few-rows kernel; 0: the simple kernel."""
+    """256 / 128: the workgroup tile the 16-bit GEMMs take for this shape now (128: its rows; where gemm16.half says so it has
+    256 columns); 64: the few-rows kernel; 0: the simple kernel."""
     return int(lib.sarek_hip_gemm16_tile(m, n, k))
 
 
 def gemm16_tile_columns(m, n, k):
-    """How many of the n columns that tile takes; the rest goes to the 128 x 128 tile or, one column, to a kernel of its own."""
+    """How many of the n columns that tile takes, with those that go to the 128 x 256 tile after it; the rest goes to the
+    128 x 128 tile or, one column, to a kernel of its own."""
     return int(lib.sarek_hip_gemm16_tile_columns(m, n, k))
 
 

@@ -386,6 +386,47 @@ def test_gemm16_both_tile_sizes(hip, oracle, torch_cuda, kind, m, n, k):
 
 
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
+@pytest.mark.parametrize("m,n,k,tile", [(128, 256, 64, 128), (1, 8, 64, 128), (127, 255, 65, 128), (129, 257, 72, 128), (300, 521, 199, 128),
+                                        (257, 264, 320, 128), (70, 1032, 384, 128), (640, 385, 449, 128), (200, 2, 32, 128),
+                                        (2048, 11264, 64, 0), (2047, 11009, 201, 0), (1921, 4099, 1200, 0), (1921, 4099, 1203, 0)])
+def test_gemm16_half_tile(hip, oracle, torch_cuda, kind, m, n, k, tile):
+    """The 128 x 256 tile for a whole product and for the columns past a round of large tiles, at the edges of its tile and of
+    its six-slab period, at any alignment of A and B: the bits of the other tiles (same products, same k order per element),
+    rows of the result against the oracle, the row sums against those of y, nothing stored outside."""
+    torch = torch_cuda
+    a, b = normal16(oracle, (m, k), m + 5, kind), normal16(oracle, (k, n), n + 6, kind)
+    bias = oracle.fill_uniform(n, seed=n + 2, lo=-0.1, hi=0.1)
+    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    dbias = dev(torch, bias)
+    rows = np.unique(np.r_[0, m // 2, max(m - 2, 0):m])
+    ref = oracle.gemm(np.ascontiguousarray(a[rows]), b)
+    hip.set_tunable("gemm16.tile", tile)
+    try:
+        for shift in (0, 1) if k >= 64 else (0,):   # elements by which both operands lie off 16 bytes
+            def placed(x):
+                flat = torch.empty(x.size + shift, device="cuda", dtype=dt)[shift:]
+                return flat.view(x.shape).copy_(dev(torch, x))
+            da, db = placed(a), placed(b)
+            got = {}
+            for half in (2, 1) if k < 1200 else (0, 1):
+                hip.set_tunable("gemm16.half", half)
+                guard = torch.full((m * n + 64,), 7.0, device="cuda")
+                c = guard[32:32 + m * n].view(m, n)
+                (hip.gemm_bf16 if kind == "bf16" else hip.gemm_f16)(da, db, out=c)
+                assert bool((guard[:32] == 7).all()) and bool((guard[32 + m * n:] == 7).all())
+                got[half] = (c,) + (hip.gemm_f16_bias_relu_rowsum(da, db, dbias) if kind == "f16" else ())
+            new, old = got[2 if k < 1200 else 0], got[1]
+            assert torch.equal(new[0], old[0])
+            assert np.abs(new[0][dev(torch, rows)].cpu().numpy() - ref).max() / np.abs(ref).max() < 1e-4
+            if kind == "f16":
+                assert torch.equal(new[1], old[1])
+                assert rowsums_ok(new[2].cpu().numpy(), new[1].double().sum(1).cpu().numpy())
+    finally:
+        hip.set_tunable("gemm16.half", 0)
+        hip.set_tunable("gemm16.tile", 0)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(2048, 8448, 64), (2047, 8195, 72), (1921, 8703, 131), (2048, 10240, 65),
                                    (8192, 2050, 70), (2300, 7425, 200)])
 def test_gemm16_columns_past_whole_rounds_of_large_tiles(hip, oracle, torch_cuda, kind, m, n, k):
