@@ -245,6 +245,7 @@ int staged_copy(bool upload, void *dst, const void *src, size_t bytes, const cha
 
 // ---- vectors of at most kSmallBytes ------------------------------------------------------------------------------
 
+#ifdef __HIP__   // compiled as host code alone (the sanitizer build) the file has no kernels, and every copy is the general one
 template <int Words>
 struct Payload {
   uint32_t words[Words];
@@ -288,9 +289,14 @@ int put(void *dst, const void *src, size_t bytes) {
                      static_cast<int>(bytes));
   return hipGetLastError() == hipSuccess ? SAREK_HIP_OK : SAREK_HIP_E_UNSUPPORTED;
 }
+#endif
 
 }  // namespace
 
+#ifndef __HIP__
+int put_small(void *, const void *, size_t) { return SAREK_HIP_E_UNSUPPORTED; }
+int get_small(void *, const void *, size_t, int) { return SAREK_HIP_E_UNSUPPORTED; }
+#else
 // One launch of 2.2 us against 11 for the driver's copy (1 KiB); the next kernel on the stream starts 2 us later for it.
 int put_small(void *dst, const void *src, size_t bytes) {
   if (bytes == 0 || bytes > kSmallBytes || tunable("transfer.small", 1) == 0) return SAREK_HIP_E_UNSUPPORTED;
@@ -333,6 +339,7 @@ int get_small(void *dst, const void *src, size_t bytes, int dev) {
   std::memcpy(dst, w.host, bytes);
   return SAREK_HIP_OK;
 }
+#endif
 
 }  // namespace sarek_hip
 
