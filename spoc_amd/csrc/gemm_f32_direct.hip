@@ -1,4 +1,4 @@
-// float32 products up to some GFLOP: C[M x N] = A[M x K] . B[K x N] on v_mfma_f32_16x16x4_f32, operands straight from
+// float32 products of up to 6 GFLOP: C[M x N] = A[M x K] . B[K x N] on v_mfma_f32_16x16x4_f32, operands straight from
 // memory to registers.
 //
 // What bounds these products is latency, not a rate: with the 64 x 64 tile of gemm_f32_dma_kernel 512^3 is 64 workgroups
@@ -32,7 +32,7 @@ constexpr int kDeviceScope = 16;
 // Workgroup -> (piece of K, tile): every XCD gets a contiguous run of the pieces' tiles, which it walks in bands of
 // `band` tile rows, column by column, the band chosen so that the patch of a run is about as tall as wide: the tiles that
 // one L2 serves then share their rows of A and columns of B.  Against tiles row by row over all XCDs (us):
-// 153 x 1216 x 1920 15.2 to 11.6, 434 x 3952 x 3328 130 to 108, 2049 x 4097 x 3000 641 to 434.  The divisions are by
+// 153 x 1216 x 1920 15.2 to 11.6, 434 x 3952 x 3328 130 to 108.  The divisions are by
 // numbers known at the launch, a multiplication by their reciprocals each (divided out they took 0.3 us of a 5 us
 // kernel): n / d = floor(n r / 2^32), r = floor(2^32 / d) + 1, is exact while n d < 2^32, so blocks stay under 2^16.
 constexpr int kMaxBlocks = 65535;
