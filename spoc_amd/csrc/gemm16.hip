@@ -596,8 +596,10 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
 // A slab is worked in two units of 16 MFMAs (rows 0-63 of the wave tile, then rows 64-127, same B fragments);
 // the barrier sits between them, and the second unit covers the fragment reads of the next slab.
 //
-// WM = 1: the upper half of the tile alone, 128 x 256 on 4 waves, with the LDS that the other half would take in deeper rings
-// (three stages of A and six slabs of B, 144 KiB): a wave has its SIMD to itself and nobody to cover a late transfer for it.
+// WM = 1: the upper half of the tile alone, 128 x 256 on 4 waves, with all 160 KiB of LDS as deeper rings: a wave has its SIMD
+// to itself and nobody to cover a late transfer for it.  Stages of A and slabs of B, three and six (144 KiB), four and six,
+// five and five, us: 4096 x 2048 x 8192 105, 99, 102; 2048 x 4096 x 4096 57.1, 53.9, 55.4; 448 x 15680 x 1728 26.4, 25.7, 26.1;
+// fused 6865 x 576 x 1472 25.1, 25.7, 24.5; ragged 256 x 24704 x 4535 62.5, 63.5, 62.0; fused 2056 x 2060 x 2547 42.2, 42.1, 41.5.
 // The same tile with a ring of 80 KiB, two workgroups to a CU, waited for its transfers: 8192^3 738 us on the large tile, 820
 // on it; 2048 x 50257 x 1024 260, 345.
 template <bool Bf16, int Epi, int Ablate = 0, bool Ragged = false, bool HalfBarriers = false, int WM = 2>
@@ -610,7 +612,8 @@ __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__
   // HalfBarriers: one barrier per A stage (K = 64) instead of one per B slab (K = 32).  A transfer may then only
   // overwrite the slab before the previous one (the waves are a whole stage apart at most), so the top of slab j
   // issues B(j - 2 + NB) and the ring is two slabs deeper, 160 KiB of LDS in all.
-  constexpr int BKA = 64, BKB = 32, NA = WM == 1 ? 3 : 2, NB = HalfBarriers || WM == 1 ? 6 : 4;
+  constexpr int BKA = 64, BKB = 32;
+  constexpr int NA = WM == 2 ? 2 : Ragged ? 5 : 4, NB = WM == 2 ? (HalfBarriers ? 6 : 4) : Ragged ? 5 : 6;
   constexpr int BEHIND = HalfBarriers ? 2 : 1;   // the slab whose stage the top of a slab refills lies this far back
   constexpr int RA = BKA / BKB;                  // B slabs per A stage
   static_assert(!HalfBarriers || RA == 2, "the barrier sits in the second slab of an A stage");
@@ -1372,12 +1375,12 @@ inline bool small_tile_wins(int m, int n) {
 // Whether n columns go to the 128 x 256 tile: where a workgroup of it per CU takes them all and 128 x 128 tiles would share
 // CUs.  Two small tiles on a CU move 64 KiB per K = 64 between them, one of these 48 (some 60 bytes a nanosecond reach a CU's
 // LDS, whichever the tile), and the 256 x 256 tile leaves CUs idle.  Measured, us, on the better of those two and on this:
-// 4096 x 2048 x 8192 118 -> 108, 2048 x 4096 x 4096 60.0 -> 57.3, 4096 x 1935 x 5504 96 -> 86, 1673 x 3642 x 7005 129 -> 101,
+// 4096 x 2048 x 8192 118 -> 103, 2048 x 4096 x 4096 61.1 -> 55.3, 4096 x 1935 x 5504 96 -> 86, 1673 x 3642 x 7005 129 -> 101,
 // 392 x 12497 x 4079 82 -> 66, 3130 x 1656 x 2304 33.9 -> 30.1, 128 x 35072 x 7296 157 -> 122.  More such tiles than CUs run in
 // two rounds and lose to the large tile (3072^3 76 us against 55), fewer than half of them leave the CUs to the small one
-// (2048^3 27 against 21).  Its prologue and its epilogue, with one wave per SIMD, take 2 us more: K = 640 15.1 -> 15.5, 1024
+// (2048^3 27 against 21).  Its prologue and its epilogue, with one wave per SIMD, take 2 us more: K = 640 15.9 -> 17.1, 1024
 // 15.2 -> 16.6 and 19.0 -> 18.2, 1274 27.2 -> 23.9, 1600 24.7 -> 24.0.  The same after whole rounds of large tiles, in the
-// second launch: one round, 2048 x 12288 x 4096 159 -> 154, x 1024 51.8 -> 51.9, x 256 25.1 -> 27.7, 2880 x 6912 x 7168 262 ->
+// second launch: one round, 2048 x 12288 x 4096 163 -> 153, x 1024 52.6 -> 54.1, x 256 25.9 -> 28.8, 2880 x 6912 x 7168 262 ->
 // 236, 6361 x 3264 x 1425 74.7 -> 70.0; two, 2880 x 13120 x 1755 137 -> 132, 5888 x 6400 x 640 60.2 -> 62.0; four, 2880 x
 // 23971 x 1579 234 -> 237; six, 5248 x 20113 x 2313 500 -> 495.  So K has to be 600 for each round and for one more; a
 // product of no whole round counts as of one.
