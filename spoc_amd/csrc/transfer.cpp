@@ -16,7 +16,8 @@
 // A vector of a few hundred elements (a histogram, a table of offsets) is bound by none of that but by what the driver
 // takes for a copy of any size: 11 us, and as much again for the launch that waits behind an upload.  put_small sends such
 // a vector in a kernel's argument block, in the order of the default stream and without a wait; get_small has a kernel
-// write it to pinned memory, with a mark that the host looks for.
+// write it to pinned memory, with a mark that the host looks for.  While a stream of the process is being captured they are
+// refused like any copy.
 #include <algorithm>
 #include <chrono>
 #include <condition_variable>
@@ -281,6 +282,15 @@ struct Window {               // per device; lives until the process ends
 Window g_windows[kMaxDevices];
 constexpr auto kLook = std::chrono::milliseconds(2);   // how long the host looks for a mark before it waits for the stream
 
+// Whether the driver takes a copy on the default stream now.  While any stream of the process is captured it does not (and
+// the capture is spoilt), but it would take the kernels that stand for a copy here.  A copy of no bytes says so at once, with
+// work queued in front or not (0.3 us).
+bool copies_taken(void *dst, const void *src, hipMemcpyKind kind) {
+  if (hipMemcpy(dst, src, 0, kind) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 template <int Words>
 int put(void *dst, const void *src, size_t bytes) {
   Payload<Words> data;
@@ -299,13 +309,15 @@ int get_small(void *, const void *, size_t, int) { return SAREK_HIP_E_UNSUPPORTE
 #else
 // One launch of 2.2 us against 11 for the driver's copy (1 KiB); the next kernel on the stream starts 2 us later for it.
 int put_small(void *dst, const void *src, size_t bytes) {
-  if (bytes == 0 || bytes > kSmallBytes || tunable("transfer.small", 1) == 0) return SAREK_HIP_E_UNSUPPORTED;
+  if (bytes == 0 || bytes > kSmallBytes || tunable("transfer.small", 1) == 0 || !copies_taken(dst, src, hipMemcpyHostToDevice))
+    return SAREK_HIP_E_UNSUPPORTED;
   return bytes <= 1024 ? put<256>(dst, src, bytes) : put<kSmallBytes / 4>(dst, src, bytes);
 }
 
 // A launch and its 1 KiB back in host memory in 10.4 us against 14.3 with the driver's copy, which is a wait for the stream.
 int get_small(void *dst, const void *src, size_t bytes, int dev) {
-  if (bytes == 0 || bytes > kSmallBytes || dev < 0 || dev >= kMaxDevices || tunable("transfer.small", 1) == 0)
+  if (bytes == 0 || bytes > kSmallBytes || dev < 0 || dev >= kMaxDevices || tunable("transfer.small", 1) == 0 ||
+      !copies_taken(dst, src, hipMemcpyDeviceToHost))
     return SAREK_HIP_E_UNSUPPORTED;
   Window &w = g_windows[dev];
   std::unique_lock<std::mutex> lock(w.mu, std::try_to_lock);

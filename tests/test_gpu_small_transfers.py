@@ -120,3 +120,39 @@ def test_threads_with_vectors_of_their_own(sarek):
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])              # hipStreamCaptureModeGlobal, ThreadLocal, Relaxed
+@pytest.mark.parametrize("small", [1, 0])
+def test_refused_while_a_stream_is_captured(hip, sarek, small, mode):
+    """A copy is an error while a stream is captured, and spoils the capture; a small one by whatever way it travels, up as
+    down, on device blocks that are there already.  Afterwards both work."""
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    runtime = C.CDLL(path)
+    hip.set_tunable("transfer.small", small)
+    try:
+        up, down, fresh = (sarek.Vector.create(sarek.Vector.float32, 256) for _ in range(3))
+        for v in (up, down, fresh):
+            v.fill_from(np.full(256, 2.0, np.float32))
+            sarek.Transfer.to_device(v)
+        sarek.Transfer.to_cpu(fresh, force=True)          # the window for downloads is there
+        up.fill_from(np.full(256, 3.0, np.float32))
+        for blocking in (True, False):
+            for copy in (lambda: sarek.Transfer.to_device(up), lambda: sarek.Transfer.to_cpu(down, force=True)):
+                stream, graph = C.c_void_p(), C.c_void_p()
+                assert runtime.hipStreamCreateWithFlags(C.byref(stream), 0 if blocking else 1) == 0
+                assert runtime.hipStreamBeginCapture(stream, mode) == 0
+                try:
+                    with pytest.raises(hip.SarekHipError, match="Capture"):
+                        copy()
+                finally:
+                    ended = runtime.hipStreamEndCapture(stream, C.byref(graph))
+                    runtime.hipGetLastError()
+                    assert runtime.hipStreamDestroy(stream) == 0
+                assert ended == 901 and not graph.value   # hipErrorStreamCaptureInvalidated
+        sarek.Transfer.to_device(up)
+        up.host[:] = 0
+        sarek.Transfer.to_cpu(up, force=True)
+        assert np.array_equal(up.host, np.full(256, 3.0, np.float32))
+    finally:
+        hip.set_tunable("transfer.small", 1)
