@@ -42,6 +42,13 @@ struct sarek_hip_host_block {
   }
 };
 
+// A vector's memory on one device.
+struct sarek_hip_device_block {
+  void *ptr = nullptr;
+  bool shown = false;      // a caller knows the address (vector_device_ptr)
+  bool in_order = false;   // an upload was left to the order of that device's default stream (put_small)
+};
+
 struct sarek_hip_vector_s {
   int kind = SAREK_HIP_KIND_FLOAT32;
   int64_t length = 0, elem_size = 4;
@@ -57,9 +64,7 @@ struct sarek_hip_vector_s {
   bool auto_sync = true;                 // Vector_types.t.auto_sync
   int location = SAREK_HIP_LOC_CPU;
   int device = -1;                       // the device of a non-CPU location
-  std::map<int, void *> buffers;         // device id -> device block (vec.device_buffers)
-  bool shown = false;                    // a caller knows a device block's address (vector_device_ptr)
-  bool in_order = false;                 // an upload was left to the order of the default stream (put_small)
+  std::map<int, sarek_hip_device_block> buffers;   // by device id (vec.device_buffers)
 };
 
 namespace sarek_hip {
@@ -86,10 +91,10 @@ int current_device(int *dev) {
 }
 
 // Transfer.ensure_buffer: the vector's block on `dev`, allocated on first use.
-int ensure_buffer(sarek_hip_vector_s *v, int dev, void **out) {
+int ensure_buffer(sarek_hip_vector_s *v, int dev, sarek_hip_device_block **out) {
   auto it = v->buffers.find(dev);
   if (it != v->buffers.end()) {
-    *out = it->second;
+    *out = &it->second;
     return SAREK_HIP_OK;
   }
   // Gpu_memory.with_retry round the allocation, track_alloc after it (Transfer.ml:184-218)
@@ -114,9 +119,9 @@ int ensure_buffer(sarek_hip_vector_s *v, int dev, void **out) {
       },
       &attempt);
   if (st != SAREK_HIP_OK) return st;
-  v->buffers[dev] = attempt.p;
+  *out = &v->buffers[dev];
+  (*out)->ptr = attempt.p;
   sarek_hip_gpu_memory_track_alloc(static_cast<int64_t>(bytes_of(v)));
-  *out = attempt.p;
   return SAREK_HIP_OK;
 }
 
@@ -127,7 +132,7 @@ int to_device(sarek_hip_vector_s *v, int dev) {
   if (on_device(v, SAREK_HIP_LOC_GPU, dev) || on_device(v, SAREK_HIP_LOC_BOTH, dev) ||
       on_device(v, SAREK_HIP_LOC_STALE_CPU, dev))
     return SAREK_HIP_OK;
-  void *buf = nullptr;
+  sarek_hip_device_block *buf = nullptr;
   int st = ensure_buffer(v, dev, &buf);
   if (st != SAREK_HIP_OK) return st;
   if (!v->zero_copy) {
@@ -135,10 +140,10 @@ int to_device(sarek_hip_vector_s *v, int dev) {
     // order; any other copy is complete on return.
     int current = -1;
     st = SAREK_HIP_E_UNSUPPORTED;
-    if (!v->shown && bytes_of(v) <= kSmallBytes && hipGetDevice(&current) == hipSuccess && current == dev)
-      st = put_small(buf, v->host, bytes_of(v));
-    v->in_order |= st == SAREK_HIP_OK;
-    if (st == SAREK_HIP_E_UNSUPPORTED) st = sarek_hip_memcpy_htod(buf, v->host, bytes_of(v));
+    if (!buf->shown && bytes_of(v) <= kSmallBytes && hipGetDevice(&current) == hipSuccess && current == dev)
+      st = put_small(buf->ptr, v->host, bytes_of(v));
+    buf->in_order |= st == SAREK_HIP_OK;
+    if (st == SAREK_HIP_E_UNSUPPORTED) st = sarek_hip_memcpy_htod(buf->ptr, v->host, bytes_of(v));
     if (st != SAREK_HIP_OK) return st;
   }
   v->location = SAREK_HIP_LOC_BOTH;
@@ -163,8 +168,8 @@ int to_cpu(sarek_hip_vector_s *v, bool force) {
   if (v->zero_copy)
     st = sarek_hip_device_synchronize();
   else if (bytes_of(v) <= kSmallBytes && hipGetDevice(&current) == hipSuccess && current == v->device)
-    st = get_small(v->host, it->second, bytes_of(v), current);
-  if (st == SAREK_HIP_E_UNSUPPORTED) st = sarek_hip_memcpy_dtoh(v->host, it->second, bytes_of(v));
+    st = get_small(v->host, it->second.ptr, bytes_of(v), current);
+  if (st == SAREK_HIP_E_UNSUPPORTED) st = sarek_hip_memcpy_dtoh(v->host, it->second.ptr, bytes_of(v));
   if (st != SAREK_HIP_OK) return st;
   v->location = SAREK_HIP_LOC_BOTH;
   return SAREK_HIP_OK;
@@ -241,7 +246,7 @@ int expand_args(const sarek_hip_varg *args, int n, int dev, bool inject_lengths,
         auto it = v->buffers.find(dev);
         if (it == v->buffers.end()) return fail(SAREK_HIP_E_INVALID_ARG, "Vector has no device buffer");
         a.kind = SAREK_HIP_ARG_BUFFER;
-        a.buffer = it->second;
+        a.buffer = it->second.ptr;
         a.length = v->length;
         out.push_back(a);
         // the length parameter of a kernel is an int32 (sarek-cuda/Sarek_ir_cuda.ml:668-672); a longer
@@ -445,7 +450,7 @@ int sarek_hip_vector_destroy(sarek_hip_vector v) {
   if (!v) return SAREK_HIP_OK;
   int first = SAREK_HIP_OK;
   for (auto &b : v->buffers) {      // what the reference's finaliser does (Gpu_memory.ml:163-178)
-    int st = sarek_hip_mem_free(b.second);
+    int st = sarek_hip_mem_free(b.second.ptr);
     if (st == SAREK_HIP_OK) sarek_hip::track_gc_free(static_cast<int64_t>(v->length * v->elem_size));
     if (first == SAREK_HIP_OK) first = st;
   }
@@ -600,9 +605,10 @@ int sarek_hip_vector_device_ptr(sarek_hip_vector v, void **dptr) {
   int st = current_device(&dev);
   if (st != SAREK_HIP_OK) return st;
   auto it = v->buffers.find(dev);
-  *dptr = it == v->buffers.end() ? nullptr : it->second;
-  if (*dptr) v->shown = true;
-  if (*dptr && v->in_order) {
+  *dptr = nullptr;
+  if (it == v->buffers.end()) return SAREK_HIP_OK;
+  it->second.shown = true;
+  if (it->second.in_order) {
     // From here on other streams may read the block: what the default stream was given is waited for, a caller's stream
     // capture left alone.
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
@@ -610,8 +616,9 @@ int sarek_hip_vector_device_ptr(sarek_hip_vector v, void **dptr) {
     const hipError_t e = hipStreamSynchronize(nullptr);
     SAREK_HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
     SAREK_HIP_TRY(e);
-    v->in_order = false;
+    it->second.in_order = false;
   }
+  *dptr = it->second.ptr;
   return SAREK_HIP_OK;
 }
 
@@ -695,7 +702,7 @@ int sarek_hip_transfer_free_buffers(sarek_hip_vector v) {
   if (!v) return fail(SAREK_HIP_E_INVALID_ARG, "free_buffers: NULL vector");
   int first = SAREK_HIP_OK;
   for (auto &b : v->buffers) {
-    int st = sarek_hip_mem_free(b.second);
+    int st = sarek_hip_mem_free(b.second.ptr);
     sarek_hip_gpu_memory_track_free(static_cast<int64_t>(v->length * v->elem_size));
     if (first == SAREK_HIP_OK) first = st;
   }
