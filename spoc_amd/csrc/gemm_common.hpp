@@ -34,11 +34,11 @@ int compute_units();
 // float32 products straight from memory to registers (gemm_f32_direct.hip): variants (row_blocks, waves) = (1, 8), (1, 4),
 // (2, 4)
 bool gemm_f32_direct_serves(int m, int n, int k);
-bool gemm_f32_direct_pays(int m, int n, int k);
+bool gemm_f32_direct_pays(int m, int n, int k, bool cuts);
 int gemm_f32_direct_pieces(int m, int n, int k, int row_blocks, int splits);
 double gemm_f32_direct_estimate(int m, int n, int k, int row_blocks, int waves, int splits);
 int launch_gemm_f32_direct(const float *a, const float *b, float *c, int m, int n, int k, int row_blocks, int waves,
-                           int splits, hipStream_t st);
+                           int splits, float *partials, hipStream_t st);   // partials: splitk_workspace's block where splits > 1
 
 // 16-bit products in tiles of at most 64 rows, straight from memory to registers (gemm16_rows.hip)
 bool gemm16_rows_serves(int m, int n, int k);

@@ -547,16 +547,20 @@ double ring_estimate(int m, int n, int k, int tile, int64_t cut, int splits) {
 // The variant and the pieces with the lowest estimate.  Pieces are tried only while they leave every wave a step (direct) or
 // three slabs (LDS).  Of the LDS tiles those past whole turns of CUs are cut: all of them where there is no whole turn, which
 // pays for the 64 x 64 tile alone.
+// block: whether there is one for the pieces' sums.  Without (stream capture, hipStreamPerThread, the seventeenth stream)
+// nothing is cut, and a tile that was chosen for its cut is not the one to run whole: in a graph 247 x 1600 x 2884 took 48 us,
+// 26 as planned here, 1380 x 3328 x 2112 236 and 156.
 // gemm_f32.direct: 1 = never, 18 / 14 / 24 = always, with (row_blocks, waves) these digits, any other value as 0;
 // gemm_f32.tile forces a tile, gemm_f32.split_k the pieces (1 = whole) of all 64 x 64 tiles or of a forced direct variant;
 // gemm_f32.cut: 1 = no tile is cut by the rule, n >= 2 = the tiles past whole rounds into n.  0 leaves the choice here.
-Plan plan_for(int m, int n, int k, bool ring_ok) {
+Plan plan_for(int m, int n, int k, bool ring_ok, bool block) {
   constexpr int kPieces[] = {1, 2, 3, 4, 6, 8, 12, 16};
   const int64_t asked = tunable("gemm_f32.direct", 0);
   const int direct = asked == 1 || asked == 18 || asked == 14 || asked == 24 ? static_cast<int>(asked) : 0;
   const int forced = static_cast<int>(tunable("gemm_f32.tile", 0));
   const int tile = forced == 0 || forced == 256 || forced == 128 ? forced : 64;
-  const int64_t split = tunable("gemm_f32.split_k", 0), cutting = tunable("gemm_f32.cut", 0);
+  int64_t split = tunable("gemm_f32.split_k", 0), cutting = tunable("gemm_f32.cut", 0);
+  if (!block) split = std::min<int64_t>(split, 1), cutting = 1;
   const bool direct_ok = gemm_f32_direct_serves(m, n, k);
   if (direct > 1 && direct_ok)
     return {direct / 10, direct % 10, 0, gemm_f32_direct_pieces(m, n, k, direct / 10, static_cast<int>(std::min<int64_t>(split, 64))), 0};
@@ -565,11 +569,11 @@ Plan plan_for(int m, int n, int k, bool ring_ok) {
   double best_us = 1e300;
   // (the clock probe of the measurement build is the ring kernels': a launch that it watches goes to them)
   const bool probed = kMeasureBuild && clock_probe(1) != nullptr;
-  if (direct == 0 && direct_ok && !(probed && ring_ok) && (!ring_ok || (tile == 0 && split == 0 && gemm_f32_direct_pays(m, n, k))))
+  if (direct == 0 && direct_ok && !(probed && ring_ok) && (!ring_ok || (tile == 0 && split == 0 && gemm_f32_direct_pays(m, n, k, block))))
     for (const auto [row_blocks, waves] : {std::pair{1, 8}, std::pair{1, 4}, std::pair{2, 4}}) {
       const int64_t tiles = ceil_div(m, 16 * row_blocks) * ceil_div(n, 64);
       for (const int pieces : kPieces) {
-        if (pieces > 1 && (k / 16 / pieces < waves || tiles * pieces > 4 * cus)) break;
+        if (pieces > 1 && (!block || k / 16 / pieces < waves || tiles * pieces > 4 * cus)) break;
         const int splits = gemm_f32_direct_pieces(m, n, k, row_blocks, pieces);
         const double us = 1.01 * gemm_f32_direct_estimate(m, n, k, row_blocks, waves, splits);
         if (us < best_us) best_us = us, best = {row_blocks, waves, 0, splits, 0};
@@ -603,7 +607,7 @@ Plan plan_for(int m, int n, int k, bool ring_ok) {
 
 extern "C" int sarek_hip_gemm_f32_k_splits(int m, int n, int k) {
   if (m < 1 || n < 1 || k < 1) return 1;
-  const Plan plan = plan_for(m, n, k, k >= 32 || k % 4 == 0);
+  const Plan plan = plan_for(m, n, k, k >= 32 || k % 4 == 0, true);
   return plan.row_blocks > 0 || (plan.tile > 0 && plan.cut_tiles == tiles_of(m, n, plan.tile)) ? plan.splits : 1;
 }
 
@@ -626,15 +630,17 @@ extern "C" int sarek_hip_gemm_f32(const float *a, const float *b, float *c, int 
   const bool c_aligned = reinterpret_cast<uintptr_t>(c) % 16 == 0;
   const bool fallback = tunable("gemm_f32.force_simple", 0) != 0 || tunable("gemm_f32.force_staged", 0) != 0;
   Plan plan{0, 0, 0, 1, 0};
-  if (!fallback) plan = plan_for(m, n, k, ring_ok);
-  if (plan.row_blocks > 0) return launch_gemm_f32_direct(a, b, c, m, n, k, plan.row_blocks, plan.waves, plan.splits, st);
+  float *partials = nullptr;
+  if (!fallback) {
+    plan = plan_for(m, n, k, ring_ok, true);
+    if (plan.splits > 1 && !(partials = splitk_workspace(st))) plan = plan_for(m, n, k, ring_ok, false);
+  }
+  if (plan.row_blocks > 0) return launch_gemm_f32_direct(a, b, c, m, n, k, plan.row_blocks, plan.waves, plan.splits, partials, st);
   if (plan.tile > 0) {
     const bool ragged = !aligned || n % 4 != 0 || k % 32 != 0 || !c_aligned;
     const int tile = plan.tile;
     const int64_t tiles = tiles_of(m, n, tile);
-    int splits = plan.splits, cut_tiles = plan.cut_tiles;
-    float *partials = cut_tiles > 0 ? splitk_workspace(st) : nullptr;
-    if (!partials) splits = 1, cut_tiles = 0;
+    const int splits = plan.splits, cut_tiles = plan.cut_tiles;
     // two workgroups to a CU where there is work for them and LDS (64 KiB for the two smaller tiles, 128 for the largest)
     const int64_t columns = compute_units(), cut_blocks = static_cast<int64_t>(cut_tiles) * splits;
     const int64_t turns = ceil_div(cut_blocks, columns) + ceil_div(tiles - cut_tiles, columns);

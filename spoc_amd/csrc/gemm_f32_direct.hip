@@ -213,9 +213,8 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_f32_direct_kernel(const floa
 }
 
 template <int MT, int W>
-int launch(const float *a, const float *b, float *c, int m, int n, int k, int splits, hipStream_t st) {
+int launch(const float *a, const float *b, float *c, int m, int n, int k, int splits, float *partials, hipStream_t st) {
   const int tiles_m = (m + 16 * MT - 1) / (16 * MT), tiles_n = (n + kCols - 1) / kCols, steps = (k + kStepK - 1) / kStepK;
-  float *partials = splits > 1 ? splitk_workspace(st) : nullptr;
   if (!partials) splits = 1;
   const int per = (steps + splits - 1) / splits;
   const double run = std::min(1.0, splits / static_cast<double>(NUM_XCD)) * tiles_m * tiles_n;
@@ -236,8 +235,8 @@ bool gemm_f32_direct_serves(int m, int n, int k) {
 }
 
 // Up to 6 GFLOP: above, the LDS kernel with its last tiles cut is level or ahead (1280 x 1644 x 960, 4 GFLOP: 41 us here, 36
-// there; 1500^3, 7: 62 and 57; 2049 x 4097 x 3000, 50: 408 and 388).
-bool gemm_f32_direct_pays(int m, int n, int k) { return static_cast<double>(m) * n * k <= 3e9; }
+// there; 1500^3, 7: 62 and 57; 2049 x 4097 x 3000, 50: 408 and 388).  Up to 10 where tiles cannot be cut.
+bool gemm_f32_direct_pays(int m, int n, int k, bool cuts) { return static_cast<double>(m) * n * k <= (cuts ? 3e9 : 5e9); }
 
 // At most `splits` pieces of K: of whole steps, none empty, their planes within the workspace and a ticket per tile.
 int gemm_f32_direct_pieces(int m, int n, int k, int row_blocks, int splits) {
@@ -270,10 +269,10 @@ double gemm_f32_direct_estimate(int m, int n, int k, int row_blocks, int waves, 
 }
 
 int launch_gemm_f32_direct(const float *a, const float *b, float *c, int m, int n, int k, int row_blocks, int waves,
-                           int splits, hipStream_t st) {
-  if (row_blocks == 2) return launch<2, 4>(a, b, c, m, n, k, splits, st);
-  if (waves == 8) return launch<1, 8>(a, b, c, m, n, k, splits, st);
-  return launch<1, 4>(a, b, c, m, n, k, splits, st);
+                           int splits, float *partials, hipStream_t st) {
+  if (row_blocks == 2) return launch<2, 4>(a, b, c, m, n, k, splits, partials, st);
+  if (waves == 8) return launch<1, 8>(a, b, c, m, n, k, splits, partials, st);
+  return launch<1, 4>(a, b, c, m, n, k, splits, partials, st);
 }
 
 }  // namespace sarek_hip

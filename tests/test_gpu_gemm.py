@@ -883,6 +883,38 @@ def test_gemm_f32_tiles_past_whole_turns(hip, torch_cuda, tile, cut, m, n, k):
             hip.set_tunable(name, 0)
 
 
+@pytest.mark.parametrize("m,n,k,knobs", [(247, 1600, 2884, dict(direct=18)), (1380, 3328, 2112, dict(tile=64)), (720, 144, 4090, dict(direct=18)),
+                                         (578, 3308, 2200, dict(direct=24))])
+def test_gemm_f32_plan_without_a_block_for_pieces(hip, torch_cuda, m, n, k, knobs):
+    """Under capture there is no block for the sums of K pieces: the product is planned as one that cannot be cut, not run
+    whole on the tile that the cut was to pay for.  The same bits as with the better of the uncut plans asked for (the plans
+    differ in the order of the sums), and not those of the eager plan, which cuts."""
+    torch = torch_cuda
+    torch.manual_seed(k)
+    a, b = torch.rand(m, k, device="cuda") * 2 - 1, torch.rand(k, n, device="cuda") * 2 - 1
+    eager = hip.gemm_f32(a, b)
+    asked = dict({"gemm_f32.split_k": 1}, **{"gemm_f32." + name: value for name, value in knobs.items()})
+    try:
+        for name, value in asked.items():
+            hip.set_tunable(name, value)
+        want = hip.gemm_f32(a, b)
+    finally:
+        for name in asked:
+            hip.set_tunable(name, 0)
+    assert not torch.equal(eager, want)
+    got, graph = torch.full((m, n), float("nan"), device="cuda"), torch.cuda.CUDAGraph()
+    side = side_stream(torch)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        hip.gemm_f32(a, b, out=got)
+    for _ in range(3):
+        got.fill_(float("nan"))
+        graph.replay()
+        assert torch.equal(hip.gemm_f32(a, b), eager)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 32), (16, 128, 256), (17, 129, 257), (15, 127, 33), (33, 3, 1000), (48, 264, 520),
                                    (49, 255, 4129), (64, 1001, 1001), (64, 640, 2048), (65, 130, 96)])
