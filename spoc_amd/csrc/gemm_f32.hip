@@ -176,7 +176,7 @@ __global__ __launch_bounds__(THREADS) void gemm_f32_staged_kernel(const float *_
 // What K is over whole slabs is at its start, outside the K loop: with it in a slab at the end, moved back over the one
 // before, every turn of the loop chose its offsets by masks (64 x 64 tile: 2049 x 4097 x 3000 428 us, now 404; 2031 x 1792 x
 // 2211 143, 135; 1500^3 77, 72).
-template <int TI, int TJ, int WMW, int WNW, int BKT, int NS, bool Ragged>
+template <int TI, int TJ, int WMW, int WNW, int BKT, int NS, bool Ragged, int Chains>
 __global__ __launch_bounds__(64 * WMW * WNW, 2) void gemm_f32_dma_kernel(
     const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int M, int N,
     int K, int tiles_m, int tiles_n, int xcd_remap, unsigned long long *probe, int columns, int cut_tiles, int pieces, int k_chunk,
@@ -262,13 +262,12 @@ __global__ __launch_bounds__(64 * WMW * WNW, 2) void gemm_f32_dma_kernel(
     const int keep = Ragged && a_lane_k < head && head < a_lane_k + 4 ? head - a_lane_k : 0;
     constexpr uint32_t kOutOfRange = 0x80000000u;
 
-    // Accumulators to an element, for the MFMA steps in turn, added at the end.  Shorter sums are closer to the product (2049 x
-    // 4097 x 3000 on the 64 x 64 tile: 6.9e-7 of the result with two, 4.8e-7 with four), and a wave with a single MFMA tile does
-    // not feed every MFMA the result of the one before.  Eight for that tile: 3.4e-7, and 0.5 to 4 % of the time.
-    constexpr int kChains = TI * TJ == 1 ? 4 : TI * TJ <= 4 ? 2 : 1;
-    f32x16 acc[kChains][TI][TJ];
+    // Chains: accumulators to an element, for the MFMA steps in turn, added at the end.  Shorter sums are closer to the product
+    // (2049 x 4097 x 3000 on the 64 x 64 tile: 6.9e-7 of the result with two, 4.8e-7 with four, 3.4e-7 with eight, which cost 0 to
+    // 2 % of the time), and a wave with a single MFMA tile does not feed every MFMA the result of the one before.
+    f32x16 acc[Chains][TI][TJ];
 #pragma unroll
-    for (int h = 0; h < kChains; ++h)
+    for (int h = 0; h < Chains; ++h)
 #pragma unroll
       for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -315,15 +314,16 @@ __global__ __launch_bounds__(64 * WMW * WNW, 2) void gemm_f32_dma_kernel(
       for (int j = 0; j < 4; ++j)
         bf[j] = *reinterpret_cast<const bvec_t *>(sb + b_addr0 + (kk * 8 + j) * B_ROW);
     };
-    auto mfma_step = [&](f32x4 (&af)[TI], bvec_t (&bf)[4]) {
+    auto mfma_step = [&](int kk, f32x4 (&af)[TI], bvec_t (&bf)[4]) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int i = 0; i < TI; ++i)
 #pragma unroll
-          for (int jn = 0; jn < TJ; ++jn)
-            acc[j % kChains][i][jn] =
-                __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][j], bf[j][jn], acc[j % kChains][i][jn], 0, 0, 0);
+          for (int jn = 0; jn < TJ; ++jn) {
+            f32x16 &chain = acc[(4 * kk + j) % Chains][i][jn];
+            chain = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][j], bf[j][jn], chain, 0, 0, 0);
+          }
     };
     // Issue order inside one k-step: behind each of the first MFMAs go the DMA instructions
     // of this k-step (NV of them; unpinned, the compiler bunches them in front of the first
@@ -355,14 +355,14 @@ __global__ __launch_bounds__(64 * WMW * WNW, 2) void gemm_f32_dma_kernel(
 #pragma unroll
       for (int kk = 0; kk + 1 < KK; ++kk) {
         load_frags(ca, cb, kk + 1, af[(kk + 1) & 1], bf[(kk + 1) & 1]);
-        mfma_step(af[kk & 1], bf[kk & 1]);
+        mfma_step(kk, af[kk & 1], bf[kk & 1]);
         interleave(std::integral_constant<int, 0>{});
       }
       __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0((NS - 2) * (A_DMA + B_DMA)));
       barrier_no_fence();
       issue(std::integral_constant<int, -1>{}, ca, cb);
       load_frags(na, nb, 0, af[0], bf[0]);
-      mfma_step(af[(KK - 1) & 1], bf[(KK - 1) & 1]);
+      mfma_step(KK - 1, af[(KK - 1) & 1], bf[(KK - 1) & 1]);
       interleave(std::integral_constant<int, A_DMA + B_DMA>{});
     };
 
@@ -414,9 +414,11 @@ __global__ __launch_bounds__(64 * WMW * WNW, 2) void gemm_f32_dma_kernel(
     for (int i = 0; i < TI; ++i)
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
+#pragma unroll
+        for (int h = 1; h < Chains; h *= 2)
+#pragma unroll
+          for (int c = 0; c + h < Chains; c += 2 * h) acc[c][i][j] += acc[c + h][i][j];
         sum[i][j] = acc[0][i][j];
-        if constexpr (kChains == 2) sum[i][j] += acc[1][i][j];
-        if constexpr (kChains == 4) sum[i][j] = (sum[i][j] + acc[1][i][j]) + (acc[2][i][j] + acc[3][i][j]);
       }
 
     // A piece's sums go to its plane, past the XCD's L2, in the order its threads hold them; the workgroup that draws a
@@ -516,6 +518,7 @@ namespace {
 struct Plan {
   int row_blocks, waves, tile, splits;
   int cut_tiles;   // of the LDS tiles, how many are cut into `splits` pieces of K: the last ones
+  int chains;      // sums an element and piece on an LDS tile
 };
 
 int64_t tiles_of(int m, int n, int tile) { return ceil_div(m, tile) * ceil_div(n, tile); }
@@ -547,6 +550,14 @@ double ring_estimate(int m, int n, int k, int tile, int64_t cut, int splits) {
 // The variant and the pieces with the lowest estimate.  Pieces are tried only while they leave every wave a step (direct) or
 // three slabs (LDS).  Of the LDS tiles those past whole turns of CUs are cut: all of them where there is no whole turn, which
 // pays for the 64 x 64 tile alone.
+// An element is the sum of shorter ones, of the waves, the chains and the pieces, and its error grows with their length, so a
+// plan is not left for a faster one with fewer sums: of the LDS tiles that are cut and of all 64 x 64 ones only those count
+// that have as many as the direct variant which would be taken up to 10 GFLOP (four to eight a piece).  The 64 x 64 tile has
+// eight chains where it would have fewer otherwise, and where products of under two turns are cut (they were all cut, into
+// three pieces or more, before their last tiles alone were).  K = 4000, some 300 tiles: eight waves 4.0e-7 of the result, four
+// chains 5.5e-7, eight 3.8e-7 (640 x 1770 x 3844: 99 us, 75.3 and 75.6).  Of 40000 products drawn over 64 .. 4100 a side one has
+// fewer sums than before there were cuts (24 for 30).  Tiles that are all cut weigh a 26th less than they are estimated at
+// against four sums of the direct kernel, for the same reason.
 // block: whether there is one for the pieces' sums.  Without (stream capture, hipStreamPerThread, the seventeenth stream)
 // nothing is cut, and a tile that was chosen for its cut is not the one to run whole: in a graph 247 x 1600 x 2884 took 48 us,
 // 26 as planned here, 1380 x 3328 x 2112 236 and 156.
@@ -563,30 +574,37 @@ Plan plan_for(int m, int n, int k, bool ring_ok, bool block) {
   if (!block) split = std::min<int64_t>(split, 1), cutting = 1;
   const bool direct_ok = gemm_f32_direct_serves(m, n, k);
   if (direct > 1 && direct_ok)
-    return {direct / 10, direct % 10, 0, gemm_f32_direct_pieces(m, n, k, direct / 10, static_cast<int>(std::min<int64_t>(split, 64))), 0};
+    return {direct / 10, direct % 10, 0, gemm_f32_direct_pieces(m, n, k, direct / 10, static_cast<int>(std::min<int64_t>(split, 64))), 0, 0};
   const int64_t cus = compute_units();
-  Plan best{0, 0, 0, 1, 0};
-  double best_us = 1e300;
+  Plan best{0, 0, 0, 1, 0, 0}, best_direct = best;
+  double best_us = 1e300, direct_us = 1e300;
   // (the clock probe of the measurement build is the ring kernels': a launch that it watches goes to them)
   const bool probed = kMeasureBuild && clock_probe(1) != nullptr;
-  if (direct == 0 && direct_ok && !(probed && ring_ok) && (!ring_ok || (tile == 0 && split == 0 && gemm_f32_direct_pays(m, n, k, block))))
+  if (direct == 0 && direct_ok && !(probed && ring_ok) && (!ring_ok || (tile == 0 && split == 0 && gemm_f32_direct_pays(m, n, k, false))))
     for (const auto [row_blocks, waves] : {std::pair{1, 8}, std::pair{1, 4}, std::pair{2, 4}}) {
       const int64_t tiles = ceil_div(m, 16 * row_blocks) * ceil_div(n, 64);
       for (const int pieces : kPieces) {
         if (pieces > 1 && (!block || k / 16 / pieces < waves || tiles * pieces > 4 * cus)) break;
         const int splits = gemm_f32_direct_pieces(m, n, k, row_blocks, pieces);
         const double us = 1.01 * gemm_f32_direct_estimate(m, n, k, row_blocks, waves, splits);
-        if (us < best_us) best_us = us, best = {row_blocks, waves, 0, splits, 0};
+        if (us < direct_us) direct_us = us, best_direct = {row_blocks, waves, 0, splits, 0, 0};
       }
     }
+  if (!ring_ok || gemm_f32_direct_pays(m, n, k, block)) best_us = direct_us, best = best_direct;
   if (!ring_ok) return best;
+  const int direct_sums = best_direct.waves * best_direct.splits;
   for (const int t : {64, 128, 256}) {
     if (tile != 0 && tile != t) continue;
     const int64_t tiles = tiles_of(m, n, t), over = tiles % cus;
     auto consider = [&](int64_t cut, int splits) {
-      if (splits < 2) cut = 0;
-      const double us = ring_estimate(m, n, k, t, cut, splits);
-      if (us < best_us) best_us = us, best = {0, 0, t, cut > 0 ? splits : 1, static_cast<int>(cut)};
+      if (splits < 2) cut = 0, splits = 1;
+      const int pieces = cut == tiles ? splits : 1;   // of every element
+      double us = ring_estimate(m, n, k, t, cut, splits);
+      if (cut == tiles && direct_sums == 4) us /= 1.04;
+      int chains = t == 256 ? 1 : t == 128 ? 2 : 4;
+      if (t == 64 && (chains * pieces < direct_sums || (cut > 0 && tiles < 2 * cus))) chains = 8;
+      if (chains * pieces < direct_sums && (t == 64 || cut > 0 || us >= direct_us)) return;
+      if (us < best_us) best_us = us, best = {0, 0, t, splits, static_cast<int>(cut), chains};
     };
     if (t == 64 && split >= 2) {
       consider(tiles, ring_pieces(tiles, k, t, split));
@@ -601,7 +619,7 @@ Plan plan_for(int m, int n, int k, bool ring_ok, bool block) {
     for (int pieces = 2; over > 0 && (t == 64 || over < tiles) && pieces <= 12 && k / pieces >= 96; ++pieces)
       consider(over, ring_pieces(over, k, t, pieces));
   }
-  return best;
+  return best.tile > 0 || best.row_blocks > 0 ? best : best_direct;
 }
 }  // namespace
 
@@ -629,7 +647,7 @@ extern "C" int sarek_hip_gemm_f32(const float *a, const float *b, float *c, int 
   const bool ring_ok = ab_ok && offsets_ok;
   const bool c_aligned = reinterpret_cast<uintptr_t>(c) % 16 == 0;
   const bool fallback = tunable("gemm_f32.force_simple", 0) != 0 || tunable("gemm_f32.force_staged", 0) != 0;
-  Plan plan{0, 0, 0, 1, 0};
+  Plan plan{0, 0, 0, 1, 0, 0};
   float *partials = nullptr;
   if (!fallback) {
     plan = plan_for(m, n, k, ring_ok, true);
@@ -647,20 +665,22 @@ extern "C" int sarek_hip_gemm_f32(const float *a, const float *b, float *c, int 
     const int64_t items = cut_blocks + tiles - cut_tiles;
     const int64_t workgroups = turns == 1 ? items : columns * (tile == 256 ? 1 : 2);
     const int k_chunk = cut_tiles > 0 ? splitk_chunk(k, slab_of(tile), splits) : k;
-#define SAREK_LAUNCH_F32(T, TI, TJ, WMW, WNW, BKT, RAGGED)                                  \
-  hipLaunchKernelGGL((gemm_f32_dma_kernel<TI, TJ, WMW, WNW, BKT, 4, RAGGED>),              \
+#define SAREK_LAUNCH_F32(T, TI, TJ, WMW, WNW, BKT, RAGGED, CHAINS)                                  \
+  hipLaunchKernelGGL((gemm_f32_dma_kernel<TI, TJ, WMW, WNW, BKT, 4, RAGGED, CHAINS>),              \
                      dim3(static_cast<unsigned>(workgroups)),                                              \
                      dim3(64 * WMW * WNW), 0, st, a, b, c, m, n, k, (m + T - 1) / T, (n + T - 1) / T, remap, \
                      cut_tiles > 0 ? nullptr : clock_probe(workgroups), static_cast<int>(columns), cut_tiles, splits, k_chunk, partials, \
                      partials ? splitk_tickets(partials) : nullptr)
     if (ragged) {
-      if (tile == 256) SAREK_LAUNCH_F32(256, 4, 2, 2, 4, 16, true);
-      else if (tile == 128) SAREK_LAUNCH_F32(128, 2, 2, 2, 2, 16, true);
-      else SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, true);
+      if (tile == 256) SAREK_LAUNCH_F32(256, 4, 2, 2, 4, 16, true, 1);
+      else if (tile == 128) SAREK_LAUNCH_F32(128, 2, 2, 2, 2, 16, true, 2);
+      else if (plan.chains == 8) SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, true, 8);
+      else SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, true, 4);
     } else {
-      if (tile == 256) SAREK_LAUNCH_F32(256, 4, 2, 2, 4, 16, false);
-      else if (tile == 128) SAREK_LAUNCH_F32(128, 2, 2, 2, 2, 16, false);
-      else SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, false);
+      if (tile == 256) SAREK_LAUNCH_F32(256, 4, 2, 2, 4, 16, false, 1);
+      else if (tile == 128) SAREK_LAUNCH_F32(128, 2, 2, 2, 2, 16, false, 2);
+      else if (plan.chains == 8) SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, false, 8);
+      else SAREK_LAUNCH_F32(64, 1, 1, 2, 2, 32, false, 4);
     }
 #undef SAREK_LAUNCH_F32
     return check_launch("gemm_f32 kernel launch");

@@ -883,6 +883,26 @@ def test_gemm_f32_tiles_past_whole_turns(hip, torch_cuda, tile, cut, m, n, k):
             hip.set_tunable(name, 0)
 
 
+@pytest.mark.parametrize("m,n,k,variant", [(270, 3915, 4063, 18), (972, 1055, 4054, 18), (439, 2616, 3950, 18), (640, 1770, 3844, 18),
+                                           (1089, 1024, 3813, 18), (2560, 1792, 1088, 24), (501, 2688, 3520, 18), (1638, 3328, 576, 24)])
+def test_gemm_f32_sums_no_longer_than_the_direct_kernel_has(hip, torch_cuda, m, n, k, variant):
+    """Products that the direct kernel computed (its variant by its digits) before their last LDS tiles could be cut: as close to
+    float64 as there.  The error of a sum of rounded additions goes with the square root of its length, the same or shorter
+    here; two random walks of some 10^6 elements differ by far less than the twentieth that is allowed."""
+    torch = torch_cuda
+    torch.manual_seed(n)
+    a, b = torch.rand(m, k, device="cuda") * 2 - 1, torch.rand(k, n, device="cuda") * 2 - 1
+    ref = a.double() @ b.double()
+    error = lambda c: float((c.double() - ref).norm() / ref.norm())  # noqa: E731
+    own = error(hip.gemm_f32(a, b))
+    try:
+        hip.set_tunable("gemm_f32.direct", variant)
+        direct = error(hip.gemm_f32(a, b))
+    finally:
+        hip.set_tunable("gemm_f32.direct", 0)
+    assert own <= 1.05 * direct, (own, direct)
+
+
 @pytest.mark.parametrize("m,n,k,knobs", [(247, 1600, 2884, dict(direct=18)), (1380, 3328, 2112, dict(tile=64)), (720, 144, 4090, dict(direct=18)),
                                          (578, 3308, 2200, dict(direct=24))])
 def test_gemm_f32_plan_without_a_block_for_pieces(hip, torch_cuda, m, n, k, knobs):
