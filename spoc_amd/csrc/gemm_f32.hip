@@ -531,15 +531,17 @@ int ring_pieces(int64_t cut, int k, int tile, int64_t splits) {
   return splitk_pieces(k, slab_of(tile), std::max<int64_t>(1, std::min<int64_t>({splits, static_cast<int64_t>(k / 32), fit})));
 }
 
-// Estimated time in us of the LDS kernels: of 300 drawn products of 0.2 to 50 GFLOP, on which every tile was timed with
-// 1 to 12 pieces, the plan with the lowest estimate takes 0.8 % more than the best one.  A 64 x 64 tile takes 0.46 us per K = 32
+// Estimated time in us of the LDS kernels, fitted to 300 drawn products of 0.2 to 50 GFLOP.  On 440 others, drawn over 64 ..
+// 4100 a side from 20 MFLOP on, the plan with the lowest estimate takes 1.2 % more than the fastest of those that were timed; 34
+// take more than 5 % and 10 more than 10 %, the worst 21 % (profiles/gemm_f32_plans.txt).  A 64 x 64 tile takes 0.46 us per K = 32
 // slab alone on its CU, and two on a CU share its matrix cores, so tiles count in turns of CUs; the larger ones take four and
-// sixteen times as long less the operand traffic they save.  Tiles that are cut come on top, in turns of their pieces, with the
-// planes to write and to add.
+// sixteen times as long less the operand traffic they save.  A turn's start and stores are 6 us on the 256 x 256 tile, whose
+// launch has one workgroup to a CU (2816 x 4096 x 90 36.2 us on it, 31.0 on 128 x 128; counted as 3 us it was taken).  Tiles that
+// are cut come on top, in turns of their pieces, with the planes to write and to add.
 double ring_estimate(int m, int n, int k, int tile, int64_t cut, int splits) {
   const int64_t tiles = tiles_of(m, n, tile), cus = compute_units();
   const double slabs = k / 32.0, c_mb = 4e-6 * m * n;
-  const double slab = tile == 64 ? 0.458 : tile == 128 ? 1.807 : 7.38, each = tile == 64 ? 1.06 : 2.96;
+  const double slab = tile == 64 ? 0.458 : tile == 128 ? 1.807 : 7.38, each = tile == 64 ? 1.06 : tile == 128 ? 2.96 : 6.0;
   double us = 3.89 + static_cast<double>(ceil_div(tiles - cut, cus)) * (slabs * slab + each) + 0.141 * c_mb;
   if (cut > 0)
     us += static_cast<double>(ceil_div(cut * splits, cus)) * (slabs / splits * slab + each) + 3.44 +

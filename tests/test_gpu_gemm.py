@@ -883,6 +883,23 @@ def test_gemm_f32_tiles_past_whole_turns(hip, torch_cuda, tile, cut, m, n, k):
             hip.set_tunable(name, 0)
 
 
+@pytest.mark.parametrize("m,n,k,tile", [(2816, 4096, 90, 128), (3904, 3904, 367, 256)])
+def test_gemm_f32_whole_tiles_at_a_short_k(hip, torch_cuda, m, n, k, tile):
+    """What a turn of the largest tile costs beside its K decides against it where K is short: the product has the bits of the
+    tile that was measured to be the faster, which are not those of the other (one sum an element, or two)."""
+    torch = torch_cuda
+    torch.manual_seed(m)
+    a, b = torch.rand(m, k, device="cuda") * 2 - 1, torch.rand(k, n, device="cuda") * 2 - 1
+    own, forced = hip.gemm_f32(a, b), {}
+    try:
+        for t in (128, 256):
+            hip.set_tunable("gemm_f32.tile", t)
+            forced[t] = hip.gemm_f32(a, b)
+    finally:
+        hip.set_tunable("gemm_f32.tile", 0)
+    assert torch.equal(own, forced[tile]) and not torch.equal(own, forced[384 - tile])
+
+
 @pytest.mark.parametrize("m,n,k,variant", [(270, 3915, 4063, 18), (972, 1055, 4054, 18), (439, 2616, 3950, 18), (640, 1770, 3844, 18),
                                            (1089, 1024, 3813, 18), (2560, 1792, 1088, 24), (501, 2688, 3520, 18), (1638, 3328, 576, 24)])
 def test_gemm_f32_sums_no_longer_than_the_direct_kernel_has(hip, torch_cuda, m, n, k, variant):
