@@ -612,8 +612,9 @@ Plan plan_for(int m, int n, int k, bool ring_ok, bool block) {
       consider(tiles, ring_pieces(tiles, k, t, split));
       continue;
     }
-    if (cutting < 2 || t == 256) consider(0, 1);
-    if (split != 0 || cutting == 1 || probed || t == 256) continue;
+    const bool may_cut = split == 0 && cutting != 1 && !probed && t != 256;
+    if (!may_cut || cutting < 2) consider(0, 1);
+    if (!may_cut) continue;
     if (cutting >= 2) {
       consider(over ? over : std::min(tiles, cus), ring_pieces(over ? over : std::min(tiles, cus), k, t, cutting));
       continue;

@@ -883,6 +883,30 @@ def test_gemm_f32_tiles_past_whole_turns(hip, torch_cuda, tile, cut, m, n, k):
             hip.set_tunable(name, 0)
 
 
+@pytest.mark.parametrize("m,n,k", [(300, 520, 448), (301, 519, 449)])
+@pytest.mark.parametrize("tile,split_k", [(64, 1), (128, 1), (128, 2)])
+def test_gemm_f32_a_forced_tile_runs_where_its_cut_is_switched_off(hip, torch_cuda, m, n, k, tile, split_k):
+    """gemm_f32.split_k = 1 keeps K whole, and a count above it is for the 64 x 64 tile: gemm_f32.cut then says nothing, and the
+    tile that was asked for is the one that runs (its bits, not those of the kernels for shapes that no tile serves)."""
+    torch = torch_cuda
+    torch.manual_seed(k)
+    a, b = torch.rand(m, k, device="cuda") * 2 - 1, torch.rand(k, n, device="cuda") * 2 - 1
+    got = []
+    try:
+        hip.set_tunable("gemm_f32.tile", tile)
+        hip.set_tunable("gemm_f32.direct", 1)
+        hip.set_tunable("gemm_f32.split_k", split_k)
+        for cut in (1, 2):
+            hip.set_tunable("gemm_f32.cut", cut)
+            got.append(hip.gemm_f32(a, b))
+        hip.set_tunable("gemm_f32.force_staged", 1)
+        other = hip.gemm_f32(a, b)
+    finally:
+        for name in ("tile", "direct", "split_k", "cut", "force_staged"):
+            hip.set_tunable("gemm_f32." + name, 0)
+    assert torch.equal(got[0], got[1]) and not torch.equal(got[0], other)
+
+
 @pytest.mark.parametrize("m,n,k,tile", [(2816, 4096, 90, 128), (3904, 3904, 367, 256)])
 def test_gemm_f32_whole_tiles_at_a_short_k(hip, torch_cuda, m, n, k, tile):
     """What a turn of the largest tile costs beside its K decides against it where K is short: the product has the bits of the
