@@ -492,7 +492,8 @@ __device__ __forceinline__ void last_products(const uint16_t *__restrict__ A, co
 // over the 16 lanes that share those rows (with TI = 8: 16+8+4+2 exchanges leave lane m with rows 2m, 2m+1 of the 32;
 // with TI = 4: 8+4+2+1 leave it with row m of the 16), the WNW waves along N through LDS.  The tile's sum of row r then
 // goes to rs_plane[r] when the launch has planes (one per tile column, added up in tile order by
-// rowsum_fold_kernel: the same bits on every run), else to rowsum[r] by atomicAdd.  add_last: the tile rows' last_products
+// rowsum_fold_kernel: the same bits on every run), else to rowsum[r] by atomicAdd.  The 128 x 256 tile has two, for its halves
+// of 128 columns: as many float32 additions in front of the fold's double as on the 128 x 128 tile, whose products it takes.  add_last: the tile rows' last_products
 // lie in `scratch` and belong to column N - 1.
 template <int Epi, int TI, int WNW, bool Ragged, int WMW = 2>   // WMW, WNW: waves along M, N
 __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restrict__ C, const float *__restrict__ bias,
@@ -567,13 +568,23 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
       scratch[wn * TROWS + wm * WROWS + (q >> 2) * 16 + 4 * g + (q & 3)] = rs[e];
     }
     __syncthreads();
-    const int t = threadIdx.x;
-    if (t < TROWS && m0 + t < M) {
-      float total;
-      if constexpr (WNW == 4) total = (scratch[t] + scratch[TROWS + t]) + (scratch[2 * TROWS + t] + scratch[3 * TROWS + t]);
-      else total = scratch[t] + scratch[TROWS + t];
-      if (rs_plane) rs_plane[m0 + t] = total;
-      else atomicAdd(rowsum + m0 + t, total);
+    if constexpr (WMW == 1) {
+      static_assert(WNW == 4 && TROWS == 128, "256 threads: a row of a half each");
+      const int t = threadIdx.x & 127, half = threadIdx.x >> 7;
+      if (m0 + t < M && col0 - wn * 64 + half * 128 < N) {
+        const float total = scratch[2 * half * TROWS + t] + scratch[(2 * half + 1) * TROWS + t];
+        if (rs_plane) rs_plane[static_cast<int64_t>(half) * M + m0 + t] = total;
+        else atomicAdd(rowsum + m0 + t, total);
+      }
+    } else {
+      const int t = threadIdx.x;
+      if (t < TROWS && m0 + t < M) {
+        float total;
+        if constexpr (WNW == 4) total = (scratch[t] + scratch[TROWS + t]) + (scratch[2 * TROWS + t] + scratch[3 * TROWS + t]);
+        else total = scratch[t] + scratch[TROWS + t];
+        if (rs_plane) rs_plane[m0 + t] = total;
+        else atomicAdd(rowsum + m0 + t, total);
+      }
     }
   }
 }
@@ -856,8 +867,8 @@ __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__
   float *scratch = reinterpret_cast<float *>(lds_ring<10, A_BYTES_S>);
   const bool add_last = Ragged && (N & 1) != 0 && n0 + BN >= N;
   if (add_last) last_products<Bf16, TBM>(A, B, M, N, K, ld, m0, 0, scratch);
-  epilogue16<Epi, 8, 4, Ragged, WM>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N,
-                                    ld, m0, wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
+  epilogue16<Epi, 8, 4, Ragged, WM>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * (WM == 1 ? 2 : 1) * M : nullptr,
+                                    M, N, ld, m0, wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
   if (kMeasureBuild && probe && tid == 0) {
     probe[2 * blockIdx.x] = static_cast<unsigned long long>(clock64() - probe_c0);
     probe[2 * blockIdx.x + 1] = static_cast<unsigned long long>(wall_clock64() - probe_t0);
@@ -1655,9 +1666,8 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   const int cut = tiled && tile_choice == 256 && nm > 0 && !(kMeasureBuild && clock_probe(1))
                       ? whole_round_columns(m, nm, k, half) : nm;
   if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
-    const int rest_tile = half ? 256 : 128;   // the columns of the tiles that take [cut, nm), or all where tile_choice is 128
-    const int first = tiled && tile_choice == 128 ? 0 : cut;
-    n_planes = tiled ? (first + 255) / 256 + (nm - first + rest_tile - 1) / rest_tile + (n - nm) : (n + 63) / 64;
+    const int first = tiled && tile_choice == 128 ? 0 : cut;   // columns in planes of 256; from there on in planes of 128
+    n_planes = tiled ? (first + 255) / 256 + (nm - first + 127) / 128 + (n - nm) : (n + 63) / 64;
     if (static_cast<int64_t>(n_planes) * m * 4 <= static_cast<int64_t>(kSplitWorkspaceBytes)) planes = splitk_workspace(st);
     if (!planes) {
       const int rc = launch_zero_f32(rowsum, m, st);

@@ -426,6 +426,39 @@ def test_gemm16_half_tile(hip, oracle, torch_cuda, kind, m, n, k, tile):
         hip.set_tunable("gemm16.tile", 0)
 
 
+@pytest.mark.parametrize("m,n,k", [(128, 256, 64), (300, 1100, 192), (257, 1024, 200), (129, 385, 96), (1000, 3201, 320), (1, 130, 64)])
+def test_gemm16_half_tile_row_sums(hip, torch_cuda, m, n, k):
+    """The fused product on the 128 x 256 tile: a plane of row sums for each 128 columns, also where the last tile's upper half
+    holds none, so the row sums are the bits of the 128 x 128 tile's.  Under capture there is no block for planes: the shares are
+    added by atomics, every row within 1e-5 of the double sum of the stored row, replay after replay."""
+    torch = torch_cuda
+    torch.manual_seed(n)
+    a, b = ((torch.randn(*s, device="cuda") * 0.2).half() for s in ((m, k), (k, n)))
+    bias = torch.rand(n, device="cuda") * 0.2 - 0.1
+    side = side_stream(torch)
+    try:
+        hip.set_tunable("gemm16.tile", 128)
+        hip.set_tunable("gemm16.half", 1)
+        y1, rs1 = hip.gemm_f16_bias_relu_rowsum(a, b, bias)
+        hip.set_tunable("gemm16.half", 2)
+        y, rs = hip.gemm_f16_bias_relu_rowsum(a, b, bias)
+        got, sums, graph = torch.empty_like(y), torch.empty_like(rs), torch.cuda.CUDAGraph()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+            hip.gemm_f16_bias_relu_rowsum(a, b, bias, out=got, rowsum=sums)
+        assert torch.equal(y, y1) and torch.equal(rs, rs1)
+        for _ in range(3):
+            got.fill_(float("nan"))
+            sums.fill_(float("nan"))
+            graph.replay()
+            assert torch.equal(hip.gemm_f16_bias_relu_rowsum(a, b, bias)[1], rs)
+            torch.cuda.synchronize()
+            assert torch.equal(got, y) and rowsums_ok(sums.cpu().numpy(), y.double().sum(1).cpu().numpy())
+    finally:
+        hip.set_tunable("gemm16.half", 0)
+        hip.set_tunable("gemm16.tile", 0)
+
+
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(2048, 8448, 64), (2047, 8195, 72), (1921, 8703, 131), (2048, 10240, 65),
                                    (8192, 2050, 70), (2300, 7425, 200)])
