@@ -636,10 +636,15 @@ int sarek_hip_gemm_f16(const uint16_t *a, const uint16_t *b, float *c, int m, in
  * No counterpart in the reference, whose tiled
  * kernel has one shape (bench_matrix_mul_tiled.ml:55-95); needs no device.  */
 int sarek_hip_gemm16_tile(int m, int n, int k);
-/* How many of the n columns that tile takes.  Columns past whole rounds of
- * 256 x 256 tiles go to the 128 x 128 tile where that pays, and a single column
- * past whole tiles to a kernel of its own where it would add a round.       */
+/* How many of the n columns that tile takes, with those that go to the 128 x
+ * 256 tile.  Columns past whole rounds of 256 x 256 tiles go to the 128 x 128
+ * or the 128 x 256 tile where that pays, and a single column past whole tiles
+ * to a kernel of its own where it would add a round.                        */
 int sarek_hip_gemm16_tile_columns(int m, int n, int k);
+/* How many of the n columns go to the 128 x 256 tile, in place of 128 x 128
+ * ones that would share CUs: all (but a last one that has a kernel of its own),
+ * those past whole rounds of 256 x 256 tiles, or none.                      */
+int sarek_hip_gemm16_half_columns(int m, int n, int k);
 /* Into how many pieces sarek_hip_gemm_bf16 / _f16 cut K for this shape now (1 =
  * none): products with few 128 x 128 tiles and a long K are spread over the
  * CUs that way, the partial tiles added up in a fixed order by a second

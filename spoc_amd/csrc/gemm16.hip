@@ -1395,10 +1395,11 @@ inline bool small_tile_wins(int m, int n) {
 // 236, 6361 x 3264 x 1425 74.7 -> 70.0; two, 2880 x 13120 x 1755 137 -> 132, 5888 x 6400 x 640 60.2 -> 62.0; four, 2880 x
 // 23971 x 1579 234 -> 237; six, 5248 x 20113 x 2313 500 -> 495.  So K has to be 600 for each round and for one more; a
 // product of no whole round counts as of one.
-// gemm16.half: 0 = this rule, 1 = never, 2 = wherever a workgroup per CU takes the columns, whatever K.
+// gemm16.half: 0 = this rule, 1 = never, 2 = in place of the 128 x 128 tile wherever a workgroup per CU takes the columns,
+// whatever K and however few small tiles they would be.  Never where K is asked to be cut (gemm16.split_k >= 2).
 inline bool half_tile_pays(int m, int n, int k, int64_t rounds) {
   const int64_t asked = tunable("gemm16.half", 0);
-  if (asked == 1 || tunable("gemm16.split_k", 0) != 0 || (kMeasureBuild && clock_probe(1))) return false;
+  if (asked == 1 || tunable("gemm16.split_k", 0) >= 2 || (kMeasureBuild && clock_probe(1))) return false;
   const int cus = compute_units();
   const int64_t rows = ceil_div(m, 128);
   if (rows * ceil_div(n, 256) > cus) return false;
@@ -1420,7 +1421,8 @@ inline bool half_tile_pays(int m, int n, int k, int64_t rounds) {
 // 132; 3712 x 39176 (9 rounds) 82 149 -> 155, 768 302 -> 313; 4160 x 8000 (2 rounds) 126 39.2 -> 42.2, 768 66.8 -> 64.7;
 // 2048 x 8448 (1 round) 82 22.6 -> 22.2, 256 24.9 -> 23.9.  So K has to be 128 times the whole rounds: of 417 drawn products
 // of up to 8192 rows the cut cost 48 more than 2 % without that and costs 6 with it.
-// gemm16.cut: 0 = this rule, 1 = never, s >= 2: a rest of up to s small tiles, whatever K.
+// gemm16.cut: 0 = this rule, 1 = never, s >= 2: a rest of up to s small tiles, whatever K.  With gemm16.half = 2 any rest that
+// the 128 x 256 tile takes is cut off.
 inline int whole_round_columns(int m, int n, int k, bool &half) {
   const int64_t asked = tunable("gemm16.cut", 0);
   if (asked == 1 || tunable("gemm16.tile", 0) != 0) return n;
@@ -1429,8 +1431,9 @@ inline int whole_round_columns(int m, int n, int k, bool &half) {
   const int64_t columns = tiles_n - ceil_div(over, tiles_m);
   if (over == 0 || columns < 1) return n;
   const int64_t rest = ceil_div(m, 128) * ceil_div(n - columns * 256, 128);
-  if (asked < 2 && k < tiles_m * tiles_n / cus * 128) return n;
-  if (rest <= (asked >= 2 ? asked : cus)) return static_cast<int>(columns * 256);
+  const bool half_forced = asked < 2 && tunable("gemm16.half", 0) == 2;
+  if (asked < 2 && !half_forced && k < tiles_m * tiles_n / cus * 128) return n;
+  if (!half_forced && rest <= (asked >= 2 ? asked : cus)) return static_cast<int>(columns * 256);
   half = asked < 2 && half_tile_pays(m, n - static_cast<int>(columns * 256), k, tiles_m * tiles_n / cus);
   return half ? static_cast<int>(columns * 256) : n;
 }
@@ -1805,9 +1808,20 @@ int sarek_hip_gemm16_tile_columns(int m, int n, int k) {
   return half ? columns : cut;
 }
 
+int sarek_hip_gemm16_half_columns(int m, int n, int k) {
+  const int tile = sarek_hip_gemm16_tile(m, n, k);
+  if ((tile != 256 && tile != 128) || n < 1) return 0;
+  const int columns = tiled_columns(m, n, tile);
+  if (columns < 1) return 0;
+  bool half = false;
+  if (tile == 128) return half_tile_pays(m, columns, k, 1) ? columns : 0;
+  const int cut = whole_round_columns(m, columns, k, half);
+  return half ? columns - cut : 0;
+}
+
 int sarek_hip_gemm16_k_splits(int m, int n, int k) {
   if (m >= 1 && n >= 1 && few_rows(m, n, k, false)) return gemm16_rows_k_splits(m, n, k);
-  return gemm16_tile_for(m, n, k) == 128 ? splitk_for(m, n, k) : 1;
+  return gemm16_tile_for(m, n, k) == 128 && sarek_hip_gemm16_half_columns(m, n, k) == 0 ? splitk_for(m, n, k) : 1;
 }
 
 int sarek_hip_gemm_bf16(const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k,

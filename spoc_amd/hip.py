@@ -148,6 +148,7 @@ SYMBOLS = {
     "sarek_hip_gemm16_tile": (_i, [_i, _i, _i]),
     "sarek_hip_gemm16_k_splits": (_i, [_i, _i, _i]),
     "sarek_hip_gemm16_tile_columns": (_i, [_i, _i, _i]),
+    "sarek_hip_gemm16_half_columns": (_i, [_i, _i, _i]),
     "sarek_hip_gemm_f16_bias_relu_rowsum": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "sarek_hip_cast_f32_to_bf16": (_i, [_vp, _vp, _i64, _vp]),
     "sarek_hip_cast_f32_to_f16": (_i, [_vp, _vp, _i64, _vp]),
@@ -756,6 +757,11 @@ def gemm16_tile_columns(m, n, k):
     """How many of the n columns that tile takes, with those that go to the 128 x 256 tile after it; the rest goes to the
     128 x 128 tile or, one column, to a kernel of its own."""
     return int(lib.sarek_hip_gemm16_tile_columns(m, n, k))
+
+
+def gemm16_half_columns(m, n, k):
+    """How many of the n columns go to the 128 x 256 tile."""
+    return int(lib.sarek_hip_gemm16_half_columns(m, n, k))
 
 
 def gemm16_k_splits(m, n, k):

@@ -63,6 +63,38 @@ def test_columns_past_whole_rounds_of_large_tiles(hip, knobs, m, n, k, columns):
         assert hip.gemm16_tile_columns(m, n, k) < n
 
 
+@pytest.mark.parametrize("m,n,k,columns", [
+    (4096, 2048, 8192, 2048), (1921, 4095, 1200, 4095), (1921, 4095, 1199, 0), (392, 12497, 4079, 12497), (3072, 3072, 3072, 0),
+    (2048, 2048, 2048, 0), (1921, 4099, 1200, 0), (2048, 12288, 4096, 4096), (2048, 11264, 1199, 0), (2048, 11264, 1200, 3072),
+    (2880, 13120, 1799, 0), (2880, 13120, 1800, 2368), (2048, 8448, 4096, 0), (1920, 4097, 2048, 4097), (16, 8192, 8192, 0), (100, 1, 64, 0)])
+def test_columns_of_the_half_tile(hip, knobs, m, n, k, columns):
+    """The 128 x 256 tile: whole products of at most one such tile to a CU, and the columns past whole rounds of large tiles, from a
+    K of 600 for each round and one more on; K is never cut beside it, and asking for pieces of K goes before it."""
+    assert hip.gemm16_half_columns(m, n, k) == columns
+    if columns:
+        assert hip.gemm16_k_splits(m, n, k) == 1
+    knobs("gemm16.split_k", 1)
+    assert hip.gemm16_half_columns(m, n, k) == columns
+    knobs("gemm16.split_k", 2)
+    assert hip.gemm16_half_columns(m, n, k) == 0
+    knobs("gemm16.split_k", 0)
+    knobs("gemm16.half", 1)
+    assert hip.gemm16_half_columns(m, n, k) == 0
+
+
+@pytest.mark.parametrize("m,n,k,columns", [(2048, 11264, 64, 3072), (2048, 8448, 64, 256), (2048, 12288, 256, 4096), (4160, 8000, 126, 320),
+                                           (3072, 3072, 64, 0), (256, 256, 4096, 256)])
+def test_half_tile_wherever_a_workgroup_per_cu_takes_the_columns(hip, knobs, m, n, k, columns):
+    """gemm16.half = 2: whatever K, and however few 128 x 128 tiles the columns would be; not against a cut that was asked for."""
+    knobs("gemm16.half", 2)
+    if hip.gemm16_tile(m, n, k) == 256:
+        assert hip.gemm16_half_columns(m, n, k) == columns
+        knobs("gemm16.cut", 1)
+        assert hip.gemm16_half_columns(m, n, k) == 0
+    else:
+        assert hip.gemm16_half_columns(m, n, k) == columns and hip.gemm16_k_splits(m, n, k) == 1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("value", [2, 34])
 def test_f32_direct_knob_of_no_variant_computes_the_same_product(hip, torch_cuda, knobs, value):
