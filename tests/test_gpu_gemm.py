@@ -386,13 +386,18 @@ def test_gemm16_both_tile_sizes(hip, oracle, torch_cuda, kind, m, n, k):
 
 
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
-@pytest.mark.parametrize("m,n,k,tile", [(128, 256, 64, 128), (1, 8, 64, 128), (127, 255, 65, 128), (129, 257, 72, 128), (300, 521, 199, 128),
-                                        (257, 264, 320, 128), (70, 1032, 384, 128), (640, 385, 449, 128), (200, 2, 32, 128),
-                                        (2048, 11264, 64, 0), (2047, 11009, 201, 0), (1921, 4099, 1200, 0), (1921, 4099, 1203, 0)])
-def test_gemm16_half_tile(hip, oracle, torch_cuda, kind, m, n, k, tile):
-    """The 128 x 256 tile for a whole product and for the columns past a round of large tiles, at the edges of its tile and of
-    its six-slab period, at any alignment of A and B: the bits of the other tiles (same products, same k order per element),
-    rows of the result against the oracle, the row sums against those of y, nothing stored outside."""
+@pytest.mark.parametrize("m,n,k,tile,half", [
+    (128, 256, 64, 128, 2), (1, 8, 64, 128, 2), (127, 255, 65, 128, 2), (129, 257, 72, 128, 2), (300, 521, 199, 128, 2),
+    (257, 264, 320, 128, 2), (70, 1032, 384, 128, 2), (640, 385, 449, 128, 2), (200, 2, 32, 128, 2),
+    (130, 264, 704, 128, 2), (128, 512, 768, 128, 2), (257, 264, 832, 128, 2), (100, 256, 1536, 128, 2), (130, 520, 1600, 128, 2),
+    (129, 257, 321, 128, 2), (130, 263, 641, 128, 2), (70, 300, 970, 128, 2),
+    (2048, 11264, 64, 0, 2), (2048, 11264, 192, 0, 2), (2047, 11009, 201, 0, 2),
+    (1921, 4095, 1200, 0, 0), (1921, 4095, 1203, 0, 0), (2048, 4096, 1216, 0, 0), (2048, 11264, 1216, 0, 0)])
+def test_gemm16_half_tile(hip, oracle, torch_cuda, kind, m, n, k, tile, half):
+    """The 128 x 256 tile for a whole product and for the columns past a round of large tiles, forced (half = 2) and by its own
+    rule (0), at the edges of its tile and of one and two turns of its rings (24 slabs of 32 where aligned, 10 where ragged), at
+    any alignment of A and B: the bits of the other tiles (same products, same k order per element), rows of the result
+    against the oracle, the row sums against those of y, nothing stored outside."""
     torch = torch_cuda
     a, b = normal16(oracle, (m, k), m + 5, kind), normal16(oracle, (k, n), n + 6, kind)
     bias = oracle.fill_uniform(n, seed=n + 2, lo=-0.1, hi=0.1)
@@ -408,14 +413,15 @@ def test_gemm16_half_tile(hip, oracle, torch_cuda, kind, m, n, k, tile):
                 return flat.view(x.shape).copy_(dev(torch, x))
             da, db = placed(a), placed(b)
             got = {}
-            for half in (2, 1) if k < 1200 else (0, 1):
-                hip.set_tunable("gemm16.half", half)
+            for arm in (half, 1):
+                hip.set_tunable("gemm16.half", arm)
+                assert (hip.gemm16_half_columns(m, n, k) > 0) == (arm != 1)
                 guard = torch.full((m * n + 64,), 7.0, device="cuda")
                 c = guard[32:32 + m * n].view(m, n)
                 (hip.gemm_bf16 if kind == "bf16" else hip.gemm_f16)(da, db, out=c)
                 assert bool((guard[:32] == 7).all()) and bool((guard[32 + m * n:] == 7).all())
-                got[half] = (c,) + (hip.gemm_f16_bias_relu_rowsum(da, db, dbias) if kind == "f16" else ())
-            new, old = got[2 if k < 1200 else 0], got[1]
+                got[arm] = (c,) + (hip.gemm_f16_bias_relu_rowsum(da, db, dbias) if kind == "f16" else ())
+            new, old = got[half], got[1]
             assert torch.equal(new[0], old[0])
             assert np.abs(new[0][dev(torch, rows)].cpu().numpy() - ref).max() / np.abs(ref).max() < 1e-4
             if kind == "f16":
@@ -1184,9 +1190,9 @@ def test_gemm_f32_direct(hip, torch_cuda, variant, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(70, 131, 200), (140, 264, 200), (129, 129, 77), (300, 257, 333), (66, 136, 131),
                                    (65, 260, 190)])
 def test_gemm_infinity_at_every_k(hip, torch_cuda, kind, tunables, m, n, k):
-    """An infinity in A at one k per row, every k of the last stages among them (the stage at the end of K is moved back
-    over the one before it: what the two share must count once and no product of it be formed twice), and rows of NaN-free
-    finite values beside them: the infinities, NaN and zeros of the float64 product, and its finite values within k 2^-24 of
+    """An infinity in A at one k per row, every k of the stages at both ends among them (what K is over whole stages is a stage of
+    its own at the start, whose transfers bring elements of the next one too: they must count once and no product of them
+    be formed twice), and rows of NaN-free finite values beside them: the infinities, NaN and zeros of the float64 product, and its finite values within k 2^-24 of
     the products' magnitudes.  B holds no zeros, so that an infinity is an infinity in every column."""
     torch = torch_cuda
     dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[kind]
@@ -1218,14 +1224,17 @@ def test_gemm_infinity_at_every_k(hip, torch_cuda, kind, tunables, m, n, k):
 
 @pytest.mark.parametrize("kind,tunables", [("bf16", {"gemm16.tile": 256}), ("f16", {"gemm16.tile": 128}),
                                            ("f16", {"gemm16.tile": 128, "gemm16.split_k": 2}),
+                                           ("bf16", {"gemm16.tile": 128, "gemm16.half": 2}),
+                                           ("f16", {"gemm16.tile": 128, "gemm16.half": 2}),
                                            ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 64}),
+                                           ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 64, "gemm_f32.cut": 2}),
                                            ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 128}),
                                            ("f32", {"gemm_f32.direct": 1, "gemm_f32.tile": 256})])
 @pytest.mark.parametrize("n,k", [(256, 65), (131, 71), (200, 72), (77, 95), (264, 96), (130, 97), (128, 127), (300, 129),
-                                 (257, 193), (96, 40), (96, 8)])
+                                 (257, 193), (96, 40), (96, 8), (270, 353)])
 def test_gemm_infinity_where_the_first_stage_ends(hip, torch_cuda, kind, tunables, n, k):
     """K over whole stages is a stage of its own at the start of K: an infinity at every k, one to a row, over first stages of
-    1 to 63, whole and part pieces of eight among them."""
+    1 to 63, whole and part pieces of eight among them, and past a whole turn of the deepest rings."""
     test_gemm_infinity_at_every_k(hip, torch_cuda, kind, tunables, k + 2, n, k)
 
 
