@@ -563,6 +563,9 @@ double ring_estimate(int m, int n, int k, int tile, int64_t cut, int splits) {
 // block: whether there is one for the pieces' sums.  Without (stream capture, hipStreamPerThread, the seventeenth stream)
 // nothing is cut, and a tile that was chosen for its cut is not the one to run whole: in a graph 247 x 1600 x 2884 took 48 us,
 // 26 as planned here, 1380 x 3328 x 2112 236 and 156.
+// Six workgroups of two row blocks share a CU (their registers), and what is over six to a CU waits for a place: from there to
+// eight the direct kernel's estimate is 5 to 24 % short (877 x 3886 x 436, 6.7 to a CU, 39.4 us, 64 x 64 tiles 34).  On 100
+// products round there, drawn apart, the chosen plan was 5.4 % above the fastest without the factor, 2.5 with it.
 // gemm_f32.direct: 1 = never, 18 / 14 / 24 = always, with (row_blocks, waves) these digits, any other value as 0;
 // gemm_f32.tile forces a tile, gemm_f32.split_k the pieces (1 = whole) of all 64 x 64 tiles or of a forced direct variant;
 // gemm_f32.cut: 1 = no tile is cut by the rule, n >= 2 = the tiles past whole rounds into n.  0 leaves the choice here.
@@ -579,7 +582,7 @@ Plan plan_for(int m, int n, int k, bool ring_ok, bool block) {
     return {direct / 10, direct % 10, 0, gemm_f32_direct_pieces(m, n, k, direct / 10, static_cast<int>(std::min<int64_t>(split, 64))), 0, 0};
   const int64_t cus = compute_units();
   Plan best{0, 0, 0, 1, 0, 0}, best_direct = best;
-  double best_us = 1e300, direct_us = 1e300;
+  double best_us = 1e300, direct_us = 1e300, uncrowded_us = 1e300;
   // (the clock probe of the measurement build is the ring kernels': a launch that it watches goes to them)
   const bool probed = kMeasureBuild && clock_probe(1) != nullptr;
   if (direct == 0 && direct_ok && !(probed && ring_ok) && (!ring_ok || (tile == 0 && split == 0 && gemm_f32_direct_pays(m, n, k, false))))
@@ -588,7 +591,9 @@ Plan plan_for(int m, int n, int k, bool ring_ok, bool block) {
       for (const int pieces : kPieces) {
         if (pieces > 1 && (!block || k / 16 / pieces < waves || tiles * pieces > 4 * cus)) break;
         const int splits = gemm_f32_direct_pieces(m, n, k, row_blocks, pieces);
-        const double us = 1.01 * gemm_f32_direct_estimate(m, n, k, row_blocks, waves, splits);
+        double us = 1.01 * gemm_f32_direct_estimate(m, n, k, row_blocks, waves, splits);
+        uncrowded_us = std::min(uncrowded_us, us);
+        if (row_blocks == 2 && tiles * splits > 6 * cus && tiles * splits <= 8 * cus) us *= 1.15;
         if (us < direct_us) direct_us = us, best_direct = {row_blocks, waves, 0, splits, 0, 0};
       }
     }
@@ -605,7 +610,7 @@ Plan plan_for(int m, int n, int k, bool ring_ok, bool block) {
       if (cut == tiles && direct_sums == 4) us /= 1.04;
       int chains = t == 256 ? 1 : t == 128 ? 2 : 4;
       if (t == 64 && (chains * pieces < direct_sums || (cut > 0 && tiles < 2 * cus))) chains = 8;
-      if (chains * pieces < direct_sums && (t == 64 || cut > 0 || us >= direct_us)) return;
+      if (chains * pieces < direct_sums && (t == 64 || cut > 0 || us >= uncrowded_us)) return;
       if (us < best_us) best_us = us, best = {0, 0, t, splits, static_cast<int>(cut), chains};
     };
     if (t == 64 && split >= 2) {
