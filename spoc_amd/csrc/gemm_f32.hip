@@ -537,13 +537,16 @@ int ring_pieces(int64_t cut, int k, int tile, int64_t splits) {
 // slab alone on its CU, and two on a CU share its matrix cores, so tiles count in turns of CUs; the larger ones take four and
 // sixteen times as long less the operand traffic they save.  A turn's start and stores are 6 us on the 256 x 256 tile, whose
 // launch has one workgroup to a CU (2816 x 4096 x 90 36.2 us on it, 31.0 on 128 x 128; counted as 3 us it was taken).  Tiles that
-// are cut come on top, in turns of their pieces, with the planes to write and to add.
+// are cut come on top, in turns of their pieces, with the planes to write and to add.  splits = 0: no less than that with any
+// number of pieces.
 double ring_estimate(int m, int n, int k, int tile, int64_t cut, int splits) {
   const int64_t tiles = tiles_of(m, n, tile), cus = compute_units();
   const double slabs = k / 32.0, c_mb = 4e-6 * m * n;
   const double slab = tile == 64 ? 0.458 : tile == 128 ? 1.807 : 7.38, each = tile == 64 ? 1.06 : tile == 128 ? 2.96 : 6.0;
   double us = 3.89 + static_cast<double>(ceil_div(tiles - cut, cus)) * (slabs * slab + each) + 0.141 * c_mb;
-  if (cut > 0)
+  if (cut > 0 && splits == 0)
+    us += static_cast<double>(cut) / static_cast<double>(cus) * slabs * slab + each + 3.44;
+  else if (cut > 0)
     us += static_cast<double>(ceil_div(cut * splits, cus)) * (slabs / splits * slab + each) + 3.44 +
           0.037 * 4e-6 * static_cast<double>(cut) * splits * tile * tile;
   return us;
@@ -624,7 +627,9 @@ Plan plan_for(int m, int n, int k, bool ring_ok, bool block) {
       consider(over ? over : std::min(tiles, cus), ring_pieces(over ? over : std::min(tiles, cus), k, t, cutting));
       continue;
     }
-    for (int pieces = 2; over > 0 && (t == 64 || over < tiles) && pieces <= 12 && k / pieces >= 96; ++pieces)
+    // (where no number of pieces can be ahead they are not gone through: 0.2 of the 0.6 us in which a small product is planned)
+    if (over == 0 || ring_estimate(m, n, k, t, over, 0) > 1.04 * best_us) continue;
+    for (int pieces = 2; (t == 64 || over < tiles) && pieces <= 12 && k / pieces >= 96; ++pieces)
       consider(over, ring_pieces(over, k, t, pieces));
   }
   return best.tile > 0 || best.row_blocks > 0 ? best : best_direct;
