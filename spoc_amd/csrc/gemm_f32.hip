@@ -628,7 +628,7 @@ Plan plan_for(int m, int n, int k, bool ring_ok, bool block) {
       continue;
     }
     // (where no number of pieces can be ahead they are not gone through: 0.2 of the 0.6 us in which a small product is planned)
-    if (over == 0 || ring_estimate(m, n, k, t, over, 0) > 1.04 * best_us) continue;
+    if (over == 0 || k / 2 < 96 || ring_estimate(m, n, k, t, over, 0) > 1.04 * best_us) continue;
     for (int pieces = 2; (t == 64 || over < tiles) && pieces <= 12 && k / pieces >= 96; ++pieces)
       consider(over, ring_pieces(over, k, t, pieces));
   }
