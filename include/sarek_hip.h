@@ -394,7 +394,10 @@ int sarek_hip_vector_set(sarek_hip_vector v, int64_t index, const void *elem);
 int sarek_hip_vector_read(sarek_hip_vector v, void *dst, int64_t first, int64_t count);
 int sarek_hip_vector_write(sarek_hip_vector v, const void *src, int64_t first, int64_t count);
 /* Transfer.set_auto, to_device (to the current device), to_cpu ?force, sync,
- * free_all_buffers, flush.                                                         */
+ * free_all_buffers, flush.  to_device of a vector of at most 3072 bytes is in the order
+ * of the device's default stream, as the launches are, and complete on return once the
+ * block's address has been asked for (vector_device_ptr waits); others are complete on
+ * return.                                                                          */
 int sarek_hip_transfer_set_auto(int enabled);
 int sarek_hip_transfer_to_device(sarek_hip_vector v);
 int sarek_hip_transfer_to_cpu(sarek_hip_vector v, int force);
