@@ -589,6 +589,142 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
   }
 }
 
+// Lanes l and l ^ W exchange: the one whose bit W is clear gets the two lanes' sum of a, the other their sum of b.
+template <int W>
+__device__ __forceinline__ float swap_and_add(float a, float b) {
+  const auto both = W == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
+                            : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(both[0]) + __uint_as_float(both[1]);
+}
+
+// The 256 x 256 tile of a C that the memory-side cache cannot hold (rows_pay), from accumulators that had B's fragments
+// as the first MFMA operand: register r of lane l holds row l%16, column 4*(l/16) + r of its 16 x 16 tile.  Whole rows of the
+// tile, 1 KiB each, are put together in LDS and stored a row to an instruction: the lines that lie within it past the caches
+// (non-temporal), the pieces of a line at its ends, whose other part belongs to the tile beside this one, through the L2.
+// What bounds it is memory, 64 MiB a round of tiles at 5 to 8 TB/s.  Stored through the caches, C pushes the operands out of them,
+// and the next tile's first transfers wait behind it: a tile of K = 1024 took 37 us, 26 of them its K loop, and takes 31, the K
+// loop 22.  256 KiB of C from one CU, us: 2.0 in whole rows, 3.9 with 16 lanes to a row and 4 bytes a lane (what A's fragments
+// first leave), 7.7 with 16 rows to an instruction; non-temporal stores of parts of lines run at 1.3 TB/s.
+// Columns past N: element by element.  place0 (32 KiB), place1, place2 (16 KiB each): of the four waves that share these rows.
+template <int Epi>
+__device__ __forceinline__ void epilogue16_rows(f32x4_t (&acc)[8][4], float *__restrict__ C, const float *__restrict__ bias,
+                                                float *__restrict__ rowsum, float *__restrict__ rs_plane, int M, int N, int ld,
+                                                int m0, int n0, int wm, int wn, int lane, float *scratch, bool add_last,
+                                                char *place0, char *place1, char *place2) {
+  constexpr uint32_t kOutOfRange = 0x80000000u;
+  constexpr int kNonTemporal = 2, TROWS = 256;
+  const int l16 = lane & 15, g = lane >> 4;
+  const int row0 = m0 + wm * 128, col0 = n0 + wn * 64, lane_col = col0 + 4 * g;
+  if (add_last) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float last = scratch[wm * 128 + i * 16 + l16];
+      const bool only = scratch[TROWS + wm * 128 + i * 16 + l16] != 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (lane_col + j * 16 + r == N - 1) acc[i][j][r] = (only ? 0.f : acc[i][j][r]) + last;
+    }
+  }
+  const bool whole = n0 + BN <= N;
+  if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x4_t b;
+      if (whole) {
+        b = *reinterpret_cast<const f32x4_u *>(bias + lane_col + j * 16);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) b[r] = lane_col + j * 16 + r < N ? bias[lane_col + j * 16 + r] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float v = acc[i][j][r] + b[r];
+          acc[i][j][r] = v > 0.f ? v : 0.f;
+        }
+    }
+  }
+  float rs[8];
+  __syncthreads();   // every wave has left the K loop (and read its last_products): the LDS ring is free
+  if (whole) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      // Turn t: row tiles 2t and 2t + 1 of both halves, 64 rows, in two places by turns: a wave that writes the next but one has
+      // passed the barrier that the readers of this one met after it.  Piece c of row r lies at place c ^ (r % 16): neither side
+      // meets a bank twice.
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        char *const to = t % 2 == 0 ? place0 + e * 16384 : e == 0 ? place1 : place2;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<f32x4_t *>(to + l16 * 1024 + (((wn * 16 + 4 * j + g) ^ l16) << 4)) = acc[2 * t + e][j];
+        if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
+          float part[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            part[j] = (acc[2 * t + e][j][0] + acc[2 * t + e][j][1]) + (acc[2 * t + e][j][2] + acc[2 * t + e][j][3]);
+          rs[2 * t + e] = (part[0] + part[1]) + (part[2] + part[3]);
+        }
+      }
+      wait_lds();
+      barrier_no_fence();
+      // rows 8 (wn % 2) .. + 7 of row tile 2t + wn / 2
+      const char *const from = (t % 2 == 0 ? place0 + (wn >> 1) * 16384 : (wn >> 1) == 0 ? place1 : place2) + (wn & 1) * 8192;
+      const int row1 = row0 + (2 * t + (wn >> 1)) * 16 + (wn & 1) * 8;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(from + q * 1024 + ((lane ^ ((wn & 1) * 8 + q)) << 4));
+        float *const row = C + static_cast<int64_t>(row1 + q) * ld + n0;
+        const int skew = static_cast<int>(reinterpret_cast<uintptr_t>(row)) & 127, off = lane * 16;
+        const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(row, row1 + q < M ? BN * 4u : 0u);
+        const bool inside = off >= ((128 - skew) & 127) && off + 16 <= BN * 4 - skew;
+        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, inside ? off : static_cast<int>(kOutOfRange), 0, kNonTemporal);
+        if (skew) __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, inside ? static_cast<int>(kOutOfRange) : off, 0, 0);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float *const row = C + static_cast<int64_t>(row0 + i * 16 + l16) * ld;
+      const bool row_ok = row0 + i * 16 + l16 < M;
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int col = lane_col + j * 16 + r;
+          if (row_ok && col < N) row[col] = acc[i][j][r];
+          sum += col < N ? acc[i][j][r] : 0.f;
+        }
+      rs[i] = sum;
+    }
+  }
+  if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
+    // lane groups g and g ^ 2, then g and g ^ 1, swap halves of their sums and add: a lane keeps row tiles
+    // q + 2 (g & 1) + 4 (g >> 1), q < 2
+#pragma unroll
+    for (int q = 0; q < 4; ++q) rs[q] = swap_and_add<32>(rs[q], rs[q + 4]);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) rs[q] = swap_and_add<16>(rs[q], rs[q + 2]);
+    wait_lds();
+    barrier_no_fence();   // the rows have been read
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      scratch[wn * TROWS + wm * 128 + (q + (g & 1) * 2 + (g >> 1) * 4) * 16 + l16] = rs[q];
+    wait_lds();
+    barrier_no_fence();
+    const int t = threadIdx.x;
+    if (t < TROWS && m0 + t < M) {
+      const float total = (scratch[t] + scratch[TROWS + t]) + (scratch[2 * TROWS + t] + scratch[3 * TROWS + t]);
+      if (rs_plane) rs_plane[m0 + t] = total;
+      else atomicAdd(rowsum + m0 + t, total);
+    }
+  }
+}
+
 // ---- direct-to-LDS kernel on v_mfma_f32_16x16x32 ---------------------------------------
 // The same tile, rings and transfers as gemm16_dma_kernel<.., 64, 32, 2, 4, 2> (256 x 256 per workgroup, 8 waves
 // of 128 x 64, A in 2 stages of K = 64, B in 4 slabs of K = 32, one barrier per B slab), but the products go
@@ -613,7 +749,9 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
 // fused 6865 x 576 x 1472 25.1, 25.7, 24.5; ragged 256 x 24704 x 4535 62.5, 63.5, 62.0; fused 2056 x 2060 x 2547 42.2, 42.1, 41.5.
 // The same tile with a ring of 80 KiB, two workgroups to a CU, waited for its transfers: 8192^3 738 us on the large tile, 820
 // on it; 2048 x 50257 x 1024 260, 345.
-template <bool Bf16, int Epi, int Ablate = 0, bool Ragged = false, bool HalfBarriers = false, int WM = 2>
+//
+// Rows: the tile is stored by epilogue16_rows.
+template <bool Bf16, int Epi, int Ablate = 0, bool Ragged = false, bool HalfBarriers = false, int WM = 2, bool Rows = false>
 __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                          float *__restrict__ C, const float *__restrict__ bias,
                                                          float *__restrict__ rowsum, int M, int N, int K, int tiles_m,
@@ -636,7 +774,13 @@ __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__
   constexpr int P = lcm_int(NB, RA * NA);
   static_assert(P % 2 == 0, "the B fragment buffers alternate by slab parity");
   static_assert((NB - 1) * DB + NA * DA < 64, "vmcnt range");
+  static_assert(NB - BEHIND <= RA * NA, "the prologue's events start with B slab 0");
 
+  // Rows: the first workgroup of a CU starts up to 9 us late, by its place in the XCD, so that the CUs do not all store at the
+  // same time in every round.  Together, then apart, us: 8192 x 8192 x 256 83.2, 69.0; x 1024 135, 125; x 2048 206, 201;
+  // 8192 x 12288 x 256 99.3, 94.4; x 1024 189, 179; 2048 x 49152 x 1024 209, 212.
+  if (Rows && blockIdx.x < NUM_XCD * 32)
+    for (int i = 0; i < static_cast<int>(blockIdx.x) / NUM_XCD * 9; ++i) __builtin_amdgcn_s_sleep(1);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -764,7 +908,8 @@ __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__
     [&]<int... Ts>(std::integer_sequence<int, Ts...>) {
       (([&] {
          constexpr int i = (First + Ts) / 4, j = i % 2 ? 3 - (First + Ts) % 4 : (First + Ts) % 4;
-         acc[i][j] = mfma16<Bf16>(af[i / 4][i % 4], bf[j], acc[i][j]);
+         // (Rows: the tile is wanted with four columns to a lane)
+         acc[i][j] = Rows ? mfma16<Bf16>(bf[j], af[i / 4][i % 4], acc[i][j]) : mfma16<Bf16>(af[i / 4][i % 4], bf[j], acc[i][j]);
        }()),
        ...);
     }(std::make_integer_sequence<int, Count>{});
@@ -867,8 +1012,14 @@ __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__
   float *scratch = reinterpret_cast<float *>(lds_ring<10, A_BYTES_S>);
   const bool add_last = Ragged && (N & 1) != 0 && n0 + BN >= N;
   if (add_last) last_products<Bf16, TBM>(A, B, M, N, K, ld, m0, 0, scratch);
-  epilogue16<Epi, 8, 4, Ragged, WM>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * (WM == 1 ? 2 : 1) * M : nullptr,
-                                    M, N, ld, m0, wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
+  float *const rs_plane = rs_planes ? rs_planes + static_cast<int64_t>(tn) * (WM == 1 ? 2 : 1) * M : nullptr;
+  if constexpr (Rows) {
+    epilogue16_rows<Epi>(acc, C, bias, rowsum, rs_plane, M, N, ld, m0, n0, wm, wn, lane, scratch, add_last,
+                         wm ? lds_ring<11, A_BYTES_S> : lds_ring<10, A_BYTES_S>, wm ? lds_ring<22, B_BYTES_S> : lds_ring<20, B_BYTES_S>,
+                         wm ? lds_ring<23, B_BYTES_S> : lds_ring<21, B_BYTES_S>);
+  } else {
+    epilogue16<Epi, 8, 4, Ragged, WM>(acc, C, bias, rowsum, rs_plane, M, N, ld, m0, wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
+  }
   if (kMeasureBuild && probe && tid == 0) {
     probe[2 * blockIdx.x] = static_cast<unsigned long long>(clock64() - probe_c0);
     probe[2 * blockIdx.x + 1] = static_cast<unsigned long long>(wall_clock64() - probe_t0);
@@ -1438,6 +1589,19 @@ inline int whole_round_columns(int m, int n, int k, bool &half) {
   return half ? static_cast<int>(columns * 256) : n;
 }
 
+// Whether the 256 x 256 tiles store C by rows, past the caches (epilogue16_rows): a C of 200 MiB or more, of the 256 MiB that the
+// memory-side cache holds, up to K = 4096 (from there on a tile's stores are lost in its K loop, and the power limit decides).
+// Measured on three products taken in turn, us, through the caches and by rows: 8192 x 8192 x 256 93 -> 66, x 1024 155 -> 126,
+// x 2048 234 -> 208, x 4096 393 -> 392; 8192 x 8191 x 1000 179 -> 162; 6223 x 29760 x 576 293 -> 243; 2048 x 50257 x 1024
+// 256 -> 251 (B, new to the caches, waits behind the stores); fused 8192 x 8192 x 1000 172 -> 145; 8192 x 6143 x 1024 (191 MiB)
+// 123 -> 121, one such product over and over, whose C the cache then holds, 106 -> 120; of 224 MiB 117 -> 121; 8192 x 6144 x 1024
+// 105 -> 97 and 96 -> 97.  Half of that, 4096 x 8192 x 256, three in turn 53 -> 47, two 35 -> 49.
+// gemm16.by_rows: 0 = this rule, 1 = never, 2 = always.
+inline bool rows_pay(int m, int n, int k) {
+  const int64_t asked = tunable("gemm16.by_rows", 0);
+  return asked == 2 || (asked == 0 && k <= 4096 && static_cast<int64_t>(m) * n * 4 >= int64_t{200} << 20);
+}
+
 // The columns that are left to the tiles when gemm16_last_column_kernel takes the last one: n - 1 for N = 1 and for whole
 // tile columns and one column more that would add a round of workgroups (4096 x 4097 x 4096: 139 us against 184).
 inline int tiled_columns(int m, int n, int tile) {
@@ -1736,6 +1900,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
     }
   } else if (nm > 0) {
     const int tiles_m = (m + BM - 1) / BM, tiles_n = (cut + BN - 1) / BN;
+    const bool by_rows = rows_pay(m, n, k);
     unsigned long long *probe = clock_probe(static_cast<int64_t>(tiles_m) * tiles_n);
 #ifdef SAREK_HIP_MEASURE
     if (Epi == EPI_STORE && !ragged && tunable("gemm16.waves", 8) == 4) {
@@ -1746,7 +1911,13 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
                          bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
     } else
 #endif
-    if (ragged)
+    if (by_rows && ragged)
+      hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, true, false, 2, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c,
+                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
+    else if (by_rows)
+      hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false, false, 2, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c,
+                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
+    else if (ragged)
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c, bias,
                          rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
     else

@@ -466,6 +466,45 @@ def test_gemm16_half_tile_row_sums(hip, torch_cuda, m, n, k):
 
 
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
+@pytest.mark.parametrize("m,n,k,rows", [(256, 256, 64, 2), (1, 8, 64, 2), (255, 257, 65, 2), (257, 511, 72, 2), (300, 521, 199, 2), (512, 768, 448, 2),
+                                        (70, 1032, 384, 2), (513, 515, 1000, 2), (200, 2, 32, 2), (129, 1025, 130, 2), (8192, 6401, 64, 0),
+                                        (6403, 8200, 200, 0)])
+def test_gemm16_stored_by_rows(hip, torch_cuda, kind, m, n, k, rows):
+    """The 256 x 256 tile that stores whole rows past the caches, forced (rows = 2) and by its own rule (0), with C, A and B at
+    several alignments (rows of C that start anywhere in a line, the last tile column cut off): the bits of the tile that stores
+    through the caches, nothing stored outside, the row sums those of y to 1e-5 of the sum of its magnitudes (float32 sums of 256
+    values and a double sum of those: 8 roundings of 2^-24)."""
+    torch = torch_cuda
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(m + n + k)
+    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    bias = torch.rand(n, device="cuda", generator=gen) * 0.2 - 0.1
+    flat = [torch.empty(size + 1, device="cuda").normal_(0, 0.02, generator=gen).to(dt) for size in (m * k, k * n)]
+    try:
+        if rows:
+            hip.set_tunable("gemm16.tile", 256)
+        for shift, c_shift in ((0, 32), (1, 33), (1, 47)) if k >= 64 else ((0, 32),):
+            a, b = flat[0][shift:shift + m * k].view(m, k), flat[1][shift:shift + k * n].view(k, n)
+            got = {}
+            for arm in (rows, 1):
+                hip.set_tunable("gemm16.by_rows", arm)
+                assert hip.gemm16_tile(m, n, k) == 256
+                guard = torch.full((m * n + 96,), 7.0, device="cuda")
+                c = guard[c_shift:c_shift + m * n].view(m, n)
+                (hip.gemm_bf16 if kind == "bf16" else hip.gemm_f16)(a, b, out=c)
+                assert bool((guard[:c_shift] == 7).all()) and bool((guard[c_shift + m * n:] == 7).all())
+                got[arm] = (c,) + (hip.gemm_f16_bias_relu_rowsum(a, b, bias) if kind == "f16" else ())
+            new, old = got[rows], got[1]
+            assert torch.equal(new[0], old[0])
+            if kind == "f16":
+                assert torch.equal(new[1], old[1])
+                assert bool(((new[2].double() - new[1].double().sum(1)).abs() <= 1e-5 * new[1].double().sum(1) + 1e-30).all())
+    finally:
+        hip.set_tunable("gemm16.by_rows", 0)
+        hip.set_tunable("gemm16.tile", 0)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(2048, 8448, 64), (2047, 8195, 72), (1921, 8703, 131), (2048, 10240, 65),
                                    (8192, 2050, 70), (2300, 7425, 200)])
 def test_gemm16_columns_past_whole_rounds_of_large_tiles(hip, oracle, torch_cuda, kind, m, n, k):
