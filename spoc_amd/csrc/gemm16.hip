@@ -605,7 +605,7 @@ __device__ __forceinline__ float swap_and_add(float a, float b) {
 // and the next tile's first transfers wait behind it: a tile of K = 1024 took 37 us, 26 of them its K loop, and takes 31, the K
 // loop 22.  256 KiB of C from one CU, us: 2.0 in whole rows, 3.9 with 16 lanes to a row and 4 bytes a lane (what A's fragments
 // first leave), 7.7 with 16 rows to an instruction; non-temporal stores of parts of lines run at 1.3 TB/s.
-// Columns past N: element by element.  place0 (32 KiB), place1, place2 (16 KiB each): of the four waves that share these rows.
+// place0 (32 KiB), place1, place2 (16 KiB each): of the four waves that share these rows.
 template <int Epi>
 __device__ __forceinline__ void epilogue16_rows(f32x4_t (&acc)[8][4], float *__restrict__ C, const float *__restrict__ bias,
                                                 float *__restrict__ rowsum, float *__restrict__ rs_plane, int M, int N, int ld,
@@ -647,59 +647,53 @@ __device__ __forceinline__ void epilogue16_rows(f32x4_t (&acc)[8][4], float *__r
         }
     }
   }
+  const int bytes = min(N - n0, BN) * 4;   // of a row that exist
   float rs[8];
   __syncthreads();   // every wave has left the K loop (and read its last_products): the LDS ring is free
-  if (whole) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      // Turn t: row tiles 2t and 2t + 1 of both halves, 64 rows, in two places by turns: a wave that writes the next but one has
-      // passed the barrier that the readers of this one met after it.  Piece c of row r lies at place c ^ (r % 16): neither side
-      // meets a bank twice.
+  for (int t = 0; t < 4; ++t) {
+    // Turn t: row tiles 2t and 2t + 1 of both halves, 64 rows, in two places by turns: a wave that writes the next but one has
+    // passed the barrier that the readers of this one met after it.  Piece c of row r lies at place c ^ (r % 16): neither side
+    // meets a bank twice.
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        char *const to = t % 2 == 0 ? place0 + e * 16384 : e == 0 ? place1 : place2;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          *reinterpret_cast<f32x4_t *>(to + l16 * 1024 + (((wn * 16 + 4 * j + g) ^ l16) << 4)) = acc[2 * t + e][j];
-        if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
-          float part[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            part[j] = (acc[2 * t + e][j][0] + acc[2 * t + e][j][1]) + (acc[2 * t + e][j][2] + acc[2 * t + e][j][3]);
-          rs[2 * t + e] = (part[0] + part[1]) + (part[2] + part[3]);
-        }
-      }
-      wait_lds();
-      barrier_no_fence();
-      // rows 8 (wn % 2) .. + 7 of row tile 2t + wn / 2
-      const char *const from = (t % 2 == 0 ? place0 + (wn >> 1) * 16384 : (wn >> 1) == 0 ? place1 : place2) + (wn & 1) * 8192;
-      const int row1 = row0 + (2 * t + (wn >> 1)) * 16 + (wn & 1) * 8;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(from + q * 1024 + ((lane ^ ((wn & 1) * 8 + q)) << 4));
-        float *const row = C + static_cast<int64_t>(row1 + q) * ld + n0;
-        const int skew = static_cast<int>(reinterpret_cast<uintptr_t>(row)) & 127, off = lane * 16;
-        const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(row, row1 + q < M ? BN * 4u : 0u);
-        const bool inside = off >= ((128 - skew) & 127) && off + 16 <= BN * 4 - skew;
-        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, inside ? off : static_cast<int>(kOutOfRange), 0, kNonTemporal);
-        if (skew) __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, inside ? static_cast<int>(kOutOfRange) : off, 0, 0);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float *const row = C + static_cast<int64_t>(row0 + i * 16 + l16) * ld;
-      const bool row_ok = row0 + i * 16 + l16 < M;
-      float sum = 0.f;
+    for (int e = 0; e < 2; ++e) {
+      char *const to = t % 2 == 0 ? place0 + e * 16384 : e == 0 ? place1 : place2;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<f32x4_t *>(to + l16 * 1024 + (((wn * 16 + 4 * j + g) ^ l16) << 4)) = acc[2 * t + e][j];
+      if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
+        float part[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int col = lane_col + j * 16 + r;
-          if (row_ok && col < N) row[col] = acc[i][j][r];
-          sum += col < N ? acc[i][j][r] : 0.f;
+        for (int j = 0; j < 4; ++j) {
+          f32x4_t y = acc[2 * t + e][j];
+          if (!whole)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y[r] = lane_col + j * 16 + r < N ? y[r] : 0.f;
+          part[j] = (y[0] + y[1]) + (y[2] + y[3]);
         }
-      rs[i] = sum;
+        rs[2 * t + e] = (part[0] + part[1]) + (part[2] + part[3]);
+      }
+    }
+    wait_lds();
+    barrier_no_fence();
+    // rows 8 (wn % 2) .. + 7 of row tile 2t + wn / 2
+    const char *const from = (t % 2 == 0 ? place0 + (wn >> 1) * 16384 : (wn >> 1) == 0 ? place1 : place2) + (wn & 1) * 8192;
+    const int row1 = row0 + (2 * t + (wn >> 1)) * 16 + (wn & 1) * 8;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const u32x4 v = *reinterpret_cast<const u32x4 *>(from + q * 1024 + ((lane ^ ((wn & 1) * 8 + q)) << 4));
+      float *const row = C + static_cast<int64_t>(row1 + q) * ld + n0;
+      const int skew = static_cast<int>(reinterpret_cast<uintptr_t>(row)) & 127, off = lane * 16;
+      const bool row_ok = row1 + q < M;
+      const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(row, row_ok ? bytes & ~15 : 0u);
+      const bool inside = off >= ((128 - skew) & 127) && off + 16 <= bytes - ((skew + bytes) & 127);
+      __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, inside ? off : static_cast<int>(kOutOfRange), 0, kNonTemporal);
+      if (skew || !whole) __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, inside ? static_cast<int>(kOutOfRange) : off, 0, 0);
+      if ((bytes & 15) != 0 && row_ok && off == (bytes & ~15)) {   // the last one to three columns
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+          if (off + 4 * d < bytes) row[lane * 4 + d] = __uint_as_float(v[d]);
+      }
     }
   }
   if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
@@ -756,7 +750,7 @@ __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__
                                                          float *__restrict__ C, const float *__restrict__ bias,
                                                          float *__restrict__ rowsum, int M, int N, int K, int tiles_m,
                                                          int tiles_n, int xcd_remap, unsigned long long *probe, int ld,
-                                                         float *__restrict__ rs_planes) {
+                                                         float *__restrict__ rs_planes, int apart = 0) {
   static_assert(WM == 2 || (WM == 1 && !HalfBarriers), "the whole tile or its upper half");
   // HalfBarriers: one barrier per A stage (K = 64) instead of one per B slab (K = 32).  A transfer may then only
   // overwrite the slab before the previous one (the waves are a whole stage apart at most), so the top of slab j
@@ -776,11 +770,9 @@ __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__
   static_assert((NB - 1) * DB + NA * DA < 64, "vmcnt range");
   static_assert(NB - BEHIND <= RA * NA, "the prologue's events start with B slab 0");
 
-  // Rows: the first workgroup of a CU starts up to 9 us late, by its place in the XCD, so that the CUs do not all store at the
-  // same time in every round.  Together, then apart, us: 8192 x 8192 x 256 83.2, 69.0; x 1024 135, 125; x 2048 206, 201;
-  // 8192 x 12288 x 256 99.3, 94.4; x 1024 189, 179; 2048 x 49152 x 1024 209, 212.
+  // The first workgroup of a CU starts `apart` times 64 cycles late for each place before it in the XCD (rows_apart)
   if (Rows && blockIdx.x < NUM_XCD * 32)
-    for (int i = 0; i < static_cast<int>(blockIdx.x) / NUM_XCD * 9; ++i) __builtin_amdgcn_s_sleep(1);
+    for (int i = 0; i < static_cast<int>(blockIdx.x) / NUM_XCD * apart; ++i) __builtin_amdgcn_s_sleep(1);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1591,16 +1583,26 @@ inline int whole_round_columns(int m, int n, int k, bool &half) {
 
 // Whether the 256 x 256 tiles store C by rows, past the caches (epilogue16_rows): a C of 200 MiB or more, of the 256 MiB that the
 // memory-side cache holds, up to K = 4096 (from there on a tile's stores are lost in its K loop, and the power limit decides).
-// Measured on three products taken in turn, us, through the caches and by rows: 8192 x 8192 x 256 93 -> 66, x 1024 155 -> 126,
-// x 2048 234 -> 208, x 4096 393 -> 392; 8192 x 8191 x 1000 179 -> 162; 6223 x 29760 x 576 293 -> 243; 2048 x 50257 x 1024
-// 256 -> 251 (B, new to the caches, waits behind the stores); fused 8192 x 8192 x 1000 172 -> 145; 8192 x 6143 x 1024 (191 MiB)
-// 123 -> 121, one such product over and over, whose C the cache then holds, 106 -> 120; of 224 MiB 117 -> 121; 8192 x 6144 x 1024
-// 105 -> 97 and 96 -> 97.  Half of that, 4096 x 8192 x 256, three in turn 53 -> 47, two 35 -> 49.
+// Measured on three products taken in turn, us, through the caches and by rows: 8192 x 8192 x 400 120 -> 89, x 1024 161 -> 136,
+// x 2048 240 -> 223, x 4096 393 -> 392; 8192 x 8191 x 1024 172 -> 143; 4096 x 14001 x 1024 156 -> 132; 8192 x 12001 x 2048 384 ->
+// 375; fused 8192 x 8192 x 1000 172 -> 145.  One product over and over, whose C the cache then holds in part: 8192 x 8192 x 1024
+// 132 -> 129, x 7168 117 -> 121, x 6143 (191 MiB) 106 -> 120.  Half of that, 4096 x 8192 x 256, three in turn 53 -> 47, two 35 -> 49.
+// A B of more than 60 MiB comes from memory while C goes there: 2048 x 50257 x 1024 268 -> 258, x 2048 413 -> 405, but with rows
+// of C of whole lines, which the caches take well enough, 2048 x 49152 x 1024 212 -> 218, x 2048 347 -> 353, 4096 x 28000 x 2048
+// 399 -> 406: those stay.
 // gemm16.by_rows: 0 = this rule, 1 = never, 2 = always.
+inline bool large_b(int n, int k) { return static_cast<int64_t>(n) * k * 2 > int64_t{60} << 20; }
 inline bool rows_pay(int m, int n, int k) {
   const int64_t asked = tunable("gemm16.by_rows", 0);
-  return asked == 2 || (asked == 0 && k <= 4096 && static_cast<int64_t>(m) * n * 4 >= int64_t{200} << 20);
+  if (asked != 0) return asked == 2;
+  return k <= 4096 && static_cast<int64_t>(m) * n * 4 >= int64_t{200} << 20 && !(large_b(n, k) && n % 32 == 0);
 }
+
+// How far apart the CUs of an XCD start on tiles that are stored by rows, times 64 cycles: by 13, 12 us from the first to the
+// last, so that they do not all store in the same part of every round.  Us, together and 14 apart: 8192 x 8191 x 400 97 -> 91,
+// x 1024 150 -> 141, x 2048 251 -> 251; 4096 x 14001 x 400 97 -> 79; 2048 x 28000 x 1024 127 -> 118.  Where B comes from memory the
+// workgroups that share a panel of it had better ask for it together: 2048 x 50257 x 1024 258 -> 275, 2048 x 49152 x 2048 353 -> 382.
+inline int rows_apart(int n, int k) { return large_b(n, k) ? 0 : 13; }
 
 // The columns that are left to the tiles when gemm16_last_column_kernel takes the last one: n - 1 for N = 1 and for whole
 // tile columns and one column more that would add a round of workgroups (4096 x 4097 x 4096: 139 us against 184).
@@ -1901,6 +1903,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   } else if (nm > 0) {
     const int tiles_m = (m + BM - 1) / BM, tiles_n = (cut + BN - 1) / BN;
     const bool by_rows = rows_pay(m, n, k);
+    const int apart = rows_apart(n, k);
     unsigned long long *probe = clock_probe(static_cast<int64_t>(tiles_m) * tiles_n);
 #ifdef SAREK_HIP_MEASURE
     if (Epi == EPI_STORE && !ragged && tunable("gemm16.waves", 8) == 4) {
@@ -1913,10 +1916,10 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
 #endif
     if (by_rows && ragged)
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, true, false, 2, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c,
-                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
+                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes, apart);
     else if (by_rows)
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false, false, 2, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c,
-                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
+                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes, apart);
     else if (ragged)
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c, bias,
                          rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
