@@ -495,10 +495,16 @@ __device__ __forceinline__ void last_products(const uint16_t *__restrict__ A, co
 // rowsum_fold_kernel: the same bits on every run), else to rowsum[r] by atomicAdd.  The 128 x 256 tile has two, for its halves
 // of 128 columns: as many float32 additions in front of the fold's double as on the 128 x 128 tile, whose products it takes.  add_last: the tile rows' last_products
 // lie in `scratch` and belong to column N - 1.
+// A row's share of a tile, where fold_rows finds it.
+__device__ __forceinline__ void store_share(float *plane, int at, float share) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(share), make_rsrc(plane, 0x7FFFFFFFu), at * 4, 0, kDeviceScope);
+}
+
 template <int Epi, int TI, int WNW, bool Ragged, int WMW = 2>   // WMW, WNW: waves along M, N
 __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restrict__ C, const float *__restrict__ bias,
                                            float *__restrict__ rowsum, float *__restrict__ rs_plane, int M, int N, int ld,
-                                           int m0, int wm, int wn, int col0, int l16, int g, float *scratch, bool add_last) {
+                                           int m0, int wm, int wn, int col0, int l16, int g, float *scratch, bool add_last,
+                                           const RowFold &fold, int tile_row, int tiles_n) {
   constexpr int WROWS = 16 * TI, TROWS = WMW * WROWS, NV = 4 * TI, E = NV / 16;
   static_assert(TI == 8 || TI == 4, "wave tiles of 128 or 64 rows");
   static_assert(WNW == 4 || WNW == 2, "four or two waves along N");
@@ -573,7 +579,7 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
       const int t = threadIdx.x & 127, half = threadIdx.x >> 7;
       if (m0 + t < M && col0 - wn * 64 + half * 128 < N) {
         const float total = scratch[2 * half * TROWS + t] + scratch[(2 * half + 1) * TROWS + t];
-        if (rs_plane) rs_plane[static_cast<int64_t>(half) * M + m0 + t] = total;
+        if (rs_plane) store_share(rs_plane, half * M + m0 + t, total);
         else atomicAdd(rowsum + m0 + t, total);
       }
     } else {
@@ -582,10 +588,11 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
         float total;
         if constexpr (WNW == 4) total = (scratch[t] + scratch[TROWS + t]) + (scratch[2 * TROWS + t] + scratch[3 * TROWS + t]);
         else total = scratch[t] + scratch[TROWS + t];
-        if (rs_plane) rs_plane[m0 + t] = total;
+        if (rs_plane) store_share(rs_plane, m0 + t, total);
         else atomicAdd(rowsum + m0 + t, total);
       }
     }
+    if (fold.tickets) fold_rows<64 * WMW * WNW, TROWS>(fold, M, m0, rowsum, tile_row, tiles_n, scratch);
   }
 }
 
@@ -610,7 +617,8 @@ template <int Epi>
 __device__ __forceinline__ void epilogue16_rows(f32x4_t (&acc)[8][4], float *__restrict__ C, const float *__restrict__ bias,
                                                 float *__restrict__ rowsum, float *__restrict__ rs_plane, int M, int N, int ld,
                                                 int m0, int n0, int wm, int wn, int lane, float *scratch, bool add_last,
-                                                char *place0, char *place1, char *place2) {
+                                                char *place0, char *place1, char *place2, const RowFold &fold, int tile_row,
+                                                int tiles_n) {
   constexpr uint32_t kOutOfRange = 0x80000000u;
   constexpr int kNonTemporal = 2, TROWS = 256;
   const int l16 = lane & 15, g = lane >> 4;
@@ -713,9 +721,10 @@ __device__ __forceinline__ void epilogue16_rows(f32x4_t (&acc)[8][4], float *__r
     const int t = threadIdx.x;
     if (t < TROWS && m0 + t < M) {
       const float total = (scratch[t] + scratch[TROWS + t]) + (scratch[2 * TROWS + t] + scratch[3 * TROWS + t]);
-      if (rs_plane) rs_plane[m0 + t] = total;
+      if (rs_plane) store_share(rs_plane, m0 + t, total);
       else atomicAdd(rowsum + m0 + t, total);
     }
+    if (fold.tickets) fold_rows<512, TROWS>(fold, M, m0, rowsum, tile_row, tiles_n, scratch);
   }
 }
 
@@ -750,7 +759,7 @@ __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__
                                                          float *__restrict__ C, const float *__restrict__ bias,
                                                          float *__restrict__ rowsum, int M, int N, int K, int tiles_m,
                                                          int tiles_n, int xcd_remap, unsigned long long *probe, int ld,
-                                                         float *__restrict__ rs_planes, int apart = 0) {
+                                                         float *__restrict__ rs_planes, RowFold fold = {}, int apart = 0) {
   static_assert(WM == 2 || (WM == 1 && !HalfBarriers), "the whole tile or its upper half");
   // HalfBarriers: one barrier per A stage (K = 64) instead of one per B slab (K = 32).  A transfer may then only
   // overwrite the slab before the previous one (the waves are a whole stage apart at most), so the top of slab j
@@ -1008,9 +1017,10 @@ __global__ __launch_bounds__(256 * WM) void gemm16_m16_kernel(const uint16_t *__
   if constexpr (Rows) {
     epilogue16_rows<Epi>(acc, C, bias, rowsum, rs_plane, M, N, ld, m0, n0, wm, wn, lane, scratch, add_last,
                          wm ? lds_ring<11, A_BYTES_S> : lds_ring<10, A_BYTES_S>, wm ? lds_ring<22, B_BYTES_S> : lds_ring<20, B_BYTES_S>,
-                         wm ? lds_ring<23, B_BYTES_S> : lds_ring<21, B_BYTES_S>);
+                         wm ? lds_ring<23, B_BYTES_S> : lds_ring<21, B_BYTES_S>, fold, tm, tiles_n);
   } else {
-    epilogue16<Epi, 8, 4, Ragged, WM>(acc, C, bias, rowsum, rs_plane, M, N, ld, m0, wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
+    epilogue16<Epi, 8, 4, Ragged, WM>(acc, C, bias, rowsum, rs_plane, M, N, ld, m0, wm, wn, n0 + wn * 64, l16, g, scratch, add_last, fold,
+                                      tm, tiles_n);
   }
   if (kMeasureBuild && probe && tid == 0) {
     probe[2 * blockIdx.x] = static_cast<unsigned long long>(clock64() - probe_c0);
@@ -1222,7 +1232,7 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
                                                                float *__restrict__ rowsum, int M, int N, int K, int tiles_m,
                                                                int tiles_n, int xcd_remap, unsigned long long *probe,
                                                                int k_chunk, float *__restrict__ partials, int ld,
-                                                               float *__restrict__ rs_planes) {
+                                                               float *__restrict__ rs_planes, RowFold fold = {}) {
   constexpr int SBM = 128, SBN = 128;
   constexpr int BKA = 64, BKB = 32, NA = 3, NB = 4;
   constexpr int RA = BKA / BKB;
@@ -1434,7 +1444,7 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   const bool add_last = Ragged && (N & 1) != 0 && n0 + SBN >= N && k0 + k_len == K;
   if (add_last) last_products<Bf16, SBM>(A, B, M, N, K, ld, m0, k0, scratch);
   epilogue16<Epi, 4, WN, Ragged>(acc, C, bias, rowsum, rs_planes ? rs_planes + static_cast<int64_t>(tn) * M : nullptr, M, N, ld, m0,
-                         wm, wn, n0 + wn * 64, l16, g, scratch, add_last);
+                         wm, wn, n0 + wn * 64, l16, g, scratch, add_last, fold, tm, tiles_n);
   if (kMeasureBuild && probe && tid == 0) {
     probe[2 * blockIdx.x] = static_cast<unsigned long long>(clock64() - probe_c0);
     probe[2 * blockIdx.x + 1] = static_cast<unsigned long long>(wall_clock64() - probe_t0);
@@ -1843,8 +1853,21 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
       if (rc != SAREK_HIP_OK) return rc;
     }
   }
+  // The last launch's own workgroups add the planes (fold_rows) where they are one round: a CU that has another tile waiting gives
+  // up on each what the launch of rowsum_fold_kernel takes once (4095 x 11008 x 4096 299 us either way, 2496 x 7821 x 331 39.5
+  // and 40.3).  gemm16.fold: 0 = this rule, 1 = never, 2 = always.
+  bool folded = false;
+  auto fold_in = [&](int tile_rows, int64_t tiles, int64_t slots) {
+    const int64_t asked = tunable("gemm16.fold", 0);
+    RowFold fold{planes, n_planes, nullptr};
+    if (planes && nm == n && tile_rows <= kFoldTickets && asked != 1 && (asked == 2 || tiles <= slots)) {
+      fold.tickets = fold_tickets(planes);
+      folded = true;
+    }
+    return fold;
+  };
   auto finish = [&](int rc) {
-    if (rc != SAREK_HIP_OK || !planes) return rc;
+    if (rc != SAREK_HIP_OK || !planes || folded) return rc;
     return launch_rowsum_fold(planes, n_planes, m, rowsum, st);
   };
 
@@ -1860,12 +1883,13 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   auto launch_half = [&](int first, int count, float *count_planes) {
     const int sm = (m + 127) / 128, sn = (count + 255) / 256;
     const float *const part_bias = Epi == EPI_BIAS_RELU_ROWSUM ? bias + first : nullptr;
+    const RowFold fold = fold_in(sm, static_cast<int64_t>(sm) * sn, compute_units());
     if (ragged)
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, true, false, 1>), dim3(sm * sn), dim3(256), 0, st, a, b + first,
-                         c + first, part_bias, rowsum, m, count, k, sm, sn, remap, nullptr, n, count_planes);
+                         c + first, part_bias, rowsum, m, count, k, sm, sn, remap, nullptr, n, count_planes, fold);
     else
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false, false, 1>), dim3(sm * sn), dim3(256), 0, st, a, b + first,
-                         c + first, part_bias, rowsum, m, count, k, sm, sn, remap, nullptr, n, count_planes);
+                         c + first, part_bias, rowsum, m, count, k, sm, sn, remap, nullptr, n, count_planes, fold);
     return check_launch("gemm16 kernel launch");
   };
   if (nm > 0 && half && tile_choice == 128) {
@@ -1892,18 +1916,20 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
       if (rc != SAREK_HIP_OK) return rc;
       rc = launch_splitk_reduce(partials, c, m, n, splits, st);
     } else {
+      const RowFold fold = fold_in(sm, static_cast<int64_t>(sm) * sn, 2 * compute_units());
       if (ragged)
         hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, true>), dim3(sm * sn), dim3(256), 0, st, a, b, c, bias,
-                           rowsum, m, nm, k, sm, sn, remap, sprobe, k, nullptr, n, planes);
+                           rowsum, m, nm, k, sm, sn, remap, sprobe, k, nullptr, n, planes, fold);
       else
         hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, false>), dim3(sm * sn), dim3(256), 0, st, a, b, c, bias,
-                           rowsum, m, nm, k, sm, sn, remap, sprobe, k, nullptr, n, planes);
+                           rowsum, m, nm, k, sm, sn, remap, sprobe, k, nullptr, n, planes, fold);
       rc = check_launch("gemm16 kernel launch");
     }
   } else if (nm > 0) {
     const int tiles_m = (m + BM - 1) / BM, tiles_n = (cut + BN - 1) / BN;
     const bool by_rows = rows_pay(m, n, k);
     const int apart = rows_apart(n, k);
+    const RowFold fold = cut < nm ? RowFold{} : fold_in(tiles_m, static_cast<int64_t>(tiles_m) * tiles_n, compute_units());
     unsigned long long *probe = clock_probe(static_cast<int64_t>(tiles_m) * tiles_n);
 #ifdef SAREK_HIP_MEASURE
     if (Epi == EPI_STORE && !ragged && tunable("gemm16.waves", 8) == 4) {
@@ -1911,34 +1937,35 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
                          tiles_n, remap);
     } else if (!ragged && tunable("gemm16.barriers", 2) == 1) {
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c,
-                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
+                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes, fold);
     } else
 #endif
     if (by_rows && ragged)
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, true, false, 2, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c,
-                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes, apart);
+                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes, fold, apart);
     else if (by_rows)
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false, false, 2, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c,
-                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes, apart);
+                         bias, rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes, fold, apart);
     else if (ragged)
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, true>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c, bias,
-                         rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
+                         rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes, fold);
     else
       hipLaunchKernelGGL((gemm16_m16_kernel<Bf16, Epi, 0, false>), dim3(tiles_m * tiles_n), dim3(512), 0, st, a, b, c, bias,
-                         rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes);
+                         rowsum, m, cut, k, tiles_m, tiles_n, remap, probe, n, planes, fold);
     rc = check_launch("gemm16 kernel launch");
     if (rc == SAREK_HIP_OK && cut < nm) {
       const int rest = nm - cut, sm = (m + 127) / 128, sn = (rest + 127) / 128;
       float *const rest_planes = planes ? planes + static_cast<int64_t>(tiles_n) * m : nullptr;
       const float *const rest_bias = Epi == EPI_BIAS_RELU_ROWSUM ? bias + cut : nullptr;
+      const RowFold rest_fold = half ? RowFold{} : fold_in(sm, static_cast<int64_t>(sm) * sn, 2 * compute_units());
       if (half)
         rc = launch_half(cut, rest, rest_planes);
       else if (ragged)
         hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, true>), dim3(sm * sn), dim3(256), 0, st, a, b + cut, c + cut,
-                           rest_bias, rowsum, m, rest, k, sm, sn, remap, nullptr, k, nullptr, n, rest_planes);
+                           rest_bias, rowsum, m, rest, k, sm, sn, remap, nullptr, k, nullptr, n, rest_planes, rest_fold);
       else
         hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, false>), dim3(sm * sn), dim3(256), 0, st, a, b + cut, c + cut,
-                           rest_bias, rowsum, m, rest, k, sm, sn, remap, nullptr, k, nullptr, n, rest_planes);
+                           rest_bias, rowsum, m, rest, k, sm, sn, remap, nullptr, k, nullptr, n, rest_planes, rest_fold);
       if (!half) rc = check_launch("gemm16 kernel launch");
     }
   }

@@ -39,8 +39,7 @@ namespace {
 
 constexpr int kTileRows = 64, kCols = 128, kStepK = 32, kWaves = 8;
 constexpr int kRedPitch = kCols + 4;   // floats per row of the waves' sums in LDS: 16 rows on different banks
-// Cache-policy bits of a buffer access: past the L2s, which the XCDs do not share; and non-temporal.
-constexpr int kDeviceScope = 16, kNonTemporal = 2;
+constexpr int kNonTemporal = 2;   // cache policy of a buffer access
 
 template <bool Bf16, int MT, int BPolicy, bool Fused>
 __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t *__restrict__ A,
@@ -50,7 +49,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
                                                                   int row_tiles, int col_tiles, int splits,
                                                                   int steps_per_split, float *__restrict__ rs_planes,
                                                                   float *__restrict__ partials,
-                                                                  unsigned *__restrict__ tickets) {
+                                                                  unsigned *__restrict__ tickets, RowFold fold) {
   __shared__ __attribute__((aligned(16))) float red[kWaves][16 * kRedPitch];
   __shared__ bool last;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -199,8 +198,11 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
 #pragma unroll
       for (int o = 16; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
       if (m < M && (lane & 31) == 0) {
-        if (rs_planes) rs_planes[static_cast<int64_t>(col_tile) * (M + m0) + m0 + m] = sum;
-        else atomicAdd(rowsum + m0 + m, sum);
+        if (rs_planes)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sum), make_rsrc(rs_planes, 0x7FFFFFFFu),
+                                                (col_tile * (M + m0) + m0 + m) * 4, 0, kDeviceScope);
+        else
+          atomicAdd(rowsum + m0 + m, sum);
       }
     }
     if (m >= M) return;
@@ -236,7 +238,15 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), p_rsrc, piece + t * (16 * kCols * 4),
                                              split * plane_bytes, kDeviceScope);
   }
-  if (splits == 1) return;
+  auto fold_here = [&] {
+    if constexpr (Fused) {
+      if (fold.tickets) fold_rows<64 * kWaves, kTileRows>(fold, M + m0, m0, rowsum, row_tile, col_tiles, &red[0][0]);
+    }
+  };
+  if (splits == 1) {
+    fold_here();
+    return;
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's pieces are where the other XCDs read them
   __syncthreads();
   if (threadIdx.x == 0)
@@ -266,6 +276,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
 #pragma unroll
   for (int t = 0; t < MT; ++t) put(t, sum[t]);
   if (threadIdx.x == 0) __hip_atomic_store(tickets + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  fold_here();
 }
 
 // Rows per tile: as few tiles of at most 64 as there can be, of equal height, in blocks of 16.
@@ -343,6 +354,8 @@ int launch(const Call &q, const Shape &s) {
       if (rc != SAREK_HIP_OK) return rc;
     }
   }
+  RowFold fold{rs_planes, s.col_tiles, nullptr};
+  if (rs_planes && s.row_tiles <= kFoldTickets && tunable("gemm16.fold", 0) != 1) fold.tickets = fold_tickets(block);
   float *partials = splits > 1 ? block + s.rs_floats : nullptr;
   unsigned *tickets = splits > 1 ? splitk_tickets(block) : nullptr;
   // B past the caches from 64 MiB on where its rows are whole 128-byte lines (100 MB: 20.2 us against 22.8, 134 MB: 26.4
@@ -353,12 +366,12 @@ int launch(const Call &q, const Shape &s) {
   const dim3 grid(static_cast<unsigned>(s.tiles * splits)), block_dim(64 * kWaves);
   if (nt)
     hipLaunchKernelGGL((gemm16_rows_kernel<Bf16, MT, kNonTemporal, Fused>), grid, block_dim, 0, q.st, q.a, q.b, q.c, q.bias,
-                       q.rowsum, q.m, q.n, q.k, s.row_tiles, s.col_tiles, splits, per, rs_planes, partials, tickets);
+                       q.rowsum, q.m, q.n, q.k, s.row_tiles, s.col_tiles, splits, per, rs_planes, partials, tickets, fold);
   else
     hipLaunchKernelGGL((gemm16_rows_kernel<Bf16, MT, 0, Fused>), grid, block_dim, 0, q.st, q.a, q.b, q.c, q.bias,
-                       q.rowsum, q.m, q.n, q.k, s.row_tiles, s.col_tiles, splits, per, rs_planes, partials, tickets);
+                       q.rowsum, q.m, q.n, q.k, s.row_tiles, s.col_tiles, splits, per, rs_planes, partials, tickets, fold);
   const int rc = check_launch("gemm16 few-rows kernel launch");
-  if (!rs_planes || rc != SAREK_HIP_OK) return rc;
+  if (!rs_planes || fold.tickets || rc != SAREK_HIP_OK) return rc;
   return launch_rowsum_fold(rs_planes, s.col_tiles, q.m, q.rowsum, q.st);
 }
 

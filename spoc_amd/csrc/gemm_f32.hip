@@ -31,7 +31,6 @@ namespace {
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-constexpr int kDeviceScope = 16;   // cache policy of loads and stores that other XCDs take part in
 constexpr int BM = 256, BN = 256, BK = 32;
 constexpr int THREADS = 512;
 constexpr int A_STRIDE = BK + 4;            // floats per A row in LDS (36)

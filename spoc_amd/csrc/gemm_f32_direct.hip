@@ -27,7 +27,6 @@ namespace {
 
 constexpr int kCols = 64, kStepK = 16;
 constexpr int kRedPitch = kCols + 4;
-constexpr int kDeviceScope = 16;
 
 // Workgroup -> (piece of K, tile): every XCD gets a contiguous run of the pieces' tiles, which it walks in bands of
 // `band` tile rows, column by column, the band chosen so that the patch of a run is about as tall as wide: the tiles that

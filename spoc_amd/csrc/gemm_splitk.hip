@@ -55,11 +55,11 @@ float *splitk_workspace(hipStream_t st) {
   if (it != blocks.end()) return static_cast<float *>(it->second);
   if (blocks.size() >= 16) return nullptr;
   void *p = nullptr;
-  if (hipMalloc(&p, kSplitWorkspaceBytes + kSplitTickets * sizeof(unsigned)) != hipSuccess) {
+  if (hipMalloc(&p, kSplitWorkspaceBytes + (kSplitTickets + kFoldTickets) * sizeof(unsigned)) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
-  hipLaunchKernelGGL(zero_tickets_kernel, dim3(kSplitTickets / 256), dim3(256), 0, st, splitk_tickets(static_cast<float *>(p)));
+  hipLaunchKernelGGL(zero_tickets_kernel, dim3((kSplitTickets + kFoldTickets) / 256), dim3(256), 0, st, splitk_tickets(static_cast<float *>(p)));
   blocks[{dev, st}] = p;
   return static_cast<float *>(p);
 }

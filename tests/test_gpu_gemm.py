@@ -504,6 +504,41 @@ def test_gemm16_stored_by_rows(hip, torch_cuda, kind, m, n, k, rows):
         hip.set_tunable("gemm16.tile", 0)
 
 
+@pytest.mark.parametrize("m,n,k,knobs", [
+    (1, 2, 32, {}), (64, 128, 64, {}), (65, 129, 100, {}), (83, 1344, 1152, {}), (512, 256, 1402, {}), (48, 2300, 520, {}),
+    (128, 128, 64, {"gemm16.tile": 128}), (129, 257, 72, {"gemm16.tile": 128}), (300, 4300, 200, {"gemm16.tile": 128}),
+    (256, 256, 64, {"gemm16.tile": 256}), (257, 4355, 131, {"gemm16.tile": 256}), (300, 1100, 192, {"gemm16.tile": 128, "gemm16.half": 2}),
+    (513, 515, 200, {"gemm16.tile": 256, "gemm16.by_rows": 2}), (2048, 8448, 512, {}), (2048, 11264, 1216, {})])
+def test_fused_row_sums_added_by_the_last_tile(hip, torch_cuda, m, n, k, knobs):
+    """Row sums that the launch's last workgroup of a row of tiles adds, on each kernel that can: the double sum of the stored
+    row to 1e-5 of it (float32 sums of at most 256 values, then doubles), the same bits again and again and on another stream at
+    the same time, and those of the launch of its own to one rounding (the doubles are added in another order)."""
+    torch = torch_cuda
+    torch.manual_seed(m + n)
+    a, b = ((torch.randn(*s, device="cuda") * 0.2).half() for s in ((m, k), (k, n)))
+    bias = torch.rand(n, device="cuda") * 0.2 - 0.1
+    side = side_stream(torch)
+    try:
+        for knob, value in knobs.items():
+            hip.set_tunable(knob, value)
+        hip.set_tunable("gemm16.fold", 1)
+        y1, rs1 = hip.gemm_f16_bias_relu_rowsum(a, b, bias)
+        for arm in (0, 2):
+            hip.set_tunable("gemm16.fold", arm)
+            torch.cuda.synchronize()
+            with torch.cuda.stream(side):
+                other = [hip.gemm_f16_bias_relu_rowsum(a, b, bias) for _ in range(3)]
+            here = [hip.gemm_f16_bias_relu_rowsum(a, b, bias) for _ in range(3)]
+            torch.cuda.synchronize()
+            for y, rs in here + other:
+                assert torch.equal(y, y1) and torch.equal(rs, here[0][1])
+                assert bool(((rs - rs1).abs() <= 2.0 ** -23 * rs1.abs()).all())
+                assert rowsums_ok(rs.cpu().numpy(), y.double().sum(1).cpu().numpy())
+    finally:
+        for knob in ("gemm16.fold", *knobs):
+            hip.set_tunable(knob, 0)
+
+
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(2048, 8448, 64), (2047, 8195, 72), (1921, 8703, 131), (2048, 10240, 65),
                                    (8192, 2050, 70), (2300, 7425, 200)])
