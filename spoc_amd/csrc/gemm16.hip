@@ -486,6 +486,14 @@ __device__ __forceinline__ void last_products(const uint16_t *__restrict__ A, co
   __syncthreads();
 }
 
+// A row's share of a tile; where fold_rows finds it if this launch folds.
+__device__ __forceinline__ void store_share(const RowFold &fold, float *plane, int at, float share) {
+  if (fold.tickets)
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(share), make_rsrc(plane, 0x7FFFFFFFu), at * 4, 0, kDeviceScope);
+  else
+    plane[at] = share;
+}
+
 // Writes one wave's (16*TI) x 64 block held as TI x 4 tiles of 16 x 16 (register r of lane l: row 4*(l/16) + r, column
 // l%16 of its tile); TI = 8 in the 256 x 256 workgroup tile (2 x 4 waves) and the 128 x 256 one (1 x 4), 4 in the 128 x 128 one (2 x 2).
 // Fused form as in `epilogue`: per lane the sum over its four columns for each of its 4*TI rows, a halving butterfly
@@ -495,11 +503,6 @@ __device__ __forceinline__ void last_products(const uint16_t *__restrict__ A, co
 // rowsum_fold_kernel: the same bits on every run), else to rowsum[r] by atomicAdd.  The 128 x 256 tile has two, for its halves
 // of 128 columns: as many float32 additions in front of the fold's double as on the 128 x 128 tile, whose products it takes.  add_last: the tile rows' last_products
 // lie in `scratch` and belong to column N - 1.
-// A row's share of a tile, where fold_rows finds it.
-__device__ __forceinline__ void store_share(float *plane, int at, float share) {
-  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(share), make_rsrc(plane, 0x7FFFFFFFu), at * 4, 0, kDeviceScope);
-}
-
 template <int Epi, int TI, int WNW, bool Ragged, int WMW = 2>   // WMW, WNW: waves along M, N
 __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restrict__ C, const float *__restrict__ bias,
                                            float *__restrict__ rowsum, float *__restrict__ rs_plane, int M, int N, int ld,
@@ -579,7 +582,7 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
       const int t = threadIdx.x & 127, half = threadIdx.x >> 7;
       if (m0 + t < M && col0 - wn * 64 + half * 128 < N) {
         const float total = scratch[2 * half * TROWS + t] + scratch[(2 * half + 1) * TROWS + t];
-        if (rs_plane) store_share(rs_plane, half * M + m0 + t, total);
+        if (rs_plane) store_share(fold, rs_plane, half * M + m0 + t, total);
         else atomicAdd(rowsum + m0 + t, total);
       }
     } else {
@@ -588,7 +591,7 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
         float total;
         if constexpr (WNW == 4) total = (scratch[t] + scratch[TROWS + t]) + (scratch[2 * TROWS + t] + scratch[3 * TROWS + t]);
         else total = scratch[t] + scratch[TROWS + t];
-        if (rs_plane) store_share(rs_plane, m0 + t, total);
+        if (rs_plane) store_share(fold, rs_plane, m0 + t, total);
         else atomicAdd(rowsum + m0 + t, total);
       }
     }
@@ -721,7 +724,7 @@ __device__ __forceinline__ void epilogue16_rows(f32x4_t (&acc)[8][4], float *__r
     const int t = threadIdx.x;
     if (t < TROWS && m0 + t < M) {
       const float total = (scratch[t] + scratch[TROWS + t]) + (scratch[2 * TROWS + t] + scratch[3 * TROWS + t]);
-      if (rs_plane) store_share(rs_plane, m0 + t, total);
+      if (rs_plane) store_share(fold, rs_plane, m0 + t, total);
       else atomicAdd(rowsum + m0 + t, total);
     }
     if (fold.tickets) fold_rows<512, TROWS>(fold, M, m0, rowsum, tile_row, tiles_n, scratch);
@@ -1650,7 +1653,7 @@ __global__ __launch_bounds__(256) void gemm16_last_column_kernel(const uint16_t 
   }
 }
 
-// K splits of the 128 x 128 kernel for a plain product with few tiles and a long K; 1 = no split.  A tile's K loop is
+// K splits of the 128 x 128 kernel for a product with few tiles and a long K, plain or fused; 1 = no split.  A tile's K loop is
 // bound by the latency of its transfers (0.19 us per K = 32 slab with one or two workgroups on a CU, measured), so
 // cutting K over idle CUs shortens it; against that stand the second launch (5 us) and the partial planes, which cost
 // 0.65 us per MiB to write and add up.  The count in {2, 4, 8, 16} with the lowest estimate is taken if it is a tenth
@@ -1694,10 +1697,12 @@ inline bool gemm16_default_kernel() {
 // Microseconds of a product on the 128 x 128 tile with at most a workgroup per CU, by an estimate: its slabs by how A's and
 // B's rows lie (on 16 bytes, on 4, on 2), the K pieces it would take.
 double small_tile_time(int m, int n, int k, bool fused) {
-  const double slab = k % 8 == 0 && n % 8 == 0 ? 0.19 : k % 2 == 0 && n % 2 == 0 ? 0.24 : 0.33;
-  const int splits = fused ? 1 : splitk_for(m, n, k);
-  return 5.5 + static_cast<double>(k) / 32 / splits * slab +
-         (splits > 1 ? 3.0 + splits * (static_cast<double>(m) * n * 4 / (1 << 20)) * 0.65 : 0.0);
+  const bool on16 = k % 8 == 0 && n % 8 == 0, on4 = k % 2 == 0 && n % 2 == 0;
+  const int splits = splitk_for(m, n, k);
+  const double slabs = static_cast<double>(k) / 32 / splits, planes = splits * (static_cast<double>(m) * n * 4 / (1 << 20));
+  if (fused)   // read off 512 drawn products, gemm16_rows_pays
+    return 6.6 + slabs * (on16 ? 0.193 : k % 2 == 0 || n % 2 == 0 ? 0.26 : 0.43) + (splits > 1 ? 0.25 + 0.5 * splits + 0.68 * planes : 0.0);
+  return 5.5 + slabs * (on16 ? 0.19 : on4 ? 0.24 : 0.33) + (splits > 1 ? 3.0 + planes * 0.65 : 0.0);
 }
 
 // The same for 17 to 64 rows and a B that is new to the caches, from 800 drawn products of that many (8 % rms): the slabs of a
@@ -1705,7 +1710,7 @@ double small_tile_time(int m, int n, int k, bool fused) {
 double narrow_tile_time(int m, int n, int k, bool fused) {
   const int align = k % 64 == 0 && n % 8 == 0 ? 0 : k % 8 == 0 && n % 8 == 0 ? 1 : k % 2 == 0 && n % 2 == 0 ? 2 : 3;
   constexpr double kSlab[] = {0.172, 0.257, 0.272, 0.334}, kMegabyte[] = {0.156, 0.125, 0.134, 0.155};
-  const int splits = fused ? 1 : splitk_for(m, n, k);
+  const int splits = splitk_for(m, n, k);
   const int64_t per_cu = ceil_div(ceil_div(n, 128) * splits, compute_units());
   const double slabs = static_cast<double>(k) / 32 / splits * kSlab[align] * static_cast<double>(per_cu);
   const double memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[align], c_mb = static_cast<double>(m) * n * 4e-6;
@@ -1853,14 +1858,17 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
       if (rc != SAREK_HIP_OK) return rc;
     }
   }
-  // The last launch's own workgroups add the planes (fold_rows) where they are one round: a CU that has another tile waiting gives
-  // up on each what the launch of rowsum_fold_kernel takes once (4095 x 11008 x 4096 299 us either way, 2496 x 7821 x 331 39.5
-  // and 40.3).  gemm16.fold: 0 = this rule, 1 = never, 2 = always.
+  // The last launch's own workgroups add the planes (fold_rows) where they are one round and their shares few: a CU that has
+  // another tile waiting gives up on each what the launch of rowsum_fold_kernel takes once (4095 x 11008 x 4096 299 us either way,
+  // 2496 x 7821 x 331 39.5 and 40.3), and many tiles in rows of many take their last workgroups longer than that launch's many
+  // (us, the launch and here, tiles x planes: 7360 x 426 x 258, 232 x 4, 12.0 and 11.5; 565 x 1344 x 647, 55 x 11, 14.3 and 13.6;
+  // 168 x 2432 x 256, 38 x 19, 9.7 and 8.3; 2457 x 1294 x 512, 220 x 11, 13.2 and 13.7; 2176 x 1600 x 896, 221 x 13, 14.6 and 15.4;
+  // 289 x 8448 x 256, 198 x 66, 10.5 and 11.8).  gemm16.fold: 0 = this rule, 1 = never, 2 = always.
   bool folded = false;
   auto fold_in = [&](int tile_rows, int64_t tiles, int64_t slots) {
     const int64_t asked = tunable("gemm16.fold", 0);
     RowFold fold{planes, n_planes, nullptr};
-    if (planes && nm == n && tile_rows <= kFoldTickets && asked != 1 && (asked == 2 || tiles <= slots)) {
+    if (planes && nm == n && tile_rows <= kFoldTickets && asked != 1 && (asked == 2 || (tiles <= slots && tiles * n_planes <= 1024))) {
       fold.tickets = fold_tickets(planes);
       folded = true;
     }
@@ -1899,22 +1907,23 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
     unsigned long long *sprobe = clock_probe(static_cast<int64_t>(sm) * sn);
     int splits = 1;
     float *partials = nullptr;
-    if constexpr (Epi == EPI_STORE) {
-      if (reinterpret_cast<uintptr_t>(c) % 16 == 0) splits = splitk_for(m, n, k);
-      if (splits > 1) partials = splitk_workspace(st);
-      if (!partials) splits = 1;
-    }
+    // (fused: the planes hold plain sums; the launch that adds them does the rest.  Us, uncut and cut: 110 x 9523 x 7936 94 -> 73,
+    // 2649 x 435 x 6243 67 -> 45, 103 x 5881 x 6427 56 on the few-rows kernel -> 32, 517 x 704 x 2995 21.8 -> 17.7)
+    if (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n) splits = splitk_for(m, n, k);
+    if (splits > 1) partials = splitk_workspace(st);
+    if (!partials) splits = 1;
     if (splits > 1) {
       const int chunk = splitk_chunk(k, 64, splits);
       if (ragged)
-        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, true>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
-                           bias, rowsum, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, planes);
+        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, true>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
+                           nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, nullptr);
       else
-        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, Epi, false>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
-                           bias, rowsum, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, planes);
+        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, false>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
+                           nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, nullptr);
       rc = check_launch("gemm16 kernel launch");
       if (rc != SAREK_HIP_OK) return rc;
-      rc = launch_splitk_reduce(partials, c, m, n, splits, st);
+      if constexpr (Epi == EPI_STORE) rc = launch_splitk_reduce(partials, c, m, n, splits, st);
+      else return launch_splitk_reduce_fused(partials, bias, c, rowsum, m, n, splits, st);
     } else {
       const RowFold fold = fold_in(sm, static_cast<int64_t>(sm) * sn, 2 * compute_units());
       if (ragged)

@@ -198,7 +198,9 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
 #pragma unroll
       for (int o = 16; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
       if (m < M && (lane & 31) == 0) {
-        if (rs_planes)
+        if (rs_planes && !fold.tickets)
+          rs_planes[static_cast<int64_t>(col_tile) * (M + m0) + m0 + m] = sum;
+        else if (rs_planes)
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sum), make_rsrc(rs_planes, 0x7FFFFFFFu),
                                                 (col_tile * (M + m0) + m0 + m) * 4, 0, kDeviceScope);
         else
@@ -355,7 +357,14 @@ int launch(const Call &q, const Shape &s) {
     }
   }
   RowFold fold{rs_planes, s.col_tiles, nullptr};
-  if (rs_planes && s.row_tiles <= kFoldTickets && tunable("gemm16.fold", 0) != 1) fold.tickets = fold_tickets(block);
+  // The last workgroup of a row of tiles adds the planes (fold_rows) while the tiles are few: the more, the longer their shares and
+  // counts take to come together, the longer with more rows (us, rowsum_fold_kernel's launch and here, K of 512: 4 x 512 10.5 and
+  // 7.3, 4 x 16384 9.7 and 8.2, 4 x 32768 10.4 and 11.9, 128 x 2048 11.4 and 11.3, 128 x 8192 11.8 and 12.8, 2000 x 512 12.3 and
+  // 12.2, 1000 x 1024 12.3 and 12.8).  gemm16.fold: 0 = this rule, 1 = never, 2 = always.
+  const int64_t asked = tunable("gemm16.fold", 0);
+  if (rs_planes && s.row_tiles <= kFoldTickets && asked != 1 &&
+      (asked == 2 || s.tiles <= (s.mt <= 2 ? 128 : 64) || s.tiles * s.col_tiles <= 512))
+    fold.tickets = fold_tickets(block);
   float *partials = splits > 1 ? block + s.rs_floats : nullptr;
   unsigned *tickets = splits > 1 ? splitk_tickets(block) : nullptr;
   // B past the caches from 64 MiB on where its rows are whole 128-byte lines (100 MB: 20.2 us against 22.8, 134 MB: 26.4
@@ -426,9 +435,11 @@ double narrow_time(const Shape &s, int n, int k, int splits) {
 // Beyond 64 rows, and with the fused epilogue at any number, where its tiles fit the CUs in one round (882 x 2401 x 4259,
 // 266 tiles: 50 us on the other tile, 108 here), at least half of the waves have a step (in tiles of 64 rows some wave has
 // two: 256 x 1280 x 191 6.8 / 8.4, 723 x 1702 x 256 7.2 / 7.9, as 21 of 118 drawn products, all but 3 of them so short), and its
-// time is below the 128 x 128 tile's by both estimates.  They were read off 50 drawn products (up to 20 % and a microsecond
-// apart from them, the better kernel taken on 45, at most 8 % lost on the others): a step costs by how A's and B's rows lie, on
-// 16 bytes, on 4, on 2.  `other`: what the tiled kernel is estimated at.
+// time is below the 128 x 128 tile's by both estimates: a step costs by how A's and B's rows lie.  The plain ones were read
+// off 50 drawn products (up to 20 % and a microsecond apart from them, the better kernel taken on 45, at most 8 % lost on the
+// others), the fused ones off 512 of both kernels (11 % rms; 8 of them more than 4 % slower than when the tile had
+// no pieces of K for them, at most 10 %, and all together 7 % faster): 419 x 1472 x 2504 25.5 on the tile, 17.4 here,
+// 180 x 256 x 2240 10.0, 13.9.  `other`: what the tiled kernel is estimated at.
 bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other, Gemm16Estimate narrow_other) {
   const Shape s = shape_of(m, n, k, fused);
   if (m <= kTileRows && !fused) {
@@ -450,11 +461,17 @@ bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other, Gem
   if (m <= kTileRows && !fused) return true;
   if (s.tiles > compute_units() || 2 * s.steps < kWaves || (s.mt == 4 && s.steps <= kWaves)) return false;
   const int splits = rows_splits_for(s, n, k);
-  const bool on16 = k % 8 == 0 && n % 8 == 0;
-  const double step = (on16 ? 0.055 : k % 2 == 0 && n % 2 == 0 ? 0.07 : 0.12) * s.mt;
   const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
-  const double here = (on16 ? 6.0 : 4.5) + rounds * s.steps / splits * step +
-                      (splits > 1 ? 2.5 + 0.15 * splits + 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0);
+  const double steps = rounds * s.steps / splits * s.mt, planes = splits > 1 ? 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0;
+  const bool on16 = k % 8 == 0 && n % 8 == 0;
+  double here;
+  if (fused) {
+    const double step = k % 2 == 0 ? 0.064 : n % 2 == 0 ? 0.098 : 0.136;
+    here = 2.95 + 1.4 * s.mt + steps * step + (splits > 1 ? 1.7 + 0.31 * splits + 0.07 * planes : 0.0);
+  } else {
+    const double step = on16 ? 0.055 : k % 2 == 0 && n % 2 == 0 ? 0.07 : 0.12;
+    here = (on16 ? 6.0 : 4.5) + steps * step + (splits > 1 ? 2.5 + 0.15 * splits + planes : 0.0);
+  }
   return here < other(m, n, k, fused);
 }
 

@@ -10,6 +10,8 @@ namespace sarek_hip {
 constexpr size_t kSplitWorkspaceBytes = 64u << 20;
 float *splitk_workspace(hipStream_t st);
 int launch_splitk_reduce(const float *partials, float *c, int m, int n, int splits, hipStream_t st);
+int launch_splitk_reduce_fused(const float *partials, const float *bias, float *y, float *rowsum, int m, int n, int splits,
+                               hipStream_t st);   // with the bias, the ReLU and the row sums
 // Floats from one partial plane to the next: planes start at 16 bytes.
 __host__ __device__ inline int64_t splitk_plane_floats(int m, int n) { return (static_cast<int64_t>(m) * n + 3) / 4 * 4; }
 // K in at most `splits` pieces of whole stages of `stage`: their length (the last one takes what is left, at least a

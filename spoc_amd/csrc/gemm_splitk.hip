@@ -26,6 +26,54 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
   }
 }
 
+// The same for the fused product: y = relu(sum of the planes + bias), and the row's sum of y, in double, in a fixed order.  Waves
+// of the four of a workgroup to a row: one where a wave's four columns a lane are a quarter of it at least, or four.  Bound by the trip
+// to the planes, which the products have left in the caches: every row is asked for at once.
+template <int Waves>
+__global__ __launch_bounds__(256) void splitk_reduce_fused_kernel(const float *__restrict__ partials, const float *__restrict__ bias,
+                                                                  float *__restrict__ y, float *__restrict__ rowsum, int m, int n,
+                                                                  int64_t plane, int splits) {
+  __shared__ double sums[4];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int row = Waves == 4 ? static_cast<int>(blockIdx.x) : static_cast<int>(blockIdx.x) * 4 + wave;
+  if (Waves == 1 && row >= m) return;
+  const float *p = partials + static_cast<int64_t>(row) * n;
+  float *out = y + static_cast<int64_t>(row) * n;
+  double sum = 0.0;
+  for (int c = (Waves == 4 ? static_cast<int>(threadIdx.x) : lane) * 4; c < n; c += Waves * 256) {
+    if (c + 4 <= n) {
+      f32x4_t acc = *reinterpret_cast<const f32x4_u *>(p + c);
+      for (int s = 1; s < splits; ++s) acc += *reinterpret_cast<const f32x4_u *>(p + s * plane + c);
+      const f32x4_t b = *reinterpret_cast<const f32x4_u *>(bias + c);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float v = acc[j] + b[j];
+        acc[j] = v > 0.f ? v : 0.f;
+        sum += static_cast<double>(acc[j]);
+      }
+      *reinterpret_cast<f32x4_u *>(out + c) = acc;
+    } else {
+      for (int j = c; j < n; ++j) {
+        float acc = p[j];
+        for (int s = 1; s < splits; ++s) acc += p[s * plane + j];
+        const float v = acc + bias[j];
+        out[j] = v > 0.f ? v : 0.f;
+        sum += static_cast<double>(v > 0.f ? v : 0.f);
+      }
+    }
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  if constexpr (Waves == 4) {
+    if (lane == 0) sums[wave] = sum;
+    __syncthreads();
+    sum = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+    if (threadIdx.x == 0) rowsum[row] = static_cast<float>(sum);
+  } else {
+    if (lane == 0) rowsum[row] = static_cast<float>(sum);
+  }
+}
+
 __global__ __launch_bounds__(256) void zero_tickets_kernel(unsigned *tickets) {
   tickets[blockIdx.x * 256 + threadIdx.x] = 0;
 }
@@ -79,6 +127,17 @@ int launch_splitk_reduce(const float *partials, float *c, int m, int n, int spli
   const int64_t mn = static_cast<int64_t>(m) * n;
   hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>((mn + 1023) / 1024)), dim3(256), 0, st, partials, c,
                      mn, splitk_plane_floats(m, n), splits);
+  return check_launch("split-K reduction launch");
+}
+
+int launch_splitk_reduce_fused(const float *partials, const float *bias, float *y, float *rowsum, int m, int n, int splits,
+                               hipStream_t st) {
+  const int64_t plane = splitk_plane_floats(m, n);
+  if (n > 1024)
+    hipLaunchKernelGGL(splitk_reduce_fused_kernel<4>, dim3(m), dim3(256), 0, st, partials, bias, y, rowsum, m, n, plane, splits);
+  else
+    hipLaunchKernelGGL(splitk_reduce_fused_kernel<1>, dim3((m + 3) / 4), dim3(256), 0, st, partials, bias, y, rowsum, m, n, plane,
+                       splits);
   return check_launch("split-K reduction launch");
 }
 

@@ -539,6 +539,53 @@ def test_fused_row_sums_added_by_the_last_tile(hip, torch_cuda, m, n, k, knobs):
             hip.set_tunable(knob, 0)
 
 
+@pytest.mark.parametrize("m,n,k,splits", [(128, 128, 256, 2), (1, 8, 128, 2), (129, 257, 200, 3), (300, 1023, 328, 2), (65, 1024, 448, 7),
+                                          (64, 1025, 320, 4), (3, 4099, 1000, 5), (103, 1881, 6427, 0), (110, 2049, 7936, 0), (5, 2, 300, 3)])
+def test_fused_products_cut_along_k(hip, oracle, torch_cuda, m, n, k, splits):
+    """The fused product on the 128 x 128 tile with K in pieces, forced and by its own rule, one wave and four to a row of the
+    launch that adds them: the oracle's y and row sums, the same bits again and on another stream at the same time; under capture
+    it runs uncut, replay after replay."""
+    torch = torch_cuda
+    a, b = normal16(oracle, (m, k), m + 21, "f16"), normal16(oracle, (k, n), n + 22, "f16")
+    bias = oracle.fill_uniform(n, seed=n + 3, lo=-0.1, hi=0.1)
+    da, db, dbias = dev(torch, a).half(), dev(torch, b).half(), dev(torch, bias)
+    y_ref, rs_ref = oracle.gemm_bias_relu_rowsum(a, b, bias)
+
+    def good(y, rs):
+        return (np.abs(y.cpu().numpy() - y_ref).max() <= 1e-4 * max(np.abs(y_ref).max(), 1e-30) and
+                rowsums_ok(rs.cpu().numpy(), y.double().sum(1).cpu().numpy()) and
+                np.abs(rs.cpu().numpy() - rs_ref).max() <= 1e-4 * np.abs(rs_ref).max())
+    side = side_stream(torch)
+    try:
+        hip.set_tunable("gemm16.rows", 1)
+        if splits:
+            hip.set_tunable("gemm16.tile", 128)
+            hip.set_tunable("gemm16.split_k", splits)
+        assert hip.gemm16_k_splits(m, n, k) > 1
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            other = [hip.gemm_f16_bias_relu_rowsum(da, db, dbias) for _ in range(3)]
+        here = [hip.gemm_f16_bias_relu_rowsum(da, db, dbias) for _ in range(3)]
+        torch.cuda.synchronize()
+        assert good(*here[0])
+        for y, rs in here + other:
+            assert torch.equal(y, here[0][0]) and torch.equal(rs, here[0][1])
+        got, sums, graph = torch.empty_like(here[0][0]), torch.empty_like(here[0][1]), torch.cuda.CUDAGraph()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+            hip.gemm_f16_bias_relu_rowsum(da, db, dbias, out=got, rowsum=sums)
+        for _ in range(3):
+            got.fill_(float("nan"))
+            sums.fill_(float("nan"))
+            graph.replay()
+            assert torch.equal(hip.gemm_f16_bias_relu_rowsum(da, db, dbias)[1], here[0][1])
+            torch.cuda.synchronize()
+            assert good(got, sums)
+    finally:
+        for knob in ("gemm16.rows", "gemm16.tile", "gemm16.split_k"):
+            hip.set_tunable(knob, 0)
+
+
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k", [(2048, 8448, 64), (2047, 8195, 72), (1921, 8703, 131), (2048, 10240, 65),
                                    (8192, 2050, 70), (2300, 7425, 200)])
