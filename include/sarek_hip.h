@@ -656,7 +656,7 @@ int sarek_hip_gemm16_half_columns(int m, int n, int k);
  * to 16 streams; calls on further streams or on hipStreamPerThread, and calls
  * under stream capture, run unsplit (same result up to the order of
  * the f32 additions).  The count is the plain products'; the fused entry point
- * splits on the few-rows kernel only.                                       */
+ * cuts K by the same rules with counts of its own.                          */
 int sarek_hip_gemm16_k_splits(int m, int n, int k);
 
 /* Fused epilogue chain: y = relu(A.B + bias[col]) (f32, [m x n]) and

@@ -1653,35 +1653,70 @@ __global__ __launch_bounds__(256) void gemm16_last_column_kernel(const uint16_t 
   }
 }
 
-// K splits of the 128 x 128 kernel for a product with few tiles and a long K, plain or fused; 1 = no split.  A tile's K loop is
-// bound by the latency of its transfers (0.19 us per K = 32 slab with one or two workgroups on a CU, measured), so
-// cutting K over idle CUs shortens it; against that stand the second launch (5 us) and the partial planes, which cost
-// 0.65 us per MiB to write and add up.  The count in {2, 4, 8, 16} with the lowest estimate is taken if it is a tenth
-// below the unsplit one; every piece is at least 256 of K and the planes fit kSplitWorkspaceBytes.
-// gemm16.split_k: 0 = this rule, 1 = never, n >= 2 forces n where the shape allows it.
-int splitk_for(int m, int n, int k) {
-  const int64_t tiles = static_cast<int64_t>((m + 127) / 128) * ((n + 127) / 128);
-  const int64_t forced = tunable("gemm16.split_k", 0);
-  if (forced == 1) return 1;
-  const int cus = compute_units();
-  const double plane_mib = static_cast<double>(m) * n * 4 / (1 << 20);
-  const int64_t fit = static_cast<int64_t>(kSplitWorkspaceBytes) / (splitk_plane_floats(m, n) * 4);
-  int64_t splits = 1;
-  if (forced >= 2) {
-    splits = std::max<int64_t>(1, std::min<int64_t>({forced, static_cast<int64_t>(k / 64), fit}));
-  } else {
-    auto estimate = [&](int64_t s) {
-      const double slabs = static_cast<double>(k) / 32 / s;
-      return 8.0 + slabs * 0.19 * (tiles * s > cus ? 1.15 : 1.0) + (s > 1 ? 5.0 + s * plane_mib * 0.65 : 0.0);
-    };
-    double best = estimate(1) * 0.9;
-    for (int64_t s = 2; s <= 16; s *= 2) {
-      if (tiles * s > 2 * cus || k / s < 256 || s > fit) break;
-      if (estimate(s) < best) best = estimate(s), splits = s;
-    }
+// Microseconds of a product on the 128 x 128 tile, plain or fused, by an estimate read off 730 plain and 520 fused products drawn
+// over 17 to 8192 rows, their operands new to the caches, each in 1 to 16 pieces of K (8 and 10 % rms): a slab of 32 of K by how
+// A's and B's rows lie (on 16 bytes, on 4, on 2), a second workgroup of a CU beside the first; the operands from memory; C; and for
+// pieces the launch that adds them, and their planes.
+struct TileTime {
+  int64_t tiles, stages, cus;
+  double stage, second, memory2, whole, launch, piece;
+
+  TileTime(int m, int n, int k, bool fused) {
+    struct Fit { double stage[3], second, memory, base, c, launch, piece, plane; };
+    constexpr Fit kPlain = {{0.336, 0.414, 0.498}, 1.75, 0.116, 4.34, 0.171, 2.05, 0.213, 0.312};
+    constexpr Fit kFused = {{0.324, 0.418, 0.498}, 1.54, 0.213, 6.68, 0.272, 0.49, 0.55, 0.318};
+    const Fit &f = fused ? kFused : kPlain;
+    tiles = ceil_div(m, 128) * ceil_div(n, 128);
+    stages = ceil_div(k, 64);
+    cus = compute_units();
+    stage = f.stage[k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2];
+    second = f.second;
+    const double memory = (static_cast<double>(m) * k + static_cast<double>(k) * n) * 2e-6 * f.memory, c_mb = static_cast<double>(m) * n * 4e-6;
+    memory2 = memory * memory;
+    whole = f.base + f.c * c_mb;
+    launch = f.launch;
+    piece = f.piece + f.plane * c_mb;
   }
-  return splitk_pieces(k, 64, splits);
+  double in(int64_t splits) const {
+    const double t = static_cast<double>(ceil_div(stages, splits)) * stage *
+                     (tiles * splits <= cus ? 1.0 : second * static_cast<double>(ceil_div(tiles * splits, 2 * cus)));
+    return whole + std::sqrt(t * t + memory2) + (splits > 1 ? launch + static_cast<double>(splits) * piece : 0.0);
+  }
+  // The count of at most `most` with the lowest estimate, if that is 3 % below the uncut one: about the root of what a piece saves
+  // over what it costs, with a workgroup per CU and with two.
+  int64_t best(int64_t most) const {
+    const double slabs = static_cast<double>(stages) * stage * (tiles <= cus ? 1.0 : second);
+    most = std::min<int64_t>({most, 16, 2 * cus / tiles});
+    if (most < 2 || slabs < 2.0 * (launch + 2.0 * piece)) return 1;   // half of the slabs saved by two pieces at most
+    int64_t splits = 1;
+    double lowest = in(1) * 0.97;
+    auto try_near = [&](double root, int64_t lo, int64_t hi) {
+      if (lo > hi) return;
+      for (int64_t s = std::clamp(static_cast<int64_t>(root), lo, hi), e = std::min(s + 1, hi); s <= e; ++s)
+        if (const double t = in(s); t < lowest) lowest = t, splits = s;
+    };
+    const double saved = static_cast<double>(stages) * stage / piece;
+    try_near(std::sqrt(saved), 2, std::min(most, cus / tiles));
+    try_near(std::sqrt(saved * second), std::max<int64_t>(2, cus / tiles + 1), most);
+    return splits;
+  }
+};
+
+// K splits of the 128 x 128 kernel for a product with few tiles and a long K, plain or fused; 1 = no split.  A tile's K loop is
+// bound by the latency of its transfers, so cutting K over idle CUs shortens it, against a launch and the partial planes: the
+// count up to 16 with the lowest estimate, of pieces that are all on the chip at once, hold a stage at least and have planes that
+// fit kSplitWorkspaceBytes.  (Powers of two by one slab's time whatever the rows, as it was, cost those products 3.9 % on the
+// average over the best count and kernel, this 0.7 %; us, then and now: 1561 x 1280 x 8121, 4 pieces and 3, 75 and 57; 522 x 2053 x
+// 4672, 4 and 3, 29.8 and 23.3; 1062 x 320 x 1984, 1 and 4, 15.4 and 12.1.)
+// gemm16.split_k: 0 = this rule (and K whole on a tile that gemm16.tile asks for), 1 = never, n >= 2 forces n where the shape
+// allows it.
+int splitk_for(int m, int n, int k, const TileTime &time) {
+  const int64_t forced = tunable("gemm16.split_k", 0);
+  if (forced == 1 || (forced == 0 && tunable("gemm16.tile", 0) != 0)) return 1;
+  const int64_t fit = std::min<int64_t>(static_cast<int64_t>(kSplitWorkspaceBytes) / (splitk_plane_floats(m, n) * 4), k / 64);
+  return splitk_pieces(k, 64, forced >= 2 ? std::max<int64_t>(1, std::min<int64_t>(forced, fit)) : time.best(fit));
 }
+inline int splitk_for(int m, int n, int k, bool fused) { return splitk_for(m, n, k, TileTime(m, n, k, fused)); }
 
 // The kernel on v_mfma_f32_16x16x32 with nothing switched off: what a call gets unless, in the measurement build, a sweep
 // knob says otherwise.
@@ -1694,28 +1729,10 @@ inline bool gemm16_default_kernel() {
 #endif
 }
 
-// Microseconds of a product on the 128 x 128 tile with at most a workgroup per CU, by an estimate: its slabs by how A's and
-// B's rows lie (on 16 bytes, on 4, on 2), the K pieces it would take.
+// The estimate in the pieces that it would take, for the choice between it and the few-rows kernel.
 double small_tile_time(int m, int n, int k, bool fused) {
-  const bool on16 = k % 8 == 0 && n % 8 == 0, on4 = k % 2 == 0 && n % 2 == 0;
-  const int splits = splitk_for(m, n, k);
-  const double slabs = static_cast<double>(k) / 32 / splits, planes = splits * (static_cast<double>(m) * n * 4 / (1 << 20));
-  if (fused)   // read off 512 drawn products, gemm16_rows_pays
-    return 6.6 + slabs * (on16 ? 0.193 : k % 2 == 0 || n % 2 == 0 ? 0.26 : 0.43) + (splits > 1 ? 0.25 + 0.5 * splits + 0.68 * planes : 0.0);
-  return 5.5 + slabs * (on16 ? 0.19 : on4 ? 0.24 : 0.33) + (splits > 1 ? 3.0 + planes * 0.65 : 0.0);
-}
-
-// The same for 17 to 64 rows and a B that is new to the caches, from 800 drawn products of that many (8 % rms): the slabs of a
-// CU's workgroups, against B from memory.  K that is no whole number of stages goes to the tile's ragged form.
-double narrow_tile_time(int m, int n, int k, bool fused) {
-  const int align = k % 64 == 0 && n % 8 == 0 ? 0 : k % 8 == 0 && n % 8 == 0 ? 1 : k % 2 == 0 && n % 2 == 0 ? 2 : 3;
-  constexpr double kSlab[] = {0.172, 0.257, 0.272, 0.334}, kMegabyte[] = {0.156, 0.125, 0.134, 0.155};
-  const int splits = splitk_for(m, n, k);
-  const int64_t per_cu = ceil_div(ceil_div(n, 128) * splits, compute_units());
-  const double slabs = static_cast<double>(k) / 32 / splits * kSlab[align] * static_cast<double>(per_cu);
-  const double memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[align], c_mb = static_cast<double>(m) * n * 4e-6;
-  return 5.17 + std::cbrt(slabs * slabs * slabs + memory * memory * memory) + 0.28 * c_mb +
-         (splits > 1 ? 4.0 + 0.38 * splits * c_mb : 0.0);
+  const TileTime time(m, n, k, fused);
+  return time.in(splitk_for(m, n, k, time));
 }
 
 // Whether a product goes to the few-rows kernel, unless a knob asks for one of the tiled kernels.  gemm16.rows: 0 = by
@@ -1725,7 +1742,7 @@ inline bool few_rows(int m, int n, int k, bool fused) {
   return asked != 1 && gemm16_default_kernel() && tunable("gemm16.tile", 0) == 0 && tunable("gemm16.split_k", 0) == 0 &&
          tunable("gemm16.force_simple", 0) == 0 && gemm16_rows_serves(m, n, k) &&
          !(kMeasureBuild && m > 64 && clock_probe(1)) &&   // the probe is the tiled kernels'
-         (asked == 2 || gemm16_rows_pays(m, n, k, fused, small_tile_time, narrow_tile_time));
+         (asked == 2 || gemm16_rows_pays(m, n, k, fused, small_tile_time));
 }
 
 // The workgroup tile of the direct-to-LDS kernels for this shape under the present tunables (256 or 128), or 0 when
@@ -1909,7 +1926,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
     float *partials = nullptr;
     // (fused: the planes hold plain sums; the launch that adds them does the rest.  Us, uncut and cut: 110 x 9523 x 7936 94 -> 73,
     // 2649 x 435 x 6243 67 -> 45, 103 x 5881 x 6427 56 on the few-rows kernel -> 32, 517 x 704 x 2995 21.8 -> 17.7)
-    if (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n) splits = splitk_for(m, n, k);
+    if (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n) splits = splitk_for(m, n, k, Epi != EPI_STORE);
     if (splits > 1) partials = splitk_workspace(st);
     if (!partials) splits = 1;
     if (splits > 1) {
@@ -2031,7 +2048,7 @@ int sarek_hip_gemm16_half_columns(int m, int n, int k) {
 
 int sarek_hip_gemm16_k_splits(int m, int n, int k) {
   if (m >= 1 && n >= 1 && few_rows(m, n, k, false)) return gemm16_rows_k_splits(m, n, k);
-  return gemm16_tile_for(m, n, k) == 128 && sarek_hip_gemm16_half_columns(m, n, k) == 0 ? splitk_for(m, n, k) : 1;
+  return gemm16_tile_for(m, n, k) == 128 && sarek_hip_gemm16_half_columns(m, n, k) == 0 ? splitk_for(m, n, k, false) : 1;
 }
 
 int sarek_hip_gemm_bf16(const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k,

@@ -361,7 +361,7 @@ int launch(const Call &q, const Shape &s) {
   // counts take to come together, the longer with more rows (us, rowsum_fold_kernel's launch and here, K of 512: 4 x 512 10.5 and
   // 7.3, 4 x 16384 9.7 and 8.2, 4 x 32768 10.4 and 11.9, 128 x 2048 11.4 and 11.3, 128 x 8192 11.8 and 12.8, 2000 x 512 12.3 and
   // 12.2, 1000 x 1024 12.3 and 12.8).  gemm16.fold: 0 = this rule, 1 = never, 2 = always.
-  const int64_t asked = tunable("gemm16.fold", 0);
+  const int64_t asked = Fused ? tunable("gemm16.fold", 0) : 1;
   if (rs_planes && s.row_tiles <= kFoldTickets && asked != 1 &&
       (asked == 2 || s.tiles <= (s.mt <= 2 ? 128 : 64) || s.tiles * s.col_tiles <= 512))
     fold.tickets = fold_tickets(block);
@@ -425,22 +425,22 @@ double narrow_time(const Shape &s, int n, int k, int splits) {
 //   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
 //   48 x 4096 x 256 6.2 / 6.1, 48 x 4096 x 1024 10.2 / 9.4, 48 x 40000 x 1024 23.0 / 26.4, 48 x 40001 x 1024 35.3 / 33.4
 //   64 x 4096 x 256 6.4 / 7.2, 64 x 4096 x 1024 10.5 / 10.5, 64 x 4096 x 4096 17.3 / 15.6, 64 x 40001 x 1024 36.3 / 37.0
-// and so does what the estimates of both kernels (narrow_other: the tile's) put 5 % apart the other way, B being new to the
+// and so does what the estimates of both kernels (other: the tile's) put 8 % apart the other way, of up to 8 column tiles 16 %, B being new to the
 // caches as in a program's loop over its weights (again and again the same B favours the tile more): 33 to 64 rows against one
-// to two hundred column tiles most of all (us, tile / here): 64 x 29028 x 2725 45.2 / 51.8, 51 x 7969 x 5857 29.5 / 34.4.  Of
-// 900 products drawn afresh 85 were more than 5 % slower here than there without the estimates and 43 are with them; nine are
-// that much slower than they were, by at most 15 % (profiles/gemm16_rows_vs_tile.txt).  An odd N of
-// few column tiles stays here whatever they say (49 x 255 x 4129 13.5 / 15.1, 64 x 1001 x 1001 15.7 / 11.4), 17 to 32 rows
+// to two hundred column tiles most of all (us, tile / here): 64 x 29028 x 2725 45.2 / 51.8, 51 x 7969 x 5857 29.5 / 34.4,
+// 63 x 17239 x 320 7.6 / 9.5, 42 x 17830 x 3328 32.4 / 40.0.  Of 900 products drawn afresh 85 were more than 5 % slower here than
+// there without estimates and 43 with them (profiles/gemm16_rows_vs_tile.txt); the tile's in any count of pieces put 10 in 167
+// right and two wrong.  An odd N of
+// up to 8 column tiles stays here whatever they say (49 x 255 x 4129 13.5 / 15.1, 64 x 1001 x 1001 15.7 / 11.4), 17 to 32 rows
 // against up to 96 column tiles do (one of 576 more than 10 % slower), and so does a product whose pieces gemm16.rows_splits sets.
 // Beyond 64 rows, and with the fused epilogue at any number, where its tiles fit the CUs in one round (882 x 2401 x 4259,
 // 266 tiles: 50 us on the other tile, 108 here), at least half of the waves have a step (in tiles of 64 rows some wave has
 // two: 256 x 1280 x 191 6.8 / 8.4, 723 x 1702 x 256 7.2 / 7.9, as 21 of 118 drawn products, all but 3 of them so short), and its
-// time is below the 128 x 128 tile's by both estimates: a step costs by how A's and B's rows lie.  The plain ones were read
-// off 50 drawn products (up to 20 % and a microsecond apart from them, the better kernel taken on 45, at most 8 % lost on the
-// others), the fused ones off 512 of both kernels (11 % rms; 8 of them more than 4 % slower than when the tile had
-// no pieces of K for them, at most 10 %, and all together 7 % faster): 419 x 1472 x 2504 25.5 on the tile, 17.4 here,
-// 180 x 256 x 2240 10.0, 13.9.  `other`: what the tiled kernel is estimated at.
-bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other, Gemm16Estimate narrow_other) {
+// time is below the 128 x 128 tile's by both estimates: a step costs by how A's and B's rows lie.  They were read off 292 plain
+// and 704 fused drawn products run on both (7 % rms, the tile's 8 and 10): 139 x 2432 x 1416 12.0 on the tile, 9.5 here,
+// 114 x 5824 x 2687 15.9, 27.2, fused 419 x 1472 x 2504 25.5, 17.4, 180 x 256 x 2240 10.0, 13.9; of those of more than 64 rows 9 in
+// 820 are more than 5 % slower by them than by the rules before.  `other`: what the tiled kernel is estimated at.
+bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other) {
   const Shape s = shape_of(m, n, k, fused);
   if (m <= kTileRows && !fused) {
     const bool odd = n % 2 != 0, one_round = s.col_tiles <= compute_units();
@@ -456,23 +456,21 @@ bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other, Gem
     if (!here) return false;
   }
   if (m > 16 && m <= kTileRows && s.col_tiles > (s.mt == 2 ? 96 : n % 2 != 0 ? 8 : 0) && tunable("gemm16.rows_splits", 0) == 0 &&
-      narrow_time(s, n, k, rows_splits_for(s, n, k)) >= 1.05 * narrow_other(m, n, k, fused))
+      narrow_time(s, n, k, rows_splits_for(s, n, k)) >= (s.col_tiles > 8 ? 1.08 : 1.16) * other(m, n, k, fused))
     return false;
   if (m <= kTileRows && !fused) return true;
   if (s.tiles > compute_units() || 2 * s.steps < kWaves || (s.mt == 4 && s.steps <= kWaves)) return false;
   const int splits = rows_splits_for(s, n, k);
+  struct Fit { double step[3], memory, base, rows, sums, piece, plane; };
+  constexpr Fit kPlain = {{0.0475, 0.0499, 0.0789}, 0.11, 2.74, 0.792, 0.94, 0.281, 0.241};
+  constexpr Fit kFused = {{0.0492, 0.0499, 0.0819}, 0.156, 4.37, 1.17, 0.55, 0.237, 0.318};
+  const Fit &f = fused ? kFused : kPlain;
+  const int align = k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2;
   const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
-  const double steps = rounds * s.steps / splits * s.mt, planes = splits > 1 ? 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0;
-  const bool on16 = k % 8 == 0 && n % 8 == 0;
-  double here;
-  if (fused) {
-    const double step = k % 2 == 0 ? 0.064 : n % 2 == 0 ? 0.098 : 0.136;
-    here = 2.95 + 1.4 * s.mt + steps * step + (splits > 1 ? 1.7 + 0.31 * splits + 0.07 * planes : 0.0);
-  } else {
-    const double step = on16 ? 0.055 : k % 2 == 0 && n % 2 == 0 ? 0.07 : 0.12;
-    here = (on16 ? 6.0 : 4.5) + steps * step + (splits > 1 ? 2.5 + 0.15 * splits + planes : 0.0);
-  }
-  return here < other(m, n, k, fused);
+  const double steps = rounds * s.steps / splits * s.mt * f.step[align], memory = static_cast<double>(k) * n * 2e-6 * f.memory;
+  const double here = f.base + f.rows * s.mt + std::sqrt(steps * steps + memory * memory) +
+                      (splits > 1 ? f.sums + splits * (f.piece + f.plane * 1e-6 * static_cast<double>(s.plane)) : 0.0);
+  return here * (s.tiles > 192 ? 1.06 : 1.0) < other(m, n, k, fused);   // (1.06: 1728 x 1034 x 1664 15.8 on the tile, 18.2 here)
 }
 
 int gemm16_rows_k_splits(int m, int n, int k) { return rows_splits_for(shape_of(m, n, k, false), n, k); }

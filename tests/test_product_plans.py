@@ -48,6 +48,22 @@ def test_16_bit_products_of_few_rows_go_where_they_are_faster(hip, m, n, k, kern
     assert hip.gemm16_tile(m, n, k) == kernel
 
 
+@pytest.mark.parametrize("m,n,k,pieces", [(1561, 1280, 8121, 3), (522, 2053, 4672, 3), (114, 5824, 2687, 4), (110, 2048, 192, 1),
+                                          (4096, 2048, 1000, 1), (128, 30000, 6000, 1), (1920, 4000, 8192, 1)])
+def test_pieces_of_k_on_the_small_tile(hip, knobs, m, n, k, pieces):
+    """The count with the lowest estimate: workgroups that fit the CUs twice over, planes that fit the workspace, a stage of 64 each;
+    K stays whole on a tile that is asked for by name."""
+    knobs("gemm16.rows", 1)
+    tiles, seen = -(-m // 128) * -(-n // 128), hip.gemm16_k_splits(m, n, k)
+    assert seen == pieces
+    for longer in (k, 2 * k, 3 * k + 1, 8 * k):
+        s = hip.gemm16_k_splits(m, n, longer)
+        assert s == 1 or (s <= 16 and tiles * s <= 512 and 4 * m * n * s <= 64 << 20 and longer // s >= 64)
+    if hip.gemm16_tile(m, n, k) == 128:
+        knobs("gemm16.tile", 128)
+        assert hip.gemm16_k_splits(m, n, k) == 1
+
+
 @pytest.mark.parametrize("m,n,k,columns", [
     (2048, 8448, 4096, 8192), (2048, 8448, 128, 8192), (2048, 8448, 127, 8448), (2048, 50257, 1024, 49152), (2048, 12288, 4096, 12288),
     (7232, 13568, 82, 13568), (7232, 13568, 767, 13568), (7232, 13568, 768, 52 * 256), (3712, 39176, 768, 39176),
