@@ -1655,21 +1655,21 @@ __global__ __launch_bounds__(256) void gemm16_last_column_kernel(const uint16_t 
 
 // Microseconds of a product on the 128 x 128 tile, plain or fused, by an estimate read off 730 plain and 520 fused products drawn
 // over 17 to 8192 rows, their operands new to the caches, each in 1 to 16 pieces of K (8 and 10 % rms): a slab of 32 of K by how
-// A's and B's rows lie (on 16 bytes, on 4, on 2), a second workgroup of a CU beside the first; the operands from memory; C; and for
+// A's and B's rows lie (on 16 bytes, both on 4, one, none), a second workgroup of a CU beside the first; the operands from memory; C; and for
 // pieces the launch that adds them, and their planes.
 struct TileTime {
   int64_t tiles, stages, cus;
   double stage, second, memory2, whole, launch, piece;
 
   TileTime(int m, int n, int k, bool fused) {
-    struct Fit { double stage[3], second, memory, base, c, launch, piece, plane; };
-    constexpr Fit kPlain = {{0.336, 0.414, 0.498}, 1.75, 0.116, 4.34, 0.171, 2.05, 0.213, 0.312};
-    constexpr Fit kFused = {{0.324, 0.418, 0.498}, 1.54, 0.213, 6.68, 0.272, 0.49, 0.55, 0.318};
+    struct Fit { double stage[4], second, memory, base, c, launch, piece, plane; };
+    constexpr Fit kPlain = {{0.335, 0.412, 0.485, 0.605}, 1.77, 0.117, 4.39, 0.163, 2.4, 0.068, 0.317};
+    constexpr Fit kFused = {{0.327, 0.423, 0.484, 0.632}, 1.57, 0.194, 6.65, 0.284, 1.29, 0.279, 0.303};
     const Fit &f = fused ? kFused : kPlain;
     tiles = ceil_div(m, 128) * ceil_div(n, 128);
     stages = ceil_div(k, 64);
     cus = compute_units();
-    stage = f.stage[k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2];
+    stage = f.stage[k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 + n % 2 + 1];
     second = f.second;
     const double memory = (static_cast<double>(m) * k + static_cast<double>(k) * n) * 2e-6 * f.memory, c_mb = static_cast<double>(m) * n * 4e-6;
     memory2 = memory * memory;

@@ -408,11 +408,11 @@ bool gemm16_rows_serves(int m, int n, int k) {
 // most workgroups by how A's and B's rows lie, against B from memory (whose stream the registers of more row blocks leave
 // fewer loads in flight), and the sums.
 double narrow_time(const Shape &s, int n, int k, int splits) {
-  const int align = k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2;
+  const int align = k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2, b_align = n % 8 == 0 ? 0 : 1 + n % 2;
   constexpr double kStep[] = {0.0125, 0.0147, 0.0288}, kMegabyte[] = {0.124, 0.147, 0.164};
   const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
   const double steps = rounds * s.steps / splits * kStep[align] * (4.0 + s.mt);
-  const double memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[align] * (1 + 0.182 * s.mt);
+  const double memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[b_align] * (1 + 0.182 * s.mt);
   return 2.94 + 0.97 * s.mt * rounds + std::cbrt(steps * steps * steps + memory * memory * memory) +
          (splits > 1 ? 1.17 + 0.31 * splits : 0.0);
 }
@@ -425,7 +425,7 @@ double narrow_time(const Shape &s, int n, int k, int splits) {
 //   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
 //   48 x 4096 x 256 6.2 / 6.1, 48 x 4096 x 1024 10.2 / 9.4, 48 x 40000 x 1024 23.0 / 26.4, 48 x 40001 x 1024 35.3 / 33.4
 //   64 x 4096 x 256 6.4 / 7.2, 64 x 4096 x 1024 10.5 / 10.5, 64 x 4096 x 4096 17.3 / 15.6, 64 x 40001 x 1024 36.3 / 37.0
-// and so does what the estimates of both kernels (other: the tile's) put 8 % apart the other way, of up to 8 column tiles 16 %, B being new to the
+// and so does what the estimates of both kernels (other: the tile's) put 4 % apart the other way, of up to 8 column tiles 25 %, B being new to the
 // caches as in a program's loop over its weights (again and again the same B favours the tile more): 33 to 64 rows against one
 // to two hundred column tiles most of all (us, tile / here): 64 x 29028 x 2725 45.2 / 51.8, 51 x 7969 x 5857 29.5 / 34.4,
 // 63 x 17239 x 320 7.6 / 9.5, 42 x 17830 x 3328 32.4 / 40.0.  Of 900 products drawn afresh 85 were more than 5 % slower here than
@@ -437,7 +437,7 @@ double narrow_time(const Shape &s, int n, int k, int splits) {
 // 266 tiles: 50 us on the other tile, 108 here), at least half of the waves have a step (in tiles of 64 rows some wave has
 // two: 256 x 1280 x 191 6.8 / 8.4, 723 x 1702 x 256 7.2 / 7.9, as 21 of 118 drawn products, all but 3 of them so short), and its
 // time is below the 128 x 128 tile's by both estimates: a step costs by how A's and B's rows lie.  They were read off 292 plain
-// and 704 fused drawn products run on both (7 % rms, the tile's 8 and 10): 139 x 2432 x 1416 12.0 on the tile, 9.5 here,
+// and 704 fused drawn products run on both (5 % rms, the tile's 8 and 9): 139 x 2432 x 1416 12.0 on the tile, 9.5 here,
 // 114 x 5824 x 2687 15.9, 27.2, fused 419 x 1472 x 2504 25.5, 17.4, 180 x 256 x 2240 10.0, 13.9; of those of more than 64 rows 9 in
 // 820 are more than 5 % slower by them than by the rules before.  `other`: what the tiled kernel is estimated at.
 bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other) {
@@ -456,18 +456,18 @@ bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other) {
     if (!here) return false;
   }
   if (m > 16 && m <= kTileRows && s.col_tiles > (s.mt == 2 ? 96 : n % 2 != 0 ? 8 : 0) && tunable("gemm16.rows_splits", 0) == 0 &&
-      narrow_time(s, n, k, rows_splits_for(s, n, k)) >= (s.col_tiles > 8 ? 1.08 : 1.16) * other(m, n, k, fused))
+      narrow_time(s, n, k, rows_splits_for(s, n, k)) >= (s.col_tiles > 8 ? 1.04 : 1.25) * other(m, n, k, fused))
     return false;
   if (m <= kTileRows && !fused) return true;
   if (s.tiles > compute_units() || 2 * s.steps < kWaves || (s.mt == 4 && s.steps <= kWaves)) return false;
   const int splits = rows_splits_for(s, n, k);
-  struct Fit { double step[3], memory, base, rows, sums, piece, plane; };
-  constexpr Fit kPlain = {{0.0475, 0.0499, 0.0789}, 0.11, 2.74, 0.792, 0.94, 0.281, 0.241};
-  constexpr Fit kFused = {{0.0492, 0.0499, 0.0819}, 0.156, 4.37, 1.17, 0.55, 0.237, 0.318};
+  struct Fit { double step[5], memory[2], base, rows, sums, piece, plane; };
+  constexpr Fit kPlain = {{0.0479, 0.0501, 0.0657, 0.0895, 0.105}, {0.091, 0.132}, 2.34, 0.878, 1.01, 0.285, 0.246};
+  constexpr Fit kFused = {{0.0489, 0.0487, 0.0638, 0.0884, 0.11}, {0.133, 0.193}, 4.4, 1.186, 0.51, 0.228, 0.335};
   const Fit &f = fused ? kFused : kPlain;
-  const int align = k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2;
+  const int align = k % 8 == 0 && n % 8 == 0 ? 0 : 1 + 2 * (k % 2) + n % 2;
   const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
-  const double steps = rounds * s.steps / splits * s.mt * f.step[align], memory = static_cast<double>(k) * n * 2e-6 * f.memory;
+  const double steps = rounds * s.steps / splits * s.mt * f.step[align], memory = static_cast<double>(k) * n * 2e-6 * f.memory[n % 8 != 0];
   const double here = f.base + f.rows * s.mt + std::sqrt(steps * steps + memory * memory) +
                       (splits > 1 ? f.sums + splits * (f.piece + f.plane * 1e-6 * static_cast<double>(s.plane)) : 0.0);
   return here * (s.tiles > 192 ? 1.06 : 1.0) < other(m, n, k, fused);   // (1.06: 1728 x 1034 x 1664 15.8 on the tile, 18.2 here)

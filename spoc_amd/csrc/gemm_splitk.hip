@@ -11,14 +11,43 @@
 namespace sarek_hip {
 namespace {
 
+// The sum of four columns' `splits` partial sums, plane 0 first, up to nine of them asked for at once: one after the other, each
+// waited a trip to the caches for the one before (us, with the products: 161 x 256 x 7182, 13 pieces, PLAIN13; 63 x 1130 x 7104,
+// PLAIN8; fused 98 x 576 x 2432 FUSED).
+template <int Count, class Vec>
+__device__ __forceinline__ void add_next(f32x4_t &acc, const float *__restrict__ p, int64_t plane) {
+  f32x4_t v[Count];
+#pragma unroll
+  for (int u = 0; u < Count; ++u) v[u] = *reinterpret_cast<const Vec *>(p + u * plane);
+#pragma unroll
+  for (int u = 0; u < Count; ++u) acc += v[u];
+}
+template <class Vec>
+__device__ __forceinline__ f32x4_t add_planes(const float *__restrict__ p, int64_t plane, int splits) {
+  f32x4_t acc = *reinterpret_cast<const Vec *>(p);
+  for (int s = 1; s < splits; s += 8) {
+    const float *next = p + s * plane;
+    switch (min(splits - s, 8)) {
+      case 1: add_next<1, Vec>(acc, next, plane); break;
+      case 2: add_next<2, Vec>(acc, next, plane); break;
+      case 3: add_next<3, Vec>(acc, next, plane); break;
+      case 4: add_next<4, Vec>(acc, next, plane); break;
+      case 5: add_next<5, Vec>(acc, next, plane); break;
+      case 6: add_next<6, Vec>(acc, next, plane); break;
+      case 7: add_next<7, Vec>(acc, next, plane); break;
+      default: add_next<8, Vec>(acc, next, plane);
+    }
+  }
+  return acc;
+}
+
 // Adds the `splits` partial planes into C, plane 0 first: a fixed order, so the result does not depend on which
 // workgroup finished when.  C is 16-byte aligned (the callers' condition).
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ partials, float *__restrict__ C,
                                                             int64_t mn, int64_t plane, int splits) {
   const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
   if (i >= mn) return;
-  f32x4_t acc = *reinterpret_cast<const f32x4_t *>(partials + i);
-  for (int s = 1; s < splits; ++s) acc += *reinterpret_cast<const f32x4_t *>(partials + s * plane + i);
+  const f32x4_t acc = add_planes<f32x4_t>(partials + i, plane, splits);
   if (i + 4 <= mn) {
     *reinterpret_cast<f32x4_t *>(C + i) = acc;
   } else {
@@ -42,8 +71,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_fused_kernel(const float *_
   double sum = 0.0;
   for (int c = (Waves == 4 ? static_cast<int>(threadIdx.x) : lane) * 4; c < n; c += Waves * 256) {
     if (c + 4 <= n) {
-      f32x4_t acc = *reinterpret_cast<const f32x4_u *>(p + c);
-      for (int s = 1; s < splits; ++s) acc += *reinterpret_cast<const f32x4_u *>(p + s * plane + c);
+      f32x4_t acc = add_planes<f32x4_u>(p + c, plane, splits);
       const f32x4_t b = *reinterpret_cast<const f32x4_u *>(bias + c);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
