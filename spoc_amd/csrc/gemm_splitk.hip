@@ -12,8 +12,8 @@ namespace sarek_hip {
 namespace {
 
 // The sum of four columns' `splits` partial sums, plane 0 first, up to nine of them asked for at once: one after the other, each
-// waited a trip to the caches for the one before (us, with the products: 161 x 256 x 7182, 13 pieces, PLAIN13; 63 x 1130 x 7104,
-// PLAIN8; fused 98 x 576 x 2432 FUSED).
+// waited a trip to the caches for the one before (us, with the products: 161 x 256 x 7182, 13 pieces, 14.2 and 12.4; 63 x 1130 x 7104,
+// 14.4, 12.6; fused 98 x 576 x 2432 13.1, 11.4).
 template <int Count, class Vec>
 __device__ __forceinline__ void add_next(f32x4_t &acc, const float *__restrict__ p, int64_t plane) {
   f32x4_t v[Count];
