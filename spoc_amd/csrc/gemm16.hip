@@ -1229,8 +1229,12 @@ __global__ __launch_bounds__(256) void gemm16_m16w4_kernel(const uint16_t *__res
 // rows of the large tile, so the same XOR swizzle keeps the transposing reads free of bank conflicts.  A slab is 16 MFMAs:
 // rows 0-31 of the wave tile before the barrier, rows 32-63 after it with the next slab's 12 fragment reads (and, every
 // other slab, the 4 transfers of an A stage) behind them; fragments are double-buffered by slab parity.
-template <bool Bf16, int Epi, bool Ragged = false>
-__global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
+// Chunked, for K in pieces: an element is the sum of sums of two slabs, kept apart in 64 registers more (two waves to a SIMD have
+// 256 each), so that a piece is as exact as the few-rows kernel's eight waves make it: rms error against float64 over the largest
+// element, 320 x 2880 x 2793, there 2.3e-8, here in one chain 4.1e-8, in chunks 2.1e-8.  The additions hide behind the MFMAs: 704 x
+// 1728 x 4591 23.2 us without, 23.7 in chunks of four slabs, 24.0 of two.
+template <bool Bf16, int Epi, bool Ragged = false, bool Chunked = false>
+__global__ __launch_bounds__(256, Chunked ? 2 : 1) void gemm16_m16_small_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                                float *__restrict__ C, const float *__restrict__ bias,
                                                                float *__restrict__ rowsum, int M, int N, int K, int tiles_m,
                                                                int tiles_n, int xcd_remap, unsigned long long *probe,
@@ -1245,6 +1249,8 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
   constexpr int NWAVES = 4, WN = 2;
   constexpr int DA = A_BYTES_S / 1024 / NWAVES, DB = B_BYTES_S / 1024 / NWAVES;
   constexpr int P = lcm_int(NB, RA * NA);
+  constexpr int kChunk = 2;   // slabs
+  static_assert(P % kChunk == 0, "a chunk ends where a turn of the rings does");
   static_assert(P % 2 == 0, "the fragment buffers alternate by slab parity");
   static_assert(2 * (NA * A_BYTES_S + NB * B_BYTES_S) <= 160 * 1024, "two workgroups per CU");
 
@@ -1308,7 +1314,13 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
-
+  f32x4_t sum[Chunked ? 4 : 1][4];   // of the chunks before this one
+  if constexpr (Chunked) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum[i][j] = acc[i][j];
+  }
   const int a_row = wm * 64 + l16;
   int a_addr0 = a_row * A_ROW + ((g ^ a_swz(a_row)) << 4);
   const int b_r = l16 >> 2;
@@ -1354,13 +1366,15 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
       bf[j] = u32x4{lo.x, lo.y, hi.x, hi.y};
     }
   };
-  // MFMAs First .. First+Count-1 of a slab's 16, in the order (row tile i, column tile j)
-  auto mfma_range = [&](auto first_c, auto count_c, u32x4 (&af)[4], u32x4 (&bf)[4]) {
+  // MFMAs First .. First+Count-1 of a slab's 16, in the order (row tile i, column tile j); `fresh`: the first slab of a chunk
+  auto mfma_range = [&](auto first_c, auto count_c, auto fresh_c, u32x4 (&af)[4], u32x4 (&bf)[4]) {
     constexpr int First = decltype(first_c)::value, Count = decltype(count_c)::value;
+    constexpr bool Fresh = decltype(fresh_c)::value;
     [&]<int... Ts>(std::integer_sequence<int, Ts...>) {
       (([&] {
          constexpr int i = (First + Ts) / 4, j = i % 2 ? 3 - (First + Ts) % 4 : (First + Ts) % 4;
-         acc[i][j] = mfma16<Bf16>(af[i], bf[j], acc[i][j]);
+         if constexpr (Fresh) sum[i][j] += acc[i][j];
+         acc[i][j] = mfma16<Bf16>(af[i], bf[j], Fresh ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[i][j]);
        }()),
        ...);
     }(std::make_integer_sequence<int, Count>{});
@@ -1395,9 +1409,10 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     constexpr int ia = (I / RA) % NA, ibp = (I + NB - 1) % NB;
     constexpr int ian = (In / RA) % NA, ibn = In % NB;
     constexpr int ksn = In % RA;
+    constexpr std::bool_constant<Chunked && I % kChunk == 0> fresh;
     asm volatile("" : "+v"(a_addr0), "+v"(b_addr0));
     issue_b(std::integral_constant<int, -1>{}, lds_ring<40 + ibp, B_BYTES_S>);
-    mfma_range(std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{}, af[I & 1], bf[I & 1]);
+    mfma_range(std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{}, fresh, af[I & 1], bf[I & 1]);
     spread(std::integral_constant<int, DB>{}, std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{});
     __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(dma_allowed_in_flight(I, RA, NA, NB, DA, DB)));
     barrier_no_fence();
@@ -1409,7 +1424,7 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     load_a1(lds_ring<30 + ian, A_BYTES_S>, ksn, 1, af[In & 1][1]);
     load_a1(lds_ring<30 + ian, A_BYTES_S>, ksn, 2, af[In & 1][2]);
     load_a1(lds_ring<30 + ian, A_BYTES_S>, ksn, 3, af[In & 1][3]);
-    mfma_range(std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{}, af[I & 1], bf[I & 1]);
+    mfma_range(std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{}, fresh, af[I & 1], bf[I & 1]);
     spread(std::integral_constant<int, (I % RA == RA - 1) ? DA : 0>{}, std::integral_constant<int, 12>{},
            std::integral_constant<int, 8>{});
   };
@@ -1443,6 +1458,12 @@ __global__ __launch_bounds__(256) void gemm16_m16_small_kernel(const uint16_t *_
     ((full + Is < nslabs ? slab(std::integral_constant<int, Is>{}, full + Is) : (void)0), ...);
   }(std::make_integer_sequence<int, P - 1>{});
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // the tail's empty transfers, before the LDS is released
+  if constexpr (Chunked) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = sum[i][j] + acc[i][j];
+  }
   float *scratch = reinterpret_cast<float *>(lds_ring<30, A_BYTES_S>);
   const bool add_last = Ragged && (N & 1) != 0 && n0 + SBN >= N && k0 + k_len == K;
   if (add_last) last_products<Bf16, SBM>(A, B, M, N, K, ld, m0, k0, scratch);
@@ -1680,7 +1701,9 @@ struct TileTime {
   double in(int64_t splits) const {
     const double t = static_cast<double>(ceil_div(stages, splits)) * stage *
                      (tiles * splits <= cus ? 1.0 : second * static_cast<double>(ceil_div(tiles * splits, 2 * cus)));
-    return whole + std::sqrt(t * t + memory2) + (splits > 1 ? launch + static_cast<double>(splits) * piece : 0.0);
+    const double us = whole + std::sqrt(t * t + memory2);
+    // (what issuing two launches takes the host: 39 x 1250 x 896 8.3 on the few-rows kernel, 8.1 to 10.2 here in pieces)
+    return splits > 1 ? std::max(9.5, us + launch + static_cast<double>(splits) * piece) : us;
   }
   // The count of at most `most` with the lowest estimate, if that is 3 % below the uncut one: about the root of what a piece saves
   // over what it costs, with a workgroup per CU and with two.
@@ -1730,19 +1753,23 @@ inline bool gemm16_default_kernel() {
 }
 
 // The estimate in the pieces that it would take, for the choice between it and the few-rows kernel.
-double small_tile_time(int m, int n, int k, bool fused) {
+Gemm16Time small_tile_time(int m, int n, int k, bool fused) {
   const TileTime time(m, n, k, fused);
-  return time.in(splitk_for(m, n, k, time));
+  const int splits = splitk_for(m, n, k, time);
+  return {time.in(splits), splits};
 }
 
 // Whether a product goes to the few-rows kernel, unless a knob asks for one of the tiled kernels.  gemm16.rows: 0 = by
 // size, 1 = never, 2 = wherever it can.
+inline int64_t few_rows_asked(int m, int n, int k) {
+  const bool can = gemm16_default_kernel() && tunable("gemm16.tile", 0) == 0 && tunable("gemm16.split_k", 0) == 0 &&
+                   tunable("gemm16.force_simple", 0) == 0 && gemm16_rows_serves(m, n, k) &&
+                   !(kMeasureBuild && m > 64 && clock_probe(1));   // the probe is the tiled kernels'
+  return can ? tunable("gemm16.rows", 0) : 1;
+}
 inline bool few_rows(int m, int n, int k, bool fused) {
-  const int64_t asked = tunable("gemm16.rows", 0);
-  return asked != 1 && gemm16_default_kernel() && tunable("gemm16.tile", 0) == 0 && tunable("gemm16.split_k", 0) == 0 &&
-         tunable("gemm16.force_simple", 0) == 0 && gemm16_rows_serves(m, n, k) &&
-         !(kMeasureBuild && m > 64 && clock_probe(1)) &&   // the probe is the tiled kernels'
-         (asked == 2 || gemm16_rows_pays(m, n, k, fused, small_tile_time));
+  const int64_t asked = few_rows_asked(m, n, k);
+  return asked != 1 && (asked == 2 || gemm16_rows_pays(m, n, k, fused, small_tile_time));
 }
 
 // The workgroup tile of the direct-to-LDS kernels for this shape under the present tunables (256 or 128), or 0 when
@@ -1926,16 +1953,21 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
     float *partials = nullptr;
     // (fused: the planes hold plain sums; the launch that adds them does the rest.  Us, uncut and cut: 110 x 9523 x 7936 94 -> 73,
     // 2649 x 435 x 6243 67 -> 45, 103 x 5881 x 6427 56 on the few-rows kernel -> 32, 517 x 704 x 2995 21.8 -> 17.7)
-    if (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n) splits = splitk_for(m, n, k, Epi != EPI_STORE);
-    if (splits > 1) partials = splitk_workspace(st);
+    splits = splitk_for(m, n, k, Epi != EPI_STORE);
+    if (splits > 1 && (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n)) partials = splitk_workspace(st);
+    // (no block under capture and past 16 streams: a product that is on this tile for its pieces is not to run whole on it)
+    if (splits > 1 && !partials && few_rows_asked(m, n, k) == 0 && gemm16_rows_more_exact(m, n, k, Epi != EPI_STORE)) {
+      if constexpr (Epi == EPI_STORE) return launch_gemm16_rows(Bf16, a, b, c, m, n, k, st);
+      else return launch_gemm16_rows_fused(a, b, bias, c, rowsum, m, n, k, st);
+    }
     if (!partials) splits = 1;
     if (splits > 1) {
       const int chunk = splitk_chunk(k, 64, splits);
       if (ragged)
-        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, true>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
+        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, true, true>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
                            nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, nullptr);
       else
-        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, false>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
+        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, false, true>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
                            nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, nullptr);
       rc = check_launch("gemm16 kernel launch");
       if (rc != SAREK_HIP_OK) return rc;

@@ -417,6 +417,34 @@ double narrow_time(const Shape &s, int n, int k, int splits) {
          (splits > 1 ? 1.17 + 0.31 * splits : 0.0);
 }
 
+// An element is one sum on the 128 x 128 tile with K whole and eight or more here, and its error there up to 2.8 times as large
+// (1280 x 1134 x 566 1.8); in pieces the tile's sums are chunked and as exact as here, up to 2048 of K (37 x 9856 x 7744, 3 pieces, 1.12).
+bool less_exact(int k, int tile_splits) { return tile_splits == 1 || k > 2048 * static_cast<int64_t>(tile_splits); }
+
+// So a product does not go there for a few per cent where it would be less exact, or cannot be cut: only where coarser estimates,
+// that put this kernel up to 2 us too low, have the tile, in 1 to 16 pieces of a plain product, ahead as well.
+bool whole_on_the_tile(const Shape &s, int m, int n, int k, bool fused) {
+  const bool on16 = k % 8 == 0 && n % 8 == 0, on4 = k % 2 == 0 && n % 2 == 0, narrow = m <= kTileRows && !fused;
+  const int align = k % 64 == 0 && n % 8 == 0 ? 0 : on16 ? 1 : on4 ? 2 : 3, cus = compute_units();
+  constexpr double kSlab[] = {0.19, 0.19, 0.24, 0.33}, kNarrowSlab[] = {0.172, 0.257, 0.272, 0.334}, kMegabyte[] = {0.156, 0.125, 0.134, 0.155};
+  const int64_t tiles = static_cast<int64_t>((m + 127) / 128) * s.col_tiles;
+  const double c_mb = static_cast<double>(m) * n * 4e-6, memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[align];
+  double tile = 1e300;
+  for (int64_t pieces = 1; pieces == 1 || (!fused && pieces <= 16 && tiles * pieces <= 2 * cus && k / pieces >= 256); pieces *= 2) {
+    const double slabs = k / 32.0 / static_cast<double>(pieces);
+    const double chain = slabs * kNarrowSlab[align] * static_cast<double>((tiles * pieces + cus - 1) / cus);
+    tile = std::min(tile, narrow ? 5.17 + std::cbrt(chain * chain * chain + memory * memory * memory) + 0.28 * c_mb +
+                                       (pieces > 1 ? 4.0 + 0.38 * static_cast<double>(pieces) * c_mb : 0.0)
+                                 : 5.5 + slabs * kSlab[align] + (pieces > 1 ? 3.0 + 0.62 * static_cast<double>(pieces) * c_mb : 0.0));
+  }
+  const int splits = rows_splits_for(s, n, k);
+  if (narrow) return narrow_time(s, n, k, splits) >= 1.05 * tile;
+  const double rounds = static_cast<double>((s.tiles * splits + cus - 1) / cus);
+  const double here = (on16 ? 6.0 : 4.5) + rounds * s.steps / splits * (on16 ? 0.055 : on4 ? 0.07 : 0.12) * s.mt +
+                      (splits > 1 ? 2.5 + 0.15 * splits + 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0);
+  return here >= tile;
+}
+
 // Whether it should.  Up to 16 rows always, but for more than 128 MiB of B in one piece of K whose rows, of an even N, share
 // lines: there the tile's transfers into LDS come in better (16 x 30000 x 4096 43.2 on the tile, 49.9 here; elsewhere the tile was
 // the faster by 4 % on 4 of 400 drawn products, operands new to the caches, this kernel by a quarter on average).  To 64 a workgroup's
@@ -456,8 +484,8 @@ bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other) {
     if (!here) return false;
   }
   if (m > 16 && m <= kTileRows && s.col_tiles > (s.mt == 2 ? 96 : n % 2 != 0 ? 8 : 0) && tunable("gemm16.rows_splits", 0) == 0 &&
-      narrow_time(s, n, k, rows_splits_for(s, n, k)) >= (s.col_tiles > 8 ? 1.04 : 1.25) * other(m, n, k, fused))
-    return false;
+      narrow_time(s, n, k, rows_splits_for(s, n, k)) >= (s.col_tiles > 8 ? 1.04 : 1.25) * other(m, n, k, fused).us)
+    return less_exact(k, other(m, n, k, fused).splits) && !whole_on_the_tile(s, m, n, k, fused);
   if (m <= kTileRows && !fused) return true;
   if (s.tiles > compute_units() || 2 * s.steps < kWaves || (s.mt == 4 && s.steps <= kWaves)) return false;
   const int splits = rows_splits_for(s, n, k);
@@ -470,7 +498,14 @@ bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other) {
   const double steps = rounds * s.steps / splits * s.mt * f.step[align], memory = static_cast<double>(k) * n * 2e-6 * f.memory[n % 8 != 0];
   const double here = f.base + f.rows * s.mt + std::sqrt(steps * steps + memory * memory) +
                       (splits > 1 ? f.sums + splits * (f.piece + f.plane * 1e-6 * static_cast<double>(s.plane)) : 0.0);
-  return here * (s.tiles > 192 ? 1.06 : 1.0) < other(m, n, k, fused);   // (1.06: 1728 x 1034 x 1664 15.8 on the tile, 18.2 here)
+  const Gemm16Time tile = other(m, n, k, fused);   // (1.06: 1728 x 1034 x 1664 15.8 on the tile, 18.2 here)
+  return here * (s.tiles > 192 ? 1.06 : 1.0) < tile.us || (less_exact(k, tile.splits) && !whole_on_the_tile(s, m, n, k, fused));
+}
+
+bool gemm16_rows_more_exact(int m, int n, int k, bool fused) {
+  const Shape s = shape_of(m, n, k, fused);
+  if (m <= kTileRows && !fused ? s.col_tiles > compute_units() : s.tiles > compute_units() || 2 * s.steps < kWaves) return false;
+  return !whole_on_the_tile(s, m, n, k, fused);
 }
 
 int gemm16_rows_k_splits(int m, int n, int k) { return rows_splits_for(shape_of(m, n, k, false), n, k); }

@@ -46,8 +46,11 @@ int launch_gemm_f32_direct(const float *a, const float *b, float *c, int m, int 
 
 // 16-bit products in tiles of at most 64 rows, straight from memory to registers (gemm16_rows.hip)
 bool gemm16_rows_serves(int m, int n, int k);
-using Gemm16Estimate = double (*)(int m, int n, int k, bool fused);   // microseconds on the 128 x 128 tile
+struct Gemm16Time { double us; int splits; };
+using Gemm16Estimate = Gemm16Time (*)(int m, int n, int k, bool fused);   // on the 128 x 128 tile, in the pieces of K it would take
 bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other);
+// Whether a product that was to go to the tile in pieces goes here if it cannot be cut.
+bool gemm16_rows_more_exact(int m, int n, int k, bool fused);
 int gemm16_rows_k_splits(int m, int n, int k);
 int launch_gemm16_rows(bool bf16, const uint16_t *a, const uint16_t *b, float *c, int m, int n, int k, hipStream_t st);
 int launch_gemm16_rows_fused(const uint16_t *a, const uint16_t *b, const float *bias, float *c, float *rowsum, int m, int n,

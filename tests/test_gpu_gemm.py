@@ -705,6 +705,35 @@ def test_gemm16_split_k_rule_and_epilogue(hip, oracle, torch_cuda):
     assert rowsums_ok(rs.cpu().numpy(), rs_ref)
 
 
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+@pytest.mark.parametrize("m,n,k,splits", [(1, 8, 128, 2), (128, 128, 192, 2), (129, 250, 200, 2), (77, 131, 449, 3), (256, 136, 832, 2),
+                                          (130, 129, 4097, 3)])
+def test_gemm16_pieces_in_chunks(hip, torch_cuda, kind, m, n, k, splits):
+    """Pieces of K of one stage, of an odd and an even count of chunks of two slabs, with a ragged first stage and more turns of the rings
+    than one.  The sum of k exact products, each addition rounded to half an ulp, is off by at most k 2^-24 times the sum of their
+    magnitudes; in chunks its error is that of chains of 64 products and k / 64 sums, half of the single chain's at the most from a
+    K of 4096 on."""
+    torch = torch_cuda
+    dt = torch.bfloat16 if kind == "bf16" else torch.float16
+    fn = hip.gemm_bf16 if kind == "bf16" else hip.gemm_f16
+    torch.manual_seed(m + n + k)
+    a, b = ((torch.randn(shape, device="cuda") * 0.02).to(dt) for shape in ((m, k), (k, n)))
+    ref, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    try:
+        hip.set_tunable("gemm16.tile", 128)
+        whole = fn(a, b)
+        hip.set_tunable("gemm16.split_k", splits)
+        assert hip.gemm16_k_splits(m, n, k) == splits
+        got = fn(a, b)
+        assert torch.equal(got, fn(a, b))
+    finally:
+        hip.set_tunable("gemm16.tile", 0)
+        hip.set_tunable("gemm16.split_k", 0)
+    assert bool(((got.double() - ref).abs() <= k * 2.0 ** -24 * size).all())
+    if k >= 4096:
+        assert (got.double() - ref).pow(2).mean() <= 0.25 * (whole.double() - ref).pow(2).mean()
+
+
 def test_gemm16_split_k_under_graph_capture(hip, torch_cuda):
     """A split-eligible product captured into a HIP graph on a stream that has no partial-plane block yet runs unsplit
     (nothing may be allocated under capture); every replay gives the eager result for the inputs of that moment."""
