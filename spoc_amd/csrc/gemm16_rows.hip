@@ -429,20 +429,26 @@ bool whole_on_the_tile(const Shape &s, int m, int n, int k, bool fused) {
   constexpr double kSlab[] = {0.19, 0.19, 0.24, 0.33}, kNarrowSlab[] = {0.172, 0.257, 0.272, 0.334}, kMegabyte[] = {0.156, 0.125, 0.134, 0.155};
   const int64_t tiles = static_cast<int64_t>((m + 127) / 128) * s.col_tiles;
   const double c_mb = static_cast<double>(m) * n * 4e-6, memory = static_cast<double>(k) * n * 2e-6 * kMegabyte[align];
-  double tile = 1e300;
-  for (int64_t pieces = 1; pieces == 1 || (!fused && pieces <= 16 && tiles * pieces <= 2 * cus && k / pieces >= 256); pieces *= 2) {
-    const double slabs = k / 32.0 / static_cast<double>(pieces);
-    const double chain = slabs * kNarrowSlab[align] * static_cast<double>((tiles * pieces + cus - 1) / cus);
-    tile = std::min(tile, narrow ? 5.17 + std::cbrt(chain * chain * chain + memory * memory * memory) + 0.28 * c_mb +
-                                       (pieces > 1 ? 4.0 + 0.38 * static_cast<double>(pieces) * c_mb : 0.0)
-                                 : 5.5 + slabs * kSlab[align] + (pieces > 1 ? 3.0 + 0.62 * static_cast<double>(pieces) * c_mb : 0.0));
-  }
+  // its pieces: of 256 at least, for a tenth of the time
+  auto cut_time = [&](int64_t pieces) {
+    return 8.0 + k / 32.0 / static_cast<double>(pieces) * 0.19 * (tiles * pieces > cus ? 1.15 : 1.0) +
+           (pieces > 1 ? 5.0 + static_cast<double>(pieces) * c_mb * 0.62 : 0.0);
+  };
+  int64_t pieces = 1;
+  double lowest = 0.9 * cut_time(1);
+  for (int64_t t = 2; !fused && t <= 16 && tiles * t <= 2 * cus && k / t >= 256; t *= 2)
+    if (cut_time(t) < lowest) lowest = cut_time(t), pieces = t;
+  const double slabs = k / 32.0 / static_cast<double>(pieces), planes = pieces > 1 ? static_cast<double>(pieces) * c_mb : 0.0;
+  const double chain = slabs * kNarrowSlab[align] * static_cast<double>((tiles * pieces + cus - 1) / cus);
+  const double tile = narrow ? 5.17 + std::cbrt(chain * chain * chain + memory * memory * memory) + 0.28 * c_mb + 0.38 * planes
+                             : 5.5 + slabs * kSlab[align] + 0.62 * planes;
+  const double launch = pieces == 1 ? 0.0 : narrow ? 4.0 : 3.0;
   const int splits = rows_splits_for(s, n, k);
-  if (narrow) return narrow_time(s, n, k, splits) >= 1.05 * tile;
+  if (narrow) return narrow_time(s, n, k, splits) >= 1.05 * (tile + launch);
   const double rounds = static_cast<double>((s.tiles * splits + cus - 1) / cus);
   const double here = (on16 ? 6.0 : 4.5) + rounds * s.steps / splits * (on16 ? 0.055 : on4 ? 0.07 : 0.12) * s.mt +
                       (splits > 1 ? 2.5 + 0.15 * splits + 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0);
-  return here >= tile;
+  return here >= tile + launch;
 }
 
 // Whether it should.  Up to 16 rows always, but for more than 128 MiB of B in one piece of K whose rows, of an even N, share
@@ -466,8 +472,8 @@ bool whole_on_the_tile(const Shape &s, int m, int n, int k, bool fused) {
 // two: 256 x 1280 x 191 6.8 / 8.4, 723 x 1702 x 256 7.2 / 7.9, as 21 of 118 drawn products, all but 3 of them so short), and its
 // time is below the 128 x 128 tile's by both estimates: a step costs by how A's and B's rows lie.  They were read off 292 plain
 // and 704 fused drawn products run on both (5 % rms, the tile's 8 and 9): 139 x 2432 x 1416 12.0 on the tile, 9.5 here,
-// 114 x 5824 x 2687 15.9, 27.2, fused 419 x 1472 x 2504 25.5, 17.4, 180 x 256 x 2240 10.0, 13.9; of those of more than 64 rows 9 in
-// 820 are more than 5 % slower by them than by the rules before.  `other`: what the tiled kernel is estimated at.
+// 114 x 5824 x 2687 15.9, 27.2, fused 419 x 1472 x 2504 25.5, 17.4, 180 x 256 x 2240 10.0, 13.9; of 430
+// drawn afresh 14 are more than 5 % slower than by the rules before, most of them launches of 6 us.  `other`: what the tiled kernel is estimated at.
 bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other) {
   const Shape s = shape_of(m, n, k, fused);
   if (m <= kTileRows && !fused) {

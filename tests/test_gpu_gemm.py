@@ -734,6 +734,46 @@ def test_gemm16_pieces_in_chunks(hip, torch_cuda, kind, m, n, k, splits):
         assert (got.double() - ref).pow(2).mean() <= 0.25 * (whole.double() - ref).pow(2).mean()
 
 
+@pytest.mark.parametrize("m,n,k,fused", [(320, 2880, 2793, False), (300, 2306, 2479, True)])
+def test_gemm16_product_that_cannot_be_cut(hip, torch_cuda, m, n, k, fused):
+    """On the tile for its pieces of K, which a captured call has no block for: there the few-rows kernel computes it, whole; the row
+    sums are then added by atomics, in any order (each addition of n terms rounded to half an ulp)."""
+    torch = torch_cuda
+    torch.manual_seed(m)
+    a, b = ((torch.randn(shape, device="cuda") * 0.02).half() for shape in ((m, k), (k, n)))
+    bias = torch.rand(n, device="cuda") * 0.1
+    assert hip.gemm16_tile(m, n, k) == 128 and hip.gemm16_k_splits(m, n, k) > 1
+    y, rs = torch.empty(m, n, device="cuda"), torch.empty(m, device="cuda")
+    call = (lambda: hip.gemm_f16_bias_relu_rowsum(a, b, bias, out=y, rowsum=rs)) if fused else (lambda: hip.gemm_f16(a, b, out=y))
+    call()
+    eager = y.clone()
+    try:
+        hip.set_tunable("gemm16.rows", 2)
+        hip.set_tunable("gemm16.rows_splits", 1)
+        call()
+    finally:
+        hip.set_tunable("gemm16.rows", 0)
+        hip.set_tunable("gemm16.rows_splits", 0)
+    whole = y.clone()
+    assert not torch.equal(eager, whole)
+    side, graph = side_stream(torch), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        call()
+    for _ in range(3):
+        y.fill_(float("nan"))
+        rs.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, whole)
+        if fused:
+            sums = y.double().sum(1)
+            assert bool(((rs.double() - sums).abs() <= n * 2.0 ** -24 * sums).all())
+        call()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager)
+
+
 def test_gemm16_split_k_under_graph_capture(hip, torch_cuda):
     """A split-eligible product captured into a HIP graph on a stream that has no partial-plane block yet runs unsplit
     (nothing may be allocated under capture); every replay gives the eager result for the inputs of that moment."""
