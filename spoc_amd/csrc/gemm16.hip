@@ -595,7 +595,7 @@ __device__ __forceinline__ void epilogue16(f32x4_t (&acc)[TI][4], float *__restr
         else atomicAdd(rowsum + m0 + t, total);
       }
     }
-    if (fold.tickets) fold_rows<64 * WMW * WNW, TROWS>(fold, M, m0, rowsum, tile_row, tiles_n, scratch);
+    if (fold.tickets) fold_rows<64 * WMW * WNW, TROWS>(fold, M, m0, TROWS, rowsum, tile_row, tiles_n, scratch);
   }
 }
 
@@ -727,7 +727,7 @@ __device__ __forceinline__ void epilogue16_rows(f32x4_t (&acc)[8][4], float *__r
       if (rs_plane) store_share(fold, rs_plane, m0 + t, total);
       else atomicAdd(rowsum + m0 + t, total);
     }
-    if (fold.tickets) fold_rows<512, TROWS>(fold, M, m0, rowsum, tile_row, tiles_n, scratch);
+    if (fold.tickets) fold_rows<512, TROWS>(fold, M, m0, TROWS, rowsum, tile_row, tiles_n, scratch);
   }
 }
 

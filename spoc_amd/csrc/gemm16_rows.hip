@@ -242,7 +242,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm16_rows_kernel(const uint16_t
   }
   auto fold_here = [&] {
     if constexpr (Fused) {
-      if (fold.tickets) fold_rows<64 * kWaves, kTileRows>(fold, M + m0, m0, rowsum, row_tile, col_tiles, &red[0][0]);
+      if (fold.tickets) fold_rows<64 * kWaves, kTileRows>(fold, M + m0, m0, 16 * MT, rowsum, row_tile, col_tiles, &red[0][0]);
     }
   };
   if (splits == 1) {

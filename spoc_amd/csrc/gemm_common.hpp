@@ -159,14 +159,15 @@ __device__ __forceinline__ void barrier_no_fence() {
 // Cache policy of a buffer access that other XCDs take part in: past the L2s, which they do not share.
 constexpr int kDeviceScope = 16;
 
-// rowsum[r] = the planes' sums of row r for the `Pitch` rows from m0 on, by the last of the `arrivals` workgroups that have put their
-// shares of these rows into planes (with kDeviceScope; this workgroup's are on their way).  In plane order, in double, one
+// rowsum[r] = the planes' sums of row r for the `rows` rows (at most Pitch) from m0 on that exist, by the last of the `arrivals`
+// workgroups that have put their shares of these rows into planes (with kDeviceScope; this workgroup's are on their way).  `rows` is
+// the height of their tiles: the rows below belong to workgroups that this counter does not count.  In plane order, in double, one
 // rounding, Threads / Pitch threads to a row: the same bits on every run.  Us, with a launch of its own for that and now: 128 x 128 x
 // 256 10.0 -> 7.4 (one launch to issue), 419 x 285 x 3370 17.3 -> 16.3, 701 x 384 x 824 12.4 -> 11.9, 5760 x 2560 x 448 25.0 -> 24.1.
 // What is left is a chain: C and the share stored, the counter's trip, the planes' loads.
 // scratch: LDS that no wave reads or writes any more when all have called this.
 template <int Threads, int Pitch>
-__device__ __forceinline__ void fold_rows(const RowFold &fold, int M, int m0, float *__restrict__ rowsum, int tile_row,
+__device__ __forceinline__ void fold_rows(const RowFold &fold, int M, int m0, int rows, float *__restrict__ rowsum, int tile_row,
                                           int arrivals, float *scratch) {
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   barrier_no_fence();
@@ -179,7 +180,7 @@ __device__ __forceinline__ void fold_rows(const RowFold &fold, int M, int m0, fl
   double *const sums = reinterpret_cast<double *>(scratch + 16);
   const int row = threadIdx.x % Pitch, part = threadIdx.x / Pitch;
   const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(fold.planes, 0x7FFFFFFFu);
-  const int at = min(m0 + row, M - 1) * 4;
+  const int end = min(M, m0 + rows), at = min(m0 + row, end - 1) * 4;
   double acc = 0.0;
   for (int t = part; t < fold.count; t += Parts * InFlight) {
     float v[InFlight];
@@ -192,7 +193,7 @@ __device__ __forceinline__ void fold_rows(const RowFold &fold, int M, int m0, fl
   sums[threadIdx.x] = acc;
   wait_lds();
   barrier_no_fence();
-  if (part == 0 && m0 + row < M) {
+  if (part == 0 && m0 + row < end) {
 #pragma unroll
     for (int q = 1; q < Parts; ++q) acc += sums[q * Pitch + row];
     rowsum[m0 + row] = static_cast<float>(acc);

@@ -539,6 +539,49 @@ def test_fused_row_sums_added_by_the_last_tile(hip, torch_cuda, m, n, k, knobs):
             hip.set_tunable(knob, 0)
 
 
+@pytest.mark.parametrize("m,n,k,splits", [
+    (65, 129, 100, 1), (65, 393, 256, 1), (80, 257, 512, 3), (96, 130, 96, 1), (96, 1500, 448, 2), (97, 300, 160, 1), (128, 300, 1000, 3),
+    (129, 257, 512, 1), (144, 700, 1024, 4), (145, 200, 256, 1), (200, 520, 640, 2), (33, 300, 256, 1), (48, 1000, 1024, 2),
+    (66, 393, 256, 0), (80, 3681, 4592, 0), (95, 2037, 4592, 0), (136, 2585, 3508, 0)])
+def test_fused_row_sums_of_each_row_tile(hip, torch_cuda, m, n, k, splits):
+    """The few-rows kernel, forced with its pieces of K and by its own rule (splits 0), whose tiles are 16 to 64 rows high: each row's
+    sum comes from the workgroups of its own tile.  Operands of three sizes take turns on a stream, so that a share that was not waited
+    for is another product's; every call's sums are those of its own y (float32 sums of at most 128 values, then doubles: 1e-5)."""
+    torch = torch_cuda
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(m * n + k)
+    sets = [tuple(torch.randn(*s, device="cuda", generator=gen).mul_(0.2).half() for s in ((m, k), (k, n))) +
+            (torch.rand(n, device="cuda", generator=gen) * scale,) for scale in (1.0, 300.0, 20.0)]
+    side = side_stream(torch)
+
+    def calls():
+        return [(i, hip.gemm_f16_bias_relu_rowsum(*sets[i])) for i in (0, 1, 2, 1, 0, 2)]
+    try:
+        if splits:
+            hip.set_tunable("gemm16.rows", 2)
+            hip.set_tunable("gemm16.rows_splits", splits)
+            hip.set_tunable("gemm16.fold", 2)
+            assert hip.gemm16_tile(m, n, k) == 64 and hip.gemm16_k_splits(m, n, k) == splits
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            other = calls()
+        here = calls()
+        torch.cuda.synchronize()
+        if not splits:   # which kernel its own rule took: the one whose bits these are
+            hip.set_tunable("gemm16.rows", 2)
+            assert torch.equal(hip.gemm_f16_bias_relu_rowsum(*sets[0])[0], here[0][1][0])
+            hip.set_tunable("gemm16.rows", 1)
+            assert not torch.equal(hip.gemm_f16_bias_relu_rowsum(*sets[0])[0], here[0][1][0])
+        first = {}
+        for i, (y, rs) in other + here:
+            assert rowsums_ok(rs.cpu().numpy(), y.double().sum(1).cpu().numpy())
+            y1, rs1 = first.setdefault(i, (y, rs))
+            assert torch.equal(y, y1) and torch.equal(rs, rs1)
+    finally:
+        for knob in ("gemm16.rows", "gemm16.rows_splits", "gemm16.fold"):
+            hip.set_tunable(knob, 0)
+
+
 @pytest.mark.parametrize("m,n,k,splits", [(128, 128, 256, 2), (1, 8, 128, 2), (129, 257, 200, 3), (300, 1023, 328, 2), (65, 1024, 448, 7),
                                           (64, 1025, 320, 4), (3, 4099, 1000, 5), (103, 1881, 6427, 0), (110, 2049, 7936, 0), (5, 2, 300, 3)])
 def test_fused_products_cut_along_k(hip, oracle, torch_cuda, m, n, k, splits):
