@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "small_window.hpp"
 #include "transfer.hpp"
 #include "tunables.hpp"
 
@@ -323,38 +324,26 @@ int get_small(void *dst, const void *src, size_t bytes, int dev) {
   if (!lock.owns_lock() || w.failed) return SAREK_HIP_E_UNSUPPORTED;
   if (!w.host) {
     void *p = nullptr;
-    if (hipHostMalloc(&p, kSmallBytes / 4 * sizeof(uint64_t), hipHostMallocCoherent) != hipSuccess) {
+    if (hipHostMalloc(&p, kWindowWords * sizeof(uint64_t), hipHostMallocCoherent) != hipSuccess) {
       (void)hipGetLastError();
       w.failed = true;
       return SAREK_HIP_E_UNSUPPORTED;
     }
-    std::memset(p, 0, kSmallBytes / 4 * sizeof(uint64_t));
+    std::memset(p, 0, kWindowWords * sizeof(uint64_t));
     w.host = static_cast<uint64_t *>(p);
   }
-  if (++w.count == 0) ++w.count;   // no word has the number 0
-  const uint32_t number = w.count;
-  const size_t words = (bytes + 3) / 4;
+  const uint32_t number = next_number(w.count);
   hipLaunchKernelGGL(get_kernel, dim3(1), dim3(256), 0, nullptr, w.host, static_cast<const uint32_t *>(src),
-                     static_cast<int>(words), number);
+                     static_cast<int>((bytes + 3) / 4), number);
   if (hipGetLastError() != hipSuccess) return SAREK_HIP_E_UNSUPPORTED;
-  const auto until = std::chrono::steady_clock::now() + kLook;
-  bool waited = false;
-  for (size_t i = 0; i < words; ++i) {
-    uint64_t word;
-    while ((word = __atomic_load_n(w.host + i, __ATOMIC_RELAXED)) >> 32 != number) {
-      for (int k = 0; k < 64 && __atomic_load_n(w.host + i, __ATOMIC_RELAXED) >> 32 != number; ++k) __builtin_ia32_pause();
-      if (!waited && std::chrono::steady_clock::now() > until) {
-        // a long kernel in front of it, or one that failed
-        const hipError_t e = hipStreamSynchronize(nullptr);
-        if (e != hipSuccess) w.failed = true;   // the kernel may still write: the window is not used again
-        if (e != hipSuccess) return check_hip(e, "download of a small vector");
-        waited = true;
-      }
-    }
-    const uint32_t low = static_cast<uint32_t>(word);
-    std::memcpy(static_cast<char *>(dst) + 4 * i, &low, std::min<size_t>(4, bytes - 4 * i));
-  }
-  return SAREK_HIP_OK;
+  hipError_t e = hipSuccess;   // of the wait: a long kernel in front of this one, or one that failed
+  const int rc = gather_words(dst, w.host, bytes, number, kLook, [&] {
+    e = hipStreamSynchronize(nullptr);
+    return e == hipSuccess ? 0 : 1;
+  });
+  if (rc == 0) return SAREK_HIP_OK;
+  w.failed = true;   // the kernel may still write, or ended without its words: the window is not used again
+  return e != hipSuccess ? check_hip(e, "download of a small vector") : SAREK_HIP_E_UNSUPPORTED;
 }
 #endif
 
