@@ -12,9 +12,13 @@ namespace sarek_hip {
 
 constexpr size_t kWindowWords = kSmallBytes / 4;
 
-// The number of the next call, never 0, which an empty window holds.
-inline uint32_t next_number(uint32_t &count) {
-  if (++count == 0) ++count;
+// The number of the next call, never 0, which an empty window holds.  When the numbers start again the window is emptied: a word
+// that no call has written since its number was used last would be taken for the data of the call that bears it now.
+inline uint32_t next_number(uint64_t *window, uint32_t &count) {
+  if (++count == 0) {
+    std::memset(window, 0, kWindowWords * sizeof(uint64_t));
+    count = 1;
+  }
   return count;
 }
 

@@ -332,7 +332,7 @@ int get_small(void *dst, const void *src, size_t bytes, int dev) {
     std::memset(p, 0, kWindowWords * sizeof(uint64_t));
     w.host = static_cast<uint64_t *>(p);
   }
-  const uint32_t number = next_number(w.count);
+  const uint32_t number = next_number(w.host, w.count);
   hipLaunchKernelGGL(get_kernel, dim3(1), dim3(256), 0, nullptr, w.host, static_cast<const uint32_t *>(src),
                      static_cast<int>((bytes + 3) / 4), number);
   if (hipGetLastError() != hipSuccess) return SAREK_HIP_E_UNSUPPORTED;

@@ -45,29 +45,35 @@ int main() {
     const size_t words = (bytes + 3) / 4;
     std::vector<unsigned char> dst(kSmallBytes + 8, 0xEE);
     // all there; word by word while the host looks; by the time the wait ends
-    uint32_t number = next_number(count);
+    uint32_t number = next_number(window, count);
     put(number, 0, words);
     expect(gather_words(dst.data(), window, bytes, number, milliseconds(2), ended) == 0 && waits == 0 && holds(dst, number, bytes), "there");
-    number = next_number(count);
+    number = next_number(window, count);
     std::thread late([&] {
       for (size_t i = words; i-- > 0;) put(number, i, i + 1);
     });
     const int rc = gather_words(dst.data(), window, bytes, number, std::chrono::seconds(20), ended);
     late.join();
     expect(rc == 0 && waits == 0 && holds(dst, number, bytes), "while it looks");
-    number = next_number(count);
+    number = next_number(window, count);
     expect(gather_words(dst.data(), window, bytes, number, microseconds(50), [&] { return put(number, 0, words), ++waits, 0; }) == 0 &&
                waits == 1 && holds(dst, number, bytes), "after the wait");
     // the last word never comes: the call ends, and dst is as it was; the same where the wait fails
     std::vector<unsigned char> kept(kSmallBytes + 8, 0xEE);
-    number = next_number(count);
+    number = next_number(window, count);
     put(number, 0, words - 1);
     expect(gather_words(kept.data(), window, bytes, number, microseconds(50), ended) == kNotDelivered && waits == 2 && untouched(kept), "never");
-    number = next_number(count);
+    number = next_number(window, count);
     put(number, 0, words - 1);
     expect(gather_words(kept.data(), window, bytes, number, microseconds(50), [] { return 7; }) == 7 && untouched(kept), "wait failed");
     waits = 0;
   }
+  // the numbers start again: what an old call with the same number left is not this call's
+  put(1, 0, kWindowWords);
+  count = 0xFFFFFFFFu;
+  const uint32_t number = next_number(window, count);
+  std::vector<unsigned char> kept(16, 0xEE);
+  expect(number == 1 && gather_words(kept.data(), window, 16, number, microseconds(50), ended) == kNotDelivered && untouched(kept), "numbers start again");
   if (failures == 0) std::printf("small window ok\n");
   return failures;
 }
