@@ -344,8 +344,9 @@ struct Call {
 template <bool Bf16, bool Fused, int MT>
 int launch(const Call &q, const Shape &s) {
   int splits = rows_splits_for(s, q.n, q.k);
-  float *block = nullptr;
-  if (Fused || splits > 1) block = splitk_workspace(q.st);
+  Workspace workspace;
+  if (Fused || splits > 1) workspace = splitk_workspace(q.st);
+  float *const block = workspace.block;
   if (!block) splits = 1;
   const int per = (s.steps + splits - 1) / splits;
   float *rs_planes = nullptr;

@@ -1,6 +1,8 @@
 // Device helpers shared by the GEMM kernels: workgroup -> tile raster, the LDS ring of
 // the direct-to-LDS pipelines, DMA and barrier primitives.
 #pragma once
+#include <mutex>
+
 #include <hip/hip_runtime.h>
 
 namespace sarek_hip {
@@ -8,7 +10,13 @@ namespace sarek_hip {
 // K-split products (gemm_splitk.hip): the per-stream block of device memory for the partial planes and the kernel that
 // adds them into C in a fixed order.
 constexpr size_t kSplitWorkspaceBytes = 64u << 20;
-float *splitk_workspace(hipStream_t st);
+// A stream's block (nullptr: none), held by one call at a time until its launches are issued: those of another thread's call on
+// the same stream would come between the launch that fills the planes and the one that adds them.
+struct Workspace {
+  float *block = nullptr;
+  std::unique_lock<std::mutex> issuing;
+};
+Workspace splitk_workspace(hipStream_t st);
 int launch_splitk_reduce(const float *partials, float *c, int m, int n, int splits, hipStream_t st);
 int launch_splitk_reduce_fused(const float *partials, const float *bias, float *y, float *rowsum, int m, int n, int splits,
                                hipStream_t st);   // with the bias, the ReLU and the row sums

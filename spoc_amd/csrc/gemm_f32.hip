@@ -662,11 +662,13 @@ extern "C" int sarek_hip_gemm_f32(const float *a, const float *b, float *c, int 
   const bool c_aligned = reinterpret_cast<uintptr_t>(c) % 16 == 0;
   const bool fallback = tunable("gemm_f32.force_simple", 0) != 0 || tunable("gemm_f32.force_staged", 0) != 0;
   Plan plan{0, 0, 0, 1, 0, 0};
-  float *partials = nullptr;
+  Workspace workspace;
   if (!fallback) {
     plan = plan_for(m, n, k, ring_ok, true);
-    if (plan.splits > 1 && !(partials = splitk_workspace(st))) plan = plan_for(m, n, k, ring_ok, false);
+    if (plan.splits > 1) workspace = splitk_workspace(st);
+    if (plan.splits > 1 && !workspace.block) plan = plan_for(m, n, k, ring_ok, false);
   }
+  float *const partials = workspace.block;
   if (plan.row_blocks > 0) return launch_gemm_f32_direct(a, b, c, m, n, k, plan.row_blocks, plan.waves, plan.splits, partials, st);
   if (plan.tile > 0) {
     const bool ragged = !aligned || n % 4 != 0 || k % 32 != 0 || !c_aligned;

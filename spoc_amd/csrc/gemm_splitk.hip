@@ -110,34 +110,42 @@ __global__ __launch_bounds__(256) void zero_tickets_kernel(unsigned *tickets) {
 
 // One block of kSplitWorkspaceBytes and its tickets per (device, stream), allocated at the first call that wants one on
 // that stream and kept until the process ends (never grown or freed, so a pointer handed out stays good whatever other threads do):
-// calls on different streams never share one, calls on one stream are ordered by it.  nullptr (the caller then works
+// calls on different streams never share one, calls on one stream are ordered by it and by the block's lock.  None (the caller then works
 // without one: no K split, row sums by atomicAdd) for a stream under capture -- a recorded graph would carry the
 // block's address to wherever it is replayed, next to eager calls or other replays that use the same block --, for
 // hipStreamPerThread (one handle, a stream to each thread: their launches are not ordered by it), past 16 streams, or when
 // the allocation fails.
-float *splitk_workspace(hipStream_t st) {
-  if (st == hipStreamPerThread) return nullptr;
+Workspace splitk_workspace(hipStream_t st) {
+  if (st == hipStreamPerThread) return {};
+  struct Block {
+    float *p;
+    std::mutex issuing;
+  };
   static std::mutex mu;
-  static std::map<std::pair<int, hipStream_t>, void *> blocks;
+  static std::map<std::pair<int, hipStream_t>, Block> blocks;   // (their places do not change)
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+  if (hipGetDevice(&dev) != hipSuccess) return {};
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
-    return nullptr;
+    return {};
   }
-  std::lock_guard<std::mutex> lock(mu);
+  std::unique_lock<std::mutex> lock(mu);
   auto it = blocks.find({dev, st});
-  if (it != blocks.end()) return static_cast<float *>(it->second);
-  if (blocks.size() >= 16) return nullptr;
+  if (it != blocks.end()) {
+    lock.unlock();   // nobody waits for another stream's call
+    return {it->second.p, std::unique_lock<std::mutex>(it->second.issuing)};
+  }
+  if (blocks.size() >= 16) return {};
   void *p = nullptr;
   if (hipMalloc(&p, kSplitWorkspaceBytes + (kSplitTickets + kFoldTickets) * sizeof(unsigned)) != hipSuccess) {
     (void)hipGetLastError();
-    return nullptr;
+    return {};
   }
   hipLaunchKernelGGL(zero_tickets_kernel, dim3((kSplitTickets + kFoldTickets) / 256), dim3(256), 0, st, splitk_tickets(static_cast<float *>(p)));
-  blocks[{dev, st}] = p;
-  return static_cast<float *>(p);
+  Block &block = blocks[{dev, st}];
+  block.p = static_cast<float *>(p);
+  return {block.p, std::unique_lock<std::mutex>(block.issuing)};
 }
 
 int compute_units() {

@@ -107,3 +107,48 @@ def test_long_folds_on_more_streams_than_the_library_has_stages(hip, torch_cuda)
             hip.check(hip.lib.sarek_hip_fold_partials_f64(x.data_ptr(), n, got[k:].data_ptr(), st.cuda_stream))
         torch.cuda.synchronize()
         assert bool((got == want).all()), (n, offset, got.tolist(), want.item())
+
+
+def test_threads_on_one_stream(hip, torch_cuda):
+    """Four threads whose products go through one stream's block of planes in two launches each: fused and plain products in pieces
+    of K, row sums with a launch of their own, a float32 product in pieces.  Another thread's launches do not come between a
+    call's two: every result is, bit for bit, the one the call gives alone."""
+    torch = torch_cuda
+    fused = [(128, 1024, 2048), (300, 1023, 1000), (110, 2049, 7936), (2304, 4352, 64)]
+    plain = [(256, 256, 4096), (512, 256, 2048), (1062, 320, 1984), (130, 512, 8192)]
+    work = []
+    for t in range(4):
+        g = torch.Generator(device="cuda")
+        g.manual_seed(7 + t)
+        (m, n, k), (pm, pn, pk) = fused[t], plain[t]
+        a, b, pa, pb = ((torch.randn(*s, device="cuda", generator=g) * 0.05).half() for s in ((m, k), (k, n), (pm, pk), (pk, pn)))
+        fa, fb = (torch.randn(*s, device="cuda", generator=g) for s in ((200, 2000), (2000, 200 + t)))
+        bias = torch.rand(n, device="cuda", generator=g) * (t + 1)
+        work.append((a, b, bias, pa, pb, fa, fb))
+        assert hip.gemm16_k_splits(pm, pn, pk) > 1 and hip.gemm_f32_k_splits(200, 200 + t, 2000) > 1
+
+    def calls(t):
+        a, b, bias, pa, pb, fa, fb = work[t]
+        return [*hip.gemm_f16_bias_relu_rowsum(a, b, bias), hip.gemm_f16(pa, pb), hip.gemm_f32(fa, fb)]
+    alone = [calls(t) for t in range(4)]
+    torch.cuda.synchronize()
+    together, errors = [[] for _ in range(4)], []
+
+    def threaded(t):
+        try:
+            together[t] = [calls(t) for _ in range(60)]
+        except Exception as e:              # noqa: BLE001 -- reported by the main thread
+            errors.append((t, repr(e)))
+
+    threads = [threading.Thread(target=threaded, args=(t,)) for t in range(4)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    assert errors == []
+    for t in range(4):
+        assert len(together[t]) == 60
+        for i, got in enumerate(together[t]):
+            for j, (x, want) in enumerate(zip(got, alone[t])):
+                assert torch.equal(x, want), (t, i, j)
