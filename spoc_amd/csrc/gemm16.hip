@@ -1884,17 +1884,37 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   const bool tiled = tile_choice != 0 && (k >= 64 || ab16);
   const int nm = tiled ? tiled_columns(m, n, tile_choice) : n;
 
+  bool half = tiled && tile_choice == 128 && half_tile_pays(m, nm, k, 1);
+  const int cut = tiled && tile_choice == 256 && nm > 0 && !(kMeasureBuild && clock_probe(1))
+                      ? whole_round_columns(m, nm, k, half) : nm;
+
+  // K in pieces on the 128 x 128 tile (fused: the planes hold plain sums; the launch that adds them does the rest.  Us, uncut and cut:
+  // 110 x 9523 x 7936 94 -> 73, 2649 x 435 x 6243 67 -> 45, 103 x 5881 x 6427 56 on the few-rows kernel -> 32, 517 x 704 x 2995
+  // 21.8 -> 17.7)
+  Workspace workspace;
+  float *partials = nullptr;
+  int splits = 1;
+  if (tiled && tile_choice == 128 && nm > 0 && !half) {
+    splits = splitk_for(m, n, k, Epi != EPI_STORE);
+    if (splits > 1 && (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n)) {
+      workspace = splitk_workspace(st);
+      partials = workspace.block;
+    }
+    // (no block under capture and past 16 streams: a product that is on this tile for its pieces is not to run whole on it)
+    if (splits > 1 && !partials && few_rows_asked(m, n, k) == 0 && gemm16_rows_more_exact(m, n, k, Epi != EPI_STORE)) {
+      if constexpr (Epi == EPI_STORE) return launch_gemm16_rows(Bf16, a, b, c, m, n, k, st);
+      else return launch_gemm16_rows_fused(a, b, bias, c, rowsum, m, n, k, st);
+    }
+    if (!partials) splits = 1;
+  }
+
   // Row sums: every tile column (every 64 columns of the simple kernel; the last column on its own) leaves its share of
   // each row in a plane of its own, and rowsum_fold_kernel adds the planes in column order, in double, with one rounding:
   // the same bits on every run.  The planes live in the stream's workspace block; a call that has none (under
   // stream capture, past the sixteenth stream, planes beyond the block's size) adds with atomicAdd in arrival order.
-  Workspace workspace;
   float *planes = nullptr;
   int n_planes = 0;
-  bool half = tiled && tile_choice == 128 && half_tile_pays(m, nm, k, 1);
-  const int cut = tiled && tile_choice == 256 && nm > 0 && !(kMeasureBuild && clock_probe(1))
-                      ? whole_round_columns(m, nm, k, half) : nm;
-  if constexpr (Epi == EPI_BIAS_RELU_ROWSUM) {
+  if (Epi == EPI_BIAS_RELU_ROWSUM && splits == 1) {
     const int first = tiled && tile_choice == 128 ? 0 : cut;   // columns in planes of 256; from there on in planes of 128
     n_planes = tiled ? (first + 255) / 256 + (nm - first + 127) / 128 + (n - nm) : (n + 63) / 64;
     if (static_cast<int64_t>(n_planes) * m * 4 <= static_cast<int64_t>(kSplitWorkspaceBytes)) workspace = splitk_workspace(st);
@@ -1951,22 +1971,6 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   } else if (nm > 0 && tile_choice == 128) {
     const int sm = (m + 127) / 128, sn = (nm + 127) / 128;
     unsigned long long *sprobe = clock_probe(static_cast<int64_t>(sm) * sn);
-    int splits = 1;
-    float *partials = nullptr;
-    // (fused: the planes hold plain sums; the launch that adds them does the rest.  Us, uncut and cut: 110 x 9523 x 7936 94 -> 73,
-    // 2649 x 435 x 6243 67 -> 45, 103 x 5881 x 6427 56 on the few-rows kernel -> 32, 517 x 704 x 2995 21.8 -> 17.7)
-    splits = splitk_for(m, n, k, Epi != EPI_STORE);
-    if (splits > 1 && (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n)) {
-      if (!workspace.block) workspace = splitk_workspace(st);
-      partials = workspace.block;
-    }
-    // (no block under capture and past 16 streams: a product that is on this tile for its pieces is not to run whole on it)
-    if (splits > 1 && !partials && few_rows_asked(m, n, k) == 0 && gemm16_rows_more_exact(m, n, k, Epi != EPI_STORE)) {
-      workspace = {};   // (that kernel asks for it itself)
-      if constexpr (Epi == EPI_STORE) return launch_gemm16_rows(Bf16, a, b, c, m, n, k, st);
-      else return launch_gemm16_rows_fused(a, b, bias, c, rowsum, m, n, k, st);
-    }
-    if (!partials) splits = 1;
     if (splits > 1) {
       const int chunk = splitk_chunk(k, 64, splits);
       if (ragged)

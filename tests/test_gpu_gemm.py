@@ -817,6 +817,22 @@ def test_gemm16_product_that_cannot_be_cut(hip, torch_cuda, m, n, k, fused):
         assert torch.equal(y, eager)
 
 
+@pytest.mark.parametrize("m,n,k", [(300, 2306, 2479), (110, 2049, 7936), (128, 128, 64)])
+def test_captured_fused_product_clears_its_row_sums_once(hip, torch_cuda, m, n, k):
+    """A graph of one fused product holds two kernels, whichever would have cut K: the row sums' clearing and the product."""
+    torch = torch_cuda
+    a, b = (torch.randn(s, device="cuda").half() for s in ((m, k), (k, n)))
+    bias, y, rs = torch.rand(n, device="cuda"), torch.empty(m, n, device="cuda"), torch.empty(m, device="cuda")
+    side, graph = side_stream(torch), torch.cuda.CUDAGraph(keep_graph=True)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        hip.gemm_f16_bias_relu_rowsum(a, b, bias, out=y, rowsum=rs)
+    runtime = C.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    nodes = C.c_size_t()
+    assert runtime.hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(nodes)) == 0
+    assert nodes.value == 2
+
+
 def test_gemm16_split_k_under_graph_capture(hip, torch_cuda):
     """A split-eligible product captured into a HIP graph on a stream that has no partial-plane block yet runs unsplit
     (nothing may be allocated under capture); every replay gives the eager result for the inputs of that moment."""
