@@ -1229,12 +1229,16 @@ __global__ __launch_bounds__(256) void gemm16_m16w4_kernel(const uint16_t *__res
 // rows of the large tile, so the same XOR swizzle keeps the transposing reads free of bank conflicts.  A slab is 16 MFMAs:
 // rows 0-31 of the wave tile before the barrier, rows 32-63 after it with the next slab's 12 fragment reads (and, every
 // other slab, the 4 transfers of an A stage) behind them; fragments are double-buffered by slab parity.
-// Chunked, for K in pieces: an element is the sum of sums of two slabs, kept apart in 64 registers more (two waves to a SIMD have
-// 256 each), so that a piece is as exact as the few-rows kernel's eight waves make it: rms error against float64 over the largest
-// element, 320 x 2880 x 2793, there 2.3e-8, here in one chain 4.1e-8, in chunks 2.1e-8.  The additions hide behind the MFMAs: 704 x
-// 1728 x 4591 23.2 us without, 23.7 in chunks of four slabs, 24.0 of two.
-template <bool Bf16, int Epi, bool Ragged = false, bool Chunked = false>
-__global__ __launch_bounds__(256, Chunked ? 2 : 1) void gemm16_m16_small_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
+// Chunk, for K in pieces: an element is the sum of sums of so many slabs, kept apart in 64 registers more (two waves to a SIMD have
+// 256 each; in chunks of two one or two are stored before the K loop and read again behind it), so that a piece is as exact as the
+// few-rows kernel's eight waves make it: rms error against float64 over the largest element, 320 x 2880 x 2793, there 2.3e-8, here in
+// one chain 7.1e-8 whole and 4.1e-8 in three pieces, in chunks 2.1e-8.  Chunks of two slabs are the more exact in short pieces (103 x 610
+// x 1022 in four 1.84e-8, of four slabs 2.07e-8), chunks of four in long ones, whose sums of chunks are longer (57 x 16274 x 3264 in two
+// 2.40e-8 and 2.24e-8): from kLongPiece of K on four.  The additions hide behind the MFMAs: 704 x 1728 x 4591 23.2 us without, 23.7 in chunks
+// of four slabs, 24.0 of two.
+constexpr int kLongPiece = 1024;
+template <bool Bf16, int Epi, bool Ragged = false, int Chunk = 0>
+__global__ __launch_bounds__(256, Chunk ? 2 : 1) void gemm16_m16_small_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
                                                                float *__restrict__ C, const float *__restrict__ bias,
                                                                float *__restrict__ rowsum, int M, int N, int K, int tiles_m,
                                                                int tiles_n, int xcd_remap, unsigned long long *probe,
@@ -1249,8 +1253,7 @@ __global__ __launch_bounds__(256, Chunked ? 2 : 1) void gemm16_m16_small_kernel(
   constexpr int NWAVES = 4, WN = 2;
   constexpr int DA = A_BYTES_S / 1024 / NWAVES, DB = B_BYTES_S / 1024 / NWAVES;
   constexpr int P = lcm_int(NB, RA * NA);
-  constexpr int kChunk = 2;   // slabs
-  static_assert(P % kChunk == 0, "a chunk ends where a turn of the rings does");
+  static_assert(Chunk == 0 || P % Chunk == 0, "a chunk ends where a turn of the rings does");
   static_assert(P % 2 == 0, "the fragment buffers alternate by slab parity");
   static_assert(2 * (NA * A_BYTES_S + NB * B_BYTES_S) <= 160 * 1024, "two workgroups per CU");
 
@@ -1314,8 +1317,8 @@ __global__ __launch_bounds__(256, Chunked ? 2 : 1) void gemm16_m16_small_kernel(
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
-  f32x4_t sum[Chunked ? 4 : 1][4];   // of the chunks before this one
-  if constexpr (Chunked) {
+  f32x4_t sum[Chunk ? 4 : 1][4];   // of the chunks before this one
+  if constexpr (Chunk != 0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1409,7 +1412,7 @@ __global__ __launch_bounds__(256, Chunked ? 2 : 1) void gemm16_m16_small_kernel(
     constexpr int ia = (I / RA) % NA, ibp = (I + NB - 1) % NB;
     constexpr int ian = (In / RA) % NA, ibn = In % NB;
     constexpr int ksn = In % RA;
-    constexpr std::bool_constant<Chunked && I % kChunk == 0> fresh;
+    constexpr std::bool_constant<Chunk != 0 && I % (Chunk ? Chunk : 1) == 0> fresh;
     asm volatile("" : "+v"(a_addr0), "+v"(b_addr0));
     issue_b(std::integral_constant<int, -1>{}, lds_ring<40 + ibp, B_BYTES_S>);
     mfma_range(std::integral_constant<int, 0>{}, std::integral_constant<int, 8>{}, fresh, af[I & 1], bf[I & 1]);
@@ -1458,7 +1461,7 @@ __global__ __launch_bounds__(256, Chunked ? 2 : 1) void gemm16_m16_small_kernel(
     ((full + Is < nslabs ? slab(std::integral_constant<int, Is>{}, full + Is) : (void)0), ...);
   }(std::make_integer_sequence<int, P - 1>{});
   __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(0));   // the tail's empty transfers, before the LDS is released
-  if constexpr (Chunked) {
+  if constexpr (Chunk != 0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1972,13 +1975,17 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
     const int sm = (m + 127) / 128, sn = (nm + 127) / 128;
     unsigned long long *sprobe = clock_probe(static_cast<int64_t>(sm) * sn);
     if (splits > 1) {
-      const int chunk = splitk_chunk(k, 64, splits);
-      if (ragged)
-        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, true, true>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
-                           nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, nullptr);
-      else
-        hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, false, true>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
-                           nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, chunk, partials, n, nullptr);
+      const int piece = splitk_chunk(k, 64, splits);
+      auto launch_pieces = [&]<int Chunk>(std::integral_constant<int, Chunk>) {
+        if (ragged)
+          hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, true, Chunk>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
+                             nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, piece, partials, n, nullptr);
+        else
+          hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, false, Chunk>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
+                             nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, piece, partials, n, nullptr);
+      };
+      if (piece < kLongPiece) launch_pieces(std::integral_constant<int, 2>{});
+      else launch_pieces(std::integral_constant<int, 4>{});
       rc = check_launch("gemm16 kernel launch");
       if (rc != SAREK_HIP_OK) return rc;
       if constexpr (Epi == EPI_STORE) rc = launch_splitk_reduce(partials, c, m, n, splits, st);

@@ -11,16 +11,22 @@
 namespace sarek_hip {
 namespace {
 
-// The sum of four columns' `splits` partial sums, plane 0 first, up to nine of them asked for at once: one after the other, each
-// waited a trip to the caches for the one before (us, with the products: 161 x 256 x 7182, 13 pieces, 14.2 and 12.4; 63 x 1130 x 7104,
-// 14.4, 12.6; fused 98 x 576 x 2432 13.1, 11.4).
+// The sum of four columns' `splits` partial sums, up to nine of them asked for at once: one after the other, each waited a trip to the
+// caches for the one before (us, with the products: 161 x 256 x 7182, 13 pieces, 14.2 and 12.4; 63 x 1130 x 7104, 14.4, 12.6; fused 98 x
+// 576 x 2432 13.1, 11.4).  What is there is added in pairs, pairs of pairs and so on, the same for every run: 14 in a row were 38 x 2250 x
+// 7680 1.03 of the few-rows kernel's error, so they are 0.96.  (In double 0.80, but a launch of 1.4 us more work: fused 67 x 4838 x 2885
+// 18.6 to 20.1 us.)
 template <int Count, class Vec>
 __device__ __forceinline__ void add_next(f32x4_t &acc, const float *__restrict__ p, int64_t plane) {
-  f32x4_t v[Count];
+  f32x4_t v[Count + 1];
+  v[0] = acc;
 #pragma unroll
-  for (int u = 0; u < Count; ++u) v[u] = *reinterpret_cast<const Vec *>(p + u * plane);
+  for (int u = 0; u < Count; ++u) v[u + 1] = *reinterpret_cast<const Vec *>(p + u * plane);
 #pragma unroll
-  for (int u = 0; u < Count; ++u) acc += v[u];
+  for (int w = 1; w <= Count; w *= 2)
+#pragma unroll
+    for (int u = 0; u + w <= Count; u += 2 * w) v[u] += v[u + w];
+  acc = v[0];
 }
 template <class Vec>
 __device__ __forceinline__ f32x4_t add_planes(const float *__restrict__ p, int64_t plane, int splits) {
@@ -41,7 +47,7 @@ __device__ __forceinline__ f32x4_t add_planes(const float *__restrict__ p, int64
   return acc;
 }
 
-// Adds the `splits` partial planes into C, plane 0 first: a fixed order, so the result does not depend on which
+// Adds the `splits` partial planes into C: a fixed order, so the result does not depend on which
 // workgroup finished when.  C is 16-byte aligned (the callers' condition).
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ partials, float *__restrict__ C,
                                                             int64_t mn, int64_t plane, int splits) {

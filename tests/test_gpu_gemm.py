@@ -750,10 +750,10 @@ def test_gemm16_split_k_rule_and_epilogue(hip, oracle, torch_cuda):
 
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("m,n,k,splits", [(1, 8, 128, 2), (128, 128, 192, 2), (129, 250, 200, 2), (77, 131, 449, 3), (256, 136, 832, 2),
-                                          (130, 129, 4097, 3)])
+                                          (130, 129, 4097, 3), (129, 130, 2048, 2), (70, 200, 2200, 2), (257, 136, 3137, 3)])
 def test_gemm16_pieces_in_chunks(hip, torch_cuda, kind, m, n, k, splits):
-    """Pieces of K of one stage, of an odd and an even count of chunks of two slabs, with a ragged first stage and more turns of the rings
-    than one.  The sum of k exact products, each addition rounded to half an ulp, is off by at most k 2^-24 times the sum of their
+    """Pieces of K of one stage, of an odd and an even count of chunks of two slabs, of chunks of four (1024 of K and more) with a rest of
+    every length, with a ragged first stage and more turns of the rings than one.  The sum of k exact products, each addition rounded to half an ulp, is off by at most k 2^-24 times the sum of their
     magnitudes; in chunks its error is that of chains of 64 products and k / 64 sums, half of the single chain's at the most from a
     K of 4096 on."""
     torch = torch_cuda
@@ -775,6 +775,30 @@ def test_gemm16_pieces_in_chunks(hip, torch_cuda, kind, m, n, k, splits):
     assert bool(((got.double() - ref).abs() <= k * 2.0 ** -24 * size).all())
     if k >= 4096:
         assert (got.double() - ref).pow(2).mean() <= 0.25 * (whole.double() - ref).pow(2).mean()
+
+
+@pytest.mark.parametrize("m,n,k,fused", [(38, 2250, 7680, False), (57, 16274, 3264, False), (40, 10279, 4066, False), (79, 563, 1641, False),
+                                         (224, 320, 5952, True), (118, 2624, 6120, True)])
+def test_pieces_on_the_tile_are_as_exact_as_the_few_rows_kernel(hip, torch_cuda, m, n, k, fused):
+    """Pieces of K of 183 to 1632 on the 128 x 128 tile, up to 14 of them: the mean square of their error against float64 is not above
+    that of the few-rows kernel, which computed such products before (70000 elements and more: its own spread is under 1 %)."""
+    torch = torch_cuda
+    torch.manual_seed(m + k)
+    a, b = ((torch.randn(shape, device="cuda") * 0.02).half() for shape in ((m, k), (k, n)))
+    bias = torch.rand(n, device="cuda") * 0.2 - 0.1
+    call = (lambda: hip.gemm_f16_bias_relu_rowsum(a, b, bias)[0]) if fused else (lambda: hip.gemm_f16(a, b))
+    ref = a.double() @ b.double()
+    if fused:
+        ref = (ref + bias.double()).clamp_min(0)
+    error = {}
+    try:
+        for rows in (1, 2):
+            hip.set_tunable("gemm16.rows", rows)
+            assert (hip.gemm16_tile(m, n, k) == 64) == (rows == 2) and hip.gemm16_k_splits(m, n, k) > 1
+            error[rows] = (call().double() - ref).pow(2).mean().item()
+    finally:
+        hip.set_tunable("gemm16.rows", 0)
+    assert error[1] <= error[2]
 
 
 @pytest.mark.parametrize("m,n,k,fused", [(320, 2880, 2793, False), (300, 2306, 2479, True)])
