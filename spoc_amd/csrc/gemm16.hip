@@ -1229,7 +1229,7 @@ __global__ __launch_bounds__(256) void gemm16_m16w4_kernel(const uint16_t *__res
 // rows of the large tile, so the same XOR swizzle keeps the transposing reads free of bank conflicts.  A slab is 16 MFMAs:
 // rows 0-31 of the wave tile before the barrier, rows 32-63 after it with the next slab's 12 fragment reads (and, every
 // other slab, the 4 transfers of an A stage) behind them; fragments are double-buffered by slab parity.
-// Chunk, for K in pieces: an element is the sum of sums of so many slabs, kept apart in 64 registers more (two waves to a SIMD have
+// Chunk, for K in pieces (and whole where TileTime::whole_in_chunks): an element is the sum of sums of so many slabs, kept apart in 64 registers more (two waves to a SIMD have
 // 256 each; in chunks of two one or two are stored before the K loop and read again behind it), so that a piece is as exact as the
 // few-rows kernel's eight waves make it: rms error against float64 over the largest element, 320 x 2880 x 2793, there 2.3e-8, here in
 // one chain 7.1e-8 whole and 4.1e-8 in three pieces, in chunks 2.1e-8.  Chunks of two slabs are the more exact in short pieces (103 x 610
@@ -1683,7 +1683,7 @@ __global__ __launch_bounds__(256) void gemm16_last_column_kernel(const uint16_t 
 // pieces the launch that adds them, and their planes.
 struct TileTime {
   int64_t tiles, stages, cus;
-  double stage, second, memory2, whole, launch, piece;
+  double stage, second, memory2, c_mb, whole, launch, piece;
 
   TileTime(int m, int n, int k, bool fused) {
     struct Fit { double stage[4], second, memory, base, c, launch, piece, plane; };
@@ -1695,7 +1695,8 @@ struct TileTime {
     cus = compute_units();
     stage = f.stage[k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 + n % 2 + 1];
     second = f.second;
-    const double memory = (static_cast<double>(m) * k + static_cast<double>(k) * n) * 2e-6 * f.memory, c_mb = static_cast<double>(m) * n * 4e-6;
+    const double memory = (static_cast<double>(m) * k + static_cast<double>(k) * n) * 2e-6 * f.memory;
+    c_mb = static_cast<double>(m) * n * 4e-6;
     memory2 = memory * memory;
     whole = f.base + f.c * c_mb;
     launch = f.launch;
@@ -1726,6 +1727,12 @@ struct TileTime {
     try_near(std::sqrt(saved * second), std::max<int64_t>(2, cus / tiles + 1), most);
     return splits;
   }
+  // Whether a plain product that is not cut sums K in chunks: a long K and a small C, a workgroup to a tile.  These had K in two pieces
+  // before any count of them was looked at; whole they are faster, but one chain of K has 1.4 times the error of two (rms over the largest
+  // element, cut in two, whole, in chunks: 49 x 26100 x 6961 7.8e-8, 10.9e-8, 3.2e-8; us 101.1, 100.7, 100.7; 12 x 30926 x 5817 82.6, 63.6,
+  // 64.0; 84 x 21952 x 8129 109.8, 97.6, 99.5).  The line takes the 471 such of 400000 drawn products and two others.  Elsewhere chunks cost up
+  // to 5 % (4457 x 448 x 3264 23.5 and 24.6).
+  bool whole_in_chunks(int k) const { return tiles <= cus && k >= 3000.0 + 640.0 * c_mb; }
 };
 
 // K splits of the 128 x 128 kernel for a product with few tiles and a long K, plain or fused; 1 = no split.  A tile's K loop is
@@ -1897,8 +1904,12 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   Workspace workspace;
   float *partials = nullptr;
   int splits = 1;
+  bool whole_in_chunks = false;
   if (tiled && tile_choice == 128 && nm > 0 && !half) {
-    splits = splitk_for(m, n, k, Epi != EPI_STORE);
+    const TileTime time(m, n, k, Epi != EPI_STORE);
+    splits = splitk_for(m, n, k, time);
+    whole_in_chunks = Epi == EPI_STORE && splits == 1 && tunable("gemm16.split_k", 0) != 1 && tunable("gemm16.tile", 0) == 0 &&
+                      time.whole_in_chunks(k);
     if (splits > 1 && (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n)) {
       workspace = splitk_workspace(st);
       partials = workspace.block;
@@ -1974,21 +1985,21 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   } else if (nm > 0 && tile_choice == 128) {
     const int sm = (m + 127) / 128, sn = (nm + 127) / 128;
     unsigned long long *sprobe = clock_probe(static_cast<int64_t>(sm) * sn);
-    if (splits > 1) {
-      const int piece = splitk_chunk(k, 64, splits);
+    if (splits > 1 || whole_in_chunks) {
+      const int piece = splits > 1 ? splitk_chunk(k, 64, splits) : k;
       auto launch_pieces = [&]<int Chunk>(std::integral_constant<int, Chunk>) {
         if (ragged)
           hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, true, Chunk>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
-                             nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, piece, partials, n, nullptr);
+                             nullptr, nullptr, m, nm, k, sm, sn, remap, splits > 1 ? nullptr : sprobe, piece, partials, n, nullptr);
         else
           hipLaunchKernelGGL((gemm16_m16_small_kernel<Bf16, EPI_STORE, false, Chunk>), dim3(sm * sn, splits), dim3(256), 0, st, a, b, c,
-                             nullptr, nullptr, m, nm, k, sm, sn, remap, nullptr, piece, partials, n, nullptr);
+                             nullptr, nullptr, m, nm, k, sm, sn, remap, splits > 1 ? nullptr : sprobe, piece, partials, n, nullptr);
       };
       if (piece < kLongPiece) launch_pieces(std::integral_constant<int, 2>{});
       else launch_pieces(std::integral_constant<int, 4>{});
       rc = check_launch("gemm16 kernel launch");
       if (rc != SAREK_HIP_OK) return rc;
-      if constexpr (Epi == EPI_STORE) rc = launch_splitk_reduce(partials, c, m, n, splits, st);
+      if constexpr (Epi == EPI_STORE) rc = splits > 1 ? launch_splitk_reduce(partials, c, m, n, splits, st) : rc;
       else return launch_splitk_reduce_fused(partials, bias, c, rowsum, m, n, splits, st);
     } else {
       const RowFold fold = fold_in(sm, static_cast<int64_t>(sm) * sn, 2 * compute_units());

@@ -801,6 +801,27 @@ def test_pieces_on_the_tile_are_as_exact_as_the_few_rows_kernel(hip, torch_cuda,
     assert error[1] <= error[2]
 
 
+@pytest.mark.parametrize("m,n,k", [(12, 30926, 5817), (147, 11697, 7903), (3, 22530, 3811), (26, 32567, 7232)])
+def test_long_k_that_is_not_cut_is_summed_in_chunks(hip, torch_cuda, m, n, k):
+    """Products of a long K and a small C that are not cut: their mean square error is at most half of the single chain's
+    (which gemm16.split_k = 1 keeps), as that of K in two pieces is."""
+    torch = torch_cuda
+    torch.manual_seed(m + k)
+    a, b = ((torch.randn(shape, device="cuda") * 0.02).half() for shape in ((m, k), (k, n)))
+    ref = a.double() @ b.double()
+    assert hip.gemm16_tile(m, n, k) == 128 and hip.gemm16_k_splits(m, n, k) == 1
+    got = hip.gemm_f16(a, b)
+    assert torch.equal(got, hip.gemm_f16(a, b))
+    try:
+        hip.set_tunable("gemm16.rows", 1)
+        hip.set_tunable("gemm16.split_k", 1)
+        chain = hip.gemm_f16(a, b)
+    finally:
+        hip.set_tunable("gemm16.rows", 0)
+        hip.set_tunable("gemm16.split_k", 0)
+    assert (got.double() - ref).pow(2).mean() <= 0.5 * (chain.double() - ref).pow(2).mean()
+
+
 @pytest.mark.parametrize("m,n,k,fused", [(320, 2880, 2793, False), (300, 2306, 2479, True)])
 def test_gemm16_product_that_cannot_be_cut(hip, torch_cuda, m, n, k, fused):
     """On the tile for its pieces of K, which a captured call has no block for: there the few-rows kernel computes it, whole; the row
