@@ -1741,11 +1741,12 @@ struct TileTime {
 // fit kSplitWorkspaceBytes.  (Powers of two by one slab's time whatever the rows, as it was, cost those products 3.9 % on the
 // average over the best count and kernel, this 0.7 %; us, then and now: 1561 x 1280 x 8121, 4 pieces and 3, 75 and 57; 522 x 2053 x
 // 4672, 4 and 3, 29.8 and 23.3; 1062 x 320 x 1984, 1 and 4, 15.4 and 12.1.)
-// gemm16.split_k: 0 = this rule (and K whole on a tile that gemm16.tile asks for), 1 = never, n >= 2 forces n where the shape
-// allows it.
+// gemm16.split_k: 0 = this rule, 1 = never, n >= 2 forces n where the shape allows it.  A tile that gemm16.tile asks for takes K whole
+// unless it is long against C (the line below which pieces of 256 and more, of a power of two, were never worth their planes): the tiles
+// are compared by their bits there.
 int splitk_for(int m, int n, int k, const TileTime &time) {
   const int64_t forced = tunable("gemm16.split_k", 0);
-  if (forced == 1 || (forced == 0 && tunable("gemm16.tile", 0) != 0)) return 1;
+  if (forced == 1 || (forced == 0 && tunable("gemm16.tile", 0) != 0 && k < 1500.0 + 640.0 * time.c_mb)) return 1;
   const int64_t fit = std::min<int64_t>(static_cast<int64_t>(kSplitWorkspaceBytes) / (splitk_plane_floats(m, n) * 4), k / 64);
   return splitk_pieces(k, 64, forced >= 2 ? std::max<int64_t>(1, std::min<int64_t>(forced, fit)) : time.best(fit));
 }
@@ -1908,8 +1909,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   if (tiled && tile_choice == 128 && nm > 0 && !half) {
     const TileTime time(m, n, k, Epi != EPI_STORE);
     splits = splitk_for(m, n, k, time);
-    whole_in_chunks = Epi == EPI_STORE && splits == 1 && tunable("gemm16.split_k", 0) != 1 && tunable("gemm16.tile", 0) == 0 &&
-                      time.whole_in_chunks(k);
+    whole_in_chunks = Epi == EPI_STORE && splits == 1 && tunable("gemm16.split_k", 0) != 1 && time.whole_in_chunks(k);
     if (splits > 1 && (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n)) {
       workspace = splitk_workspace(st);
       partials = workspace.block;

@@ -52,7 +52,7 @@ def test_16_bit_products_of_few_rows_go_where_they_are_faster(hip, m, n, k, kern
                                           (4096, 2048, 1000, 1), (128, 30000, 6000, 1), (1920, 4000, 8192, 1)])
 def test_pieces_of_k_on_the_small_tile(hip, knobs, m, n, k, pieces):
     """The count with the lowest estimate: workgroups that fit the CUs twice over, planes that fit the workspace, a stage of 64 each;
-    K stays whole on a tile that is asked for by name."""
+    where the tile is asked for by name, K is whole unless it is long against C."""
     knobs("gemm16.rows", 1)
     tiles, seen = -(-m // 128) * -(-n // 128), hip.gemm16_k_splits(m, n, k)
     assert seen == pieces
@@ -61,7 +61,15 @@ def test_pieces_of_k_on_the_small_tile(hip, knobs, m, n, k, pieces):
         assert s == 1 or (s <= 16 and tiles * s <= 512 and 4 * m * n * s <= 64 << 20 and longer // s >= 64)
     if hip.gemm16_tile(m, n, k) == 128:
         knobs("gemm16.tile", 128)
-        assert hip.gemm16_k_splits(m, n, k) == 1
+        assert hip.gemm16_k_splits(m, n, k) == (pieces if k >= 1500 + 640 * m * n * 4e-6 else 1)
+
+
+@pytest.mark.parametrize("m,n,k,pieces", [(64, 64, 1536, 4), (256, 256, 8192, 16), (16, 8192, 8192, 8), (100, 256, 1536, 1), (130, 520, 1600, 1)])
+def test_pieces_of_k_on_a_tile_asked_for_by_name(hip, knobs, m, n, k, pieces):
+    """A K that is long against C is cut there too, into half as many pieces at least as when they were powers of two (a sum in chunks
+    is the more exact by more than that)."""
+    knobs("gemm16.tile", 128)
+    assert (hip.gemm16_k_splits(m, n, k) == 1) == (pieces == 1) and 2 * hip.gemm16_k_splits(m, n, k) >= pieces
 
 
 @pytest.mark.parametrize("m,n,k,columns", [
