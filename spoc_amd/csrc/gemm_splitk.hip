@@ -62,8 +62,11 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
 }
 
 // The same for the fused product: y = relu(sum of the planes + bias), and the row's sum of y, in double, in a fixed order.  Waves
-// of the four of a workgroup to a row: one where a wave's four columns a lane are a quarter of it at least, or four.  Bound by the trip
-// to the planes, which the products have left in the caches: every row is asked for at once.
+// of the four of a workgroup to a row: one or four.  Bound by the trips to the planes, which the products have left in the caches: a wave
+// takes 256 columns a turn, so of more it makes several trips where four waves make one.  Us, one wave and four: 205 x 875 x 6932 22.9 and
+// 20.2 (20.9 before such products were cut), 133 x 958 x 4595 20.1 and 16.8, 300 x 300 x 4000 13.9 and 13.1; up to 256 columns three of the
+// four would have none (2000 x 150 x 3000 16.1 and 17.4), and many rows of up to 512 had better be fewer workgroups (2690 x 350 x 7071
+// 42.0 and 43.2, 1472 x 384 x 1600 15.2 and 14.7).
 template <int Waves>
 __global__ __launch_bounds__(256) void splitk_reduce_fused_kernel(const float *__restrict__ partials, const float *__restrict__ bias,
                                                                   float *__restrict__ y, float *__restrict__ rowsum, int m, int n,
@@ -175,7 +178,7 @@ int launch_splitk_reduce(const float *partials, float *c, int m, int n, int spli
 int launch_splitk_reduce_fused(const float *partials, const float *bias, float *y, float *rowsum, int m, int n, int splits,
                                hipStream_t st) {
   const int64_t plane = splitk_plane_floats(m, n);
-  if (n > 1024)
+  if (n > 512 || (n > 256 && m <= 2048))
     hipLaunchKernelGGL(splitk_reduce_fused_kernel<4>, dim3(m), dim3(256), 0, st, partials, bias, y, rowsum, m, n, plane, splits);
   else
     hipLaunchKernelGGL(splitk_reduce_fused_kernel<1>, dim3((m + 3) / 4), dim3(256), 0, st, partials, bias, y, rowsum, m, n, plane,
