@@ -407,9 +407,9 @@ bool gemm16_rows_serves(int m, int n, int k) {
 
 // Microseconds of a product of 17 to 64 rows whose B is new to the caches, by an estimate read off 800 drawn ones (9 % rms): the steps of the CU with the
 // most workgroups by how A's and B's rows lie, against B from memory (whose stream the registers of more row blocks leave
-// fewer loads in flight), and the sums.
-double narrow_time(const Shape &s, int n, int k, int splits) {
-  const int align = k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2, b_align = n % 8 == 0 ? 0 : 1 + n % 2;
+// fewer loads in flight), and the sums.  coarse: B's share by how A's rows lie too.
+double narrow_time(const Shape &s, int n, int k, int splits, bool coarse = false) {
+  const int align = k % 8 == 0 && n % 8 == 0 ? 0 : k % 2 == 0 && n % 2 == 0 ? 1 : 2, b_align = coarse ? align : n % 8 == 0 ? 0 : 1 + n % 2;
   constexpr double kStep[] = {0.0125, 0.0147, 0.0288}, kMegabyte[] = {0.124, 0.147, 0.164};
   const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
   const double steps = rounds * s.steps / splits * kStep[align] * (4.0 + s.mt);
@@ -445,7 +445,7 @@ bool whole_on_the_tile(const Shape &s, int m, int n, int k, bool fused) {
                              : 5.5 + slabs * kSlab[align] + 0.62 * planes;
   const double launch = pieces == 1 ? 0.0 : narrow ? 4.0 : 3.0;
   const int splits = rows_splits_for(s, n, k);
-  if (narrow) return narrow_time(s, n, k, splits) >= 1.05 * (tile + launch);
+  if (narrow) return narrow_time(s, n, k, splits, true) >= 1.05 * (tile + launch);
   const double rounds = static_cast<double>((s.tiles * splits + cus - 1) / cus);
   const double here = (on16 ? 6.0 : 4.5) + rounds * s.steps / splits * (on16 ? 0.055 : on4 ? 0.07 : 0.12) * s.mt +
                       (splits > 1 ? 2.5 + 0.15 * splits + 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0);

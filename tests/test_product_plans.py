@@ -42,7 +42,8 @@ def test_16_bit_pieces_forced_where_there_is_no_room(hip, knobs, m, n, k, room, 
 @pytest.mark.parametrize("m,n,k,kernel", [(64, 27136, 2432, 128), (64, 20992, 4160, 128), (51, 7969, 5857, 128), (64, 29028, 2725, 128),
                                           (64, 31360, 2624, 128), (256, 1280, 191, 128), (723, 1702, 256, 128),
                                           (16, 30000, 4096, 128), (16, 30016, 4096, 64), (16, 27136, 2432, 64), (16, 8192, 8192, 64), (32, 4096, 4096, 64), (48, 4096, 1024, 64),
-                                          (64, 1001, 1001, 64), (64, 576, 1064, 64), (77, 2332, 1920, 64), (130, 4608, 140, 64)])
+                                          (64, 1001, 1001, 64), (64, 576, 1064, 64), (62, 23936, 1305, 128), (60, 20992, 2483, 128),
+                                          (35, 27888, 858, 128), (38, 24064, 2749, 128), (77, 2332, 1920, 64), (130, 4608, 140, 64)])
 def test_16_bit_products_of_few_rows_go_where_they_are_faster(hip, m, n, k, kernel):
     """The few-rows kernel (64) or the 128 x 128 tile, whichever was measured to be the faster at these sizes."""
     assert hip.gemm16_tile(m, n, k) == kernel
