@@ -418,14 +418,44 @@ double narrow_time(const Shape &s, int n, int k, int splits, bool coarse = false
          (splits > 1 ? 1.17 + 0.31 * splits : 0.0);
 }
 
-// An element is one sum on the 128 x 128 tile with K whole and eight or more here, and its error there up to 2.8 times as large
-// (1280 x 1134 x 566 1.8); in pieces the tile's sums are chunked and as exact as here, up to 2048 of K (37 x 9856 x 7744, 3 pieces, 1.12).
-bool less_exact(int k, int tile_splits) { return tile_splits == 1 || k > 2048 * static_cast<int64_t>(tile_splits); }
+// What does not go by estimates.  Up to 16 rows always here, but for more than 128 MiB of B in one piece of K whose rows, of an even N, share
+// lines: there the tile's transfers into LDS come in better (16 x 30000 x 4096 43.2 on the tile, 49.9 here; elsewhere the tile was
+// the faster by 4 % on 4 of 400 drawn products, operands new to the caches, this kernel by a quarter on average).  To 64 a workgroup's
+// sums through LDS cost it 0.5 us per 16 rows and its registers leave room for one workgroup per CU, so short K and more
+// column tiles than CUs belong to the 128 x 128 tile unless N is odd (us, 128 tile / here):
+//   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
+//   48 x 4096 x 256 6.2 / 6.1, 48 x 4096 x 1024 10.2 / 9.4, 48 x 40000 x 1024 23.0 / 26.4, 48 x 40001 x 1024 35.3 / 33.4
+//   64 x 4096 x 256 6.4 / 7.2, 64 x 4096 x 1024 10.5 / 10.5, 64 x 4096 x 4096 17.3 / 15.6, 64 x 40001 x 1024 36.3 / 37.0
+// An odd N of up to 8 column tiles stays here (49 x 255 x 4129 13.5 / 15.1, 64 x 1001 x 1001 15.7 / 11.4), 17 to 32 rows against up to 96
+// column tiles do (one of 576 more than 10 % slower), and so does a product whose pieces gemm16.rows_splits sets.  Beyond 64 rows, and with
+// the fused epilogue at any number, its tiles have to fit the CUs in one round (882 x 2401 x 4259, 266 tiles: 50 us on the other tile, 108
+// here) and half of the waves to have a step at least (in tiles of 64 rows some wave two: 256 x 1280 x 191 6.8 / 8.4, 723 x 1702 x 256 7.2 /
+// 7.9, as 21 of 118 drawn products, all but 3 of them so short).
+enum class Kernel { rows, tile, by_estimate };
+bool narrow_counts(const Shape &s, int m, int n) {
+  return m > 16 && m <= kTileRows && s.col_tiles > (s.mt == 2 ? 96 : n % 2 != 0 ? 8 : 0) && tunable("gemm16.rows_splits", 0) == 0;
+}
+Kernel outright(const Shape &s, int m, int n, int k, bool fused) {
+  if (m > kTileRows || fused)
+    return s.tiles > compute_units() || 2 * s.steps < kWaves || (s.mt == 4 && s.steps <= kWaves) ? Kernel::tile : Kernel::by_estimate;
+  const bool odd = n % 2 != 0, one_round = s.col_tiles <= compute_units();
+  bool here = true;
+  switch (s.mt) {
+    case 1:
+      here = n % 64 == 0 || odd || static_cast<int64_t>(k) * n * 2 <= (int64_t{128} << 20) || rows_splits_for(s, n, k) > 1 ||
+             tunable("gemm16.rows_splits", 0) != 0;
+      return here ? Kernel::rows : Kernel::tile;
+    case 2: here = odd || one_round; break;
+    case 3: here = one_round ? odd || k >= 512 : odd && k >= 1024; break;
+    default: here = one_round && (odd || k >= 1024);
+  }
+  return !here ? Kernel::tile : narrow_counts(s, m, n) ? Kernel::by_estimate : Kernel::rows;
+}
 
-// So a product does not go there for a few per cent where it would be less exact, or cannot be cut: only where coarser estimates,
-// that put this kernel up to 2 us too low, have the tile, in 1 to 16 pieces of a plain product, ahead as well.
-bool whole_on_the_tile(const Shape &s, int m, int n, int k, bool fused) {
-  const bool on16 = k % 8 == 0 && n % 8 == 0, on4 = k % 2 == 0 && n % 2 == 0, narrow = m <= kTileRows && !fused;
+// The same by coarser estimates of both kernels, that put this one up to 2 us too low, of the tile in 1 to 16 pieces of a plain product,
+// powers of two: what decides where the tile would be the less exact, and where a product cannot be cut.
+bool coarsely_on_the_tile(const Shape &s, int m, int n, int k, bool fused, int splits) {
+  const bool on16 = k % 8 == 0 && n % 8 == 0, on4 = k % 2 == 0 && n % 2 == 0, narrow = narrow_counts(s, m, n);
   const int align = k % 64 == 0 && n % 8 == 0 ? 0 : on16 ? 1 : on4 ? 2 : 3, cus = compute_units();
   constexpr double kSlab[] = {0.19, 0.19, 0.24, 0.33}, kNarrowSlab[] = {0.172, 0.257, 0.272, 0.334}, kMegabyte[] = {0.156, 0.125, 0.134, 0.155};
   const int64_t tiles = static_cast<int64_t>((m + 127) / 128) * s.col_tiles;
@@ -439,80 +469,60 @@ bool whole_on_the_tile(const Shape &s, int m, int n, int k, bool fused) {
   double lowest = 0.9 * cut_time(1);
   for (int64_t t = 2; !fused && t <= 16 && tiles * t <= 2 * cus && k / t >= 256; t *= 2)
     if (cut_time(t) < lowest) lowest = cut_time(t), pieces = t;
+  pieces = splitk_pieces(k, 64, pieces);
   const double slabs = k / 32.0 / static_cast<double>(pieces), planes = pieces > 1 ? static_cast<double>(pieces) * c_mb : 0.0;
-  const double chain = slabs * kNarrowSlab[align] * static_cast<double>((tiles * pieces + cus - 1) / cus);
-  const double tile = narrow ? 5.17 + std::cbrt(chain * chain * chain + memory * memory * memory) + 0.28 * c_mb + 0.38 * planes
-                             : 5.5 + slabs * kSlab[align] + 0.62 * planes;
-  const double launch = pieces == 1 ? 0.0 : narrow ? 4.0 : 3.0;
-  const int splits = rows_splits_for(s, n, k);
-  if (narrow) return narrow_time(s, n, k, splits, true) >= 1.05 * (tile + launch);
+  if (narrow) {
+    const double chain = slabs * kNarrowSlab[align] * static_cast<double>((tiles * pieces + cus - 1) / cus);
+    const double tile = 5.17 + std::cbrt(chain * chain * chain + memory * memory * memory) + 0.28 * c_mb + 0.38 * planes + (pieces == 1 ? 0.0 : 4.0);
+    const bool behind = narrow_time(s, n, k, splits, true) >= 1.05 * tile;
+    if (behind || !fused) return behind;
+  }
   const double rounds = static_cast<double>((s.tiles * splits + cus - 1) / cus);
   const double here = (on16 ? 6.0 : 4.5) + rounds * s.steps / splits * (on16 ? 0.055 : on4 ? 0.07 : 0.12) * s.mt +
                       (splits > 1 ? 2.5 + 0.15 * splits + 2.0 * static_cast<double>(splits * s.plane) / 2.7e6 : 0.0);
-  return here >= tile + launch;
+  return here >= 5.5 + slabs * kSlab[align] + 0.62 * planes + (pieces == 1 ? 0.0 : 3.0);
 }
 
-// Whether it should.  Up to 16 rows always, but for more than 128 MiB of B in one piece of K whose rows, of an even N, share
-// lines: there the tile's transfers into LDS come in better (16 x 30000 x 4096 43.2 on the tile, 49.9 here; elsewhere the tile was
-// the faster by 4 % on 4 of 400 drawn products, operands new to the caches, this kernel by a quarter on average).  To 64 a workgroup's
-// sums through LDS cost it 0.5 us per 16 rows and its registers leave room for one workgroup per CU, so short K and more
-// column tiles than CUs belong to the 128 x 128 tile unless N is odd (us, 128 tile / here):
-//   32 x 512 x 64 4.8 / 4.0, 32 x 4096 x 4096 15.7 / 12.0, 32 x 40000 x 1024 22.0 / 23.8, 32 x 40001 x 1024 34.5 / 29.9
-//   48 x 4096 x 256 6.2 / 6.1, 48 x 4096 x 1024 10.2 / 9.4, 48 x 40000 x 1024 23.0 / 26.4, 48 x 40001 x 1024 35.3 / 33.4
-//   64 x 4096 x 256 6.4 / 7.2, 64 x 4096 x 1024 10.5 / 10.5, 64 x 4096 x 4096 17.3 / 15.6, 64 x 40001 x 1024 36.3 / 37.0
-// and so does what the estimates of both kernels (other: the tile's) put 4 % apart the other way, of up to 8 column tiles 25 %, B being new to the
-// caches as in a program's loop over its weights (again and again the same B favours the tile more): 33 to 64 rows against one
-// to two hundred column tiles most of all (us, tile / here): 64 x 29028 x 2725 45.2 / 51.8, 51 x 7969 x 5857 29.5 / 34.4,
-// 63 x 17239 x 320 7.6 / 9.5, 42 x 17830 x 3328 32.4 / 40.0.  Of 900 products drawn afresh 85 were more than 5 % slower here than
-// there without estimates and 43 with them (profiles/gemm16_rows_vs_tile.txt); the tile's in any count of pieces put 10 in 167
-// right and two wrong.  An odd N of
-// up to 8 column tiles stays here whatever they say (49 x 255 x 4129 13.5 / 15.1, 64 x 1001 x 1001 15.7 / 11.4), 17 to 32 rows
-// against up to 96 column tiles do (one of 576 more than 10 % slower), and so does a product whose pieces gemm16.rows_splits sets.
-// Beyond 64 rows, and with the fused epilogue at any number, where its tiles fit the CUs in one round (882 x 2401 x 4259,
-// 266 tiles: 50 us on the other tile, 108 here), at least half of the waves have a step (in tiles of 64 rows some wave has
-// two: 256 x 1280 x 191 6.8 / 8.4, 723 x 1702 x 256 7.2 / 7.9, as 21 of 118 drawn products, all but 3 of them so short), and its
-// time is below the 128 x 128 tile's by both estimates: a step costs by how A's and B's rows lie.  They were read off 292 plain
-// and 704 fused drawn products run on both (5 % rms, the tile's 8 and 9): 139 x 2432 x 1416 12.0 on the tile, 9.5 here,
-// 114 x 5824 x 2687 15.9, 27.2, fused 419 x 1472 x 2504 25.5, 17.4, 180 x 256 x 2240 10.0, 13.9; of 430
-// drawn afresh 14 are more than 5 % slower than by the rules before, most of them launches of 6 us.  `other`: what the tiled kernel is estimated at.
+// An element is one sum on the 128 x 128 tile with K whole and eight or more here, and its error there up to 2.8 times as large
+// (1280 x 1134 x 566 1.8); in pieces the tile's sums are chunked and as exact as here, up to 2048 of K (37 x 9856 x 7744, 3 pieces, 1.12).
+bool less_exact(int k, int tile_splits) { return tile_splits == 1 || k > 2048 * static_cast<int64_t>(tile_splits); }
+
+// Whether a product goes here: by what both kernels are estimated to take, B being new to the caches as in a program's loop over its
+// weights (again and again the same B favours the tile more).  17 to 64 rows, us, tile and here: 64 x 29028 x 2725 45.2, 51.8, 51 x 7969 x
+// 5857 29.5, 34.4, 63 x 17239 x 320 7.6, 9.5, 42 x 17830 x 3328 32.4, 40.0 (4 % to this kernel's favour, 25 % of up to 8 column tiles:
+// profiles/gemm16_rows_vs_tile.txt).  Beyond, and fused, a step costs by how A's and B's rows lie: read off 292 plain and 704 fused drawn
+// products run on both (5 % rms, the same on 4000 drawn later; from three quarters of the CUs on 178 of those took 5 % longer): 139 x 2432 x
+// 1416 12.0 on the tile, 9.5 here, 114 x 5824 x 2687 15.9, 27.2, fused 419 x 1472 x 2504 25.5, 17.4, 180 x 256 x 2240 10.0, 13.9.  Where
+// that moved a product it is 9 % (plain) and 16 % (fused) faster on the average, 3 % of the 6000 looked at are more than 5 % slower.  Fitting it
+// all again to those 6000 moves as many the wrong way as the right one.  `other`: what the tiled kernel is estimated at.
 bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other) {
   const Shape s = shape_of(m, n, k, fused);
-  if (m <= kTileRows && !fused) {
-    const bool odd = n % 2 != 0, one_round = s.col_tiles <= compute_units();
-    bool here = true;
-    switch (s.mt) {
-      case 1:
-        return n % 64 == 0 || odd || static_cast<int64_t>(k) * n * 2 <= (int64_t{128} << 20) || rows_splits_for(s, n, k) > 1 ||
-               tunable("gemm16.rows_splits", 0) != 0;
-      case 2: here = odd || one_round; break;
-      case 3: here = one_round ? odd || k >= 512 : odd && k >= 1024; break;
-      default: here = one_round && (odd || k >= 1024);
-    }
-    if (!here) return false;
-  }
-  if (m > 16 && m <= kTileRows && s.col_tiles > (s.mt == 2 ? 96 : n % 2 != 0 ? 8 : 0) && tunable("gemm16.rows_splits", 0) == 0 &&
-      narrow_time(s, n, k, rows_splits_for(s, n, k)) >= (s.col_tiles > 8 ? 1.04 : 1.25) * other(m, n, k, fused).us)
-    return less_exact(k, other(m, n, k, fused).splits) && !whole_on_the_tile(s, m, n, k, fused);
-  if (m <= kTileRows && !fused) return true;
-  if (s.tiles > compute_units() || 2 * s.steps < kWaves || (s.mt == 4 && s.steps <= kWaves)) return false;
+  const Kernel kernel = outright(s, m, n, k, fused);
+  if (kernel != Kernel::by_estimate) return kernel == Kernel::rows;
+  const Gemm16Time tile = other(m, n, k, fused);
   const int splits = rows_splits_for(s, n, k);
-  struct Fit { double step[5], memory[2], base, rows, sums, piece, plane; };
-  constexpr Fit kPlain = {{0.0479, 0.0501, 0.0657, 0.0895, 0.105}, {0.091, 0.132}, 2.34, 0.878, 1.01, 0.285, 0.246};
-  constexpr Fit kFused = {{0.0489, 0.0487, 0.0638, 0.0884, 0.11}, {0.133, 0.193}, 4.4, 1.186, 0.51, 0.228, 0.335};
-  const Fit &f = fused ? kFused : kPlain;
-  const int align = k % 8 == 0 && n % 8 == 0 ? 0 : 1 + 2 * (k % 2) + n % 2;
-  const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
-  const double steps = rounds * s.steps / splits * s.mt * f.step[align], memory = static_cast<double>(k) * n * 2e-6 * f.memory[n % 8 != 0];
-  const double here = f.base + f.rows * s.mt + std::sqrt(steps * steps + memory * memory) +
-                      (splits > 1 ? f.sums + splits * (f.piece + f.plane * 1e-6 * static_cast<double>(s.plane)) : 0.0);
-  const Gemm16Time tile = other(m, n, k, fused);   // (1.06: 1728 x 1034 x 1664 15.8 on the tile, 18.2 here)
-  return here * (s.tiles > 192 ? 1.06 : 1.0) < tile.us || (less_exact(k, tile.splits) && !whole_on_the_tile(s, m, n, k, fused));
+  double ratio = 0.0;   // this kernel's time over the tile's
+  if (narrow_counts(s, m, n)) ratio = narrow_time(s, n, k, splits) / (s.col_tiles > 8 ? 1.04 : 1.25) / tile.us;
+  if (m > kTileRows || fused) {
+    struct Fit { double step[5], memory[2], base, rows, sums, piece, plane; };
+    constexpr Fit kPlain = {{0.0479, 0.0501, 0.0657, 0.0895, 0.105}, {0.091, 0.132}, 2.34, 0.878, 1.01, 0.285, 0.246};
+    constexpr Fit kFused = {{0.0489, 0.0487, 0.0638, 0.0884, 0.11}, {0.133, 0.193}, 4.4, 1.186, 0.51, 0.228, 0.335};
+    const Fit &f = fused ? kFused : kPlain;
+    const int align = k % 8 == 0 && n % 8 == 0 ? 0 : 1 + 2 * (k % 2) + n % 2;
+    const double rounds = static_cast<double>((s.tiles * splits + compute_units() - 1) / compute_units());
+    const double steps = rounds * s.steps / splits * s.mt * f.step[align], memory = static_cast<double>(k) * n * 2e-6 * f.memory[n % 8 != 0];
+    const double here = f.base + f.rows * s.mt + std::sqrt(steps * steps + memory * memory) +
+                        (splits > 1 ? f.sums + splits * (f.piece + f.plane * 1e-6 * static_cast<double>(s.plane)) : 0.0);
+    ratio = std::max(ratio, here * (4 * s.tiles > 3 * compute_units() ? 1.06 : 1.0) / tile.us);
+  }
+  return ratio < 1.0 || (less_exact(k, tile.splits) && !coarsely_on_the_tile(s, m, n, k, fused, splits));
 }
 
 bool gemm16_rows_more_exact(int m, int n, int k, bool fused) {
   const Shape s = shape_of(m, n, k, fused);
-  if (m <= kTileRows && !fused ? s.col_tiles > compute_units() : s.tiles > compute_units() || 2 * s.steps < kWaves) return false;
-  return !whole_on_the_tile(s, m, n, k, fused);
+  const Kernel kernel = outright(s, m, n, k, fused);
+  if (kernel != Kernel::by_estimate) return kernel == Kernel::rows;
+  return !coarsely_on_the_tile(s, m, n, k, fused, rows_splits_for(s, n, k));
 }
 
 int gemm16_rows_k_splits(int m, int n, int k) { return rows_splits_for(shape_of(m, n, k, false), n, k); }

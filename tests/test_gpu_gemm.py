@@ -864,6 +864,32 @@ def test_gemm16_product_that_cannot_be_cut(hip, torch_cuda, m, n, k, fused):
         assert torch.equal(y, eager)
 
 
+@pytest.mark.parametrize("m,n,k", [(61, 512, 859), (59, 320, 767)])
+def test_gemm16_product_that_cannot_be_cut_and_is_too_short_for_the_few_rows_kernel(hip, torch_cuda, m, n, k):
+    """49 to 64 rows and a K below 1024 are the tile's whether K can be cut or not: in a graph it runs whole there."""
+    torch = torch_cuda
+    torch.manual_seed(m + n)
+    a, b = ((torch.randn(shape, device="cuda") * 0.02).half() for shape in ((m, k), (k, n)))
+    assert hip.gemm16_tile(m, n, k) == 128 and hip.gemm16_k_splits(m, n, k) > 1
+    try:
+        hip.set_tunable("gemm16.tile", 128)
+        hip.set_tunable("gemm16.split_k", 1)
+        whole = hip.gemm_f16(a, b)
+    finally:
+        hip.set_tunable("gemm16.tile", 0)
+        hip.set_tunable("gemm16.split_k", 0)
+    c, side, graph = torch.empty_like(whole), side_stream(torch), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        hip.gemm_f16(a, b, out=c)
+    for _ in range(3):
+        c.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, whole)
+        hip.gemm_f16(a, b)
+
+
 @pytest.mark.parametrize("m,n,k", [(300, 2306, 2479), (110, 2049, 7936), (128, 128, 64)])
 def test_captured_fused_product_clears_its_row_sums_once(hip, torch_cuda, m, n, k):
     """A graph of one fused product holds two kernels, whichever would have cut K: the row sums' clearing and the product."""
