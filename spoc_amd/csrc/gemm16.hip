@@ -1731,8 +1731,14 @@ struct TileTime {
   // before any count of them was looked at; whole they are faster, but one chain of K has 1.4 times the error of two (rms over the largest
   // element, cut in two, whole, in chunks: 49 x 26100 x 6961 7.8e-8, 10.9e-8, 3.2e-8; us 101.1, 100.7, 100.7; 12 x 30926 x 5817 82.6, 63.6,
   // 64.0; 84 x 21952 x 8129 109.8, 97.6, 99.5).  The line takes the 471 such of 400000 drawn products and two others.  Elsewhere chunks cost up
-  // to 5 % (4457 x 448 x 3264 23.5 and 24.6).
-  bool whole_in_chunks(int k) const { return tiles <= cus && k >= 3000.0 + 640.0 * c_mb; }
+  // to 5 % (4457 x 448 x 3264 23.5 and 24.6).  And 17 to 64 rows, on about half of the CUs
+  // and more, of an A whose rows start at other places than B's: the few-rows kernel's finer estimate has it ahead there, up to two thirds
+  // wrongly (62 x 18432 x 1897 32.4 us, here in one chain 19.1, in chunks 19.7), but its sums are short (2.4e-8, 5.6e-8, 2.2e-8).  With fewer
+  // tiles the chunks cost 12 % of a short K (53 x 960 x 778 9.6 and 10.7).
+  bool whole_in_chunks(int m, int n, int k) const {
+    const bool apart = (n % 8 == 0 && k % 8 != 0) || (n % 2 == 0 && k % 2 != 0);
+    return tiles <= cus && (k >= 3000.0 + 640.0 * c_mb || (k >= 512 && m > 16 && m <= 64 && apart && 2 * tiles > cus - 8));
+  }
 };
 
 // K splits of the 128 x 128 kernel for a product with few tiles and a long K, plain or fused; 1 = no split.  A tile's K loop is
@@ -1909,7 +1915,7 @@ int launch_gemm16(const uint16_t *a, const uint16_t *b, float *c, const float *b
   if (tiled && tile_choice == 128 && nm > 0 && !half) {
     const TileTime time(m, n, k, Epi != EPI_STORE);
     splits = splitk_for(m, n, k, time);
-    whole_in_chunks = Epi == EPI_STORE && splits == 1 && tunable("gemm16.split_k", 0) != 1 && time.whole_in_chunks(k);
+    whole_in_chunks = Epi == EPI_STORE && splits == 1 && tunable("gemm16.split_k", 0) != 1 && time.whole_in_chunks(m, n, k);
     if (splits > 1 && (Epi == EPI_STORE ? reinterpret_cast<uintptr_t>(c) % 16 == 0 : nm == n)) {
       workspace = splitk_workspace(st);
       partials = workspace.block;

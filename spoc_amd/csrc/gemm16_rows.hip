@@ -453,8 +453,9 @@ Kernel outright(const Shape &s, int m, int n, int k, bool fused) {
 }
 
 // The same by coarser estimates of both kernels, that put this one up to 2 us too low, of the tile in 1 to 16 pieces of a plain product,
-// powers of two: what decides where the tile would be the less exact, and where a product cannot be cut.
-bool coarsely_on_the_tile(const Shape &s, int m, int n, int k, bool fused, int splits) {
+// powers of two: what decides where the tile would be the less exact, and where a product cannot be cut.  pieces_asked: it is about pieces
+// of more than 2048 of K, for which this kernel is not left where its finer estimate of 17 to 64 rows has it ahead.
+bool coarsely_on_the_tile(const Shape &s, int m, int n, int k, bool fused, int splits, bool pieces_asked = false) {
   const bool on16 = k % 8 == 0 && n % 8 == 0, on4 = k % 2 == 0 && n % 2 == 0, narrow = narrow_counts(s, m, n);
   const int align = k % 64 == 0 && n % 8 == 0 ? 0 : on16 ? 1 : on4 ? 2 : 3, cus = compute_units();
   constexpr double kSlab[] = {0.19, 0.19, 0.24, 0.33}, kNarrowSlab[] = {0.172, 0.257, 0.272, 0.334}, kMegabyte[] = {0.156, 0.125, 0.134, 0.155};
@@ -474,7 +475,7 @@ bool coarsely_on_the_tile(const Shape &s, int m, int n, int k, bool fused, int s
   if (narrow) {
     const double chain = slabs * kNarrowSlab[align] * static_cast<double>((tiles * pieces + cus - 1) / cus);
     const double tile = 5.17 + std::cbrt(chain * chain * chain + memory * memory * memory) + 0.28 * c_mb + 0.38 * planes + (pieces == 1 ? 0.0 : 4.0);
-    const bool behind = narrow_time(s, n, k, splits, true) >= 1.05 * tile;
+    const bool behind = narrow_time(s, n, k, splits, !pieces_asked) >= 1.05 * tile;
     if (behind || !fused) return behind;
   }
   const double rounds = static_cast<double>((s.tiles * splits + cus - 1) / cus);
@@ -515,7 +516,7 @@ bool gemm16_rows_pays(int m, int n, int k, bool fused, Gemm16Estimate other) {
                         (splits > 1 ? f.sums + splits * (f.piece + f.plane * 1e-6 * static_cast<double>(s.plane)) : 0.0);
     ratio = std::max(ratio, here * (4 * s.tiles > 3 * compute_units() ? 1.06 : 1.0) / tile.us);
   }
-  return ratio < 1.0 || (less_exact(k, tile.splits) && !coarsely_on_the_tile(s, m, n, k, fused, splits));
+  return ratio < 1.0 || (less_exact(k, tile.splits) && !coarsely_on_the_tile(s, m, n, k, fused, splits, tile.splits > 1));
 }
 
 bool gemm16_rows_more_exact(int m, int n, int k, bool fused) {

@@ -803,7 +803,7 @@ def test_pieces_on_the_tile_are_as_exact_as_the_few_rows_kernel(hip, torch_cuda,
     assert error[1] <= error[2]
 
 
-@pytest.mark.parametrize("m,n,k", [(12, 30926, 5817), (147, 11697, 7903), (3, 22530, 3811), (26, 32567, 7232)])
+@pytest.mark.parametrize("m,n,k", [(12, 30926, 5817), (147, 11697, 7903), (3, 22530, 3811), (26, 32567, 7232), (62, 18432, 1897), (35, 27888, 858)])
 def test_long_k_that_is_not_cut_is_summed_in_chunks(hip, torch_cuda, m, n, k):
     """Products of a long K and a small C that are not cut: their mean square error is at most half of the single chain's
     (which gemm16.split_k = 1 keeps), as that of K in two pieces is."""
