@@ -1,8 +1,10 @@
 // What the GEMMs share when tiles are cut along K over several workgroups each: device memory for the partial tiles and
 // tickets for the kernels whose last workgroup of a tile adds them, and, for the 16-bit tiles, the kernel that adds partial
 // M x N planes up.
+#include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "common.hpp"
@@ -22,6 +24,7 @@ __device__ __forceinline__ void add_next(f32x4_t &acc, const float *__restrict__
   v[0] = acc;
 #pragma unroll
   for (int u = 0; u < Count; ++u) v[u + 1] = *reinterpret_cast<const Vec *>(p + u * plane);
+  __builtin_amdgcn_sched_barrier(0);   // (the first pair would be waited for before the other planes are asked for: fused 88 x 4928 x 3823 1.1 us)
 #pragma unroll
   for (int w = 1; w <= Count; w *= 2)
 #pragma unroll
@@ -62,53 +65,61 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
 }
 
 // The same for the fused product: y = relu(sum of the planes + bias), and the row's sum of y, in double, in a fixed order.  Waves
-// of the four of a workgroup to a row: one or four.  Bound by the trips to the planes, which the products have left in the caches: a wave
-// takes 256 columns a turn, so of more it makes several trips where four waves make one.  Us, one wave and four: 205 x 875 x 6932 22.9 and
-// 20.2 (20.9 before such products were cut), 133 x 958 x 4595 20.1 and 16.8, 300 x 300 x 4000 13.9 and 13.1; up to 256 columns three of the
-// four would have none (2000 x 150 x 3000 16.1 and 17.4), and many rows of up to 512 had better be fewer workgroups (2690 x 350 x 7071
-// 42.0 and 43.2, 1472 x 384 x 1600 15.2 and 14.7).
+// of the four of a workgroup to a row.  Bound by the trips to the planes, which the products have left in the caches: a wave takes 256
+// columns a turn, so of more it makes several trips where two or four waves make one.  Us, products whole and planes added with one wave, two
+// and four: 205 x 875 x 6932 20.2, 18.5, 17.3 (20.6 when such products were not cut), 133 x 958 x 4595 18.3, 16.3, 15.0 (17.5), 361 x 512 x 2112
+// 12.2, 11.9, 13.6; with many rows the workgroups count: 2690 x 350 x 7071 41.4, 42.4, 43.3, 2000 x 1025 x 2000 31.4, 31.5, 32.8, 4642 x 583 x 6966 81, 84, -.  The last one
+// to three columns of an odd N are read four at a time too, with some of those before them: one by one they waited for every plane (205 x
+// 875 x 6932 20.2, 17.3 now).
 template <int Waves>
 __global__ __launch_bounds__(256) void splitk_reduce_fused_kernel(const float *__restrict__ partials, const float *__restrict__ bias,
                                                                   float *__restrict__ y, float *__restrict__ rowsum, int m, int n,
                                                                   int64_t plane, int splits) {
   __shared__ double sums[4];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = Waves == 4 ? static_cast<int>(blockIdx.x) : static_cast<int>(blockIdx.x) * 4 + wave;
-  if (Waves == 1 && row >= m) return;
-  const float *p = partials + static_cast<int64_t>(row) * n;
-  float *out = y + static_cast<int64_t>(row) * n;
+  const int row = static_cast<int>(blockIdx.x) * (4 / Waves) + wave / Waves;
   double sum = 0.0;
-  for (int c = (Waves == 4 ? static_cast<int>(threadIdx.x) : lane) * 4; c < n; c += Waves * 256) {
-    if (c + 4 <= n) {
-      f32x4_t acc = add_planes<f32x4_u>(p + c, plane, splits);
-      const f32x4_t b = *reinterpret_cast<const f32x4_u *>(bias + c);
+  if (row < m) {
+    const float *p = partials + static_cast<int64_t>(row) * n;
+    float *out = y + static_cast<int64_t>(row) * n;
+    for (int c = (wave % Waves * 64 + lane) * 4; c < n; c += Waves * 256) {
+      if (n >= 4) {
+        const int at = min(c, n - 4);   // the last columns with some of those before them: one by one they wait for each plane
+        const f32x4_t b = *reinterpret_cast<const f32x4_u *>(bias + at);
+        f32x4_t acc = add_planes<f32x4_u>(p + at, plane, splits);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float v = acc[j] + b[j];
-        acc[j] = v > 0.f ? v : 0.f;
-        sum += static_cast<double>(acc[j]);
-      }
-      *reinterpret_cast<f32x4_u *>(out + c) = acc;
-    } else {
-      for (int j = c; j < n; ++j) {
-        float acc = p[j];
-        for (int s = 1; s < splits; ++s) acc += p[s * plane + j];
-        const float v = acc + bias[j];
-        out[j] = v > 0.f ? v : 0.f;
-        sum += static_cast<double>(v > 0.f ? v : 0.f);
+        for (int j = 0; j < 4; ++j) {
+          const float v = acc[j] + b[j];
+          acc[j] = v > 0.f ? v : 0.f;
+          sum += at + j >= c ? static_cast<double>(acc[j]) : 0.0;
+        }
+        if (at == c) {
+          *reinterpret_cast<f32x4_u *>(out + c) = acc;
+        } else {
+#pragma unroll
+          for (int j = 1; j < 4; ++j)
+            if (at + j >= c) out[at + j] = acc[j];
+        }
+      } else {
+        for (int j = c; j < n; ++j) {
+          float acc = p[j];
+          for (int s = 1; s < splits; ++s) acc += p[s * plane + j];
+          const float v = acc + bias[j];
+          out[j] = v > 0.f ? v : 0.f;
+          sum += static_cast<double>(v > 0.f ? v : 0.f);
+        }
       }
     }
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
-  if constexpr (Waves == 4) {
+  if constexpr (Waves > 1) {
     if (lane == 0) sums[wave] = sum;
     __syncthreads();
-    sum = (sums[0] + sums[1]) + (sums[2] + sums[3]);
-    if (threadIdx.x == 0) rowsum[row] = static_cast<float>(sum);
-  } else {
-    if (lane == 0) rowsum[row] = static_cast<float>(sum);
+    if constexpr (Waves == 4) sum = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+    else sum = sums[wave] + sums[wave ^ 1];
   }
+  if (lane == 0 && wave % Waves == 0 && row < m) rowsum[row] = static_cast<float>(sum);
 }
 
 __global__ __launch_bounds__(256) void zero_tickets_kernel(unsigned *tickets) {
@@ -178,11 +189,15 @@ int launch_splitk_reduce(const float *partials, float *c, int m, int n, int spli
 int launch_splitk_reduce_fused(const float *partials, const float *bias, float *y, float *rowsum, int m, int n, int splits,
                                hipStream_t st) {
   const int64_t plane = splitk_plane_floats(m, n);
-  if (n > 512 || (n > 256 && m <= 2048))
-    hipLaunchKernelGGL(splitk_reduce_fused_kernel<4>, dim3(m), dim3(256), 0, st, partials, bias, y, rowsum, m, n, plane, splits);
-  else
-    hipLaunchKernelGGL(splitk_reduce_fused_kernel<1>, dim3((m + 3) / 4), dim3(256), 0, st, partials, bias, y, rowsum, m, n, plane,
-                       splits);
+  auto launch = [&]<int Waves>(std::integral_constant<int, Waves>) {
+    hipLaunchKernelGGL(splitk_reduce_fused_kernel<Waves>, dim3((m + 4 / Waves - 1) / (4 / Waves)), dim3(256), 0, st, partials, bias, y,
+                       rowsum, m, n, plane, splits);
+  };
+  const int by_columns = n <= 256 ? 1 : n <= 512 ? 2 : 4, by_rows = m < 1280 ? 4 : m <= 2048 || n > 1024 ? 2 : 1;
+  const int waves = std::min(by_columns, by_rows);
+  if (waves == 4) launch(std::integral_constant<int, 4>{});
+  else if (waves == 2) launch(std::integral_constant<int, 2>{});
+  else launch(std::integral_constant<int, 1>{});
   return check_launch("split-K reduction launch");
 }
 

@@ -584,9 +584,10 @@ def test_fused_row_sums_of_each_row_tile(hip, torch_cuda, m, n, k, splits):
 
 @pytest.mark.parametrize("m,n,k,splits", [(128, 128, 256, 2), (1, 8, 128, 2), (129, 257, 200, 3), (300, 1023, 328, 2), (65, 1024, 448, 7),
                                           (64, 1025, 320, 4), (3, 4099, 1000, 5), (103, 1881, 6427, 0), (110, 2049, 7936, 0), (5, 2, 300, 3),
-                                          (2048, 300, 200, 2), (2049, 301, 200, 2), (2050, 513, 200, 2), (30, 512, 600, 9), (31, 256, 1088, 16)])
+                                          (2048, 300, 200, 2), (2049, 301, 200, 2), (2050, 513, 200, 2), (30, 512, 600, 9), (31, 256, 1088, 16),
+                                          (9, 5, 200, 2), (70, 3, 300, 2), (6, 6, 300, 4), (1281, 519, 200, 3), (1280, 1026, 200, 2), (33, 1031, 1500, 12), (2051, 1029, 200, 2), (2051, 1023, 200, 2)])
 def test_fused_products_cut_along_k(hip, oracle, torch_cuda, m, n, k, splits):
-    """The fused product on the 128 x 128 tile with K in pieces, forced and by its own rule, one wave and four to a row of the
+    """The fused product on the 128 x 128 tile with K in pieces, forced and by its own rule, one, two and four waves to a row of the
     launch that adds them: the oracle's y and row sums, the same bits again and on another stream at the same time; under capture
     it runs uncut, replay after replay."""
     torch = torch_cuda
