@@ -648,6 +648,9 @@ int sarek_hip_gemm16_tile_columns(int m, int n, int k);
  * ones that would share CUs: all (but a last one that has a kernel of its own),
  * those past whole rounds of 256 x 256 tiles, or none.                      */
 int sarek_hip_gemm16_half_columns(int m, int n, int k);
+/* Whether its 256 x 256 tiles store C by whole rows, past the caches (tunable
+ * gemm16.by_rows): a C of 200 MiB and more.                                 */
+int sarek_hip_gemm16_by_rows(int m, int n, int k);
 /* Into how many pieces sarek_hip_gemm_bf16 / _f16 cut K for this shape now (1 =
  * none): products with few 128 x 128 tiles and a long K are spread over the
  * CUs that way, the partial tiles added up in a fixed order by a second

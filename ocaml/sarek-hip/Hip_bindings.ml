@@ -197,6 +197,7 @@ let gemm_f32_k_splits = bind "sarek_hip_gemm_f32_k_splits" (int @-> int @-> int 
 let gemm16_tile = bind "sarek_hip_gemm16_tile" (int @-> int @-> int @-> returning int)
 let gemm16_tile_columns = bind "sarek_hip_gemm16_tile_columns" (int @-> int @-> int @-> returning int)
 let gemm16_half_columns = bind "sarek_hip_gemm16_half_columns" (int @-> int @-> int @-> returning int)
+let gemm16_by_rows = bind "sarek_hip_gemm16_by_rows" (int @-> int @-> int @-> returning int)
 let gemm16_k_splits = bind "sarek_hip_gemm16_k_splits" (int @-> int @-> int @-> returning int)
 let gemm_f16_bias_relu_rowsum =
   bind "sarek_hip_gemm_f16_bias_relu_rowsum"

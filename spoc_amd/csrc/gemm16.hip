@@ -2112,6 +2112,10 @@ int sarek_hip_gemm16_half_columns(int m, int n, int k) {
   return half ? columns - cut : 0;
 }
 
+int sarek_hip_gemm16_by_rows(int m, int n, int k) {
+  return sarek_hip_gemm16_tile(m, n, k) == 256 && tiled_columns(m, n, 256) > 0 && rows_pay(m, n, k) ? 1 : 0;
+}
+
 int sarek_hip_gemm16_k_splits(int m, int n, int k) {
   if (m >= 1 && n >= 1 && few_rows(m, n, k, false)) return gemm16_rows_k_splits(m, n, k);
   return gemm16_tile_for(m, n, k) == 128 && sarek_hip_gemm16_half_columns(m, n, k) == 0 ? splitk_for(m, n, k, false) : 1;

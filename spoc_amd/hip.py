@@ -149,6 +149,7 @@ SYMBOLS = {
     "sarek_hip_gemm16_k_splits": (_i, [_i, _i, _i]),
     "sarek_hip_gemm16_tile_columns": (_i, [_i, _i, _i]),
     "sarek_hip_gemm16_half_columns": (_i, [_i, _i, _i]),
+    "sarek_hip_gemm16_by_rows": (_i, [_i, _i, _i]),
     "sarek_hip_gemm_f16_bias_relu_rowsum": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "sarek_hip_cast_f32_to_bf16": (_i, [_vp, _vp, _i64, _vp]),
     "sarek_hip_cast_f32_to_f16": (_i, [_vp, _vp, _i64, _vp]),
@@ -762,6 +763,11 @@ def gemm16_tile_columns(m, n, k):
 def gemm16_half_columns(m, n, k):
     """How many of the n columns go to the 128 x 256 tile."""
     return int(lib.sarek_hip_gemm16_half_columns(m, n, k))
+
+
+def gemm16_by_rows(m, n, k):
+    """1 where the 256 x 256 tiles store C by whole rows, past the caches."""
+    return int(lib.sarek_hip_gemm16_by_rows(m, n, k))
 
 
 def gemm16_k_splits(m, n, k):

@@ -488,7 +488,7 @@ def test_gemm16_stored_by_rows(hip, torch_cuda, kind, m, n, k, rows):
             got = {}
             for arm in (rows, 1):
                 hip.set_tunable("gemm16.by_rows", arm)
-                assert hip.gemm16_tile(m, n, k) == 256
+                assert hip.gemm16_tile(m, n, k) == 256 and hip.gemm16_by_rows(m, n, k) == (arm != 1)
                 guard = torch.full((m * n + 96,), 7.0, device="cuda")
                 c = guard[c_shift:c_shift + m * n].view(m, n)
                 (hip.gemm_bf16 if kind == "bf16" else hip.gemm_f16)(a, b, out=c)

@@ -88,6 +88,20 @@ def test_columns_past_whole_rounds_of_large_tiles(hip, knobs, m, n, k, columns):
         assert hip.gemm16_tile_columns(m, n, k) < n
 
 
+@pytest.mark.parametrize("m,n,k,rows", [
+    (8192, 6401, 64, 1), (8192, 6400, 64, 1), (8192, 6399, 64, 0), (6400, 8192, 1024, 1), (8192, 8191, 4096, 1), (8192, 8191, 4097, 0), (8192, 8192, 4096, 0),
+    (2048, 50257, 625, 1), (2048, 50257, 1024, 1), (2048, 50272, 625, 1), (2048, 50272, 626, 0), (2048, 50256, 1024, 1),
+    (4096, 4096, 256, 0), (16, 8192, 8192, 0), (128, 128, 128, 0)])
+def test_c_stored_by_rows(hip, knobs, m, n, k, rows):
+    """A C of 200 MiB and more (8192 x 6400), up to a K of 4096, and not where its rows are whole lines and B has more than 60 MiB
+    (50272 columns: from a K of 626 on); never and always where asked, on the 256 x 256 tile alone."""
+    assert hip.gemm16_by_rows(m, n, k) == rows
+    knobs("gemm16.by_rows", 1)
+    assert hip.gemm16_by_rows(m, n, k) == 0
+    knobs("gemm16.by_rows", 2)
+    assert hip.gemm16_by_rows(m, n, k) == (hip.gemm16_tile(m, n, k) == 256)
+
+
 @pytest.mark.parametrize("m,n,k,columns", [
     (4096, 2048, 8192, 2048), (1921, 4095, 1200, 4095), (1921, 4095, 1199, 0), (392, 12497, 4079, 12497), (3072, 3072, 3072, 0),
     (2048, 2048, 2048, 0), (1921, 4099, 1200, 0), (2048, 12288, 4096, 4096), (2048, 11264, 1199, 0), (2048, 11264, 1200, 3072),
