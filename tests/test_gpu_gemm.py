@@ -505,34 +505,42 @@ def test_gemm16_stored_by_rows(hip, torch_cuda, kind, m, n, k, rows):
 
 
 @pytest.mark.parametrize("m,n,k,knobs", [
-    (1, 2, 32, {}), (64, 128, 64, {}), (65, 129, 100, {}), (83, 1344, 1152, {}), (512, 256, 1402, {}), (48, 2300, 520, {}),
+    (1, 2, 32, {"gemm16.rows": 2}), (64, 128, 64, {"gemm16.rows": 2}), (65, 129, 100, {"gemm16.rows": 2}),
+    (83, 1344, 1152, {"gemm16.rows": 2}), (512, 256, 1402, {"gemm16.rows": 2}), (48, 2300, 520, {"gemm16.rows": 2}),
     (128, 128, 64, {"gemm16.tile": 128}), (129, 257, 72, {"gemm16.tile": 128}), (300, 4300, 200, {"gemm16.tile": 128}),
     (256, 256, 64, {"gemm16.tile": 256}), (257, 4355, 131, {"gemm16.tile": 256}), (300, 1100, 192, {"gemm16.tile": 128, "gemm16.half": 2}),
     (513, 515, 200, {"gemm16.tile": 256, "gemm16.by_rows": 2}), (2048, 8448, 512, {}), (2048, 11264, 1216, {})])
 def test_fused_row_sums_added_by_the_last_tile(hip, torch_cuda, m, n, k, knobs):
     """Row sums that the launch's last workgroup of a row of tiles adds, on each kernel that can: the double sum of the stored
     row to 1e-5 of it (float32 sums of at most 256 values, then doubles), the same bits again and again and on another stream at
-    the same time, and those of the launch of its own to one rounding (the doubles are added in another order)."""
+    the same time, and those of the launch of its own to one rounding (the doubles are added in another order).  Products of two
+    sizes take turns, so that a share that was not waited for is the other one's."""
     torch = torch_cuda
     torch.manual_seed(m + n)
-    a, b = ((torch.randn(*s, device="cuda") * 0.2).half() for s in ((m, k), (k, n)))
-    bias = torch.rand(n, device="cuda") * 0.2 - 0.1
+    sets = [tuple((torch.randn(*s, device="cuda") * 0.2).half() for s in ((m, k), (k, n))) + (torch.rand(n, device="cuda") * scale - 0.1,)
+            for scale in (0.2, 100.0)]
     side = side_stream(torch)
+
+    def calls():
+        return [(i, hip.gemm_f16_bias_relu_rowsum(*sets[i])) for i in (0, 1, 0, 1, 1, 0)]
     try:
         for knob, value in knobs.items():
             hip.set_tunable(knob, value)
+        assert hip.gemm16_tile(m, n, k) == (64 if "gemm16.rows" in knobs else knobs.get("gemm16.tile", 256))
+        assert (hip.gemm16_half_columns(m, n, k) > 0) == ("gemm16.half" in knobs or (m, n) == (2048, 11264))
         hip.set_tunable("gemm16.fold", 1)
-        y1, rs1 = hip.gemm_f16_bias_relu_rowsum(a, b, bias)
+        apart = [hip.gemm_f16_bias_relu_rowsum(*x) for x in sets]
         for arm in (0, 2):
             hip.set_tunable("gemm16.fold", arm)
             torch.cuda.synchronize()
             with torch.cuda.stream(side):
-                other = [hip.gemm_f16_bias_relu_rowsum(a, b, bias) for _ in range(3)]
-            here = [hip.gemm_f16_bias_relu_rowsum(a, b, bias) for _ in range(3)]
+                other = calls()
+            here = calls()
             torch.cuda.synchronize()
-            for y, rs in here + other:
-                assert torch.equal(y, y1) and torch.equal(rs, here[0][1])
-                assert bool(((rs - rs1).abs() <= 2.0 ** -23 * rs1.abs()).all())
+            first = dict(reversed(here))
+            for i, (y, rs) in here + other:
+                assert torch.equal(y, apart[i][0]) and torch.equal(rs, first[i][1])
+                assert bool(((rs - apart[i][1]).abs() <= 2.0 ** -23 * apart[i][1].abs()).all())
                 assert rowsums_ok(rs.cpu().numpy(), y.double().sum(1).cpu().numpy())
     finally:
         for knob in ("gemm16.fold", *knobs):
