@@ -68,7 +68,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
 // of the four of a workgroup to a row.  Bound by the trips to the planes, which the products have left in the caches: a wave takes 256
 // columns a turn, so of more it makes several trips where two or four waves make one.  Us, products whole and planes added with one wave, two
 // and four: 205 x 875 x 6932 20.2, 18.5, 17.3 (20.6 when such products were not cut), 133 x 958 x 4595 18.3, 16.3, 15.0 (17.5), 361 x 512 x 2112
-// 12.2, 11.9, 13.6; with many rows the workgroups count: 2690 x 350 x 7071 41.4, 42.4, 43.3, 2000 x 1025 x 2000 31.4, 31.5, 32.8, 4642 x 583 x 6966 81, 84, -.  The last one
+// 12.2, 11.9, 13.6; with many rows the workgroups count: 2690 x 350 x 7071 in two pieces 41.4, 42.4, 43.3, 2000 x 1025 x 2000 31.4, 31.5, 32.8, 4642 x 583 x 6966 81, 84, -.  The last one
 // to three columns of an odd N are read four at a time too, with some of those before them: one by one they waited for every plane (205 x
 // 875 x 6932 20.2, 17.3 now).
 template <int Waves>
