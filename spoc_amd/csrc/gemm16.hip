@@ -1229,13 +1229,13 @@ __global__ __launch_bounds__(256) void gemm16_m16w4_kernel(const uint16_t *__res
 // rows of the large tile, so the same XOR swizzle keeps the transposing reads free of bank conflicts.  A slab is 16 MFMAs:
 // rows 0-31 of the wave tile before the barrier, rows 32-63 after it with the next slab's 12 fragment reads (and, every
 // other slab, the 4 transfers of an A stage) behind them; fragments are double-buffered by slab parity.
-// Chunk, for K in pieces (and whole where TileTime::whole_in_chunks): an element is the sum of sums of so many slabs, kept apart in 64 registers more (two waves to a SIMD have
-// 256 each; in chunks of two one or two are stored before the K loop and read again behind it), so that a piece is as exact as the
-// few-rows kernel's eight waves make it: rms error against float64 over the largest element, 320 x 2880 x 2793, there 2.3e-8, here in
-// one chain 7.1e-8 whole and 4.1e-8 in three pieces, in chunks 2.1e-8.  Chunks of two slabs are the more exact in short pieces (103 x 610
-// x 1022 in four 1.84e-8, of four slabs 2.07e-8), chunks of four in long ones, whose sums of chunks are longer (57 x 16274 x 3264 in two
-// 2.40e-8 and 2.24e-8): from kLongPiece of K on four.  The additions hide behind the MFMAs: 704 x 1728 x 4591 23.2 us without, 23.7 in chunks
-// of four slabs, 24.0 of two.
+// Chunk, for K in pieces (and whole where TileTime::whole_in_chunks): an element is the sum of sums of so many slabs, kept apart in 64
+// registers more (two waves to a SIMD have 256 each; in chunks of two, one or two are stored before the K loop and read again behind
+// it), so that a piece is as exact as the few-rows kernel's eight waves make it: rms error against float64 over the largest element,
+// 320 x 2880 x 2793, there 2.3e-8, here in one chain 7.1e-8 whole and 4.1e-8 in three pieces, in chunks 2.1e-8.  Chunks of two slabs are
+// the more exact in short pieces (103 x 610 x 1022 in four 1.84e-8, of four slabs 2.07e-8), chunks of four in long ones, whose sums of
+// chunks are longer (57 x 16274 x 3264 in two 2.40e-8 and 2.24e-8): from kLongPiece of K on four.  The additions hide behind the MFMAs:
+// 704 x 1728 x 4591 23.2 us without, 23.7 in chunks of four slabs, 24.0 of two.
 constexpr int kLongPiece = 1024;
 template <bool Bf16, int Epi, bool Ragged = false, int Chunk = 0>
 __global__ __launch_bounds__(256, Chunk ? 2 : 1) void gemm16_m16_small_kernel(const uint16_t *__restrict__ A, const uint16_t *__restrict__ B,
@@ -1731,10 +1731,10 @@ struct TileTime {
   // before any count of them was looked at; whole they are faster, but one chain of K has 1.4 times the error of two (rms over the largest
   // element, cut in two, whole, in chunks: 49 x 26100 x 6961 7.8e-8, 10.9e-8, 3.2e-8; us 101.1, 100.7, 100.7; 12 x 30926 x 5817 82.6, 63.6,
   // 64.0; 84 x 21952 x 8129 109.8, 97.6, 99.5).  The line takes the 471 such of 400000 drawn products and two others.  Elsewhere chunks cost up
-  // to 5 % (4457 x 448 x 3264 23.5 and 24.6).  And 17 to 64 rows, on about half of the CUs
-  // and more, of an A whose rows start at other places than B's: the few-rows kernel's finer estimate has it ahead there, up to two thirds
-  // wrongly (62 x 18432 x 1897 32.4 us, here in one chain 19.1, in chunks 19.7), but its sums are short (2.4e-8, 5.6e-8, 2.2e-8).  With fewer
-  // tiles the chunks cost 12 % of a short K (53 x 960 x 778 9.6 and 10.7).
+  // to 5 % (4457 x 448 x 3264 23.5 and 24.6).
+  // And 17 to 64 rows of an A whose rows start at other places than B's, on about half of the CUs and more: the few-rows kernel was taken there
+  // for a while, up to two thirds slower (62 x 18432 x 1897 32.4 us, here in one chain 19.1, in chunks 19.7) but with short sums (2.4e-8,
+  // 5.6e-8, 2.2e-8).  With fewer tiles the chunks cost 12 % of a short K (53 x 960 x 778 9.6 and 10.7).
   bool whole_in_chunks(int m, int n, int k) const {
     const bool apart = (n % 8 == 0 && k % 8 != 0) || (n % 2 == 0 && k % 2 != 0);
     return tiles <= cus && (k >= 3000.0 + 640.0 * c_mb || (k >= 512 && m > 16 && m <= 64 && apart && 2 * tiles > cus - 8));

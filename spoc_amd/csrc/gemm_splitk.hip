@@ -24,7 +24,8 @@ __device__ __forceinline__ void add_next(f32x4_t &acc, const float *__restrict__
   v[0] = acc;
 #pragma unroll
   for (int u = 0; u < Count; ++u) v[u + 1] = *reinterpret_cast<const Vec *>(p + u * plane);
-  __builtin_amdgcn_sched_barrier(0);   // (the first pair would be waited for before the other planes are asked for: fused 88 x 4928 x 3823 1.1 us)
+  // (without it the first pair is waited for before the other planes are asked for: fused 88 x 4928 x 3823 20.5 us, 18.5 with it)
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int w = 1; w <= Count; w *= 2)
 #pragma unroll
@@ -66,11 +67,11 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
 
 // The same for the fused product: y = relu(sum of the planes + bias), and the row's sum of y, in double, in a fixed order.  Waves
 // of the four of a workgroup to a row.  Bound by the trips to the planes, which the products have left in the caches: a wave takes 256
-// columns a turn, so of more it makes several trips where two or four waves make one.  Us, products whole and planes added with one wave, two
-// and four: 205 x 875 x 6932 20.2, 18.5, 17.3 (20.6 when such products were not cut), 133 x 958 x 4595 18.3, 16.3, 15.0 (17.5), 361 x 512 x 2112
-// 12.2, 11.9, 13.6; with many rows the workgroups count: 2690 x 350 x 7071 in two pieces 41.4, 42.4, 43.3, 2000 x 1025 x 2000 31.4, 31.5, 32.8, 4642 x 583 x 6966 81, 84, -.  The last one
-// to three columns of an odd N are read four at a time too, with some of those before them: one by one they waited for every plane (205 x
-// 875 x 6932 20.2, 17.3 now).
+// columns a turn, so of more it makes several trips where two or four waves make one.  Us, products with one wave to a row, two and four:
+// 205 x 875 x 6932 20.2, 18.5, 17.3 (20.6 when such products were not cut), 133 x 958 x 4595 18.3, 16.3, 15.0 (17.5), 361 x 512 x 2112 12.2,
+// 11.9, 13.6; with many rows the workgroups count: 2690 x 350 x 7071 in two pieces 41.4, 42.4, 43.3, 2000 x 1025 x 2000 31.4, 31.5, 32.8,
+// 4642 x 583 x 6966 81 and 84.  The last one to three columns of an odd N are read four at a time too, with some of those before them: one by
+// one they waited for every plane (205 x 875 x 6932 20.2, 17.3 now).
 template <int Waves>
 __global__ __launch_bounds__(256) void splitk_reduce_fused_kernel(const float *__restrict__ partials, const float *__restrict__ bias,
                                                                   float *__restrict__ y, float *__restrict__ rowsum, int m, int n,
